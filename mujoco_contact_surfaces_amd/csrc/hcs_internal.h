@@ -77,9 +77,9 @@ struct Plan {
   std::vector<int> order; /* items by decreasing measured work (empty: item order) */
 };
 
-/* Scratch of hcs_taxel_sensor_update. */
+/* Scratch of hcs_taxel_sensor_update and hcs_curved_sensor_update. */
 struct TaxelSensorBufs {
-  DBuf mask, k64, kp, idx, cnt, nfan, fan_off, tmp, tris, surf, scnt, soff, P, E, taxel, val;
+  DBuf mask, k64, kp, idx, cnt, nfan, fan_off, tmp, tris, surf, scnt, soff, P, E, taxel, val, hits;
 };
 
 struct Ctx {

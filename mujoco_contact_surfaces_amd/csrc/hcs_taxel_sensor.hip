@@ -247,79 +247,166 @@ __global__ __launch_bounds__(64) void k_ts_taxel(const double* __restrict__ P, c
   }
 }
 
-/* CurvedSensor ray of one surface sample (one thread): the sample moved by
- * X (normal rotated, not renormalised), ray from p + n 1e-8 along -n,
- * Moeller-Trumbore (S/src/bvh.cpp:49-74) in FP64 over the fan triangles,
- * nearest t (first triangle in order on ties); raw pressure when 0 < t <
- * margin.  Triangles whose box misses the box of the ray segment
- * [0, margin] (widened by 1e-9 of its largest coordinate) are skipped: they
- * cannot give an accepted hit, and one with t >= margin never changes
- * whether the nearest hit is accepted. */
-__global__ __launch_bounds__(256) void k_cs_rays(const double* __restrict__ tris, int64_t nt, CsArgs a,
-                                                 const double* __restrict__ pts, const double* __restrict__ nrms,
-                                                 int m, double* __restrict__ raw, unsigned char* __restrict__ hit) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= m) return;
-  double pw[3], nw[3], O[3], D[3];
-  xform(a.X, pts + 3 * (size_t)j, pw);
-  rot(a.X, nrms + 3 * (size_t)j, nw);
+/* The nearest hit of a ray in one slice of the triangles. */
+struct CsHit {
+  double t, u, v; /* t = 1e30: none */
+  long long tri;
+};
+
+/* CurvedSensor rays: the sample moved by X (normal rotated, not
+ * renormalised), ray from p + n 1e-8 along -n, Moeller-Trumbore
+ * (S/src/bvh.cpp:49-74) in FP64 over the fan triangles, nearest t (first
+ * triangle in order on ties).
+ *
+ * Triangles whose bounding sphere (centre C, radius r) the ray's line misses
+ * are skipped.  The computed barycentrics err by at most
+ * 16 eps (|s| + L) L^2 / |det| in position, s the vector from the triangle to
+ * the ray's origin, L <= 2r the longest edge, and the hit test rejects
+ * |det| < 1e-10, so an accepted hit lies within 3.6e-5 (|s| + L) L^2 of the
+ * triangle; the sphere is widened by more than four times that (|s| bounded
+ * through the largest coordinates), by 1e-9 of the ray's largest coordinate,
+ * and the comparison by 1e-14 |s|^2 for the cancellation in |s|^2 - (s.D)^2.
+ * A NaN or infinity fails the comparison, so nothing is skipped on it.
+ *
+ * One lane per ray, one wave per (64 rays, slice of the triangles): with a
+ * thread walking every triangle, 2601 rays were 41 waves on 256 CUs, each a
+ * chain of 11k triangle loads (5522 us); blockIdx.y cuts the chain so that
+ * about 4096 waves run (see cs_slices).  The wave stages 64 triangles'
+ * spheres in LDS (one per lane), so the inner loop is a broadcast read and
+ * 16 FP64 operations, which bound it; each lane then hit-tests the triangles
+ * of its own mask, so a round serves one triangle of every lane.  (The box of the ray segment
+ * against the triangle's box, the test before, let a fifth of the triangles
+ * through for rays oblique to the axes, so most triangles were hit-tested
+ * for some lane: 67 us.)  2601 rays on 11.5k triangles: 5522 -> 44 us. */
+__global__ __launch_bounds__(64) void k_cs_rays(const double* __restrict__ tris, int64_t nt, CsArgs a,
+                                                const double* __restrict__ pts, const double* __restrict__ nrms, int m,
+                                                CsHit* __restrict__ part) {
+  __shared__ double sph[64][6];
+  const int lane = threadIdx.x, j = blockIdx.x * 64 + lane, jr = j < m ? j : m - 1;
+  double pw[3], nw[3], O[3], D[3], sc = 0.0;
+  xform(a.X, pts + 3 * (size_t)jr, pw);
+  rot(a.X, nrms + 3 * (size_t)jr, nw);
 #pragma unroll
-  for (int c = 0; c < 3; ++c) O[c] = pw[c] + nw[c] * 1e-8, D[c] = -nw[c];
-  double slo[3], shi[3], E[3], sc = 0.0;
-#pragma unroll
-  for (int c = 0; c < 3; ++c) E[c] = O[c] + D[c] * a.margin, sc = fmax(sc, fmax(fabs(O[c]), fabs(E[c])));
-  /* one slack for all axes, on the scale of the largest coordinate: the
-   * rounding of t moves the computed hit along every axis by that much */
-  const double sl = 1e-9 * sc + 1e-300;
-#pragma unroll
-  for (int c = 0; c < 3; ++c) slo[c] = fmin(O[c], E[c]) - sl, shi[c] = fmax(O[c], E[c]) + sl;
+  for (int c = 0; c < 3; ++c) O[c] = pw[c] + nw[c] * 1e-8, D[c] = -nw[c], sc = fmax(sc, fabs(O[c]));
+  const double iD2 = 1.0 / dot3(D, D), sl = 1e-9 * sc + 1e-300;
   double best = 1e30, bu = 0.0, bv = 0.0;
   int64_t bt = -1;
-  for (int64_t t = 0; t < nt; ++t) {
-    const double* T = tris + HCS_TS_TRI * t;
-    bool out = false;
+  const int64_t t0 = nt * blockIdx.y / gridDim.y, t1 = nt * (blockIdx.y + 1) / gridDim.y;
+  for (int64_t c0 = t0; c0 < t1; c0 += 64) {
+    const int cn = (int)(t1 - c0 < 64 ? t1 - c0 : 64);
+    __syncthreads();
+    if (lane < cn) {
+      const double* T = tris + HCS_TS_TRI * (c0 + lane);
+      double C[3], tm = 0.0, r2 = 0.0;
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      const double lo = fmin(fmin(T[c], T[3 + c]), T[6 + c]), hi = fmax(fmax(T[c], T[3 + c]), T[6 + c]);
-      out = out || hi < slo[c] || lo > shi[c];
+      for (int c = 0; c < 3; ++c)
+        C[c] = ((T[c] + T[3 + c]) + T[6 + c]) * (1.0 / 3.0),
+        tm = fmax(tm, fmax(fabs(T[c]), fmax(fabs(T[3 + c]), fabs(T[6 + c]))));
+#pragma unroll
+      for (int v = 0; v < 3; ++v) {
+        const double d[3] = {T[3 * v] - C[0], T[3 * v + 1] - C[1], T[3 * v + 2] - C[2]};
+        r2 = fmax(r2, dot3(d, d));
+      }
+      const double r = sqrt(r2), k = 1.2e-3 * r2;
+      sph[lane][0] = C[0], sph[lane][1] = C[1], sph[lane][2] = C[2];
+      sph[lane][3] = r + k * (tm + r), sph[lane][4] = k;
     }
-    if (out) continue;
-    const double e1[3] = {T[3] - T[0], T[4] - T[1], T[5] - T[2]}, e2[3] = {T[6] - T[0], T[7] - T[1], T[8] - T[2]};
-    double h[3];
-    cross3(D, e2, h);
-    const double det = dot3(e1, h);
-    if (fabs(det) < 1e-10) continue;
-    const double f = 1.0 / det;
-    const double sv[3] = {O[0] - T[0], O[1] - T[1], O[2] - T[2]};
-    const double u = f * dot3(sv, h);
-    if (u < 0.0 || u > 1.0) continue;
-    double qv[3];
-    cross3(sv, e1, qv);
-    const double v = f * dot3(D, qv);
-    if (v < 0.0 || u + v > 1.0) continue;
-    const double tt = f * dot3(e2, qv);
-    if (tt > 0.0 && tt < best) best = tt, bu = u, bv = v, bt = t;
+    __syncthreads();
+    /* the lane's triangles of the tile, then their hit tests in order */
+    unsigned long long todo = 0;
+#pragma unroll 8
+    for (int k = 0; k < 64; ++k) {
+      const double* b = sph[k];
+      const double s[3] = {b[0] - O[0], b[1] - O[1], b[2] - O[2]};
+      const double ss = dot3(s, s), sd = dot3(s, D), re = (b[3] + b[4] * sc) + sl;
+      todo |= ss - (sd * sd) * iD2 > re * re + 1e-14 * ss ? 0ull : 1ull << k;
+    }
+    todo &= ~0ull >> (64 - cn);
+    while (todo) {
+      const int64_t t = c0 + __builtin_ctzll(todo);
+      todo &= todo - 1;
+      const double* T = tris + HCS_TS_TRI * t;
+      const double e1[3] = {T[3] - T[0], T[4] - T[1], T[5] - T[2]}, e2[3] = {T[6] - T[0], T[7] - T[1], T[8] - T[2]};
+      double h[3];
+      cross3(D, e2, h);
+      const double det = dot3(e1, h);
+      if (fabs(det) < 1e-10) continue;
+      const double f = 1.0 / det;
+      const double sv[3] = {O[0] - T[0], O[1] - T[1], O[2] - T[2]};
+      const double u = f * dot3(sv, h);
+      if (u < 0.0 || u > 1.0) continue;
+      double qv[3];
+      cross3(sv, e1, qv);
+      const double v = f * dot3(D, qv);
+      if (v < 0.0 || u + v > 1.0) continue;
+      const double tt = f * dot3(e2, qv);
+      if (tt > 0.0 && tt < best) best = tt, bu = u, bv = v, bt = t;
+    }
   }
-  const bool ok = bt >= 0 && best < a.margin && best > 0.0;
+  if (j < m) part[(size_t)blockIdx.y * m + j] = CsHit{best, bu, bv, bt};
+}
+
+/* Per ray, the nearest of its slices' hits, the first triangle on ties; raw
+ * pressure when 0 < t < margin.  16 rays per wave, the slices shared by four
+ * lanes each (one lane per ray left 41 waves with 50 dependent loads). */
+__global__ __launch_bounds__(64) void k_cs_hits(const double* __restrict__ tris, const CsHit* __restrict__ part,
+                                                int nslice, double margin, int m, double* __restrict__ raw,
+                                                unsigned char* __restrict__ hit) {
+  const int j = blockIdx.x * 16 + (threadIdx.x & 15);
+  CsHit b{1e30, 0.0, 0.0, 0x7fffffffffffffffll};
+  if (j < m)
+    for (int s = threadIdx.x >> 4; s < nslice; s += 4) {
+      const CsHit h = part[(size_t)s * m + j];
+      if (h.tri >= 0 && h.t < b.t) b = h;
+    }
+#pragma unroll
+  for (int o = 16; o <= 32; o <<= 1) {
+    const CsHit h{__shfl_xor(b.t, o, 64), __shfl_xor(b.u, o, 64), __shfl_xor(b.v, o, 64), __shfl_xor(b.tri, o, 64)};
+    if (h.t < b.t || (h.t == b.t && h.tri < b.tri)) b = h;
+  }
+  if (j >= m || threadIdx.x >= 16) return;
+  const bool ok = b.t < 1e30 && b.t < margin && b.t > 0.0;
   double r = 0.0;
   if (ok) {
-    const double* T = tris + HCS_TS_TRI * bt;
-    const double b0 = 1 - bu - bv;
-    r = (b0 * T[9] + bu * T[10]) + bv * T[11];
+    const double* T = tris + HCS_TS_TRI * b.tri;
+    const double b0 = 1 - b.u - b.v;
+    r = (b0 * T[9] + b.u * T[10]) + b.v * T[11];
   }
   raw[j] = r;
   hit[j] = ok ? 1 : 0;
 }
 
-/* taxel i: sum over its samples of weight * raw, in list order */
+/* Triangle slices of the ray kernel: enough for about 4096 waves (four per
+ * SIMD), at least 64 triangles (one staged tile) each. */
+static int cs_slices(int m, int64_t nt) {
+  const int64_t groups = (m + 63) / 64;
+  return (int)std::max<int64_t>(1, std::min<int64_t>(4096 / std::max<int64_t>(1, groups), nt / 64));
+}
+
+/* taxel i: sum over its samples of weight * raw, in list order; four entries
+ * are loaded before they are added, so the chain of dependent loads (entry,
+ * sample) is a quarter as long */
 __global__ void k_cs_taxels(const int* __restrict__ ptr, const int* __restrict__ idx, const double* __restrict__ w,
                             int n, const double* __restrict__ raw, const unsigned char* __restrict__ hit,
                             double* __restrict__ values) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
+  const int k1 = ptr[i + 1];
   double pr = 0.0;
-  for (int k = ptr[i]; k < ptr[i + 1]; ++k)
-    if (hit[idx[k]]) pr += w[k] * raw[idx[k]];
+  for (int k = ptr[i]; k < k1; k += 4) {
+    double term[4];
+    bool on[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int q = k + u < k1 ? k + u : k;
+      const int j = idx[q];
+      on[u] = k + u < k1 && hit[j];
+      term[u] = w[q] * raw[j];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (on[u]) pr += term[u];
+  }
   values[i] = pr;
 }
 
@@ -492,10 +579,11 @@ int hcs_curved_sensor_update(hcs_ctx* h, const hcs_curved_sensor* S, double* val
   }
   const int m = S->nsamples;
   const size_t m1 = (size_t)std::max(1, m), n1 = (size_t)S->ntaxels, z1 = (size_t)std::max(1, nnz);
+  const int nslice = cs_slices(m, ntri);
   if ((rc = ensure(c, B.P, sizeof(double) * 6 * m1)) || (rc = ensure(c, B.E, sizeof(double) * m1)) ||
       (rc = ensure(c, B.mask, m1)) || (rc = ensure(c, B.taxel, sizeof(double) * z1)) ||
       (rc = ensure(c, B.val, sizeof(double) * n1)) || (rc = ensure(c, B.scnt, sizeof(int) * (n1 + 1))) ||
-      (rc = ensure(c, B.soff, sizeof(int) * z1)))
+      (rc = ensure(c, B.soff, sizeof(int) * z1)) || (rc = ensure(c, B.hits, sizeof(CsHit) * m1 * nslice)))
     return rc;
   double* pts = (double*)B.P.ptr;
   rc = hip_check(c, hipMemcpyAsync(pts, S->points, sizeof(double) * 3 * m, hipMemcpyHostToDevice, s), "ul");
@@ -511,10 +599,13 @@ int hcs_curved_sensor_update(hcs_ctx* h, const hcs_curved_sensor* S, double* val
   CsArgs a;
   std::memcpy(a.X, S->X_W_sensor, sizeof a.X);
   a.margin = S->include_margin;
-  if (m > 0)
-    hipLaunchKernelGGL(k_cs_rays, dim3((m + 255) / 256), dim3(256), 0, s, (const double*)B.tris.ptr, (int64_t)ntri, a,
-                       pts, pts + 3 * m1, m, (double*)B.E.ptr, (unsigned char*)B.mask.ptr);
-  hipLaunchKernelGGL(k_cs_taxels, dim3((S->ntaxels + 255) / 256), dim3(256), 0, s, (const int*)B.scnt.ptr,
+  if (m > 0) {
+    hipLaunchKernelGGL(k_cs_rays, dim3((m + 63) / 64, nslice), dim3(64), 0, s, (const double*)B.tris.ptr, (int64_t)ntri,
+                       a, pts, pts + 3 * m1, m, (CsHit*)B.hits.ptr);
+    hipLaunchKernelGGL(k_cs_hits, dim3((m + 15) / 16), dim3(64), 0, s, (const double*)B.tris.ptr,
+                       (const CsHit*)B.hits.ptr, nslice, a.margin, m, (double*)B.E.ptr, (unsigned char*)B.mask.ptr);
+  }
+  hipLaunchKernelGGL(k_cs_taxels, dim3((S->ntaxels + 63) / 64), dim3(64), 0, s, (const int*)B.scnt.ptr,
                      (const int*)B.soff.ptr, (const double*)B.taxel.ptr, S->ntaxels, (const double*)B.E.ptr,
                      (const unsigned char*)B.mask.ptr, (double*)B.val.ptr);
   rc = hip_check(c, hipGetLastError(), "curved sensor");
