@@ -5,8 +5,9 @@
  * (mujoco_contact_surface_sensors/src/taxel_sensor.cpp:158-478) over the
  * contact polygons kept by the last contact step:
  *   1. the polygons of the pairs touching the sensor geometry, in key order
- *      (pair, element of A, element of B) -- two stable radix passes -- and
- *      their kTriangle fans (v_k, v_{k+1}, C), the surface's triangles;
+ *      (pair, element of A, element of B) -- by rank, or radix passes over the
+ *      packed key -- and their kTriangle fans (v_k, v_{k+1}, C), the surface's
+ *      triangles;
  *   2. samples on every triangle: DEFAULT (:174-203), the reference's loops
  *      a, b += 1/st from 0 while <= 1 with st from |v1 - v0| and |v2 - v0|
  *      (both st1 and st2 from v2 - v0), one thread per triangle after a
@@ -43,18 +44,26 @@ namespace hcs {
 
 #define HCS_TS_TRI 12 /* fan triangle: v0, v1, v2 (W), e0, e1, e2 */
 
-/* selected polygons get their key, others sort last */
-__global__ void k_ts_keys(const int64_t* __restrict__ key, int64_t np, const unsigned char* __restrict__ mask,
-                          unsigned long long* __restrict__ k64, unsigned* __restrict__ kp, int* __restrict__ idx,
-                          unsigned* __restrict__ cnt) {
+/* Sort keys of the kept polygons: (pair, element of A, element of B) packed
+ * into the bits the pairs and meshes need when those fit 64 (ba, bb >= 0:
+ * bits of the elements), else (element of A, element of B) with the pair in
+ * kp.  Unselected polygons sort last.  For the rank sort, its counters are
+ * cleared here and every place is empty (-1) until a polygon takes it. */
+__global__ void k_ts_keys(const int64_t* __restrict__ key, int64_t np, const unsigned char* __restrict__ mask, int ba,
+                          int bb, unsigned long long* __restrict__ k64, unsigned* __restrict__ kp,
+                          int* __restrict__ idx, unsigned* __restrict__ rank) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= np) return;
-  const int64_t pair = key[3 * i], a = key[3 * i + 1], b = key[3 * i + 2];
+  const unsigned long long pair = key[3 * i], a = key[3 * i + 1], b = key[3 * i + 2];
   const bool on = mask[pair] != 0;
-  k64[i] = ((unsigned long long)(unsigned)a << 32) | (unsigned long long)(unsigned)b;
-  kp[i] = on ? (unsigned)pair : 0xffffffffu;
-  idx[i] = (int)i;
-  if (on) atomicAdd(cnt, 1u);
+  if (ba >= 0) {
+    k64[i] = on ? (((pair << ba) | a) << bb) | b : ~0ull;
+  } else {
+    k64[i] = (a << 32) | b;
+    kp[i] = on ? (unsigned)pair : 0xffffffffu;
+  }
+  idx[i] = rank ? -1 : (int)i;
+  if (rank) rank[i] = 0;
 }
 
 __global__ void k_ts_gather_u32(const unsigned* __restrict__ src, const int* __restrict__ idx, int64_t n,
@@ -63,18 +72,54 @@ __global__ void k_ts_gather_u32(const unsigned* __restrict__ src, const int* __r
   if (i < n) dst[i] = src[idx[i]];
 }
 
-__global__ void k_ts_nfan(const double* __restrict__ poly, const int* __restrict__ order, int n,
+/* Rank sort, for up to HCS_TS_RANK polygons: the keys are distinct (one
+ * polygon per element pair; the unselected share the largest key and need no
+ * order), so a polygon's place is the number of smaller keys.  One thread
+ * per polygon, blockIdx.y a slice of the keys it is compared with, staged in
+ * LDS.  n^2 compares are cheaper than the radix sort's launches at these
+ * sizes: 6.8k polygons 60 launches, about 300 us (12 passes of 5) -> 2
+ * launches, 12 us; at 16k the compares take about 30 us, as much as the
+ * radix sort on packed keys. */
+#define HCS_TS_RANK 16384
+__global__ __launch_bounds__(256) void k_ts_rank(const unsigned long long* __restrict__ k64, int n, int per,
+                                                 unsigned* __restrict__ rank) {
+  __shared__ unsigned long long tile[256];
+  const int t = threadIdx.x, i = blockIdx.x * 256 + t;
+  const unsigned long long k = i < n ? k64[i] : 0ull;
+  const int j1 = min(n, (int)(blockIdx.y + 1) * per);
+  unsigned less = 0;
+  for (int j0 = blockIdx.y * per; j0 < j1; j0 += 256) {
+    __syncthreads();
+    tile[t] = j0 + t < j1 ? k64[j0 + t] : ~0ull;
+    __syncthreads();
+#pragma unroll 8
+    for (int u = 0; u < 256; ++u) less += tile[u] < k;
+  }
+  if (i < n && less && k != ~0ull) atomicAdd(rank + i, less);
+}
+
+/* order by rank; the places after the last selected polygon stay -1 */
+__global__ void k_ts_order(const unsigned long long* __restrict__ k64, const unsigned* __restrict__ rank, int n,
+                           int* __restrict__ order) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n && k64[i] != ~0ull) order[rank[i]] = i;
+}
+
+/* fans of the i-th polygon in order: 0 for an unselected one */
+__global__ void k_ts_nfan(const double* __restrict__ poly, const int64_t* __restrict__ key,
+                          const unsigned char* __restrict__ mask, const int* __restrict__ order, int n,
                           unsigned* __restrict__ nt) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) nt[i] = (unsigned)poly[HCS_PREC * (size_t)order[i]];
-  if (i == n) nt[i] = 0;
+  if (i > n) return;
+  const int q = i < n ? order[i] : -1;
+  nt[i] = q >= 0 && mask[key[3 * (size_t)q]] ? (unsigned)poly[HCS_PREC * (size_t)q] : 0u;
 }
 
 __global__ void k_ts_fans(const double* __restrict__ poly, const int64_t* __restrict__ key,
                           const int* __restrict__ order, int n, const unsigned* __restrict__ off,
                           double* __restrict__ tris, int* __restrict__ surf) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  if (i >= n || off[i] == off[i + 1]) return;
   const double* P = poly + HCS_PREC * (size_t)order[i];
   const int nv = (int)P[0];
   for (int k = 0; k < nv; ++k) {
@@ -414,6 +459,13 @@ __global__ void k_cs_taxels(const int* __restrict__ ptr, const int* __restrict__
 
 extern "C" {
 
+/* Bits that hold the values 0 .. n. */
+static int key_bits(int64_t n) {
+  int b = 1;
+  while (b < 62 && (n >> b) != 0) ++b;
+  return b;
+}
+
 /* The kTriangle fan triangles of the kept polygons of the pairs touching
  * geometry geom, in key order, into c->ts.tris / c->ts.surf. */
 static int sensor_fans(Ctx* c, int32_t geom, unsigned& ntri) {
@@ -432,39 +484,58 @@ static int sensor_fans(Ctx* c, int32_t geom, unsigned& ntri) {
       (rc = ensure(c, B.fan_off, sizeof(unsigned) * (n1 + 1))))
     return rc;
   rc = hip_check(c, hipMemcpyAsync(B.mask.ptr, mask.data(), mask.size(), hipMemcpyHostToDevice, s), "upload mask");
-  if (!rc) rc = hip_check(c, hipMemsetAsync(B.cnt.ptr, 0, 64, s), "memset");
   if (rc) return rc;
   unsigned long long* k64 = (unsigned long long*)B.k64.ptr;
   unsigned* kp = (unsigned*)B.kp.ptr;
-  int* idx = (int*)B.idx.ptr;
-  unsigned nsel = 0;
-  if (np > 0) {
-    hipLaunchKernelGGL(k_ts_keys, dim3((np + 255) / 256), dim3(256), 0, s, (const int64_t*)c->d_poly_key.ptr, np,
-                       (const unsigned char*)B.mask.ptr, k64, kp, idx, (unsigned*)B.cnt.ptr);
-    /* stable LSD passes: (element of A, element of B), then pair */
-    const size_t b1 = sort_temp_bytes(np, 8), b2 = sort_temp_bytes(np, 4);
-    if ((rc = ensure(c, B.tmp, std::max<size_t>(8, std::max(b1, b2))))) return rc;
-    if (radix_sort_pairs_u64(s, k64, k64 + n1, idx, idx + n1, np, 0, 64, B.tmp.ptr, B.tmp.bytes) != 0)
-      return set_err(c, HCS_ERR_LIMIT, "sensor: too many polygons to sort");
-    hipLaunchKernelGGL(k_ts_gather_u32, dim3((np + 255) / 256), dim3(256), 0, s, kp, idx + n1, np, kp + n1);
-    if (radix_sort_pairs_u32(s, kp + n1, kp, idx + n1, idx, np, 0, 32, B.tmp.ptr, B.tmp.bytes) != 0)
-      return set_err(c, HCS_ERR_LIMIT, "sensor: too many polygons to sort");
-    rc = hip_check(c, hipGetLastError(), "select polygons");
-    if (!rc) rc = hip_check(c, hipMemcpyAsync(&nsel, B.cnt.ptr, sizeof(unsigned), hipMemcpyDeviceToHost, s), "dl");
-    if (!rc) rc = hip_check(c, hipStreamSynchronize(s), "sync");
-    if (rc) return rc;
-  }
-  /* fan triangles of the selected polygons, in order */
+  int *idx = (int*)B.idx.ptr, *order = idx + n1;
+  const unsigned char* dmask = (const unsigned char*)B.mask.ptr;
   ntri = 0;
-  if (nsel > 0) {
-    hipLaunchKernelGGL(k_ts_nfan, dim3((nsel + 1 + 255) / 256), dim3(256), 0, s, (const double*)c->d_poly_rec.ptr,
-                       idx, (int)nsel, (unsigned*)B.nfan.ptr);
-    if ((rc = ensure(c, B.tmp, std::max<size_t>(scan_temp_bytes((long long)nsel + 1), 8)))) return rc;
-    if (exclusive_scan_u32(s, (const unsigned*)B.nfan.ptr, (unsigned*)B.fan_off.ptr, (long long)nsel + 1, B.tmp.ptr,
+  if (np > 0) {
+    /* bits of the packed key: pair numbers, and the element counts of the
+     * pairs' meshes */
+    int64_t ma = 1, mb = 1;
+    for (int e = 0; e < npairs; ++e) {
+      ma = std::max<int64_t>(ma, c->meshes[c->last_geoms[2 * e]].nelem);
+      mb = std::max<int64_t>(mb, c->meshes[c->last_geoms[2 * e + 1]].nelem);
+    }
+    const int bp = key_bits(npairs), ba = key_bits(ma), bb = key_bits(mb);
+    const bool packed = bp + ba + bb < 64;
+    const bool rank = packed && np <= HCS_TS_RANK;
+    const unsigned nb = (unsigned)((np + 255) / 256);
+    hipLaunchKernelGGL(k_ts_keys, dim3(nb), dim3(256), 0, s, (const int64_t*)c->d_poly_key.ptr, np, dmask,
+                       packed ? ba : -1, bb, k64, kp, rank ? order : idx, rank ? kp : nullptr);
+    if (rank) {
+      const int slices = (int)std::max<int64_t>(1, std::min<int64_t>(nb, 512 / nb));
+      const int per = (int)((np + slices - 1) / slices);
+      hipLaunchKernelGGL(k_ts_rank, dim3(nb, slices), dim3(256), 0, s, k64, (int)np, per, kp);
+      hipLaunchKernelGGL(k_ts_order, dim3(nb), dim3(256), 0, s, k64, kp, (int)np, order);
+    } else if (packed) {
+      const size_t b = sort_temp_bytes(np, 8);
+      if ((rc = ensure(c, B.tmp, std::max<size_t>(8, b)))) return rc;
+      /* one bit more than the keys need: the unselected polygons' */
+      if (radix_sort_pairs_u64(s, k64, k64 + n1, idx, order, np, 0, bp + ba + bb + 1, B.tmp.ptr, B.tmp.bytes) != 0)
+        return set_err(c, HCS_ERR_LIMIT, "sensor: too many polygons to sort");
+    } else {
+      /* stable LSD passes: (element of A, element of B), then pair */
+      const size_t b1 = sort_temp_bytes(np, 8), b2 = sort_temp_bytes(np, 4);
+      if ((rc = ensure(c, B.tmp, std::max<size_t>(8, std::max(b1, b2))))) return rc;
+      if (radix_sort_pairs_u64(s, k64, k64 + n1, idx, order, np, 0, 64, B.tmp.ptr, B.tmp.bytes) != 0)
+        return set_err(c, HCS_ERR_LIMIT, "sensor: too many polygons to sort");
+      hipLaunchKernelGGL(k_ts_gather_u32, dim3(nb), dim3(256), 0, s, kp, order, np, kp + n1);
+      if (radix_sort_pairs_u32(s, kp + n1, kp, order, idx, np, 0, 32, B.tmp.ptr, B.tmp.bytes) != 0)
+        return set_err(c, HCS_ERR_LIMIT, "sensor: too many polygons to sort");
+      order = idx;
+    }
+    /* fan triangles of the selected polygons, in order */
+    hipLaunchKernelGGL(k_ts_nfan, dim3((unsigned)((np + 1 + 255) / 256)), dim3(256), 0, s,
+                       (const double*)c->d_poly_rec.ptr, (const int64_t*)c->d_poly_key.ptr, dmask, order, (int)np,
+                       (unsigned*)B.nfan.ptr);
+    if ((rc = ensure(c, B.tmp, std::max<size_t>(scan_temp_bytes((long long)np + 1), 8)))) return rc;
+    if (exclusive_scan_u32(s, (const unsigned*)B.nfan.ptr, (unsigned*)B.fan_off.ptr, (long long)np + 1, B.tmp.ptr,
                            B.tmp.bytes) != 0)
       return set_err(c, HCS_ERR_LIMIT, "sensor: too many polygons to scan");
-    rc = hip_check(c, hipMemcpyAsync(&ntri, (unsigned*)B.fan_off.ptr + nsel, sizeof(unsigned), hipMemcpyDeviceToHost,
-                                     s), "dl");
+    rc = hip_check(c, hipMemcpyAsync(&ntri, (unsigned*)B.fan_off.ptr + np, sizeof(unsigned), hipMemcpyDeviceToHost, s),
+                   "dl");
     if (!rc) rc = hip_check(c, hipStreamSynchronize(s), "sync");
     if (rc) return rc;
   }
@@ -473,9 +544,9 @@ static int sensor_fans(Ctx* c, int32_t geom, unsigned& ntri) {
       (rc = ensure(c, B.scnt, sizeof(unsigned) * (nt1 + 1))) || (rc = ensure(c, B.soff, sizeof(unsigned) * (nt1 + 1))))
     return rc;
   if (ntri > 0)
-    hipLaunchKernelGGL(k_ts_fans, dim3((nsel + 255) / 256), dim3(256), 0, s, (const double*)c->d_poly_rec.ptr,
-                       (const int64_t*)c->d_poly_key.ptr, idx, (int)nsel, (const unsigned*)B.fan_off.ptr,
-                       (double*)B.tris.ptr, (int*)B.surf.ptr);
+    hipLaunchKernelGGL(k_ts_fans, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, s,
+                       (const double*)c->d_poly_rec.ptr, (const int64_t*)c->d_poly_key.ptr, order, (int)np,
+                       (const unsigned*)B.fan_off.ptr, (double*)B.tris.ptr, (int*)B.surf.ptr);
   return hip_check(c, hipGetLastError(), "sensor triangles");
 }
 
