@@ -1246,7 +1246,7 @@ int hcs_destroy(hcs_ctx* h) {
     if (b->ptr) (void)hipFree(b->ptr);
   TaxelSensorBufs& T = c->ts;
   for (DBuf* b : {&T.mask, &T.k64, &T.kp, &T.idx, &T.cnt, &T.nfan, &T.fan_off, &T.tmp, &T.tris, &T.surf, &T.scnt, &T.soff,
-                  &T.P, &T.E, &T.taxel, &T.val, &T.hits})
+                  &T.P, &T.E, &T.taxel, &T.val, &T.hits, &T.area, &T.acc, &T.pair_u})
     if (b->ptr) (void)hipFree(b->ptr);
   (void)hipStreamDestroy(c->stream);
   delete h;

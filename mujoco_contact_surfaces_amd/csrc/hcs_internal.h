@@ -79,7 +79,7 @@ struct Plan {
 
 /* Scratch of hcs_taxel_sensor_update and hcs_curved_sensor_update. */
 struct TaxelSensorBufs {
-  DBuf mask, k64, kp, idx, cnt, nfan, fan_off, tmp, tris, surf, scnt, soff, P, E, taxel, val, hits;
+  DBuf mask, k64, kp, idx, cnt, nfan, fan_off, tmp, tris, surf, scnt, soff, P, E, taxel, val, hits, area, acc, pair_u;
 };
 
 struct Ctx {

@@ -13,16 +13,17 @@
  *      (both st1 and st2 from v2 - v0), one thread per triangle after a
  *      count and a scan; or AREA_IMPORTANCE (:205-246), a single sequential
  *      stream of libstdc++'s default_random_engine through
- *      uniform_real_distribution<double>(0, 1), one thread;
- *   3. one wavefront per taxel: dist = (-2 t.p + |t|^2) + |p|^2 to every
+ *      uniform_real_distribution<double>(0, 1), its running sums in
+ *      order and its samples in parallel;
+ *   3. taxels against samples: dist = (-2 t.p + |t|^2) + |p|^2 to every
  *      sample; CLOSEST (:285-319) takes the first nearest sample, and within
  *      the margin writes its pressure when visualize is set and |p| > 1e-6,
  *      else 0; WEIGHTED and MEAN fall through to SQUARED (:320-457, no
  *      break): sum of max(0, margin - sqrt(dist))^2 |p| over the samples in
  *      the margin, times sample_resolution.  A taxel no sample reaches keeps
  *      its value; with no sample at all every taxel is 0 (:458-477).
- * Sums over samples run lane-strided in sample order and then in a fixed
- * butterfly, so results are deterministic.
+ * Sums over samples run lane-strided within fixed slices of the samples, then
+ * in a fixed butterfly and over the slices, so results are deterministic.
  */
 #include <hip/hip_runtime.h>
 
@@ -202,42 +203,125 @@ struct TsRng {
   }
 };
 
-/* AREA_IMPORTANCE, one thread: write = false counts the samples into *m */
-__global__ void k_ts_area(const double* __restrict__ tris, const int* __restrict__ surf, int64_t nt, double res,
-                          bool write, double* __restrict__ P, double* __restrict__ E,
-                          unsigned long long* __restrict__ m) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  TsRng gen;
-  unsigned long long j = 0;
-  for (int64_t t0 = 0; t0 < nt;) {
-    int64_t t1 = t0;
-    double total = 0.0;
-    while (t1 < nt && surf[t1] == surf[t0]) {
-      const double* T = tris + HCS_TS_TRI * t1;
-      double e1[3] = {T[3] - T[0], T[4] - T[1], T[5] - T[2]}, e2[3] = {T[6] - T[0], T[7] - T[1], T[8] - T[2]}, cr[3];
-      cross3(e1, e2, cr);
-      total += 0.5 * sqrt(dot3(cr, cr));
-      ++t1;
-    }
-    const double area_resolution = res * total;
-    double acc = 0.0, at = 0.0;
-    for (int64_t t = t0; t < t1; ++t) {
-      const double* T = tris + HCS_TS_TRI * t;
-      double e1[3] = {T[3] - T[0], T[4] - T[1], T[5] - T[2]}, e2[3] = {T[6] - T[0], T[7] - T[1], T[8] - T[2]}, cr[3];
-      cross3(e1, e2, cr);
-      at += 0.5 * sqrt(dot3(cr, cr));
-      while (acc < at) {
-        acc += area_resolution;
-        const double u0 = gen.next(), u1 = gen.next();
-        const double a = 1.0 - sqrt(u0);
-        const double b = (1.0 - a) * u1;
-        if (write) ts_sample(T, a, (1 - a) * (1 - b), (1 - a) * b, P + 3 * j, E + j);
-        ++j;
-      }
-    }
-    t0 = t1;
+/* AREA_IMPORTANCE (:205-246).  Per surface the reference walks the triangles
+ * adding areas (at) and, while a running sum acc of resolution * total area is
+ * below at, draws a sample on the current triangle, all from one random
+ * stream.  The running sums are chains of rounded additions that decide which
+ * triangle a sample falls on and how many there are, so they are added in
+ * that order; everything else is parallel:
+ *   k_ts_areas  the triangles' areas;
+ *   k_ts_chain  one wave per surface: the prefix sums of its areas (the last
+ *               is the total), then the chain of acc below the total, counted
+ *               (write = false) or stored (write = true);
+ *   k_ts_draw   one thread per sample: its triangle is the first whose prefix
+ *               sum exceeds its acc, its random numbers come from jumping the
+ *               generator ahead to its place in the stream.
+ * One thread doing all of it, twice, took 28 ms for 25k triangles and 500
+ * samples; the chain kernel's two passes take 0.5 ms (FP64 add latency). */
+__global__ void k_ts_areas(const double* __restrict__ tris, const int* __restrict__ surf, int64_t nt,
+                           double* __restrict__ area, int* __restrict__ surf0, unsigned* __restrict__ nsurf) {
+  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (t >= nt) return;
+  const double* T = tris + HCS_TS_TRI * t;
+  double e1[3] = {T[3] - T[0], T[4] - T[1], T[5] - T[2]}, e2[3] = {T[6] - T[0], T[7] - T[1], T[8] - T[2]}, cr[3];
+  cross3(e1, e2, cr);
+  area[t] = 0.5 * sqrt(dot3(cr, cr));
+  /* the first triangle of every surface (in no order) */
+  if (t == 0 || surf[t] != surf[t - 1]) surf0[atomicAdd(nsurf, 1u)] = (int)t;
+}
+
+#define HCS_TS_CHAIN 1024
+__global__ __launch_bounds__(64) void k_ts_chain(const int* __restrict__ surf, int64_t nt,
+                                                 const int* __restrict__ surf0, unsigned* __restrict__ nsurf,
+                                                 double res, bool write, double* __restrict__ at,
+                                                 unsigned* __restrict__ count, const unsigned* __restrict__ off,
+                                                 double* __restrict__ acc_out, int2* __restrict__ tri_out) {
+  __shared__ double L[HCS_TS_CHAIN];
+  const int lane = threadIdx.x;
+  if (blockIdx.x >= *nsurf) return;
+  const int64_t t0 = surf0[blockIdx.x];
+  const int id = surf[t0];
+  /* the surface's end (the triangles are ordered by surface) */
+  int64_t t1 = t0 + 1;
+  for (int64_t hi = nt; t1 < hi;) {
+    const int64_t mid = (t1 + hi) >> 1;
+    if (surf[mid] == id) t1 = mid + 1;
+    else hi = mid;
   }
-  if (!write) *m = j;
+  if (!write) {
+    /* prefix sums in place of the areas, a tile of LDS at a time (padded with
+     * zeros, which leave the sum as it is): every lane adds the same chain
+     * (broadcast reads), lane 0 stores it */
+    double total = 0.0;
+    for (int64_t c0 = t0; c0 < t1; c0 += HCS_TS_CHAIN) {
+      const int cn = (int)(t1 - c0 < HCS_TS_CHAIN ? t1 - c0 : HCS_TS_CHAIN);
+      __syncthreads();
+      for (int k = lane; k < HCS_TS_CHAIN; k += 64) L[k] = k < cn ? at[c0 + k] : 0.0;
+      __syncthreads();
+      for (int k = 0; k < cn; k += 16) {
+        double v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = L[k + u];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = total = total + v[u];
+        if (lane == 0) {
+#pragma unroll
+          for (int u = 0; u < 16; ++u) L[k + u] = v[u];
+        }
+      }
+      __syncthreads();
+      for (int k = lane; k < cn; k += 64) at[c0 + k] = L[k];
+    }
+    __syncthreads();
+  }
+  /* a sample is drawn while acc is below some prefix sum: the total, or the
+   * last that is a number (fmax passes over a NaN area and what follows it) */
+  double top = 0.0;
+#pragma unroll 8
+  for (int64_t t = t0 + lane; t < t1; t += 64) top = fmax(top, at[t]);
+  top = wave_max(top);
+  const double step = res * at[t1 - 1];
+  const unsigned base = write ? off[id] : 0u;
+  unsigned n = 0;
+  for (double acc = 0.0; acc < top; ++n) {
+    if (write && lane == 0) acc_out[base + n] = acc, tri_out[base + n] = make_int2((int)t0, (int)t1 - 1);
+    const double next = acc + step;
+    if (next == acc) {
+      /* a step below the rounding of acc would never reach the end */
+      if (lane == 0) nsurf[1] = 1u;
+      break;
+    }
+    acc = next;
+  }
+  if (!write && lane == 0) count[id] = n;
+}
+
+/* x * 16807^e modulo 2^31 - 1 */
+__device__ inline unsigned long long minstd_jump(unsigned long long x, unsigned long long e) {
+  for (unsigned long long g = 16807ull; e; e >>= 1, g = (g * g) % 2147483647ull)
+    if (e & 1) x = (x * g) % 2147483647ull;
+  return x;
+}
+
+__global__ void k_ts_draw(const double* __restrict__ tris, const double* __restrict__ at,
+                          const double* __restrict__ acc, const int2* __restrict__ range, int64_t m,
+                          double* __restrict__ P, double* __restrict__ E) {
+  const int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (j >= m) return;
+  /* prefix sums do not decrease (a NaN counts as exceeding) */
+  const double a0 = acc[j];
+  int64_t lo = range[j].x, hi = range[j].y;
+  while (lo < hi) {
+    const int64_t mid = (lo + hi) >> 1;
+    if (at[mid] <= a0) lo = mid + 1;
+    else hi = mid;
+  }
+  TsRng gen;
+  gen.x = minstd_jump(gen.x, 4ull * (unsigned long long)j);
+  const double u0 = gen.next(), u1 = gen.next();
+  const double a = 1.0 - sqrt(u0);
+  const double b = (1.0 - a) * u1;
+  ts_sample(tris + HCS_TS_TRI * lo, a, (1 - a) * (1 - b), (1 - a) * b, P + 3 * j, E + j);
 }
 
 struct CsArgs {
@@ -251,45 +335,100 @@ struct TsTaxelArgs {
   int method, visualize;
 };
 
+/* One wave's result for a taxel over its slice of the samples: squared: the
+ * weighted sum and the samples in the margin; closest: the least distance
+ * and its first sample (n < 0: none). */
+struct TsPart {
+  double v;
+  long long n;
+};
+
+/* Taxels against samples.  A wave takes HCS_TS_TX taxels and a slice of the
+ * samples (blockIdx.y), a lane every 64th sample of it: a sample is loaded
+ * once for the wave's taxels, and the slices fill the chip whatever the
+ * number of taxels (one wave per taxel over all samples was 256 waves, each
+ * a chain of 1600 loads of its own: 501 us for 256 taxels and 104k samples,
+ * -> 24 us).  FP64 multiplies and adds bound it. */
+#define HCS_TS_TX 8
+template <bool CLOSEST>
 __global__ __launch_bounds__(64) void k_ts_taxel(const double* __restrict__ P, const double* __restrict__ E,
-                                                 int64_t m, TsTaxelArgs a, const double* __restrict__ taxels,
-                                                 double* __restrict__ values) {
-  const int i = blockIdx.x, lane = threadIdx.x;
-  double tw[3];
-  xform(a.X, taxels + 3 * (size_t)i, tw);
-  const double tt = dot3(tw, tw), msq = a.margin * a.margin;
-  if (a.method == 0) {
-    double bd = __builtin_inf();
-    long long bj = 0x7fffffffffffffffll;
-    for (int64_t j = lane; j < m; j += 64) {
-      const double* p = P + 3 * j;
-      const double d = ((-2.0 * dot3(tw, p)) + tt) + dot3(p, p);
-      if (d < bd) bd = d, bj = j;
-    }
-    /* first nearest sample: (distance, index) lexicographic minimum */
+                                                 int64_t m, TsTaxelArgs a, const double* __restrict__ taxels, int nx,
+                                                 TsPart* __restrict__ part) {
+  const int i0 = blockIdx.x * HCS_TS_TX, lane = threadIdx.x;
+  double tw[HCS_TS_TX][3], tt[HCS_TS_TX], v[HCS_TS_TX];
+  int64_t n[HCS_TS_TX];
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      const double od = __shfl_xor(bd, o, 64);
-      const long long oj = __shfl_xor(bj, o, 64);
-      if (od < bd || (od == bd && oj < bj)) bd = od, bj = oj;
-    }
-    if (lane == 0 && bd < msq) values[i] = (a.visualize && fabs(E[bj]) > 1e-6) ? E[bj] : 0.0;
-  } else {
-    double sum = 0.0;
-    long long ws = 0;
-    for (int64_t j = lane; j < m; j += 64) {
-      const double* p = P + 3 * j;
-      const double d = ((-2.0 * dot3(tw, p)) + tt) + dot3(p, p);
-      if (d < msq) {
+  for (int k = 0; k < HCS_TS_TX; ++k) {
+    const int i = i0 + k < nx ? i0 + k : nx - 1;
+    xform(a.X, taxels + 3 * (size_t)i, tw[k]);
+    tt[k] = dot3(tw[k], tw[k]);
+    v[k] = CLOSEST ? __builtin_inf() : 0.0;
+    n[k] = CLOSEST ? 0x7fffffffffffffffll : 0;
+  }
+  const double msq = a.margin * a.margin;
+  const int64_t s0 = m * blockIdx.y / gridDim.y, s1 = m * (blockIdx.y + 1) / gridDim.y;
+  for (int64_t j = s0 + lane; j < s1; j += 64) {
+    const double p[3] = {P[3 * j], P[3 * j + 1], P[3 * j + 2]};
+    const double e = CLOSEST ? 0.0 : fabs(E[j]);
+    const double pp = dot3(p, p);
+#pragma unroll
+    for (int k = 0; k < HCS_TS_TX; ++k) {
+      const double d = ((-2.0 * dot3(tw[k], p)) + tt[k]) + pp;
+      if (CLOSEST) {
+        if (d < v[k]) v[k] = d, n[k] = j;
+      } else if (d < msq) {
         const double w0 = fmax(0.0, a.margin - sqrt(d));
-        sum += (w0 * w0) * fabs(E[j]);
-        ++ws;
+        v[k] += (w0 * w0) * e;
+        ++n[k];
       }
     }
-    sum = wave_sum<double>(sum);
-    ws = wave_sum_i(ws);
-    if (lane == 0 && ws > 0) values[i] = sum * a.res;
   }
+#pragma unroll
+  for (int k = 0; k < HCS_TS_TX; ++k) {
+    if (CLOSEST) {
+      /* first nearest sample: (distance, index) lexicographic minimum */
+#pragma unroll
+      for (int o = 32; o >= 1; o >>= 1) {
+        const double od = __shfl_xor(v[k], o, 64);
+        const int64_t oj = __shfl_xor((long long)n[k], o, 64);
+        if (od < v[k] || (od == v[k] && oj < n[k])) v[k] = od, n[k] = oj;
+      }
+    } else {
+      v[k] = wave_sum<double>(v[k]);
+      n[k] = wave_sum_i(n[k]);
+    }
+    if (lane == 0 && i0 + k < nx) part[(size_t)blockIdx.y * nx + i0 + k] = TsPart{v[k], (long long)n[k]};
+  }
+}
+
+/* Per taxel, the slices' results in order, four lanes per taxel and then a
+ * fixed butterfly; a taxel no sample reaches keeps its value. */
+template <bool CLOSEST>
+__global__ __launch_bounds__(64) void k_ts_combine(const TsPart* __restrict__ part, int nslice, int nx, TsTaxelArgs a,
+                                                   const double* __restrict__ E, double* __restrict__ values) {
+  const int i = blockIdx.x * 16 + (threadIdx.x & 15);
+  TsPart b{CLOSEST ? __builtin_inf() : 0.0, CLOSEST ? 0x7fffffffffffffffll : 0};
+  auto add = [&](const TsPart& q) {
+    if (!CLOSEST) b.v += q.v, b.n += q.n;
+    else if (q.v < b.v || (q.v == b.v && q.n < b.n)) b = q;
+  };
+  if (i < nx)
+    for (int s = threadIdx.x >> 4; s < nslice; s += 4) add(part[(size_t)s * nx + i]);
+#pragma unroll
+  for (int o = 16; o <= 32; o <<= 1) add(TsPart{__shfl_xor(b.v, o, 64), __shfl_xor(b.n, o, 64)});
+  if (i >= nx || threadIdx.x >= 16) return;
+  if (CLOSEST) {
+    if (b.v < a.margin * a.margin) values[i] = (a.visualize && fabs(E[b.n]) > 1e-6) ? E[b.n] : 0.0;
+  } else if (b.n > 0) {
+    values[i] = b.v * a.res;
+  }
+}
+
+/* Sample slices of the taxel kernel: enough for about 2048 waves, at least
+ * 256 samples each. */
+static int ts_slices(int nx, int64_t m) {
+  const int64_t groups = (nx + HCS_TS_TX - 1) / HCS_TS_TX;
+  return (int)std::max<int64_t>(1, std::min<int64_t>(2048 / groups, m / 256));
 }
 
 /* The nearest hit of a ray in one slice of the triangles. */
@@ -565,6 +704,8 @@ int hcs_taxel_sensor_update(hcs_ctx* h, const hcs_taxel_sensor* S, double* value
   if ((rc = sensor_fans(c, S->geom, ntri))) return rc;
   /* samples */
   unsigned long long m = 0;
+  unsigned *nsurf = nullptr, *soff = nullptr;
+  int* surf0 = nullptr;
   if (ntri > 0 && S->sample_method == 0) {
     hipLaunchKernelGGL(k_ts_count, dim3((ntri + 1 + 255) / 256), dim3(256), 0, s, (const double*)B.tris.ptr,
                        (int64_t)ntri, S->sample_resolution, (unsigned*)B.scnt.ptr);
@@ -579,12 +720,29 @@ int hcs_taxel_sensor_update(hcs_ctx* h, const hcs_taxel_sensor* S, double* value
     if (rc) return rc;
     m = m32;
   } else if (ntri > 0) {
-    hipLaunchKernelGGL(k_ts_area, dim3(1), dim3(64), 0, s, (const double*)B.tris.ptr, (const int*)B.surf.ptr,
-                       (int64_t)ntri, S->sample_resolution, false, nullptr, nullptr,
-                       (unsigned long long*)B.cnt.ptr);
-    rc = hip_check(c, hipMemcpyAsync(&m, B.cnt.ptr, sizeof(m), hipMemcpyDeviceToHost, s), "dl");
+    /* areas and prefix sums; per pair the first triangle (in no order), the
+     * sample count and its scan; [surfaces, stalled] */
+    const size_t np1 = c->last_pairs.size() + 1;
+    if ((rc = ensure(c, B.area, sizeof(double) * ntri)) || (rc = ensure(c, B.pair_u, sizeof(unsigned) * (3 * np1 + 2))) ||
+        (rc = ensure(c, B.tmp, std::max<size_t>(scan_temp_bytes((long long)np1), 8))))
+      return rc;
+    unsigned* cnt = (unsigned*)B.pair_u.ptr;
+    nsurf = cnt + np1, soff = nsurf + 2, surf0 = (int*)(soff + np1);
+    launch_fill_u32(s, cnt, 0u, (int)np1 + 2);
+    hipLaunchKernelGGL(k_ts_areas, dim3((ntri + 255) / 256), dim3(256), 0, s, (const double*)B.tris.ptr,
+                       (const int*)B.surf.ptr, (int64_t)ntri, (double*)B.area.ptr, surf0, nsurf);
+    hipLaunchKernelGGL(k_ts_chain, dim3((unsigned)c->last_pairs.size()), dim3(64), 0, s, (const int*)B.surf.ptr,
+                       (int64_t)ntri, surf0, nsurf, S->sample_resolution, false, (double*)B.area.ptr, cnt,
+                       (const unsigned*)soff, (double*)nullptr, (int2*)nullptr);
+    if (exclusive_scan_u32(s, cnt, soff, (long long)np1, B.tmp.ptr, B.tmp.bytes) != 0)
+      return set_err(c, HCS_ERR_LIMIT, "sensor: too many pairs to scan");
+    unsigned got[2] = {0, 0}; /* stalled, samples */
+    rc = hip_check(c, hipMemcpyAsync(got, nsurf + 1, sizeof(unsigned), hipMemcpyDeviceToHost, s), "dl");
+    if (!rc) rc = hip_check(c, hipMemcpyAsync(got + 1, soff + np1 - 1, sizeof(unsigned), hipMemcpyDeviceToHost, s), "dl");
     if (!rc) rc = hip_check(c, hipStreamSynchronize(s), "sync");
     if (rc) return rc;
+    if (got[0]) return set_err(c, HCS_ERR_LIMIT, "sensor: sample_resolution is below the rounding of the surface's area");
+    m = got[1];
   }
   if (nsamples) *nsamples = (int64_t)m;
   if (m == 0) {
@@ -598,10 +756,17 @@ int hcs_taxel_sensor_update(hcs_ctx* h, const hcs_taxel_sensor* S, double* value
   if (S->sample_method == 0)
     hipLaunchKernelGGL(k_ts_gen, dim3((ntri + 255) / 256), dim3(256), 0, s, (const double*)B.tris.ptr, (int64_t)ntri,
                        S->sample_resolution, (const unsigned*)B.soff.ptr, (double*)B.P.ptr, (double*)B.E.ptr);
-  else
-    hipLaunchKernelGGL(k_ts_area, dim3(1), dim3(64), 0, s, (const double*)B.tris.ptr, (const int*)B.surf.ptr,
-                       (int64_t)ntri, S->sample_resolution, true, (double*)B.P.ptr, (double*)B.E.ptr,
-                       (unsigned long long*)B.cnt.ptr);
+  else {
+    if ((rc = ensure(c, B.acc, (sizeof(double) + sizeof(int2)) * m))) return rc;
+    double* acc = (double*)B.acc.ptr;
+    int2* range = (int2*)(acc + m);
+    hipLaunchKernelGGL(k_ts_chain, dim3((unsigned)c->last_pairs.size()), dim3(64), 0, s, (const int*)B.surf.ptr,
+                       (int64_t)ntri, surf0, nsurf, S->sample_resolution, true, (double*)B.area.ptr,
+                       (unsigned*)nullptr, (const unsigned*)soff, acc, range);
+    hipLaunchKernelGGL(k_ts_draw, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, (const double*)B.tris.ptr,
+                       (const double*)B.area.ptr, (const double*)acc, (const int2*)range, (int64_t)m,
+                       (double*)B.P.ptr, (double*)B.E.ptr);
+  }
   if (S->ntaxels == 0) return hip_check(c, hipGetLastError(), "samples");
   TsTaxelArgs a;
   std::memcpy(a.X, S->X_W_sensor, sizeof a.X);
@@ -612,8 +777,22 @@ int hcs_taxel_sensor_update(hcs_ctx* h, const hcs_taxel_sensor* S, double* value
     rc = hip_check(c, hipMemcpyAsync(B.val.ptr, values, sizeof(double) * S->ntaxels, hipMemcpyHostToDevice, s),
                    "upload values");
   if (rc) return rc;
-  hipLaunchKernelGGL(k_ts_taxel, dim3(S->ntaxels), dim3(64), 0, s, (const double*)B.P.ptr, (const double*)B.E.ptr,
-                     (int64_t)m, a, (const double*)B.taxel.ptr, (double*)B.val.ptr);
+  const int nx = S->ntaxels, nslice = ts_slices(nx, (int64_t)m);
+  if ((rc = ensure(c, B.hits, sizeof(TsPart) * (size_t)nx * nslice))) return rc;
+  TsPart* part = (TsPart*)B.hits.ptr;
+  const dim3 grid((nx + HCS_TS_TX - 1) / HCS_TS_TX, nslice), cgrid((nx + 15) / 16);
+  const double *P = (const double*)B.P.ptr, *E = (const double*)B.E.ptr;
+  if (a.method == 0) {
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_ts_taxel<true>), grid, dim3(64), 0, s, P, E, (int64_t)m, a,
+                       (const double*)B.taxel.ptr, nx, part);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_ts_combine<true>), cgrid, dim3(64), 0, s, (const TsPart*)part, nslice, nx, a,
+                       E, (double*)B.val.ptr);
+  } else {
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_ts_taxel<false>), grid, dim3(64), 0, s, P, E, (int64_t)m, a,
+                       (const double*)B.taxel.ptr, nx, part);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_ts_combine<false>), cgrid, dim3(64), 0, s, (const TsPart*)part, nslice, nx, a,
+                       E, (double*)B.val.ptr);
+  }
   rc = hip_check(c, hipGetLastError(), "taxel sensor");
   if (!rc)
     rc = hip_check(c, hipMemcpyAsync(values, B.val.ptr, sizeof(double) * S->ntaxels, hipMemcpyDeviceToHost, s), "dl");
