@@ -1170,6 +1170,31 @@ __device__ inline void run_cand(CandLds& L, const QueryArgs& A, int it, const It
   }
 }
 
+/* The lane's tet of a half-space item (64 consecutive leaves): the same tests
+ * in the same order as run_cand's half-space branch (candidate when the tet's
+ * AABB straddles B's plane, then survives()). */
+__device__ inline void plane_test(const QueryArgs& A, const Item& item, int& a, bool& hit, bool& keep) {
+  const int lane = threadIdx.x & 63;
+  a = 0, hit = keep = false;
+  if (lane >= item.count) return;
+  const EnvDesc& E = A.envs[item.env];
+  const double* X = A.xf + 12 * (size_t)item.env;
+  a = E.leafA[item.first + lane];
+  const HCS_GPTR double* lb = E.boxLA + 6 * (size_t)(item.first + lane); /* = boxA of tet a */
+  const double ez[3] = {0.0, 0.0, 1.0};
+  double nS[3];
+  rot(X, ez, nS);
+  const double off = -dot3(nS, X + 9);
+  double dist = off, rad = 0.0;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    dist += nS[c] * (0.5 * (lb[c] + lb[3 + c]));
+    rad += fabs(nS[c]) * (0.5 * (lb[3 + c] - lb[c]));
+  }
+  hit = !(fabs(dist) > rad);
+  if (hit) keep = survives<KIND_PLANE>(E, X, a, 0, nullptr, nullptr);
+}
+
 /* ===================================================================
  * k_clip: one survivor per thread -> contribution at item_off + seq
  * =================================================================== */
