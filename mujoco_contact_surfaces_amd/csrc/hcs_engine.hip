@@ -28,6 +28,7 @@
 #include "hcs_internal.h"
 #include "hcs_prim.h"
 #include "hcs_query.h"
+#include "hcs_reduce.h"
 
 #pragma clang fp contract(off)
 
@@ -67,6 +68,20 @@ int ensure(Ctx* c, DBuf& b, size_t bytes) {
   size_t n = std::max<size_t>(bytes, 256);
   HCHK(c, hipMalloc(&b.ptr, n));
   b.bytes = n;
+  return HCS_OK;
+}
+
+/* Grow-only pinned host memory, readable and writable by the device. */
+int pinned(Ctx* c, void*& p, size_t& have, size_t bytes) {
+  if (p && bytes <= have) return HCS_OK;
+  if (p) {
+    HCHK(c, hipStreamSynchronize(c->stream));
+    HCHK(c, hipHostFree(p));
+    p = nullptr, have = 0;
+  }
+  bytes += bytes / 2;
+  HCHK(c, hipHostMalloc(&p, bytes, hipHostMallocDefault));
+  have = bytes;
   return HCS_OK;
 }
 
@@ -300,34 +315,55 @@ __global__ void k_gather_boxes(const double* __restrict__ box, const int* __rest
   for (int c = 0; c < 6; ++c) boxL[6 * (size_t)i + c] = box[6 * (size_t)idx[i] + c];
 }
 
-/* Per step, one block per tet-query pair: its rigid triangles moved into
- * A's frame (vertices by xform, unit normal by rot, and their AABB), the
- * same arithmetic the candidate and clip stages use. */
+/* Per step, one block per tet-query pair: its triangles moved. */
 __global__ __launch_bounds__(64) void k_xtri(const EnvDesc* __restrict__ envs, const int* __restrict__ xenv,
                                              const double* __restrict__ xf, double* __restrict__ xtri) {
   const int e = xenv[blockIdx.x];
-  const EnvDesc& E = envs[e];
-  const double* X = xf + 12 * (size_t)e;
-  for (int t = threadIdx.x; t < E.nB; t += blockDim.x) {
-    double* o = xtri + HCS_XTRI * (size_t)(E.xtri_off + t);
-    const int32_t* f = E.FB + 3 * (size_t)t;
-    double lo[3], hi[3];
+  move_triangles(envs[e], xf + 12 * (size_t)e, xtri, 64);
+}
+
+/* Boxes of a mesh's chunks of 64 elements (nv vertices each) in the order
+ * `order`, in the mesh's own frame, one wave per chunk. */
+__global__ __launch_bounds__(64) void k_chunk_boxes(const double* __restrict__ V, const int32_t* __restrict__ el, int nv,
+                                                    const int32_t* __restrict__ order, int n,
+                                                    double* __restrict__ cbox) {
+  const int i = blockIdx.x * 64 + threadIdx.x;
+  const double inf = __builtin_inf();
+  double lo[3] = {inf, inf, inf}, hi[3] = {-inf, -inf, -inf};
+  if (i < n) {
+    const int32_t* f = el + (size_t)nv * order[i];
+    for (int k = 0; k < nv; ++k) {
+      const double* v = V + 3 * (size_t)f[k];
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      double y[3];
-      xform(X, hcs_plain(E.VB + 3 * (size_t)f[i]), y);
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        o[3 * i + c] = y[c];
-        lo[c] = i == 0 ? y[c] : fmin(lo[c], y[c]);
-        hi[c] = i == 0 ? y[c] : fmax(hi[c], y[c]);
-      }
+      for (int c = 0; c < 3; ++c) lo[c] = fmin(lo[c], v[c]), hi[c] = fmax(hi[c], v[c]);
     }
-    double nS[3];
-    rot(X, hcs_plain(E.nrmB + 3 * (size_t)t), nS);
-#pragma unroll
-    for (int c = 0; c < 3; ++c) o[9 + c] = nS[c], o[12 + c] = lo[c], o[15 + c] = hi[c];
   }
+#pragma unroll
+  for (int c = 0; c < 3; ++c) lo[c] = wave_min(lo[c]), hi[c] = wave_max(hi[c]);
+  if (threadIdx.x < 6) {
+    double v = lo[0];
+#pragma unroll
+    for (int c = 1; c < 6; ++c) v = threadIdx.x == c ? (c < 3 ? lo[c] : hi[c - 3]) : v;
+    cbox[6 * (size_t)blockIdx.x + threadIdx.x] = v;
+  }
+}
+
+/* The LBVH's frontiers (HCS_ROOTS), one block, level by level. */
+__global__ __launch_bounds__(HCS_ROOTS / 2) void k_frontiers(const Node* __restrict__ nodes, int n_int, int32_t* __restrict__ heap) {
+  __shared__ int32_t h[HCS_ROOTS];
+  const int t = threadIdx.x;
+  if (t < 2) h[t] = t == 1 ? 0 : HCS_WNONE;
+  __syncthreads();
+  for (int d = 0; d < HCS_ROOT_DEPTH; ++d) {
+    if (t < (1 << d)) {
+      const int i = (1 << d) + t, c = h[i];
+      const bool node = c >= 0 && n_int > 0;
+      h[2 * i] = node ? nodes[c].c[0] : c;
+      h[2 * i + 1] = node ? nodes[c].c[1] : HCS_WNONE;
+    }
+    __syncthreads();
+  }
+  heap[t] = h[t], heap[HCS_ROOTS / 2 + t] = h[HCS_ROOTS / 2 + t];
 }
 
 /* Static boxes of one item per wave: [0..5] its query elements in their own
@@ -510,7 +546,7 @@ template <int MODE, int KS>
 __global__ __launch_bounds__(64, KS == KIND_TRI ? 3 : 2) void k_cand(QueryArgs A) {
   __shared__ CandLds L;
   unsigned long long s_next = 0, s_end = 0; /* this wave's survivor slots */
-  const int nq = A.live ? A.nqueues : 1;
+  const int nq = A.live_cnt ? A.nqueues : 1;
   const int lane = threadIdx.x & 63;
   if (A.counter == nullptr) {
     /* one item per block, queues back to back */
@@ -528,7 +564,7 @@ __global__ __launch_bounds__(64, KS == KIND_TRI ? 3 : 2) void k_cand(QueryArgs A
       }
       v -= n;
     }
-  } else if (A.live && nq == 1) {
+  } else if (A.live_cnt && nq == 1) {
     /* persistent, one queue.  Block b's first three items are items b,
      * b + G and b + 2G (G = gridDim.x), and the counter hands out the
      * items from 3G on: every wave starts at the launch, and one atomic per
@@ -539,12 +575,12 @@ __global__ __launch_bounds__(64, KS == KIND_TRI ? 3 : 2) void k_cand(QueryArgs A
      * issued after its first item, when the waves no longer run in step,
      * and its result is needed only after the second. */
     const unsigned n = A.live_cnt[0], G = gridDim.x;
-    const int base = A.qseg[0];
+    const int base = A.live ? A.qseg[0] : 0;
     const unsigned v = blockIdx.x;
     /* tet and half-space items are alike and short: dealt out by index */
     constexpr bool fixed = KS == KIND_PLANE || KS == KIND_TET;
     if (v < n) {
-      int idx = A.live[base + v];
+      int idx = A.live ? A.live[base + v] : (int)v;
       int4 rec = A.live_item[base + v];
       unsigned vn = v + G;
       for (int k = 0;; ++k) {
@@ -552,7 +588,7 @@ __global__ __launch_bounds__(64, KS == KIND_TRI ? 3 : 2) void k_cand(QueryArgs A
         int4 nrec = make_int4(0, 0, 0, 0);
         unsigned raw = 0;
         if (vn < n) {
-          nidx = A.live[base + vn];
+          nidx = A.live ? A.live[base + vn] : (int)vn;
           nrec = A.live_item[base + vn];
           if (!fixed && k > 0 && lane == 0) raw = atomicAdd(A.counter, 1u);
         }
@@ -626,9 +662,9 @@ __global__ __launch_bounds__(64 * HCS_PLANE_WAVES) void k_cand_plane(QueryArgs A
   __shared__ unsigned tot[HCS_PLANE_WAVES];
   __shared__ unsigned long long base;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int nq = A.live ? A.nqueues : 1;
+  const int nq = A.live_cnt ? A.nqueues : 1;
   for (int x = 0; x < nq; ++x) {
-    const unsigned n = A.live ? A.live_cnt[x] : (unsigned)A.nitems;
+    const unsigned n = A.live_cnt ? A.live_cnt[x] : (unsigned)A.nitems;
     const int q0 = A.live ? A.qseg[x] : 0;
     for (unsigned r0 = blockIdx.x * HCS_PLANE_ITEMS; r0 < n; r0 += gridDim.x * HCS_PLANE_ITEMS) {
       unsigned long long t_begin[HCS_PLANE_PER], w_begin[HCS_PLANE_PER];
@@ -642,10 +678,10 @@ __global__ __launch_bounds__(64 * HCS_PLANE_WAVES) void k_cand_plane(QueryArgs A
         Item item{0, 0, 0, 0};
         it[u] = -1;
         if (v < n) {
-          if (A.live) {
+          if (A.live_cnt) {
             const int4 rec = A.live_item[q0 + v];
             item = Item{rec.x, rec.y, rec.z, rec.w};
-            it[u] = A.live[q0 + v];
+            it[u] = A.live ? A.live[q0 + v] : (int)v;
           } else {
             item = A.items[v];
             it[u] = (int)v;
@@ -725,7 +761,7 @@ __global__ __launch_bounds__(64) void k_env_reduce(const EnvDesc* __restrict__ e
                                                    const Contrib* __restrict__ contrib, int64_t stride,
                                                    RedPart* __restrict__ part) {
   const int4 w = rtab[blockIdx.x];
-  const int e = w.x, j = w.y, K = w.z, d = blockIdx.y, lane = threadIdx.x;
+  const int e = w.x, j = w.y, K = w.z, d = blockIdx.y;
   const int first = envs[e].item_first, cnt = envs[e].item_count;
   /* on survivor-list overflow the offsets run past the contribution slots:
    * sum nothing, the status reports the overflow */
@@ -734,36 +770,8 @@ __global__ __launch_bounds__(64) void k_env_reduce(const EnvDesc* __restrict__ e
    * it whatever the offsets hold) */
   const unsigned capu = (unsigned)(surv_cap < 0xffffffffLL ? surv_cap : 0xffffffffLL);
   const unsigned lo = min(off[first], capu), hi = over ? lo : max(lo, min(off[first + cnt], capu));
-  const uint64_t len = hi - lo;
-  const unsigned s0 = lo + (unsigned)(len * j / K), s1 = lo + (unsigned)(len * (j + 1) / K);
-  const int i0 = first + (int)((int64_t)cnt * j / K), i1 = first + (int)((int64_t)cnt * (j + 1) / K);
-  const Contrib* cb = contrib + (int64_t)d * stride;
-  double F[3] = {0, 0, 0}, tA[3] = {0, 0, 0}, tB[3] = {0, 0, 0};
-  int64_t np = 0, nf = 0, nc = 0;
-  auto add = [&](const Contrib& q) {
-#pragma unroll
-    for (int c = 0; c < 3; ++c) F[c] = F[c] + q.F[c], tA[c] = tA[c] + q.tA[c], tB[c] = tB[c] + q.tB[c];
-    np += q.np, nf += q.nf;
-  };
-  /* lane-strided in slot order; four slots loaded before they are added,
-   * so four loads are in flight per lane */
-  unsigned i = s0 + lane;
-  for (; i < s1 && s1 - i > 192; i += 256) {
-    const Contrib q0 = cb[i], q1 = cb[i + 64], q2 = cb[i + 128], q3 = cb[i + 192];
-    add(q0), add(q1), add(q2), add(q3);
-  }
-  for (; i < s1; i += 64) add(cb[i]);
-  for (int i = i0 + lane; i < i1; i += 64) nc += item_ncand[i];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) F[c] = wave_sum(F[c]), tA[c] = wave_sum(tA[c]), tB[c] = wave_sum(tB[c]);
-  np = wave_sum_i(np), nf = wave_sum_i(nf), nc = wave_sum_i(nc);
-  if (lane == 0) {
-    RedPart r;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) r.F[c] = F[c], r.tA[c] = tA[c], r.tB[c] = tB[c];
-    r.np = np, r.nf = nf, r.nc = nc;
-    part[(int64_t)d * nred + w.w + j] = r;
-  }
+  const RedPart r = reduce_slice(contrib + (int64_t)d * stride, lo, hi, j, K, item_ncand, first, cnt);
+  if (threadIdx.x == 0) part[(int64_t)d * nred + w.w + j] = r;
 }
 
 /* One thread per (pair, direction): the pair's slices in order. */
@@ -900,6 +908,22 @@ void launch_cand(hipStream_t s, const QueryArgs& a, int grid, int mode) {
   else launch_cand_mode<CAND_STEP>(s, a, grid);
 }
 
+/* The forward clip kernel, built for the launch's kind. */
+void launch_clip(Ctx* c, const Pipe& p, const QueryArgs& a, int clip_grid) {
+  const ClipArgs C{(const unsigned*)p.off.ptr, nullptr, nullptr, p.cap};
+  const dim3 g(std::max(1, clip_grid));
+  Contrib* out = (Contrib*)p.contrib.ptr;
+  const int64_t zero = 0;
+  hipStream_t s = c->stream;
+  switch (launch_kind(a)) {
+    case KIND_TRI: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_clip<double, KIND_TRI>), g, dim3(256), 0, s, a, C, -1, out, zero); break;
+    case KIND_SOFT: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_clip<double, KIND_SOFT>), g, dim3(256), 0, s, a, C, -1, out, zero); break;
+    case KIND_TET: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_clip<double, KIND_TET>), g, dim3(256), 0, s, a, C, -1, out, zero); break;
+    case KIND_PLANE: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_clip<double, KIND_PLANE>), g, dim3(256), 0, s, a, C, -1, out, zero); break;
+    default: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_clip<double, -1>), g, dim3(256), 0, s, a, C, -1, out, zero); break;
+  }
+}
+
 /* Scan of the per-item survivor counts, [event e_clip], clip (double, or
  * Dual over ndir directions), [event e_reduce], per-pair reduction. */
 static void pipe_back(Ctx* c, Pipe& p, const QueryArgs& a, int npairs, int clip_grid, int ndir,
@@ -909,27 +933,13 @@ static void pipe_back(Ctx* c, Pipe& p, const QueryArgs& a, int npairs, int clip_
   (void)exclusive_scan_u32(s, (const unsigned*)p.nsurv.ptr, (unsigned*)p.off.ptr, (long long)a.nitems + 1,
                            p.scan_tmp.ptr, p.scan_bytes);
   if (e_clip) (void)hipEventRecord(e_clip, s);
-  ClipArgs C{(const unsigned*)p.off.ptr, dstar_dE, invE, p.cap};
-  const int g = std::max(1, clip_grid);
-  const int kind = launch_kind(a);
-  if (ndir > 0)
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_clip<Dual, -1>), dim3(g, ndir), dim3(256), 0, s, a, C, dir0,
+  if (ndir > 0) {
+    const ClipArgs C{(const unsigned*)p.off.ptr, dstar_dE, invE, p.cap};
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_clip<Dual, -1>), dim3(std::max(1, clip_grid), ndir), dim3(256), 0, s, a, C, dir0,
                        (Contrib*)p.contrib.ptr, (int64_t)p.cap);
-  else if (kind == KIND_TRI)
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_clip<double, KIND_TRI>), dim3(g), dim3(256), 0, s, a, C, -1,
-                       (Contrib*)p.contrib.ptr, (int64_t)0);
-  else if (kind == KIND_SOFT)
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_clip<double, KIND_SOFT>), dim3(g), dim3(256), 0, s, a, C, -1,
-                       (Contrib*)p.contrib.ptr, (int64_t)0);
-  else if (kind == KIND_TET)
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_clip<double, KIND_TET>), dim3(g), dim3(256), 0, s, a, C, -1,
-                       (Contrib*)p.contrib.ptr, (int64_t)0);
-  else if (kind == KIND_PLANE)
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_clip<double, KIND_PLANE>), dim3(g), dim3(256), 0, s, a, C, -1,
-                       (Contrib*)p.contrib.ptr, (int64_t)0);
-  else
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_clip<double, -1>), dim3(g), dim3(256), 0, s, a, C, -1,
-                       (Contrib*)p.contrib.ptr, (int64_t)0);
+  } else {
+    launch_clip(c, p, a, clip_grid);
+  }
   if (e_reduce) (void)hipEventRecord(e_reduce, s);
   if (npairs > 0 && p.nred > 0) {
     const int nd = std::max(1, ndir);
@@ -1036,7 +1046,7 @@ int pipe_plan(Ctx* c, Pipe& p, const EnvDesc* envs, const Item* items, const Pla
 void pipe_free(Pipe& p) {
   for (DBuf* b : {&p.counter, &p.surv, &p.surv_cnt, &p.ncand, &p.nsurv, &p.off, &p.scan_tmp, &p.contrib, &p.out, &p.err,
                   &p.xf, &p.ibox, &p.live, &p.live_item, &p.qseg, &p.xtri, &p.xenv, &p.order, &p.item_o, &p.part, &p.rtab,
-                  &p.ptab})
+                  &p.ptab, &p.blob, &p.gen_cnt, &p.gen_mask, &p.gen_item, &p.pair_lo})
     if (b->ptr) (void)hipFree(b->ptr), b->ptr = nullptr, b->bytes = 0;
 }
 
@@ -1190,20 +1200,66 @@ static int build_bvh(Ctx* c, Mesh& m) {
   return rc;
 }
 
+/* Chunk boxes (with room for one more) over the elements in `order`. */
+static int build_chunk_boxes(Ctx* c, Mesh& m, int nv, const int32_t* order) {
+  const int chunks = (m.nelem + 63) / 64;
+  HCHK(c, hipMalloc((void**)&m.cbox, 6 * sizeof(double) * ((size_t)chunks + 1)));
+  hipLaunchKernelGGL(k_chunk_boxes, dim3(chunks), dim3(64), 0, c->stream, m.V, m.E, nv, order, m.nelem, m.cbox);
+  return hip_check(c, hipGetLastError(), "k_chunk_boxes");
+}
+
+/* A soft mesh's tables for the work items: boxes of its chunks of 64 leaves,
+ * and its LBVH's frontiers. */
+static int build_item_tables(Ctx* c, Mesh& m) {
+  int rc = build_chunk_boxes(c, m, 4, m.leaf);
+  if (!rc) rc = hip_check(c, hipMalloc((void**)&m.roots, sizeof(int32_t) * HCS_ROOTS), "hipMalloc");
+  if (rc) return rc;
+  hipLaunchKernelGGL(k_frontiers, dim3(1), dim3(HCS_ROOTS / 2), 0, c->stream, m.nodes, m.nelem - 1, m.roots);
+  rc = hip_check(c, hipGetLastError(), "k_frontiers");
+  if (!rc)
+    rc = hip_check(c, hipMemcpyAsync(m.roots_h, m.roots, sizeof(int32_t) * HCS_ROOTS, hipMemcpyDeviceToHost, c->stream),
+                   "memcpy");
+  return rc ? rc : hip_check(c, hipStreamSynchronize(c->stream), "sync");
+}
+
 static void free_mesh(Mesh& m) {
   for (void* p : {(void*)m.V, (void*)m.E, (void*)m.p, (void*)m.rec, (void*)m.box, (void*)m.nodes, (void*)m.nrm,
-                  (void*)m.leaf, (void*)m.boxL, (void*)m.qorder, (void*)m.fpl, (void*)m.wnodes})
+                  (void*)m.leaf, (void*)m.boxL, (void*)m.qorder, (void*)m.fpl, (void*)m.wnodes, (void*)m.cbox,
+                  (void*)m.roots})
     if (p) (void)hipFree(p);
   m = Mesh();
 }
 
-int build_plan(Ctx* c, int npairs, const int32_t* geoms, const hcs_step_opts* o, int tet_max, Plan& plan) {
+/* Frontier depth of each triangle / soft pair's items, chosen from sizes
+ * alone (a per-call step cannot measure first): subtrees of at most
+ * HCS_SUBTREE tets, as far as the launch's items stay within the budget (a
+ * common depth limit otherwise). */
+#define HCS_SUBTREE 256
+#define HCS_STATIC_DEPTH 6
+static void static_depths(Plan& plan) {
+  auto want = [](const EnvDesc& E) {
+    int d = 0;
+    if (E.kind == KIND_TRI || E.kind == KIND_SOFT)
+      while (d < HCS_STATIC_DEPTH && (E.ntA >> d) > HCS_SUBTREE) ++d;
+    return d;
+  };
+  int lim = HCS_STATIC_DEPTH;
+  for (; lim > 0; --lim) {
+    int64_t n = 0;
+    for (const EnvDesc& E : plan.envs) n += (int64_t)E.item_count << std::min(lim, want(E));
+    if (n <= HCS_ITEM_BUDGET) break;
+  }
+  for (EnvDesc& E : plan.envs) E.depth = std::min(lim, want(E));
+}
+
+int build_plan(Ctx* c, int npairs, const int32_t* geoms, const hcs_step_opts* o, int tet_max, Plan& plan,
+               PlanItems mode) {
   plan.envs.assign(npairs, EnvDesc{});
+  plan.blocks.clear();
   plan.items.clear();
   plan.xenv.clear();
   plan.ntx = 0;
   plan.pair_kind.assign(npairs, 0);
-  const int per_item = 64;
   for (int e = 0; e < npairs; ++e) {
     const int ha = geoms[2 * e], hb = geoms[2 * e + 1];
     if (ha < 0 || hb < 0 || ha >= (int)c->meshes.size() || hb >= (int)c->meshes.size() ||
@@ -1250,6 +1306,7 @@ int build_plan(Ctx* c, int npairs, const int32_t* geoms, const hcs_step_opts* o,
       const double den = m1 + m2;
       E.mu = den == 0.0 ? 0.0 : 2 * m1 * m2 / den;
     }
+    E.rootsA = hcs_gptr((const int32_t*)A.roots);
     int nq, chunk;
     if (B.kind == 3) {
       /* rigid half-space (plane geom): A's tets in Morton chunks */
@@ -1259,7 +1316,7 @@ int build_plan(Ctx* c, int npairs, const int32_t* geoms, const hcs_step_opts* o,
     } else if (E.b_soft) {
       E.kind = KIND_SOFT;
       nq = B.nelem;
-      chunk = per_item;
+      chunk = 64;
     } else if (B.nelem <= tet_max) {
       E.kind = KIND_TET;
       nq = A.nelem;
@@ -1270,14 +1327,38 @@ int build_plan(Ctx* c, int npairs, const int32_t* geoms, const hcs_step_opts* o,
     } else {
       E.kind = KIND_TRI;
       nq = B.nelem;
-      chunk = per_item;
+      chunk = 64;
     }
     plan.pair_kind[e] = E.kind;
-    E.item_first = (int)plan.items.size();
-    for (int q = 0; q < nq; q += chunk) plan.items.push_back(Item{e, q, std::min(chunk, nq - q), 0});
-    /* (root 0: the whole LBVH of A) */
-    E.item_count = (int)plan.items.size() - E.item_first;
+    const bool tree = E.kind == KIND_TRI || E.kind == KIND_SOFT;
+    E.cboxQ = hcs_gptr((const double*)(tree ? B.cbox : A.cbox));
+    E.boxB = hcs_gptr((const double*)(E.kind == KIND_TET ? B.cbox + 6 * (size_t)((B.nelem + 63) / 64) : nullptr));
+    E.item_count = (nq + chunk - 1) / chunk;
   }
+  if (mode != ITEMS_WHOLE) static_depths(plan);
+  int64_t total = 0;
+  for (int e = 0; e < npairs; ++e) {
+    EnvDesc& E = plan.envs[e];
+    const int chunks = E.item_count;
+    const int nq = E.kind == KIND_TRI || E.kind == KIND_SOFT ? E.nB : E.ntA;
+    E.item_first = (int)total;
+    if (mode == ITEMS_IMPLICIT) {
+      E.item_count = chunks << E.depth;
+      for (int i = 0; i < E.item_count; i += HCS_GEN_THREADS) plan.blocks.push_back(make_int2(e, i));
+    } else {
+      /* (root 0: the whole LBVH of A) */
+      const int32_t* roots = c->meshes[geoms[2 * e]].roots_h + (1 << E.depth);
+      for (int k = 0; k < chunks; ++k)
+        for (int s = 0; s < (1 << E.depth); ++s) {
+          const int32_t root = E.depth ? roots[s] : 0;
+          if (root != HCS_WNONE) plan.items.push_back(Item{e, 64 * k, std::min(64, nq - 64 * k), root});
+        }
+      E.item_count = (int)plan.items.size() - E.item_first;
+    }
+    total += E.item_count;
+    if (total > INT32_MAX - 64) return set_err(c, HCS_ERR_LIMIT, "too many work items");
+  }
+  plan.nitems = (int)total;
   return HCS_OK;
 }
 
@@ -1317,8 +1398,11 @@ int hcs_create(hcs_ctx** out, int device) {
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, device) == hipSuccess) c->num_cu = prop.multiProcessorCount;
   if (c->num_cu <= 0) c->num_cu = 256;
-  if (scratch_setup(c) != HCS_OK) {
+  if (scratch_setup(c) != HCS_OK || pinned(c, c->pin_up, c->pin_up_bytes, 64 << 10) != HCS_OK ||
+      pinned(c, c->pin_down, c->pin_down_bytes, 64 << 10) != HCS_OK) {
     g_create_err = c->err;
+    for (void* p : {c->pin_up, c->pin_down})
+      if (p) (void)hipHostFree(p);
     (void)hipStreamDestroy(c->stream);
     delete h;
     return HCS_ERR_HIP;
@@ -1343,6 +1427,8 @@ int hcs_destroy(hcs_ctx* h) {
   for (DBuf* b : {&T.mask, &T.k64, &T.kp, &T.idx, &T.cnt, &T.nfan, &T.fan_off, &T.tmp, &T.tris, &T.surf, &T.scnt, &T.soff,
                   &T.P, &T.E, &T.taxel, &T.val, &T.hits, &T.area, &T.acc, &T.pair_u})
     if (b->ptr) (void)hipFree(b->ptr);
+  for (void* p : {c->pin_up, c->pin_down})
+    if (p) (void)hipHostFree(p);
   (void)hipStreamDestroy(c->stream);
   delete h;
   return HCS_OK;
@@ -1389,6 +1475,7 @@ static int make_soft(Ctx* c, const double* V, int32_t nv, const int32_t* T, int3
     rc = hip_check(c, hipGetLastError(), "k_tet_precompute");
   }
   if (rc == HCS_OK) rc = build_bvh(c, m);
+  if (rc == HCS_OK) rc = build_item_tables(c, m);
   if (rc != HCS_OK) {
     (void)hipStreamSynchronize(c->stream);
     free_mesh(m);
@@ -1449,6 +1536,15 @@ static int make_rigid(Ctx* c, const double* V, int32_t nv, const int32_t* F, int
   if (rc == HCS_OK) {
     hipLaunchKernelGGL(k_tri_normals, dim3((ntri + 127) / 128), dim3(128), 0, c->stream, m.V, m.E, ntri, m.nrm);
     rc = hip_check(c, hipGetLastError(), "k_tri_normals");
+  }
+  double vbox[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+  if (rc == HCS_OK) rc = build_chunk_boxes(c, m, 3, m.qorder);
+  if (rc == HCS_OK) {
+    for (int32_t v = 0; v < nv; ++v)
+      for (int k = 0; k < 3; ++k)
+        vbox[k] = std::fmin(vbox[k], V[3 * (size_t)v + k]), vbox[3 + k] = std::fmax(vbox[3 + k], V[3 * (size_t)v + k]);
+    rc = hip_check(c, hipMemcpyAsync(m.cbox + 6 * (size_t)((ntri + 63) / 64), vbox, sizeof vbox, hipMemcpyHostToDevice,
+                                     c->stream), "upload");
   }
   if (rc == HCS_OK) rc = hip_check(c, hipStreamSynchronize(c->stream), "sync");
   if (rc != HCS_OK) free_mesh(m);
@@ -1554,8 +1650,9 @@ int hcs_mesh_tet_records(hcs_ctx* h, int32_t handle, double* out) {
 
 namespace hcs {
 
-/* Uploads plan and state of npairs pairs into the context scratch. */
-int stage_pairs(Ctx* c, int npairs, const hcs_pair_in* in, const hcs_step_opts* opts, Plan& plan, DBuf* dst) {
+/* Uploads plan and state of npairs pairs into the context scratch (tangent
+ * pass). */
+int stage_pairs(Ctx* c, int npairs, const hcs_pair_in* in, const hcs_step_opts* opts, Plan& plan) {
   HCHK(c, hipSetDevice(c->device));
   std::vector<int32_t> geoms(2 * (size_t)npairs);
   std::vector<double> state((size_t)HCS_STATE * npairs);
@@ -1570,9 +1667,7 @@ int stage_pairs(Ctx* c, int npairs, const hcs_pair_in* in, const hcs_step_opts* 
   int rc = build_plan(c, npairs, geoms.data(), opts, c->tet_mode_max_tris, plan);
   if (rc) return rc;
   const int nitems = (int)plan.items.size();
-  DBuf& envs = dst ? dst[0] : c->d_envs;
-  DBuf& st = dst ? dst[1] : c->d_state;
-  DBuf& items = dst ? dst[2] : c->d_items;
+  DBuf &envs = c->d_envs, &st = c->d_state, &items = c->d_items;
   if ((rc = ensure(c, envs, sizeof(EnvDesc) * npairs)) || (rc = ensure(c, st, state.size() * 8)) ||
       (rc = ensure(c, items, sizeof(Item) * std::max(1, nitems))))
     return rc;
@@ -1580,7 +1675,6 @@ int stage_pairs(Ctx* c, int npairs, const hcs_pair_in* in, const hcs_step_opts* 
   HCHK(c, hipMemcpyAsync(st.ptr, state.data(), state.size() * 8, hipMemcpyHostToDevice, c->stream));
   if (nitems)
     HCHK(c, hipMemcpyAsync(items.ptr, plan.items.data(), sizeof(Item) * nitems, hipMemcpyHostToDevice, c->stream));
-  c->last_geoms = geoms;
   return HCS_OK;
 }
 
@@ -1593,13 +1687,23 @@ int clip_grid_for(const Ctx* c, int64_t cap) {
  * pipeline over npairs pairs (keys: candidate-key mode). */
 static int run_pairs(Ctx* c, int npairs, const hcs_pair_in* in, const hcs_step_opts* opts, hcs_pair_out* out,
                      hcs_faces* faces, int64_t* keys, int64_t key_cap, int64_t* key_count) {
+  HCHK(c, hipSetDevice(c->device));
   Plan plan;
-  int rc = stage_pairs(c, npairs, in, opts, plan);
+  std::vector<int32_t> geoms(2 * (size_t)npairs);
+  for (int e = 0; e < npairs; ++e) geoms[2 * e] = in[e].geom_a, geoms[2 * e + 1] = in[e].geom_b;
+  int rc = build_plan(c, npairs, geoms.data(), opts, c->tet_mode_max_tris, plan, ITEMS_IMPLICIT);
   if (rc) return rc;
-  const int nitems = (int)plan.items.size();
   Pipe& P = c->pipe;
-  if ((rc = pipe_reserve(c, P, nitems, npairs, std::max<int64_t>(P.cap, 4096), 0))) return rc;
-  if ((rc = pipe_plan(c, P, (const EnvDesc*)c->d_envs.ptr, (const Item*)c->d_items.ptr, plan))) return rc;
+  CallBlob blob;
+  const size_t tail_at = sizeof(PairOut) * npairs;
+  if ((rc = pinned(c, c->pin_up, c->pin_up_bytes, call_blob_bytes(plan, blob))) ||
+      (rc = pinned(c, c->pin_down, c->pin_down_bytes, tail_at + sizeof(CallTail))) ||
+      (rc = call_reserve(c, P, plan, blob, std::max<int64_t>(P.cap, 4096))))
+    return rc;
+  call_blob_fill(plan, in, blob, (char*)c->pin_up);
+  blob.src = c->pin_up;
+  PairOut* res = (PairOut*)c->pin_down;
+  CallTail* tail = (CallTail*)((char*)c->pin_down + tail_at);
   if ((rc = ensure(c, c->d_face_cnt, 64)) || (rc = ensure(c, c->d_poly_cnt, 64)) || (rc = ensure(c, c->d_cand_cnt, 64)))
     return rc;
   const bool keep = opts && opts->keep_polygons && !keys;
@@ -1617,14 +1721,10 @@ static int run_pairs(Ctx* c, int npairs, const hcs_pair_in* in, const hcs_step_o
         (rc = ensure(c, c->d_poly_key, sizeof(int64_t) * 3 * poly_cap)))
       return rc;
   }
-  std::vector<PairOut> res(npairs);
   unsigned long long nface = 0, ncand = 0, npoly = 0, nsurv = 0;
+  int err = 0;
   for (int attempt = 0; attempt < 3; ++attempt) {
-    HCHK(c, hipMemsetAsync(c->d_face_cnt.ptr, 0, 64, c->stream));
-    HCHK(c, hipMemsetAsync(c->d_poly_cnt.ptr, 0, 64, c->stream));
-    HCHK(c, hipMemsetAsync(c->d_cand_cnt.ptr, 0, 64, c->stream));
-    QueryArgs a = pipe_args(P, (const EnvDesc*)c->d_envs.ptr, (const double*)c->d_state.ptr,
-                            (const Item*)c->d_items.ptr, nitems, false);
+    QueryArgs a = call_args(P, plan, blob);
     if (want_faces) {
       a.face_rec = (double*)c->d_face_rec.ptr;
       a.face_key = (int64_t*)c->d_face_key.ptr;
@@ -1642,18 +1742,19 @@ static int run_pairs(Ctx* c, int npairs, const hcs_pair_in* in, const hcs_step_o
       a.cand_cnt = (unsigned long long*)c->d_cand_cnt.ptr;
       a.cand_cap = key_cap;
     }
-    pipe_enqueue(c, P, a, npairs, nitems, clip_grid_for(c, P.cap), 0, nullptr, nullptr, keys != nullptr, 0);
+    unsigned* const counters[] = {(unsigned*)c->d_face_cnt.ptr, (unsigned*)c->d_poly_cnt.ptr,
+                                  (unsigned*)c->d_cand_cnt.ptr};
+    if ((rc = call_enqueue(c, P, a, plan, blob, counters, 3, keys != nullptr, res, tail))) return rc;
     HCHK(c, hipGetLastError());
-    HCHK(c, hipMemcpyAsync(&nsurv, P.surv_cnt.ptr, 8, hipMemcpyDeviceToHost, c->stream));
-    HCHK(c, hipMemcpyAsync(&npoly, c->d_poly_cnt.ptr, 8, hipMemcpyDeviceToHost, c->stream));
-    HCHK(c, hipMemcpyAsync(&nface, c->d_face_cnt.ptr, 8, hipMemcpyDeviceToHost, c->stream));
-    HCHK(c, hipMemcpyAsync(&ncand, c->d_cand_cnt.ptr, 8, hipMemcpyDeviceToHost, c->stream));
-    if (!keys)
-      HCHK(c, hipMemcpyAsync(res.data(), P.out.ptr, sizeof(PairOut) * npairs, hipMemcpyDeviceToHost, c->stream));
+    if (keys) {
+      HCHK(c, hipMemcpyAsync(&ncand, c->d_cand_cnt.ptr, 8, hipMemcpyDeviceToHost, c->stream));
+      HCHK(c, hipMemcpyAsync(&err, P.err.ptr, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    }
     HCHK(c, hipStreamSynchronize(c->stream));
+    if (!keys) nsurv = tail->nsurv, npoly = tail->npoly, nface = tail->nface, err = tail->err;
     bool again = false;
     if (!keys && (int64_t)nsurv > P.cap) {
-      if ((rc = pipe_reserve(c, P, nitems, npairs, (int64_t)nsurv + (int64_t)nsurv / 4 + 1024, 0))) return rc;
+      if ((rc = call_reserve(c, P, plan, blob, (int64_t)nsurv + (int64_t)nsurv / 4 + 1024))) return rc;
       again = true;
     }
     if (keep && (int64_t)npoly > poly_cap) {
@@ -1679,9 +1780,6 @@ static int run_pairs(Ctx* c, int npairs, const hcs_pair_in* in, const hcs_step_o
   } else if (faces) {
     faces->count = 0;
   }
-  int err = 0;
-  HCHK(c, hipMemcpyAsync(&err, P.err.ptr, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  HCHK(c, hipStreamSynchronize(c->stream));
   if (keys) {
     const int64_t nw = std::min<int64_t>((int64_t)ncand, key_cap);
     if (nw > 0) {
@@ -1695,9 +1793,10 @@ static int run_pairs(Ctx* c, int npairs, const hcs_pair_in* in, const hcs_step_o
       return set_err(c, HCS_ERR_CAPACITY, "key buffer too small: " + std::to_string(ncand) + " keys");
     return HCS_OK;
   }
-  if (out) std::memcpy(out, res.data(), sizeof(PairOut) * npairs);
+  if (out) std::memcpy(out, res, sizeof(PairOut) * npairs);
   if (keep) {
     c->last_valid = 1;
+    c->last_geoms = geoms;
     c->last_pairs.assign(in, in + npairs);
   }
   if (err) return set_err(c, HCS_ERR_LIMIT, "traversal stack overflow");

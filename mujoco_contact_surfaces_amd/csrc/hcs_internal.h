@@ -30,6 +30,9 @@ struct Mesh {
   int32_t* qorder = nullptr; /* rigid: triangles in Morton order of their centroids */
   double* boxL = nullptr;   /* their AABBs in that order */
   double* nrm = nullptr;
+  double* cbox = nullptr;    /* boxes of the chunks of 64 elements in leaf / query order, then (rigid) of the vertices */
+  int32_t* roots = nullptr;  /* soft: LBVH frontiers (HCS_ROOTS) */
+  int32_t roots_h[HCS_ROOTS] = {}; /* their host copy */
 };
 
 /* Grow-only device buffer.  A fixed buffer is a view of memory the library
@@ -48,7 +51,11 @@ struct Pipe {
   DBuf counter /* [0..7] work counters, [8..15] live items per queue */, surv, surv_cnt, ncand, nsurv, off, scan_tmp,
       contrib, out, err, xf, ibox /* item boxes, in the work order when ordered */, live, live_item, qseg, xtri, xenv,
       order, item_o /* the items in the work order (ordered plans) */, part /* per-slice sums */,
-      rtab /* reduction waves (pair, slice, slices, first partial) */, ptab /* per pair (first partial, slices) */;
+      rtab /* reduction waves (pair, slice, slices, first partial) */, ptab /* per pair (first partial, slices) */,
+      /* per-call steps: the uploaded descriptors, state and tables; kept
+       * items per block and their lane masks, and the items of the first
+       * cull; first live item per pair */
+      blob, gen_cnt, gen_mask, gen_item, pair_lo;
   int64_t cap = 0;
   size_t scan_bytes = 0;
   std::vector<int> qseg_host; /* host copy of the queue segments (the upload source) */
@@ -67,10 +74,12 @@ int set_err(Ctx* c, int code, const std::string& msg);
 int hip_check(Ctx* c, hipError_t e, const char* what);
 int ensure(Ctx* c, DBuf& b, size_t bytes);
 
-/* Per-call plan: env descriptors and items for a set of pairs. */
+/* Env descriptors and items for a set of pairs. */
 struct Plan {
   std::vector<EnvDesc> envs;
-  std::vector<Item> items;
+  int nitems = 0;
+  std::vector<Item> items;  /* empty in an implicit plan: the items are enumerated on the device */
+  std::vector<int2> blocks; /* implicit plan: (pair, first item of the pair) per block of HCS_GEN_THREADS items */
   std::vector<int> pair_kind;
   std::vector<int> xenv; /* pairs in tet-query mode */
   int64_t ntx = 0;       /* their triangles in total */
@@ -102,6 +111,10 @@ struct Ctx {
   std::vector<hcs_pair_in> last_pairs;
   std::vector<int32_t> last_geoms; /* per pair: geom_a, geom_b */
   int tet_mode_max_tris = 64;
+  /* pinned host memory of the per-call steps, mapped on the device: the
+   * uploaded blob, and the results that the last kernel writes */
+  void *pin_up = nullptr, *pin_down = nullptr;
+  size_t pin_up_bytes = 0, pin_down_bytes = 0;
   /* device address and size of the static scratch array on this device */
   void* scratch = nullptr;
   size_t scratch_bytes = 0;
@@ -111,8 +124,46 @@ struct Ctx {
 
 /* Builds env descriptors and work items (chunks of 64 queries, one per
  * lane of the candidate kernel's wave).  Returns HCS_OK or an error. */
+enum PlanItems {
+  ITEMS_WHOLE,    /* one item per chunk over A's whole tree (measured splitting follows) */
+  ITEMS_SPLIT,    /* over the static frontiers of static_depths() */
+  ITEMS_IMPLICIT, /* the same items, enumerated on the device */
+};
 int build_plan(Ctx* c, int npairs, const int32_t* geoms, const hcs_step_opts* o, int tet_mode_max_tris,
-               Plan& plan);
+               Plan& plan, PlanItems mode = ITEMS_WHOLE);
+
+/* Per-call steps: threads (items) per block of the item enumeration; items
+ * that a split may lead to in all; sizes of the tables that follow from a
+ * plan (blocks of both culls, places of live items, reduction slices). */
+#define HCS_GEN_THREADS 256
+#define HCS_ITEM_BUDGET 65536
+#define HCS_EXPAND_BUDGET 16384
+struct CallSizes {
+  size_t blocks1, blocks2, items, live;
+  int slices;
+};
+CallSizes call_sizes(const Plan& plan);
+
+/* What a per-call step reports beside the pairs' results. */
+struct CallTail {
+  unsigned long long nsurv, npoly, nface, ncand;
+  int err, pad;
+};
+/* A per-call step (hcs_contact_step and its no-allocation form): the host
+ * image of its uploaded blob (descriptors, state, block table, tet-query
+ * pairs) and the offsets in it. */
+struct CallBlob {
+  size_t state, blocks, xenv, bytes;
+  const void* src = nullptr; /* device-readable: pinned host memory, or the device blob itself once uploaded */
+};
+size_t call_blob_bytes(const Plan& plan, CallBlob& b);
+void call_blob_fill(const Plan& plan, const hcs_pair_in* in, const CallBlob& b, char* dst);
+/* Enqueues the step; the last kernel writes out[0..npairs) and *tail (device
+ * or mapped host memory).  keys: candidate keys only, nothing is written. */
+int call_enqueue(Ctx* c, Pipe& p, QueryArgs& a, const Plan& plan, const CallBlob& b, unsigned* const* counters,
+                 int ncounters, bool keys, PairOut* out, CallTail* tail);
+int call_reserve(Ctx* c, Pipe& p, const Plan& plan, const CallBlob& b, int64_t cap);
+QueryArgs call_args(const Pipe& p, const Plan& plan, const CallBlob& b);
 
 int pipe_reserve(Ctx* c, Pipe& p, int nitems, int npairs, int64_t cap, int ndir);
 QueryArgs pipe_args(const Pipe& p, const EnvDesc* envs, const double* state, const Item* items, int nitems,
@@ -135,13 +186,13 @@ int split_roots(Ctx* c, const EnvDesc* envs, const Item* items, const std::vecto
 void pipe_free(Pipe& p);
 /* mode: CandMode */
 void launch_cand(hipStream_t s, const QueryArgs& a, int grid, int mode);
+void launch_clip(Ctx* c, const Pipe& p, const QueryArgs& a, int clip_grid);
+int pinned(Ctx* c, void*& p, size_t& have, size_t bytes);
 void launch_clip_reduce(Ctx* c, Pipe& p, const QueryArgs& a, int npairs, int clip_grid, hipEvent_t e_clip,
                         hipEvent_t e_reduce);
 /* Builds the plan of npairs pairs and uploads env descriptors, state and
- * items into the context's scratch buffers, or into dst[0..2] (envs, state,
- * items) when given. */
-int stage_pairs(Ctx* c, int npairs, const hcs_pair_in* in, const hcs_step_opts* opts, Plan& plan,
-                DBuf* dst = nullptr);
+ * items into the context's scratch buffers (tangent pass). */
+int stage_pairs(Ctx* c, int npairs, const hcs_pair_in* in, const hcs_step_opts* opts, Plan& plan);
 /* The per-pair reduction waves of a plan (see pipe_plan). */
 void reduction_slices(const Plan& plan, std::vector<int4>& rt, std::vector<int2>& pt);
 /* The static scratch array of the no-allocation entry point on the

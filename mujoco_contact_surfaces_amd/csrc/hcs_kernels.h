@@ -141,9 +141,21 @@ struct EnvDesc {
   int32_t a_is_M, repr, apply, b_soft;
   double mu, dstar, dt;
   int32_t item_first, item_count;
+  const HCS_GPTR double* cboxQ; /* boxes of the chunks of 64 queries, in their own frame (6 doubles each) */
+  const HCS_GPTR double* boxB;  /* tet queries: B's vertex box */
+  const HCS_GPTR int32_t* rootsA; /* A's LBVH frontiers (HCS_ROOTS) */
+  int32_t depth;    /* triangle / soft queries: items over the frontier of depth `depth` */
+  int32_t pad;
   int64_t xtri_off; /* tet-query mode: first of this pair's triangles in the
                        per-step moved-triangle buffer (HCS_XTRI doubles each) */
 };
+
+/* The frontiers of an LBVH below its root as a heap: entries [2^d, 2^(d+1))
+ * are the nodes at depth d <= HCS_ROOT_DEPTH (the code of Node::c), a leaf
+ * reached earlier standing once at every deeper level, HCS_WNONE elsewhere.
+ * The subtrees of one depth hold each leaf exactly once. */
+#define HCS_ROOT_DEPTH 10
+#define HCS_ROOTS (2 << HCS_ROOT_DEPTH)
 
 /* A work item: queries first .. first+count-1 of pair env.  Triangle and
  * soft queries walk A's LBVH from node root (0: the whole tree; < 0: the
@@ -192,13 +204,16 @@ struct QueryArgs {
   unsigned* item_nsurv;
   /* items whose static boxes overlap this step, in nqueues queues (the
    * items of pair e go to queue e % nqueues; queue x holds live_cnt[x]
-   * items from live + qseg[x]); nullptr: all items, one queue */
+   * items from live + qseg[x]); live_cnt nullptr: all items, one queue; live
+   * nullptr: the live items are numbered by their place (items = live_item) */
   const int* live;
   const unsigned* live_cnt;
   const int* qseg;
   int32_t nqueues;
   const int4* live_item; /* the live items' Item records, same order as live */
   const double* xtri;    /* per-step moved triangles of tet-query pairs */
+  int32_t exact_slots;   /* survivor slots reserved as needed (one atomic per
+                            flush, no padding) instead of per wave in chunks */
   int32_t kinds;         /* bit k set: some pair is of EnvKind k; a launch
                             whose pairs share one kind runs a kernel built
                             for it (0: not known, the general kernel) */

@@ -6,9 +6,8 @@
  * hipMalloc).
  *
  * Every device buffer of the step (env descriptors, state, work items, the
- * pipeline's counters, item boxes, live lists, survivors, contributions,
- * scan storage, reduction partials and per-pair outputs) is a slice of one
- * file-scope array, `scratch`, of HCS_SCRATCH_BYTES on each device.  Its
+ * pipeline's counters, survivors, contributions, scan storage, reduction
+ * partials and per-pair outputs) is a slice of one file-scope array, `scratch`, of HCS_SCRATCH_BYTES on each device.  Its
  * device address comes from hipGetSymbolAddress, taken once per device
  * with that device current (hcs_create calls scratch_setup); host code only
  * ever uses that address.  The slices are laid out per call from the call's
@@ -32,11 +31,14 @@
 #include "hcs_internal.h"
 #include "hcs_prim.h"
 
-/* 64 MiB per device: room for about 690k survivors of the exact
- * rejections after the per-call tables of a few hundred pairs. */
+/* What a call may use: 64 MiB per device, room for about 690k survivors of
+ * the exact rejections after the per-call tables of a few hundred pairs.  The
+ * array holds a little more: the work items of the engine's own splitting (at
+ * most its item budget, 44 bytes each) are not the caller's to pay for. */
 #define HCS_SCRATCH_BYTES (64ull << 20)
+#define HCS_SCRATCH_EXTRA (4ull << 20)
 
-static __device__ __align__(256) unsigned char scratch[HCS_SCRATCH_BYTES];
+static __device__ __align__(256) unsigned char scratch[HCS_SCRATCH_BYTES + HCS_SCRATCH_EXTRA];
 
 namespace hcs {
 
@@ -59,7 +61,7 @@ int scratch_setup(Ctx* c) {
     g_scratch_ptr[c->device] = p;
   }
   c->scratch = g_scratch_ptr[c->device];
-  c->scratch_bytes = HCS_SCRATCH_BYTES;
+  c->scratch_bytes = HCS_SCRATCH_BYTES + HCS_SCRATCH_EXTRA;
   return HCS_OK;
 }
 
@@ -85,6 +87,35 @@ struct Carver {
   size_t left() const { return size > ((used + 255) & ~(size_t)255) ? size - ((used + 255) & ~(size_t)255) : 0; }
 };
 
+/* Survivors a call may have, by a fixed price list: bytes per pair, work item
+ * (64 queries, unsplit), moved triangle and reduction slice (8 items, at most
+ * 64 per pair), slices of 256 bytes, the rest 96 bytes per survivor.  Which
+ * calls fit is thus a matter of their sizes, whatever tables the engine keeps
+ * for them.  Negative: the tables alone do not fit. */
+int64_t admitted_survivors(const Plan& plan) {
+  const size_t np = plan.envs.size();
+  size_t ni = 0, slices = 0;
+  for (const EnvDesc& E : plan.envs) {
+    const size_t n = (size_t)(E.item_count >> E.depth);
+    ni += n;
+    slices += std::max<size_t>(1, std::min<size_t>(64, (n + 7) / 8));
+  }
+  ni = std::max<size_t>(1, ni);
+  size_t used = 0;
+  auto take = [&](size_t bytes) { used = ((used + 255) & ~(size_t)255) + std::max<size_t>(bytes, 8); };
+  for (size_t per : {184, 288}) take(per * np);
+  take(16 * ni);
+  for (int k = 0; k < 3; ++k) take(64);
+  take(96 * np), take(4 * ni), take(4 * (ni + 1)), take(4 * (ni + 1)), take(128 * np);
+  take(scan_temp_bytes((long long)ni + 1));
+  take(96 * ni), take(4 * ni), take(16 * ni), take(36);
+  take(144 * (size_t)std::max<int64_t>(1, plan.ntx)), take(4 * std::max<size_t>(1, plan.xenv.size())), take(8);
+  take(16 * slices), take(8 * np), take(672 * slices);
+  used = (used + 255) & ~(size_t)255;
+  if (used + 512 > HCS_SCRATCH_BYTES) return -1;
+  return (int64_t)((HCS_SCRATCH_BYTES - used - 512) / (sizeof(int4) + sizeof(Contrib)));
+}
+
 }  // namespace
 
 }  // namespace hcs
@@ -105,70 +136,80 @@ extern "C" int hcs_contact_step_noalloc(hcs_ctx* h, int32_t npairs, const hcs_pa
   std::vector<int32_t> geoms(2 * (size_t)npairs);
   for (int e = 0; e < npairs; ++e) geoms[2 * e] = in[e].geom_a, geoms[2 * e + 1] = in[e].geom_b;
   Plan plan;
-  if ((rc = build_plan(c, npairs, geoms.data(), opts, c->tet_mode_max_tris, plan))) return rc;
-  const size_t ni = std::max<size_t>(1, plan.items.size());
-  std::vector<int4> rt;
-  std::vector<int2> pt;
-  reduction_slices(plan, rt, pt);
-  const size_t scan_bytes = scan_temp_bytes((long long)ni + 1);
+  if ((rc = build_plan(c, npairs, geoms.data(), opts, c->tet_mode_max_tris, plan, ITEMS_IMPLICIT))) return rc;
+  const int64_t cap = admitted_survivors(plan);
+  if (cap < 4096) {
+    size_t items = 0;
+    for (const EnvDesc& E : plan.envs) items += (size_t)(E.item_count >> E.depth);
+    return set_err(c, HCS_ERR_CAPACITY,
+                   "hcs_contact_step_noalloc: " + std::to_string(npairs) + " pairs and " + std::to_string(items) +
+                       " work items do not fit the " + std::to_string(HCS_SCRATCH_BYTES >> 20) + " MiB scratch array");
+  }
+  CallBlob blob;
+  const CallSizes z = call_sizes(plan);
+  const size_t np = npairs, nb = z.blocks1 + z.blocks2;
+  const size_t blob_bytes = call_blob_bytes(plan, blob), out_bytes = sizeof(PairOut) * np + sizeof(CallTail);
   Carver cv{(unsigned char*)c->scratch, c->scratch_bytes};
-  DBuf staged[3];
   Pipe P;
-  cv.take(staged[0], sizeof(EnvDesc) * npairs);
-  cv.take(staged[1], sizeof(double) * HCS_STATE * npairs);
-  cv.take(staged[2], sizeof(Item) * ni);
+  cv.take(P.blob, blob_bytes);
   cv.take(P.counter, 64);
   cv.take(P.surv_cnt, 64);
   cv.take(P.err, 64);
-  cv.take(P.xf, sizeof(double) * 12 * npairs);
-  cv.take(P.ncand, sizeof(int) * ni);
-  cv.take(P.nsurv, sizeof(unsigned) * (ni + 1));
-  cv.take(P.off, sizeof(unsigned) * (ni + 1));
-  cv.take(P.out, sizeof(PairOut) * npairs);
-  cv.take(P.scan_tmp, std::max<size_t>(scan_bytes, 8));
-  cv.take(P.ibox, sizeof(double) * 12 * ni);
-  cv.take(P.live, sizeof(int) * ni);
-  cv.take(P.live_item, sizeof(Item) * ni);
-  cv.take(P.qseg, sizeof(int) * (HCS_QUEUES + 1));
+  cv.take(P.xf, sizeof(double) * 12 * np);
   cv.take(P.xtri, sizeof(double) * HCS_XTRI * std::max<int64_t>(1, plan.ntx));
-  cv.take(P.xenv, sizeof(int) * std::max<size_t>(1, plan.xenv.size()));
-  cv.take(P.order, 8);
-  cv.take(P.rtab, sizeof(int4) * std::max<size_t>(1, rt.size()));
-  cv.take(P.ptab, sizeof(int2) * pt.size());
-  cv.take(P.part, sizeof(RedPart) * HCS_MAXDIR * std::max<size_t>(1, rt.size()));
-  /* the rest: survivors (16 B) and their contributions (80 B), less the
-   * alignment of the two slices */
-  const int64_t cap = (int64_t)(cv.left() > 512 ? (cv.left() - 512) / (sizeof(int4) + sizeof(Contrib)) : 0);
-  if (!cv.ok || cap < 4096)
-    return set_err(c, HCS_ERR_CAPACITY,
-                   "hcs_contact_step_noalloc: " + std::to_string(npairs) + " pairs and " + std::to_string(ni) +
-                       " work items do not fit the " + std::to_string(c->scratch_bytes >> 20) + " MiB scratch array");
+  cv.take(P.gen_cnt, sizeof(unsigned) * (nb + 1));
+  cv.take(P.gen_mask, sizeof(unsigned long long) * nb * (HCS_GEN_THREADS / 64));
+  cv.take(P.gen_item, sizeof(int4) * z.items);
+  cv.take(P.pair_lo, sizeof(int) * (np + 1));
+  cv.take(P.live_item, sizeof(int4) * z.live);
+  cv.take(P.ncand, sizeof(int) * z.live);
+  cv.take(P.nsurv, sizeof(unsigned) * (z.live + 1));
+  cv.take(P.off, sizeof(unsigned) * (z.live + 1));
+  cv.take(P.scan_tmp, scan_temp_bytes((long long)z.live + 1));
+  cv.take(P.part, sizeof(RedPart) * np * z.slices);
+  cv.take(P.out, out_bytes);
   cv.take(P.surv, sizeof(int4) * cap);
   cv.take(P.contrib, sizeof(Contrib) * cap);
   if (!cv.ok) return set_err(c, HCS_ERR_CAPACITY, "hcs_contact_step_noalloc: scratch layout");
-  if ((rc = stage_pairs(c, npairs, in, opts, plan, staged))) return rc;
-  const int nitems = (int)plan.items.size();
   /* every request below fits its slice (ensure() on a fixed slice never
    * allocates and reports anything larger as HCS_ERR_CAPACITY) */
-  if ((rc = pipe_reserve(c, P, nitems, npairs, cap, 0))) return rc;
-  if ((rc = pipe_plan(c, P, (const EnvDesc*)staged[0].ptr, (const Item*)staged[2].ptr, plan))) return rc;
-  QueryArgs a = pipe_args(P, (const EnvDesc*)staged[0].ptr, (const double*)staged[1].ptr, (const Item*)staged[2].ptr,
-                          nitems, false);
-  pipe_enqueue(c, P, a, npairs, nitems, clip_grid_for(c, P.cap), 0, nullptr, nullptr, false, 0);
+  if ((rc = call_reserve(c, P, plan, blob, cap))) return rc;
+  /* the blob goes through the context's pinned memory as long as that holds
+   * it (it is not grown here), else by a copy from ordinary memory */
+  std::vector<char> image;
+  if (blob_bytes <= c->pin_up_bytes) {
+    call_blob_fill(plan, in, blob, (char*)c->pin_up);
+    blob.src = c->pin_up;
+  } else {
+    image.resize(blob_bytes);
+    call_blob_fill(plan, in, blob, image.data());
+    rc = hip_check(c, hipMemcpyAsync(P.blob.ptr, image.data(), blob_bytes, hipMemcpyHostToDevice, c->stream), "upload");
+    if (rc) return rc;
+    blob.src = P.blob.ptr;
+  }
+  const bool direct = out_bytes <= c->pin_down_bytes;
+  char* down = direct ? (char*)c->pin_down : (char*)P.out.ptr;
+  CallTail tail{};
+  QueryArgs a = call_args(P, plan, blob);
+  if ((rc = call_enqueue(c, P, a, plan, blob, nullptr, 0, false, (PairOut*)down,
+                         (CallTail*)(down + sizeof(PairOut) * np))))
+    return rc;
   rc = hip_check(c, hipGetLastError(), "noalloc step");
-  unsigned long long nsurv = 0;
-  int err = 0;
-  if (!rc) rc = hip_check(c, hipMemcpyAsync(&nsurv, P.surv_cnt.ptr, 8, hipMemcpyDeviceToHost, c->stream), "dl");
-  if (!rc) rc = hip_check(c, hipMemcpyAsync(&err, P.err.ptr, sizeof(int), hipMemcpyDeviceToHost, c->stream), "dl");
   static_assert(sizeof(hcs_pair_out) == sizeof(PairOut), "pair_out layout");
-  if (!rc)
-    rc = hip_check(c, hipMemcpyAsync(out, P.out.ptr, sizeof(PairOut) * npairs, hipMemcpyDeviceToHost, c->stream),
+  if (!rc && !direct)
+    rc = hip_check(c, hipMemcpyAsync(out, down, sizeof(PairOut) * np, hipMemcpyDeviceToHost, c->stream), "dl");
+  if (!rc && !direct)
+    rc = hip_check(c, hipMemcpyAsync(&tail, down + sizeof(PairOut) * np, sizeof tail, hipMemcpyDeviceToHost, c->stream),
                    "dl");
   if (!rc) rc = hip_check(c, hipStreamSynchronize(c->stream), "sync");
   if (rc) return rc;
-  if (err) return set_err(c, HCS_ERR_LIMIT, "traversal stack overflow");
-  if ((int64_t)nsurv > P.cap)
-    return set_err(c, HCS_ERR_CAPACITY, "hcs_contact_step_noalloc: " + std::to_string(nsurv) +
+  if (direct) {
+    std::memcpy(out, down, sizeof(PairOut) * np);
+    std::memcpy(&tail, down + sizeof(PairOut) * np, sizeof tail);
+  }
+  if (tail.err) return set_err(c, HCS_ERR_LIMIT, "traversal stack overflow");
+  if ((int64_t)tail.nsurv > P.cap)
+    return set_err(c, HCS_ERR_CAPACITY, "hcs_contact_step_noalloc: " + std::to_string(tail.nsurv) +
                                             " survivors exceed the scratch array's room for " +
                                             std::to_string(P.cap));
   return HCS_OK;

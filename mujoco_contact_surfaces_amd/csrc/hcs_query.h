@@ -761,6 +761,32 @@ __device__ inline bool box_may_meet_plane(const double* X, const double* Q) {
   return !(fabs(dist) > rad + (1e-9 * mag + 1e-300));
 }
 
+/* The rigid triangles of one tet-query pair moved into A's frame (vertices by
+ * xform, unit normal by rot, and their AABB), strided over the block: the same
+ * arithmetic the candidate and clip stages use. */
+__device__ inline void move_triangles(const EnvDesc& E, const double* X, double* xtri, int threads) {
+  for (int t = threadIdx.x; t < E.nB; t += threads) {
+    double* o = xtri + HCS_XTRI * (size_t)(E.xtri_off + t);
+    const HCS_GPTR int32_t* f = E.FB + 3 * (size_t)t;
+    double lo[3], hi[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      double y[3];
+      xform(X, hcs_plain(E.VB + 3 * (size_t)f[i]), y);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        o[3 * i + c] = y[c];
+        lo[c] = i == 0 ? y[c] : fmin(lo[c], y[c]);
+        hi[c] = i == 0 ? y[c] : fmax(hi[c], y[c]);
+      }
+    }
+    double nS[3];
+    rot(X, hcs_plain(E.nrmB + 3 * (size_t)t), nS);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) o[9 + c] = nS[c], o[12 + c] = lo[c], o[15 + c] = hi[c];
+  }
+}
+
 /* ===================================================================
  * k_cand: candidate generation, exact cheap tests, survivor compaction
  * =================================================================== */
@@ -1113,12 +1139,14 @@ __device__ inline void run_cand(CandLds& L, const QueryArgs& A, int it, const It
         const int take = q2n >= 64 ? 64 : q2n;
         const int base = q2n - take;
         if (s_next + take > s_end) {
-          /* new chunk of survivor slots; the rest of the old one is padded */
+          /* new chunk of survivor slots; the rest of the old one is padded
+           * (exact_slots: just these slots, no rest) */
           fill_sentinels(A, s_next, s_end);
           unsigned long long v = 0;
-          if (lane == 0) v = atomicAdd(A.surv_cnt, (unsigned long long)HCS_SURV_CHUNK);
+          const unsigned long long chunk = A.exact_slots ? take : HCS_SURV_CHUNK;
+          if (lane == 0) v = atomicAdd(A.surv_cnt, chunk);
           s_next = __shfl(v, 0, 64);
-          s_end = s_next + HCS_SURV_CHUNK;
+          s_end = s_next + chunk;
         }
         const unsigned long long slot0 = s_next;
         s_next += take;

@@ -1,0 +1,84 @@
+"""The per-call step's work items, enumerated and culled on the device:
+element counts around a chunk of 64, one-tet bodies, pairs without contact
+between others, and calls whose items exceed the splitting budget, against
+the oracle and against calls of one pair."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import oracle as O
+from mujoco_contact_surfaces_amd import _abi as A
+from mujoco_contact_surfaces_amd import scenes as S
+from mujoco_contact_surfaces_amd.engine import _opts, _pair
+from test_gpu_parity import add_scene, assert_wrench_close, oracle_soft_rigid, pair_of
+
+pytestmark = pytest.mark.gpu
+
+
+# triangles: a tet-query pair (50), one chunk and a part (72), two chunks
+# (128), many; tets: one layer of 20 up to subtrees below every frontier
+@pytest.mark.parametrize("m", [5, 6, 8, 40])
+@pytest.mark.parametrize("L,K", [(0, 1), (1, 1), (2, 2), (4, 3)])
+def test_items_of_one_pair(engine, L, K, m):
+    print("[case] items", L, K, m, flush=True)
+    sc = S.tactile_pad(7, L=L, K=K, m=m, depth=0.006)
+    ha, hb = add_scene(engine, sc)
+    ref = oracle_soft_rigid(sc)
+    W, cnt = engine.contact_step([pair_of(sc, ha, hb)])
+    np.testing.assert_array_equal(cnt[0], ref["counts"])
+    assert ref["counts"][1] > 0
+    assert_wrench_close(W[0], ref["wrench"])
+    keys = engine.candidates(pair_of(sc, ha, hb))
+    assert keys.size == ref["counts"][0] and np.unique(keys).size == keys.size
+
+
+def test_one_tet_body(engine):
+    V = np.array([[0.0, 0, 0], [0.1, 0, 0], [0, 0.1, 0], [0, 0, 0.1]])
+    T = np.array([[0, 1, 2, 3]], np.int32)
+    p = np.array([0.0, 0, 0, 1e4])
+    VR, FR = S.rigid_mesh(1, 9, 0.4)  # 162 triangles
+    sp = dict(S.SOFT_PROPS, hydroelastic_modulus=1e5)
+    ha, hb = engine.add_soft_mesh(V, T, p, sp, 0), engine.add_rigid_mesh(VR, FR, S.RIGID_PROPS, 1)
+    XA, XB, z = S.pose(np.eye(3), [0.013, 0.007, -0.02]), S.pose(np.eye(3), [0, 0, 0]), np.zeros(6)
+    W, cnt = engine.contact_step([(ha, hb, XA, XB, z, z)])
+    ref = O.soft_rigid(V, T, p, VR, FR, XA, XB, z, z, 1e5, sp["dissipation"], sp["dynamic_friction"],
+                       S.RIGID_PROPS["dynamic_friction"])
+    np.testing.assert_array_equal(cnt[0], ref["counts"])
+    assert cnt[0, 1] > 0
+    assert_wrench_close(W[0], ref["wrench"])
+
+
+def _scenes(engine):
+    out = []
+    for sc in (S.sphere_box(1), S.tactile_pad(2, L=3, K=3, m=20), S.soft_soft_env(3, 0, nt_range=(3e3, 6e3))):
+        ha, hb = add_scene(engine, sc)
+        out.append(pair_of(sc, ha, hb))
+    return out
+
+
+@pytest.mark.parametrize("n", [7, 300, 1100])
+def test_many_pairs_with_and_without_contact(engine, n):
+    """Every third pair lifted away; 1100 pairs hold more items than the
+    splitting budget, so nothing is split there.  Results are those of calls
+    of one pair (the sums' order differs)."""
+    print("[case] pairs", n, flush=True)
+    base = _scenes(engine)
+    away = [(a, b, XA + np.r_[np.zeros(11), 5.0], XB, VA, VB) for a, b, XA, XB, VA, VB in base]
+    W1, c1 = zip(*[engine.contact_step([p]) for p in base])
+    W0, c0 = zip(*[engine.contact_step([p]) for p in away])
+    pairs = [(away if k % 3 == 1 else base)[k // 3 % 3] for k in range(n)]
+    W, cnt = engine.contact_step(pairs)
+    for k in range(n):
+        w, c = ((W0, c0) if k % 3 == 1 else (W1, c1))
+        w, c = w[k // 3 % 3][0], c[k // 3 % 3][0]
+        np.testing.assert_array_equal(cnt[k], c)
+        assert_wrench_close(W[k], w, rtol=1e-12)
+    assert cnt[0, 1] > 0 and cnt[1, 1] == 0
+    # the no-allocation form runs the same items in the same order
+    arr = (A.PairIn * n)(*[_pair(*p) for p in pairs])
+    got, o = (A.PairOut * n)(), _opts()
+    rc = engine.lib.hcs_contact_step_noalloc(engine.h, n, arr, C.byref(o), got)
+    assert rc == 0, engine.lib.hcs_last_error(engine.h)
+    Wn = np.frombuffer(got, np.float64).reshape(n, 16)[:, :12]
+    np.testing.assert_array_equal(Wn, W)
