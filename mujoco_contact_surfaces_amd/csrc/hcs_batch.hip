@@ -40,7 +40,14 @@ struct hcs_batch {
    * the persistent launch depends on) */
   int order_mode = 0;
   bool has_state = false;
+  bool shape_set = false; /* hcs_batch_set_config or hcs_batch_tune chose the shape */
+  bool whole = false;     /* plan whole items without a measurement (item statistics) */
   DBuf envs, state, items;
+  /* Until a step can be measured (a shape set or tuned with a state), the
+   * items are enumerated, culled and split on the device in every step, as in
+   * a per-call step: an unmeasured plan has no way to tell the heavy items. */
+  bool implicit = false;
+  CallBlob blob;
   Pipe pipe;
   BatchTaxels tx; /* flat tactile sensors (hcs_batch_set_sensors) */
   hipGraph_t graph = nullptr;
@@ -60,9 +67,22 @@ static int grid_of(const hcs_batch* b) {
   return std::max(1, std::min(nitems, b->c->num_cu * b->blocks_per_cu));
 }
 
+/* Blocks of the candidate kernel: an unmeasured batch whose shape was not set
+ * fills the chip. */
+static int cand_grid(const hcs_batch* b) {
+  if (!b->implicit) return grid_of(b);
+  return b->c->num_cu * (b->shape_set ? b->blocks_per_cu : 12);
+}
+
 static QueryArgs batch_args(hcs_batch* b) {
-  QueryArgs a = pipe_args(b->pipe, (const EnvDesc*)b->envs.ptr, (const double*)b->state.ptr,
-                          (const Item*)b->items.ptr, (int)b->plan.items.size(), true);
+  QueryArgs a;
+  if (b->implicit) {
+    a = call_args(b->pipe, b->plan, b->blob);
+    a.state = (const double*)b->state.ptr;
+  } else {
+    a = pipe_args(b->pipe, (const EnvDesc*)b->envs.ptr, (const double*)b->state.ptr,
+                  (const Item*)b->items.ptr, (int)b->plan.items.size(), true);
+  }
   if (b->tx.n > 0) {
     /* the clip kernel keeps the polygons of the pairs that carry a sensor */
     a.poly_rec = (double*)b->tx.poly_rec.ptr;
@@ -76,10 +96,39 @@ static QueryArgs batch_args(hcs_batch* b) {
 
 /* Enqueues one step on the context stream. */
 static void batch_enqueue(hcs_batch* b, const QueryArgs& a) {
+  if (b->implicit) {
+    /* sizes were checked when the buffers were reserved */
+    unsigned* const counters[] = {(unsigned*)b->tx.poly_cnt.ptr};
+    (void)call_enqueue(b->c, b->pipe, a, b->plan, b->blob, counters, b->tx.n > 0 ? 1 : 0, false, cand_grid(b),
+                       (PairOut*)b->pipe.out.ptr, (CallTail*)((PairOut*)b->pipe.out.ptr + b->npairs));
+    batch_taxels_enqueue(b->c, b->tx, (const double*)b->state.ptr);
+    return;
+  }
   if (b->tx.n > 0) launch_fill_u32(b->c->stream, (unsigned*)b->tx.poly_cnt.ptr, 0u, 2);
   pipe_enqueue(b->c, b->pipe, a, b->npairs, grid_of(b), clip_grid_for(b->c, b->pipe.cap), 0, nullptr, nullptr,
                false, 0);
   batch_taxels_enqueue(b->c, b->tx, (const double*)b->state.ptr);
+}
+
+/* Survivor slots of the batch's step (both forms). */
+static int batch_reserve(hcs_batch* b, int64_t cap) {
+  if (!b->implicit) return pipe_reserve(b->c, b->pipe, (int)b->plan.items.size(), b->npairs, cap, 0);
+  int rc = ensure(b->c, b->pipe.out, sizeof(PairOut) * b->npairs + sizeof(CallTail));
+  return rc ? rc : call_reserve(b->c, b->pipe, b->plan, b->blob, cap);
+}
+
+/* Uploads the tables of an implicit plan. */
+static int batch_upload_implicit(hcs_batch* b) {
+  Ctx* c = b->c;
+  std::vector<char> image(call_blob_bytes(b->plan, b->blob));
+  b->blob.src = nullptr;
+  int rc = ensure(c, b->state, sizeof(double) * HCS_STATE * b->npairs);
+  if (!rc) rc = batch_reserve(b, std::max<int64_t>(b->pipe.cap, 65536));
+  if (rc) return rc;
+  call_blob_fill(b->plan, nullptr, b->blob, image.data());
+  rc = hip_check(c, hipMemcpyAsync(b->pipe.blob.ptr, image.data(), image.size(), hipMemcpyHostToDevice, c->stream),
+                 "upload plan");
+  return rc ? rc : hip_check(c, hipStreamSynchronize(c->stream), "sync");
 }
 
 /* Uploads envs and items of b->plan and computes the static item boxes. */
@@ -237,8 +286,11 @@ static int batch_split(hcs_batch* b) {
  * set, heavy items are split and all items ordered by measured steps. */
 static int batch_plan(hcs_batch* b) {
   batch_free_graph(b);
-  int rc = build_plan(b->c, b->npairs, b->geoms.data(), &b->opts, b->tet_max, b->plan);
+  b->implicit = !b->has_state && !b->whole;
+  int rc = build_plan(b->c, b->npairs, b->geoms.data(), &b->opts, b->tet_max, b->plan,
+                      b->implicit ? ITEMS_IMPLICIT : ITEMS_WHOLE);
   b->plan.order.clear();
+  if (b->implicit) return rc ? rc : batch_upload_implicit(b);
   if (!rc) rc = batch_upload(b);
   if (!rc && b->has_state) rc = batch_split(b);
   if (!rc && b->has_state) rc = batch_order(b);
@@ -271,7 +323,7 @@ static int batch_settle(hcs_batch* b) {
     const bool over_tx = b->tx.n > 0 && (npoly > b->tx.poly_cap || nlist > b->tx.list_cap);
     if ((int64_t)n <= b->pipe.cap && !over_tx) return HCS_OK;
     if ((int64_t)n > b->pipe.cap)
-      rc = pipe_reserve(c, b->pipe, (int)b->plan.items.size(), b->npairs, (int64_t)n + (int64_t)n / 4 + 4096, 0);
+      rc = batch_reserve(b, (int64_t)n + (int64_t)n / 4 + 4096);
     else
       rc = batch_taxels_reserve(c, b->tx, std::max(b->tx.poly_cap, npoly + npoly / 4 + 4096),
                                 std::max(b->tx.list_cap, nlist + nlist / 4 + 4096));
@@ -292,16 +344,13 @@ int hcs::batches_refresh(Ctx* c, int handle) {
   return HCS_OK;
 }
 
-extern "C" {
-
-int hcs_batch_create(hcs_ctx* h, int32_t npairs, const int32_t* geoms, const hcs_step_opts* opts,
-                     hcs_batch** out) {
-  if (!h || !geoms || !out || npairs <= 0) return HCS_ERR_ARG;
-  *out = nullptr;
-  Ctx* c = &h->c;
+static int batch_create(Ctx* c, int npairs, const int32_t* geoms, const hcs_step_opts* opts, int tet_max, bool whole,
+                        hcs_batch** out) {
   int rc = hip_check(c, hipSetDevice(c->device), "hipSetDevice");
   if (rc) return rc;
   hcs_batch* b = new hcs_batch();
+  b->whole = whole;
+  if (tet_max >= 0) b->tet_max = tet_max;
   b->c = c;
   c->batches.insert(b);
   b->npairs = npairs;
@@ -329,6 +378,15 @@ int hcs_batch_create(hcs_ctx* h, int32_t npairs, const int32_t* geoms, const hcs
   }
   *out = b;
   return HCS_OK;
+}
+
+extern "C" {
+
+int hcs_batch_create(hcs_ctx* h, int32_t npairs, const int32_t* geoms, const hcs_step_opts* opts,
+                     hcs_batch** out) {
+  if (!h || !geoms || !out || npairs <= 0) return HCS_ERR_ARG;
+  *out = nullptr;
+  return batch_create(&h->c, npairs, geoms, opts, -1, false, out);
 }
 
 int hcs_batch_destroy(hcs_batch* b) {
@@ -446,6 +504,7 @@ int hcs_batch_set_config(hcs_batch* b, const int32_t* cfg) {
     return set_err(b->c, HCS_ERR_ARG, "queries_per_lane must be 1 (items of more than 64 queries are switched off)");
   b->blocks_per_cu = cfg[0], b->qpl = cfg[1], b->tet_max = cfg[2], b->split_target = cfg[3], b->queues = cfg[4];
   b->order_mode = cfg[5];
+  b->shape_set = true;
   int rc = batch_plan(b);
   if (!rc) rc = batch_capture(b);
   return rc;
@@ -475,6 +534,7 @@ int hcs_batch_tune(hcs_batch* b, int32_t reps, double* best_ms) {
   const int tets[] = {0, 64, 256};
   const int splits[] = {0, 512, 1024, 2048, 4096};
   double best = 1e300;
+  b->shape_set = true;
   int bb = b->blocks_per_cu, bq = b->queues, bt = b->tet_max, bs = b->split_target, bo = b->order_mode;
   auto try_plan = [&](const int* ks, int nk) -> int {
     int rc = batch_plan(b);
@@ -527,6 +587,22 @@ int hcs_batch_tune(hcs_batch* b, int32_t reps, double* best_ms) {
 int hcs_batch_item_stats(hcs_batch* b, int64_t* out, int64_t capacity, int64_t* nitems) {
   if (!b || !nitems || capacity < 0 || (capacity > 0 && !out)) return HCS_ERR_ARG;
   Ctx* c = b->c;
+  if (b->implicit) {
+    /* per item of a plan of whole items: a batch of its own for the call */
+    hcs_batch* w = nullptr;
+    int rc = batch_create(c, b->npairs, b->geoms.data(), &b->opts, b->tet_max, true, &w);
+    if (!rc)
+      rc = hip_check(c, hipMemcpyAsync(w->state.ptr, b->state.ptr, sizeof(double) * HCS_STATE * b->npairs,
+                                       hipMemcpyDeviceToDevice, c->stream), "copy state");
+    if (!rc && capacity > 0) {
+      rc = hcs_batch_step(w);
+      std::vector<hcs_pair_out> o(b->npairs);
+      if (!rc) rc = hcs_batch_get(w, o.data());
+    }
+    if (!rc) rc = hcs_batch_item_stats(w, out, capacity, nitems);
+    if (w) hcs_batch_destroy(w);
+    return rc;
+  }
   const int n = (int)b->plan.items.size();
   *nitems = n;
   if (capacity < n) return capacity == 0 ? HCS_OK : set_err(c, HCS_ERR_CAPACITY, "item stats buffer too small");
@@ -597,11 +673,15 @@ int hcs_batch_kernel_times(hcs_batch* b, int32_t reps, double* ms) {
     QueryArgs a = batch_args(b);
     Pipe& P = b->pipe;
     if (b->tx.n > 0) launch_fill_u32(s, (unsigned*)b->tx.poly_cnt.ptr, 0u, 2);
-    pipe_front(c, P, a, b->npairs);
+    if (b->implicit) (void)call_front(c, P, a, b->plan, b->blob, nullptr, 0);
+    else pipe_front(c, P, a, b->npairs);
     (void)hipEventRecord(ev[0], s);
-    launch_cand(s, a, grid_of(b), CAND_STEP);
+    launch_cand(s, a, cand_grid(b), CAND_STEP);
     (void)hipEventRecord(ev[1], s);
-    launch_clip_reduce(c, P, a, b->npairs, clip_grid_for(c, P.cap), ev[2], ev[4]);
+    if (b->implicit)
+      (void)call_back(c, P, a, b->plan, (PairOut*)P.out.ptr, (CallTail*)((PairOut*)P.out.ptr + b->npairs), ev[2], ev[4]);
+    else
+      launch_clip_reduce(c, P, a, b->npairs, clip_grid_for(c, P.cap), ev[2], ev[4]);
     batch_taxels_enqueue(c, b->tx, (const double*)b->state.ptr);
     (void)hipEventRecord(ev[3], s);
     rc = hip_check(c, hipEventSynchronize(ev[3]), "sync");

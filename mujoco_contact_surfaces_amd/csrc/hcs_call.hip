@@ -109,9 +109,9 @@ __device__ inline int levels_below(const EnvDesc& E, int e) {
   while (n < e && E.depth + n < HCS_ROOT_DEPTH && (E.ntA >> (E.depth + n)) > 32) ++n;
   return n;
 }
-__device__ inline int expand_levels(unsigned n1) {
+__device__ inline int expand_levels(unsigned n1, unsigned budget) {
   int e = 0;
-  while (e < HCS_ROOT_DEPTH && ((unsigned long long)n1 << (e + 1)) <= HCS_EXPAND_BUDGET) ++e;
+  while (e < HCS_ROOT_DEPTH && ((unsigned long long)n1 << (e + 1)) <= budget) ++e;
   return e;
 }
 
@@ -206,13 +206,13 @@ __global__ __launch_bounds__(HCS_GEN_THREADS) void k_call_place1(const EnvDesc* 
 }
 
 /* Second cull: the kept items cut e levels deeper, e the same for the launch
- * (2^e n1 items within HCS_EXPAND_BUDGET).  The contact lies in a few of the
+ * (2^e n1 items within the budget).  The contact lies in a few of the
  * first frontier's subtrees: a pad's 33k candidates came from 110 chunks and
  * 4 to 8 subtrees, 1000 and more per item; cut again where the boxes meet, the
  * longest item falls to a tenth and about a thousand waves share the work. */
 __device__ inline bool second_item(const EnvDesc* __restrict__ envs, const int4* __restrict__ item, unsigned n1,
-                                   unsigned t, int& i, int& sub, int& node) {
-  const int e = expand_levels(n1);
+                                   unsigned budget, unsigned t, int& i, int& sub, int& node) {
+  const int e = expand_levels(n1, budget);
   i = (int)(t >> e), sub = (int)(t & ((1u << e) - 1));
   if ((unsigned)i >= n1) return false;
   const int4 it = item[i];
@@ -223,11 +223,11 @@ __device__ inline bool second_item(const EnvDesc* __restrict__ envs, const int4*
 __global__ __launch_bounds__(HCS_GEN_THREADS) void k_call_cull2(const EnvDesc* __restrict__ envs,
                                                                 const double* __restrict__ xf,
                                                                 const int4* __restrict__ item,
-                                                                const unsigned* __restrict__ n1,
+                                                                const unsigned* __restrict__ n1, unsigned budget,
                                                                 unsigned* __restrict__ cnt,
                                                                 unsigned long long* __restrict__ mask) {
   int i, sub, node;
-  bool keep = second_item(envs, item, *n1, blockIdx.x * HCS_GEN_THREADS + threadIdx.x, i, sub, node);
+  bool keep = second_item(envs, item, *n1, budget, blockIdx.x * HCS_GEN_THREADS + threadIdx.x, i, sub, node);
   if (keep) {
     const int4 it = item[i];
     const EnvDesc& E = envs[it.x];
@@ -243,7 +243,7 @@ __global__ __launch_bounds__(HCS_GEN_THREADS) void k_call_cull2(const EnvDesc* _
 /* The live items in order, and each pair's first. */
 __global__ __launch_bounds__(HCS_GEN_THREADS) void k_call_place2(const EnvDesc* __restrict__ envs,
                                                                  const int4* __restrict__ item,
-                                                                 const unsigned* __restrict__ n1p,
+                                                                 const unsigned* __restrict__ n1p, unsigned budget,
                                                                  const unsigned* __restrict__ cnt, bool scanned,
                                                                  const unsigned long long* __restrict__ mask,
                                                                  int npairs, int4* __restrict__ live_item,
@@ -259,7 +259,7 @@ __global__ __launch_bounds__(HCS_GEN_THREADS) void k_call_place2(const EnvDesc* 
     for (int e = n1 ? item[n1 - 1].x + 1 : 0; e <= npairs; ++e) pair_lo[e] = (int)through;
   }
   int i, sub, node;
-  const bool on = second_item(envs, item, n1, t, i, sub, node);
+  const bool on = second_item(envs, item, n1, budget, t, i, sub, node);
   if (on && sub == 0) {
     /* the first item of a pair: its place, also for the pairs without items
      * before it */
@@ -373,7 +373,8 @@ CallSizes call_sizes(const Plan& plan) {
   CallSizes z;
   z.blocks1 = plan.blocks.size();
   z.items = (size_t)std::max(1, plan.nitems);
-  z.live = std::max<size_t>(z.items, HCS_EXPAND_BUDGET);
+  z.expand = HCS_EXPAND_BUDGET;
+  z.live = std::max<size_t>(z.items, z.expand);
   z.blocks2 = (z.live + HCS_GEN_THREADS - 1) / HCS_GEN_THREADS;
   /* slices of a pair's contributions: about 1024 waves in all, at most 64 per
    * pair */
@@ -391,7 +392,7 @@ size_t call_blob_bytes(const Plan& plan, CallBlob& b) {
 
 void call_blob_fill(const Plan& plan, const hcs_pair_in* in, const CallBlob& b, char* dst) {
   std::memcpy(dst, plan.envs.data(), sizeof(EnvDesc) * plan.envs.size());
-  for (size_t e = 0; e < plan.envs.size(); ++e) {
+  for (size_t e = 0; in && e < plan.envs.size(); ++e) {
     double* st = (double*)(dst + b.state) + HCS_STATE * e;
     std::memcpy(st, in[e].X_WA, 12 * sizeof(double));
     std::memcpy(st + 12, in[e].X_WB, 12 * sizeof(double));
@@ -451,13 +452,19 @@ QueryArgs call_args(const Pipe& p, const Plan& plan, const CallBlob& b) {
   return a;
 }
 
-int call_enqueue(Ctx* c, Pipe& p, QueryArgs& a, const Plan& plan, const CallBlob& b, unsigned* const* counters,
-                 int ncounters, bool keys, PairOut* out, CallTail* tail) {
+/* Clears, pose composition (with the blob's upload when it has a source) and
+ * the two culls. */
+int call_front(Ctx* c, Pipe& p, const QueryArgs& a, const Plan& plan, const CallBlob& b, unsigned* const* counters,
+               int ncounters) {
   hipStream_t s = c->stream;
   const int np = (int)plan.envs.size(), nblk = (int)plan.blocks.size();
   FrontArgs f{};
-  f.src = (const uint4*)b.src, f.dst = (uint4*)p.blob.ptr, f.n16 = (int64_t)(b.bytes / 16);
-  f.state = (const double*)((const char*)b.src + b.state);
+  if (b.src) {
+    f.src = (const uint4*)b.src, f.dst = (uint4*)p.blob.ptr, f.n16 = (int64_t)(b.bytes / 16);
+    f.state = (const double*)((const char*)b.src + b.state);
+  } else {
+    f.state = a.state;
+  }
   f.xf = (double*)p.xf.ptr, f.npairs = np;
   for (DBuf* d : {&p.counter, &p.surv_cnt, &p.err}) f.counters[f.ncounters++] = (unsigned*)d->ptr;
   for (int k = 0; k < ncounters && f.ncounters < kMaxCounters; ++k) f.counters[f.ncounters++] = counters[k];
@@ -480,15 +487,25 @@ int call_enqueue(Ctx* c, Pipe& p, QueryArgs& a, const Plan& plan, const CallBlob
                      blocks, nblk, (const unsigned*)cnt1, scan1, (const unsigned long long*)mask1,
                      (const int*)(blob + b.xenv), a.xf, (double*)p.xtri.ptr, item, n1);
   const dim3 g2((unsigned)z.blocks2);
+  const unsigned budget = (unsigned)z.expand;
   hipLaunchKernelGGL(k_call_cull2, g2, dim3(HCS_GEN_THREADS), 0, s, a.envs, a.xf, (const int4*)item,
-                     (const unsigned*)n1, cnt2, mask2);
+                     (const unsigned*)n1, budget, cnt2, mask2);
   if (scan2) rc |= exclusive_scan_u32(s, cnt2, cnt2, (long long)z.blocks2, p.scan_tmp.ptr, p.scan_bytes);
   if (rc) return set_err(c, HCS_ERR_LIMIT, "too many work items to scan");
   hipLaunchKernelGGL(k_call_place2, g2, dim3(HCS_GEN_THREADS), 0, s, a.envs, (const int4*)item, (const unsigned*)n1,
-                     (const unsigned*)cnt2, scan2, (const unsigned long long*)mask2, np, (int4*)p.live_item.ptr,
-                     live_cnt, (int*)p.pair_lo.ptr);
-  launch_cand(s, a, std::min(a.nitems, c->num_cu * 12), keys ? CAND_KEYS : CAND_STEP);
-  if (keys) return HCS_OK;
+                     budget, (const unsigned*)cnt2, scan2, (const unsigned long long*)mask2, np,
+                     (int4*)p.live_item.ptr, live_cnt, (int*)p.pair_lo.ptr);
+  return HCS_OK;
+}
+
+/* Scan of the live items' survivor counts, [event e_clip], clip, [event
+ * e_reduce], per-pair reduction into out[0..npairs) and *tail (device or
+ * mapped host memory). */
+int call_back(Ctx* c, Pipe& p, const QueryArgs& a, const Plan& plan, PairOut* out, CallTail* tail, hipEvent_t e_clip,
+              hipEvent_t e_reduce) {
+  hipStream_t s = c->stream;
+  const CallSizes z = call_sizes(plan);
+  const int np = (int)plan.envs.size();
   unsigned* off = (unsigned*)p.off.ptr;
   if (z.live <= (size_t)kScanThreads * kScanPer * 8) {
     hipLaunchKernelGGL(k_call_scan, dim3(1), dim3(kScanThreads), 0, s, (const unsigned*)a.item_nsurv,
@@ -497,7 +514,9 @@ int call_enqueue(Ctx* c, Pipe& p, QueryArgs& a, const Plan& plan, const CallBlob
     /* (entries past the live items are not read) */
     return set_err(c, HCS_ERR_LIMIT, "too many work items to scan");
   }
+  if (e_clip) (void)hipEventRecord(e_clip, s);
   launch_clip(c, p, a, clip_grid_for(c, p.cap));
+  if (e_reduce) (void)hipEventRecord(e_reduce, s);
   const int K = z.slices;
   hipLaunchKernelGGL(k_call_reduce, dim3(np * K), dim3(64), 0, s, (const int*)p.pair_lo.ptr, K, (const unsigned*)off,
                      (const int*)a.item_ncand, (const unsigned long long*)a.surv_cnt, p.cap,
@@ -512,6 +531,14 @@ int call_enqueue(Ctx* c, Pipe& p, QueryArgs& a, const Plan& plan, const CallBlob
   q.cand_cnt = a.cand_cnt ? a.cand_cnt : zero;
   hipLaunchKernelGGL(k_call_combine, dim3(np), dim3(64), 0, s, q);
   return HCS_OK;
+}
+
+int call_enqueue(Ctx* c, Pipe& p, const QueryArgs& a, const Plan& plan, const CallBlob& b, unsigned* const* counters,
+                 int ncounters, bool keys, int cand_grid, PairOut* out, CallTail* tail) {
+  int rc = call_front(c, p, a, plan, b, counters, ncounters);
+  if (rc) return rc;
+  launch_cand(c->stream, a, std::min(a.nitems, cand_grid), keys ? CAND_KEYS : CAND_STEP);
+  return keys ? HCS_OK : call_back(c, p, a, plan, out, tail, nullptr, nullptr);
 }
 
 }  // namespace hcs

@@ -1260,6 +1260,15 @@ int build_plan(Ctx* c, int npairs, const int32_t* geoms, const hcs_step_opts* o,
   plan.xenv.clear();
   plan.ntx = 0;
   plan.pair_kind.assign(npairs, 0);
+  /* Items over frontiers serve small rigid meshes as well as tet queries do
+   * (a ball on 12 triangles: 12 against 14 us), and a launch of one kind runs
+   * the kernel built for it: tet queries only where every rigid mesh of the
+   * call is small enough for them. */
+  if (mode == ITEMS_IMPLICIT)
+    for (int e = 0; e < npairs && tet_max > 0; ++e) {
+      const int hb = geoms[2 * e + 1];
+      if (hb >= 0 && hb < (int)c->meshes.size() && c->meshes[hb].kind == 2 && c->meshes[hb].nelem > tet_max) tet_max = 0;
+    }
   for (int e = 0; e < npairs; ++e) {
     const int ha = geoms[2 * e], hb = geoms[2 * e + 1];
     if (ha < 0 || hb < 0 || ha >= (int)c->meshes.size() || hb >= (int)c->meshes.size() ||
@@ -1744,7 +1753,7 @@ static int run_pairs(Ctx* c, int npairs, const hcs_pair_in* in, const hcs_step_o
     }
     unsigned* const counters[] = {(unsigned*)c->d_face_cnt.ptr, (unsigned*)c->d_poly_cnt.ptr,
                                   (unsigned*)c->d_cand_cnt.ptr};
-    if ((rc = call_enqueue(c, P, a, plan, blob, counters, 3, keys != nullptr, res, tail))) return rc;
+    if ((rc = call_enqueue(c, P, a, plan, blob, counters, 3, keys != nullptr, c->num_cu * 12, res, tail))) return rc;
     HCHK(c, hipGetLastError());
     if (keys) {
       HCHK(c, hipMemcpyAsync(&ncand, c->d_cand_cnt.ptr, 8, hipMemcpyDeviceToHost, c->stream));

@@ -139,7 +139,7 @@ int build_plan(Ctx* c, int npairs, const int32_t* geoms, const hcs_step_opts* o,
 #define HCS_ITEM_BUDGET 65536
 #define HCS_EXPAND_BUDGET 16384
 struct CallSizes {
-  size_t blocks1, blocks2, items, live;
+  size_t blocks1, blocks2, items, live, expand;
   int slices;
 };
 CallSizes call_sizes(const Plan& plan);
@@ -154,14 +154,19 @@ struct CallTail {
  * pairs) and the offsets in it. */
 struct CallBlob {
   size_t state, blocks, xenv, bytes;
-  const void* src = nullptr; /* device-readable: pinned host memory, or the device blob itself once uploaded */
+  /* device-readable: pinned host memory, or the device blob itself once
+   * uploaded; nullptr: the blob stays, the state is elsewhere (a batch) */
+  const void* src = nullptr;
 };
 size_t call_blob_bytes(const Plan& plan, CallBlob& b);
 void call_blob_fill(const Plan& plan, const hcs_pair_in* in, const CallBlob& b, char* dst);
-/* Enqueues the step; the last kernel writes out[0..npairs) and *tail (device
- * or mapped host memory).  keys: candidate keys only, nothing is written. */
-int call_enqueue(Ctx* c, Pipe& p, QueryArgs& a, const Plan& plan, const CallBlob& b, unsigned* const* counters,
-                 int ncounters, bool keys, PairOut* out, CallTail* tail);
+int call_front(Ctx* c, Pipe& p, const QueryArgs& a, const Plan& plan, const CallBlob& b, unsigned* const* counters,
+               int ncounters);
+int call_back(Ctx* c, Pipe& p, const QueryArgs& a, const Plan& plan, PairOut* out, CallTail* tail, hipEvent_t e_clip,
+              hipEvent_t e_reduce);
+/* The whole step (keys: candidate keys only, nothing is written). */
+int call_enqueue(Ctx* c, Pipe& p, const QueryArgs& a, const Plan& plan, const CallBlob& b, unsigned* const* counters,
+                 int ncounters, bool keys, int cand_grid, PairOut* out, CallTail* tail);
 int call_reserve(Ctx* c, Pipe& p, const Plan& plan, const CallBlob& b, int64_t cap);
 QueryArgs call_args(const Pipe& p, const Plan& plan, const CallBlob& b);
 

@@ -191,7 +191,7 @@ extern "C" int hcs_contact_step_noalloc(hcs_ctx* h, int32_t npairs, const hcs_pa
   char* down = direct ? (char*)c->pin_down : (char*)P.out.ptr;
   CallTail tail{};
   QueryArgs a = call_args(P, plan, blob);
-  if ((rc = call_enqueue(c, P, a, plan, blob, nullptr, 0, false, (PairOut*)down,
+  if ((rc = call_enqueue(c, P, a, plan, blob, nullptr, 0, false, c->num_cu * 12, (PairOut*)down,
                          (CallTail*)(down + sizeof(PairOut) * np))))
     return rc;
   rc = hip_check(c, hipGetLastError(), "noalloc step");
