@@ -154,12 +154,6 @@ __global__ void k_tet_precompute(const double* __restrict__ V, const int32_t* __
   }
 }
 
-/* 4-wide nodes of the LBVH's n_int internal nodes. */
-__global__ void k_wide_nodes(const Node* __restrict__ nodes, int n_int, WNode* __restrict__ w) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n_int) make_wide_node(nodes, i, w[i]);
-}
-
 /* Unit triangle normals (Drake's TriangleSurfaceMesh face normals). */
 __global__ void k_tri_normals(const double* __restrict__ V, const int32_t* __restrict__ F, int ntri,
                               double* __restrict__ nrm) {
@@ -208,12 +202,32 @@ __device__ inline int delta(const unsigned* codes, int n, int i, int j) {
   return __clz(a ^ b);
 }
 
-/* Karras radix-tree construction over sorted Morton codes: internal node i
- * covers a key range whose split is the highest differing bit. */
-__global__ void k_karras(const unsigned* __restrict__ codes, const int* __restrict__ idx, int n,
-                         Node* __restrict__ nodes, int* __restrict__ node_parent, int* __restrict__ leaf_parent) {
+/* The LBVH build's outcome, read once at its end. */
+struct BuildOut {
+  int bad;    /* the sort did not return a permutation in code order: nothing is built on it */
+  int height; /* of the tree: the depth of its deepest leaf */
+  int32_t roots[HCS_ROOTS];
+};
+
+/* The leaf order must be a permutation in code order before a tree is built
+ * on it (the kernels below index by it, and do nothing when it is not). */
+__global__ void k_check_order(const unsigned* __restrict__ codes, const int* __restrict__ idx, int n,
+                              unsigned* __restrict__ seen, BuildOut* __restrict__ out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n - 1) return;
+  if (i >= n) return;
+  const int t = idx[i];
+  const bool ok = t >= 0 && t < n && (i == 0 || codes[i - 1] <= codes[i]) && atomicOr(seen + t, 1u) == 0u;
+  if (!ok) out->bad = 1;
+}
+
+/* Karras radix-tree construction over sorted Morton codes: internal node i
+ * covers a key range whose split is the highest differing bit.  The range is
+ * kept for the boxes. */
+__global__ void k_karras(const unsigned* __restrict__ codes, const int* __restrict__ idx, int n,
+                         const BuildOut* __restrict__ out, Node* __restrict__ nodes, int* __restrict__ node_parent,
+                         int* __restrict__ leaf_parent, int2* __restrict__ range) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n - 1 || out->bad) return;
   const int d = (delta(codes, n, i, i + 1) - delta(codes, n, i, i - 1)) >= 0 ? 1 : -1;
   const int dmin = delta(codes, n, i, i - d);
   int lmax = 2;
@@ -230,60 +244,153 @@ __global__ void k_karras(const unsigned* __restrict__ codes, const int* __restri
   } while (t > 1);
   const int gamma = i + s * d + (d < 0 ? -1 : 0);
   const int lo = i < j ? i : j, hi = i < j ? j : i;
+  range[i] = make_int2(lo, hi);
   Node* N = nodes + i;
+  N->h[0] = N->h[1] = 0;
   if (lo == gamma) {
     N->c[0] = ~idx[gamma];
-    leaf_parent[gamma] = 2 * i;
+    leaf_parent[gamma] = i;
   } else {
     N->c[0] = gamma;
-    node_parent[gamma] = 2 * i;
+    node_parent[gamma] = i;
   }
   if (hi == gamma + 1) {
     N->c[1] = ~idx[gamma + 1];
-    leaf_parent[gamma + 1] = 2 * i + 1;
+    leaf_parent[gamma + 1] = i;
   } else {
     N->c[1] = gamma + 1;
-    node_parent[gamma + 1] = 2 * i + 1;
+    node_parent[gamma + 1] = i;
   }
 }
 
-/* Bottom-up refit: the second thread to reach a node writes its union box
- * and height into the parent's child slot.  Counter RMWs are acq_rel at
- * agent scope, which orders the slot stores/loads between the two threads. */
-__global__ void k_refit(const double* __restrict__ box, const int* __restrict__ idx, int n, Node* nodes,
-                        const int* __restrict__ node_parent, const int* __restrict__ leaf_parent, int* flags,
-                        int* root_height) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n) return;
-  const double* b = box + 6 * (size_t)idx[j];
-  int pc = leaf_parent[j];
-  int p = pc >> 1, side = pc & 1;
-  Node* N = nodes + p;
+__device__ inline void box_union(double* u, const double* b) {
 #pragma unroll
-  for (int c = 0; c < 6; ++c) N->b[6 * side + c] = b[c];
-  N->h[side] = 0;
-  for (int guard = 0; guard < n; ++guard) {
-    const int old = __hip_atomic_fetch_add(flags + p, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-    if (old == 0) return;
-    N = nodes + p;
-    double u[6];
+  for (int c = 0; c < 3; ++c) u[c] = fmin(u[c], b[c]), u[3 + c] = fmax(u[3 + c], b[3 + c]);
+}
+
+/* Boxes of the leaves in Morton order and of their chunks of 64, one wave per
+ * chunk. */
+__global__ __launch_bounds__(64) void k_leaf_boxes(const double* __restrict__ box, const int* __restrict__ idx, int n,
+                                                   const BuildOut* __restrict__ out, double* __restrict__ boxL,
+                                                   double* __restrict__ cbox) {
+  const int i = blockIdx.x * 64 + threadIdx.x;
+  const double inf = __builtin_inf();
+  double u[6] = {inf, inf, inf, -inf, -inf, -inf};
+  if (out->bad) return;
+  if (i < n) {
+    const double* b = box + 6 * (size_t)idx[i];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      u[c] = fmin(N->b[c], N->b[6 + c]);
-      u[3 + c] = fmax(N->b[3 + c], N->b[9 + c]);
-    }
-    const int h = 1 + (N->h[0] > N->h[1] ? N->h[0] : N->h[1]);
-    if (p == 0) {
-      *root_height = h;
-      return;
-    }
-    pc = node_parent[p];
-    p = pc >> 1, side = pc & 1;
-    Node* P = nodes + p;
-#pragma unroll
-    for (int c = 0; c < 6; ++c) P->b[6 * side + c] = u[c];
-    P->h[side] = h;
+    for (int c = 0; c < 6; ++c) u[c] = b[c], boxL[6 * (size_t)i + c] = u[c];
   }
+#pragma unroll
+  for (int c = 0; c < 3; ++c) u[c] = wave_min(u[c]), u[3 + c] = wave_max(u[3 + c]);
+  if (threadIdx.x < 6) {
+    double v = u[0];
+#pragma unroll
+    for (int c = 1; c < 6; ++c) v = threadIdx.x == c ? u[c] : v;
+    cbox[6 * (size_t)blockIdx.x + threadIdx.x] = v;
+  }
+}
+
+/* Boxes of the chunks of 64 boxes of `in`, one wave per chunk. */
+__global__ __launch_bounds__(64) void k_box_chunks(const double* __restrict__ in, int n, double* __restrict__ o) {
+  const int i = blockIdx.x * 64 + threadIdx.x;
+  const double inf = __builtin_inf();
+  double u[6] = {inf, inf, inf, -inf, -inf, -inf};
+  if (i < n) box_union(u, in + 6 * (size_t)i);
+#pragma unroll
+  for (int c = 0; c < 3; ++c) u[c] = wave_min(u[c]), u[3 + c] = wave_max(u[3 + c]);
+  if (threadIdx.x < 6) {
+    double v = u[0];
+#pragma unroll
+    for (int c = 1; c < 6; ++c) v = threadIdx.x == c ? u[c] : v;
+    o[6 * (size_t)blockIdx.x + threadIdx.x] = v;
+  }
+}
+
+/* The box of every internal node, from its range of leaves: the leaves up to
+ * the next chunk boundary on either side, whole chunks, whole chunks of chunks
+ * (at most 126 + 126 + n / 4096 boxes; most nodes hold a few leaves).  Minima
+ * and maxima are exact, so these are the boxes a bottom-up refit gives, without
+ * its counters: one acquire-release atomic per node visit, which writes back
+ * and invalidates the L2s, made that 240 us for 51k tets (this: 22 us, and 13 for the height). */
+__global__ __launch_bounds__(64) void k_node_boxes(const double* __restrict__ boxL, const double* __restrict__ cbox,
+                                                   const double* __restrict__ sbox, const int2* __restrict__ range,
+                                                   int n_int, const BuildOut* __restrict__ out,
+                                                   double* __restrict__ ubox) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n_int || out->bad) return;
+  const int2 r = range[i];
+  const double inf = __builtin_inf();
+  double u[6] = {inf, inf, inf, -inf, -inf, -inf};
+  /* [a, b) of one level; what lies between chunk boundaries goes up a level */
+  auto level = [&](const double* B, int& a, int& b, bool top) {
+    const int a1 = top ? b : min(b, (a + 63) & ~63), b1 = top ? b : max(a1, b & ~63);
+#pragma unroll 4
+    for (int k = a; k < a1; ++k) box_union(u, B + 6 * (size_t)k);
+#pragma unroll 4
+    for (int k = b1; k < b; ++k) box_union(u, B + 6 * (size_t)k);
+    a = a1 >> 6, b = b1 >> 6;
+  };
+  int a = r.x, b = r.y + 1;
+  level(boxL, a, b, false);
+  if (a < b) level(cbox, a, b, false);
+  if (a < b) level(sbox, a, b, true);
+#pragma unroll
+  for (int c = 0; c < 6; ++c) ubox[6 * (size_t)i + c] = u[c];
+}
+
+/* The children's boxes of every internal node, and its 4-wide node (the
+ * layout of make_wide_node: grandchildren, a leaf child standing for itself). */
+__global__ __launch_bounds__(256) void k_fill_nodes(const double* __restrict__ ubox, const double* __restrict__ box,
+                                                    int n_int, const BuildOut* __restrict__ out, Node* nodes,
+                                                    WNode* __restrict__ wide) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n_int || out->bad) return;
+  WNode& w = wide[i];
+  int m = 0;
+  auto put = [&](int ch) {
+    const double* b = ch < 0 ? box + 6 * (size_t)~ch : ubox + 6 * (size_t)ch;
+#pragma unroll
+    for (int c = 0; c < 6; ++c) w.b[6 * m + c] = b[c];
+    w.ch[m++] = ch;
+  };
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const int ch = nodes[i].c[s];
+    const double* b = ch < 0 ? box + 6 * (size_t)~ch : ubox + 6 * (size_t)ch;
+#pragma unroll
+    for (int c = 0; c < 6; ++c) nodes[i].b[6 * s + c] = b[c];
+    if (ch < 0) {
+      put(ch);
+    } else {
+      const int g0 = nodes[ch].c[0], g1 = nodes[ch].c[1];
+      put(g0);
+      put(g1);
+    }
+  }
+  for (; m < 4; ++m) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) w.b[6 * m + c] = __builtin_inf(), w.b[6 * m + 3 + c] = -__builtin_inf();
+    w.ch[m] = HCS_WNONE;
+  }
+#pragma unroll
+  for (int k = 0; k < 12; ++k) w.pad[k] = 0;
+}
+
+/* Depth of the deepest leaf: every leaf counts its ancestors. */
+__global__ void k_tree_height(const int* __restrict__ leaf_parent, const int* __restrict__ node_parent, int n,
+                              BuildOut* __restrict__ out) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (out->bad) return;
+  int h = 0;
+  if (j < n) {
+    int p = leaf_parent[j];
+    for (h = 1; p != 0 && h < n; ++h) p = node_parent[p];
+  }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) h = max(h, __shfl_xor(h, o, 64));
+  if ((threadIdx.x & 63) == 0) atomicMax(&out->height, h);
 }
 
 /* ===================================================================
@@ -304,15 +411,6 @@ __global__ void k_prep(const EnvDesc* __restrict__ envs, const double* __restric
   compose_SR(st, st + 12, X);
 #pragma unroll
   for (int i = 0; i < 12; ++i) xf[12 * (size_t)e + i] = X[i];
-}
-
-/* AABBs of a soft mesh's tets in Morton (leaf) order. */
-__global__ void k_gather_boxes(const double* __restrict__ box, const int* __restrict__ idx, int n,
-                               double* __restrict__ boxL) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-#pragma unroll
-  for (int c = 0; c < 6; ++c) boxL[6 * (size_t)i + c] = box[6 * (size_t)idx[i] + c];
 }
 
 /* Per step, one block per tet-query pair: its triangles moved. */
@@ -349,9 +447,11 @@ __global__ __launch_bounds__(64) void k_chunk_boxes(const double* __restrict__ V
 }
 
 /* The LBVH's frontiers (HCS_ROOTS), one block, level by level. */
-__global__ __launch_bounds__(HCS_ROOTS / 2) void k_frontiers(const Node* __restrict__ nodes, int n_int, int32_t* __restrict__ heap) {
+__global__ __launch_bounds__(HCS_ROOTS / 2) void k_frontiers(const Node* __restrict__ nodes, int n_int,
+                                                             BuildOut* __restrict__ out, int32_t* __restrict__ heap) {
   __shared__ int32_t h[HCS_ROOTS];
   const int t = threadIdx.x;
+  if (out->bad) return;
   if (t < 2) h[t] = t == 1 ? 0 : HCS_WNONE;
   __syncthreads();
   for (int d = 0; d < HCS_ROOT_DEPTH; ++d) {
@@ -363,7 +463,8 @@ __global__ __launch_bounds__(HCS_ROOTS / 2) void k_frontiers(const Node* __restr
     }
     __syncthreads();
   }
-  heap[t] = h[t], heap[HCS_ROOTS / 2 + t] = h[HCS_ROOTS / 2 + t];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) heap[k * (HCS_ROOTS / 2) + t] = out->roots[k * (HCS_ROOTS / 2) + t] = h[k * (HCS_ROOTS / 2) + t];
 }
 
 /* Static boxes of one item per wave: [0..5] its query elements in their own
@@ -1087,147 +1188,115 @@ static bool is_rigid(const hcs_props& p) {
   return !(p.hydroelastic_modulus > 0) || std::isinf(p.hydroelastic_modulus);
 }
 
-static int upload(Ctx* c, void** dst, const void* src, size_t bytes) {
-  HCHK(c, hipMalloc(dst, std::max<size_t>(bytes, 8)));
-  if (bytes) HCHK(c, hipMemcpyAsync(*dst, src, bytes, hipMemcpyHostToDevice, c->stream));
+/* A mesh's device arrays are slices of one allocation (256-byte aligned). */
+struct Slices {
+  size_t bytes = 0;
+  template <class T>
+  size_t take(size_t n) {
+    const size_t at = bytes;
+    bytes += (sizeof(T) * std::max<size_t>(n, 1) + 255) & ~(size_t)255;
+    return at;
+  }
+};
+
+/* Memory for a mesh: the context's spare block when it fits without much
+ * waste (a geom that is re-meshed at run time asks for about the same size
+ * again and again), else a new allocation. */
+static int mesh_alloc(Ctx* c, Mesh& m, size_t bytes) {
+  if (c->spare && c->spare_bytes >= bytes && c->spare_bytes / 2 <= bytes) {
+    m.mem = c->spare, m.mem_bytes = c->spare_bytes;
+    c->spare = nullptr, c->spare_bytes = 0;
+    return HCS_OK;
+  }
+  HCHK(c, hipMalloc(&m.mem, bytes));
+  m.mem_bytes = bytes;
   return HCS_OK;
 }
 
-static int build_bvh(Ctx* c, Mesh& m) {
-  const int n = m.nelem;
-  m.height = 0;
-  if (n == 1) {
-    HCHK(c, hipMalloc((void**)&m.nodes, sizeof(Node)));
-    const int32_t zero = 0;
-    int rc = upload(c, (void**)&m.leaf, &zero, sizeof(int32_t));
-    if (!rc) rc = hip_check(c, hipMalloc((void**)&m.boxL, 6 * sizeof(double)), "hipMalloc");
-    if (!rc)
-      rc = hip_check(c, hipMemcpyAsync(m.boxL, m.box, 6 * sizeof(double), hipMemcpyDeviceToDevice, c->stream), "copy");
-    return rc ? rc : hip_check(c, hipStreamSynchronize(c->stream), "sync");
+static void free_mesh(Mesh& m) {
+  if (m.mem) (void)hipFree(m.mem);
+  m = Mesh();
+}
+
+/* A replaced mesh: its memory becomes the context's spare block (one block,
+ * at most HCS_SPARE_BYTES; the one before it is given back).  Nothing in
+ * flight uses it. */
+#define HCS_SPARE_BYTES (256ull << 20)
+static void retire_mesh(Ctx* c, Mesh& m) {
+  if (m.mem && m.mem_bytes <= HCS_SPARE_BYTES) {
+    if (c->spare) (void)hipFree(c->spare);
+    c->spare = m.mem, c->spare_bytes = m.mem_bytes;
+    m.mem = nullptr;
   }
+  free_mesh(m);
+}
+
+/* Builds the leaf order, the LBVH and the work items' tables (chunk boxes,
+ * frontiers) of a soft mesh whose records and boxes are enqueued.  V: its
+ * vertices on the host.  One wait, at the end. */
+static int build_bvh(Ctx* c, Mesh& m, const double* V) {
+  const int n = m.nelem, chunks = (n + 63) / 64, schunks = (chunks + 63) / 64;
+  hipStream_t s = c->stream;
   /* Scene bounds from the vertices (they bound every tet AABB). */
-  std::vector<double> Vh(3 * (size_t)m.nv);
-  HCHK(c, hipMemcpyAsync(Vh.data(), m.V, Vh.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HCHK(c, hipStreamSynchronize(c->stream));
   double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
   for (int v = 0; v < m.nv; ++v)
-    for (int k = 0; k < 3; ++k) lo[k] = std::min(lo[k], Vh[3 * v + k]), hi[k] = std::max(hi[k], Vh[3 * v + k]);
+    for (int k = 0; k < 3; ++k)
+      lo[k] = std::min(lo[k], V[3 * (size_t)v + k]), hi[k] = std::max(hi[k], V[3 * (size_t)v + k]);
   double sc[3];
   for (int k = 0; k < 3; ++k) sc[k] = hi[k] > lo[k] ? 1024.0 / (hi[k] - lo[k]) : 0.0;
-  unsigned *codes = nullptr, *codes2 = nullptr;
-  int *idx = nullptr, *idx2 = nullptr, *np = nullptr, *lp = nullptr, *flags = nullptr, *rh = nullptr;
-  void* tmp = nullptr;
-  size_t tmp_bytes = 0;
-  int rc = HCS_OK;
-  auto fail = [&](hipError_t e, const char* w) {
-    if (rc == HCS_OK) rc = hip_check(c, e, w);
-  };
-  fail(hipMalloc((void**)&codes, n * sizeof(unsigned)), "hipMalloc");
-  fail(hipMalloc((void**)&codes2, n * sizeof(unsigned)), "hipMalloc");
-  fail(hipMalloc((void**)&idx, n * sizeof(int)), "hipMalloc");
-  fail(hipMalloc((void**)&idx2, n * sizeof(int)), "hipMalloc");
-  fail(hipMalloc((void**)&np, n * sizeof(int)), "hipMalloc");
-  fail(hipMalloc((void**)&lp, n * sizeof(int)), "hipMalloc");
-  fail(hipMalloc((void**)&flags, n * sizeof(int)), "hipMalloc");
-  fail(hipMalloc((void**)&rh, sizeof(int)), "hipMalloc");
-  fail(hipMalloc((void**)&m.nodes, (size_t)(n - 1) * sizeof(Node)), "hipMalloc");
-  if (rc == HCS_OK) {
-    hipLaunchKernelGGL(k_morton, dim3((n + 255) / 256), dim3(256), 0, c->stream, m.box, n, lo[0], lo[1], lo[2],
-                       sc[0], sc[1], sc[2], codes, idx);
-    fail(hipGetLastError(), "k_morton");
-    tmp_bytes = sort_temp_bytes(n, sizeof(unsigned));
-    fail(hipMalloc(&tmp, std::max<size_t>(tmp_bytes, 8)), "hipMalloc");
-  }
-  if (rc == HCS_OK) {
-    if (radix_sort_pairs_u32(c->stream, codes, codes2, idx, idx2, n, 0, 30, tmp, tmp_bytes) != 0)
-      fail(hipErrorInvalidValue, "radix sort size");
-  }
-  if (rc == HCS_OK) {
-    /* the leaf order must be a permutation in code order before the tree
-     * is built on it */
-    std::vector<unsigned> hc(n);
-    std::vector<int> hi(n);
-    fail(hipMemcpyAsync(hc.data(), codes2, n * sizeof(unsigned), hipMemcpyDeviceToHost, c->stream), "memcpy");
-    fail(hipMemcpyAsync(hi.data(), idx2, n * sizeof(int), hipMemcpyDeviceToHost, c->stream), "memcpy");
-    fail(hipStreamSynchronize(c->stream), "sync");
-    if (rc == HCS_OK) {
-      std::vector<char> seen(n, 0);
-      bool ok = true;
-      for (int i = 0; i < n && ok; ++i) {
-        ok = hi[i] >= 0 && hi[i] < n && !seen[hi[i]] && (i == 0 || hc[i - 1] <= hc[i]);
-        if (ok) seen[hi[i]] = 1;
-      }
-      if (!ok) rc = set_err(c, HCS_ERR_HIP, "LBVH build: the Morton sort returned an invalid order");
-    }
-  }
-  if (rc == HCS_OK) {
-    fail(hipMemsetAsync(flags, 0, n * sizeof(int), c->stream), "memset");
-    hipLaunchKernelGGL(k_karras, dim3((n - 1 + 255) / 256), dim3(256), 0, c->stream, codes2, idx2, n, m.nodes, np,
-                       lp);
-    fail(hipGetLastError(), "k_karras");
-    hipLaunchKernelGGL(k_refit, dim3((n + 255) / 256), dim3(256), 0, c->stream, m.box, idx2, n, m.nodes, np, lp,
-                       flags, rh);
-    fail(hipGetLastError(), "k_refit");
-    int h = 0;
-    fail(hipMemcpyAsync(&h, rh, sizeof(int), hipMemcpyDeviceToHost, c->stream), "memcpy");
-    fail(hipStreamSynchronize(c->stream), "sync");
-    m.height = h;
-  }
-  if (rc == HCS_OK) {
-    fail(hipMalloc((void**)&m.wnodes, (size_t)(n - 1) * sizeof(WNode)), "hipMalloc");
-    if (rc == HCS_OK) {
-      hipLaunchKernelGGL(k_wide_nodes, dim3((n - 1 + 255) / 256), dim3(256), 0, c->stream, m.nodes, n - 1, m.wnodes);
-      fail(hipGetLastError(), "k_wide_nodes");
-    }
-  }
-  if (rc == HCS_OK) {
-    fail(hipMalloc((void**)&m.boxL, 6 * sizeof(double) * (size_t)n), "hipMalloc");
-    if (rc == HCS_OK) {
-      hipLaunchKernelGGL(k_gather_boxes, dim3((n + 255) / 256), dim3(256), 0, c->stream, m.box, idx2, n, m.boxL);
-      fail(hipGetLastError(), "k_gather_boxes");
-      fail(hipStreamSynchronize(c->stream), "sync");
-    }
-  }
-  if (rc == HCS_OK) {
-    m.leaf = idx2; /* kept: Morton order of the tets */
-    idx2 = nullptr;
-  }
-  for (void* ptr : {(void*)codes, (void*)codes2, (void*)idx, (void*)idx2, (void*)np, (void*)lp, (void*)flags,
-                    (void*)rh, tmp})
-    if (ptr) (void)hipFree(ptr);
-  if (rc == HCS_OK && 3 * ((m.height + 1) / 2) + 1 > HCS_STACK)
-    rc = set_err(c, HCS_ERR_LIMIT, "LBVH height " + std::to_string(m.height) + " exceeds the traversal stack");
-  return rc;
-}
-
-/* Chunk boxes (with room for one more) over the elements in `order`. */
-static int build_chunk_boxes(Ctx* c, Mesh& m, int nv, const int32_t* order) {
-  const int chunks = (m.nelem + 63) / 64;
-  HCHK(c, hipMalloc((void**)&m.cbox, 6 * sizeof(double) * ((size_t)chunks + 1)));
-  hipLaunchKernelGGL(k_chunk_boxes, dim3(chunks), dim3(64), 0, c->stream, m.V, m.E, nv, order, m.nelem, m.cbox);
-  return hip_check(c, hipGetLastError(), "k_chunk_boxes");
-}
-
-/* A soft mesh's tables for the work items: boxes of its chunks of 64 leaves,
- * and its LBVH's frontiers. */
-static int build_item_tables(Ctx* c, Mesh& m) {
-  int rc = build_chunk_boxes(c, m, 4, m.leaf);
-  if (!rc) rc = hip_check(c, hipMalloc((void**)&m.roots, sizeof(int32_t) * HCS_ROOTS), "hipMalloc");
+  /* scratch of the build, kept by the context while it is small */
+  Slices S;
+  const size_t o_out = S.take<BuildOut>(1), o_seen = S.take<unsigned>(n), o_codes = S.take<unsigned>(n),
+               o_codes2 = S.take<unsigned>(n), o_idx = S.take<int>(n), o_np = S.take<int>(n), o_lp = S.take<int>(n),
+               o_range = S.take<int2>(n), o_ubox = S.take<double>(6 * (size_t)n), o_sbox = S.take<double>(6 * (size_t)schunks);
+  const size_t sort_bytes = sort_temp_bytes(n, sizeof(unsigned));
+  const size_t o_sort = S.take<char>(sort_bytes);
+  int rc = ensure(c, c->d_build, S.bytes);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_frontiers, dim3(1), dim3(HCS_ROOTS / 2), 0, c->stream, m.nodes, m.nelem - 1, m.roots);
-  rc = hip_check(c, hipGetLastError(), "k_frontiers");
-  if (!rc)
-    rc = hip_check(c, hipMemcpyAsync(m.roots_h, m.roots, sizeof(int32_t) * HCS_ROOTS, hipMemcpyDeviceToHost, c->stream),
-                   "memcpy");
-  return rc ? rc : hip_check(c, hipStreamSynchronize(c->stream), "sync");
-}
-
-static void free_mesh(Mesh& m) {
-  for (void* p : {(void*)m.V, (void*)m.E, (void*)m.p, (void*)m.rec, (void*)m.box, (void*)m.nodes, (void*)m.nrm,
-                  (void*)m.leaf, (void*)m.boxL, (void*)m.qorder, (void*)m.fpl, (void*)m.wnodes, (void*)m.cbox,
-                  (void*)m.roots})
-    if (p) (void)hipFree(p);
-  m = Mesh();
+  char* B = (char*)c->d_build.ptr;
+  BuildOut* out = (BuildOut*)(B + o_out);
+  unsigned *codes = (unsigned*)(B + o_codes), *codes2 = (unsigned*)(B + o_codes2);
+  int *idx = (int*)(B + o_idx), *np = (int*)(B + o_np), *lp = (int*)(B + o_lp);
+  int2* range = (int2*)(B + o_range);
+  double *ubox = (double*)(B + o_ubox), *sbox = (double*)(B + o_sbox);
+  const dim3 g((n + 255) / 256), gi((n - 1 + 255) / 256), t(256);
+  /* out and seen are adjacent */
+  launch_fill_u32(s, (unsigned*)out, 0u, (int)((o_codes - o_out) / 4));
+  hipLaunchKernelGGL(k_morton, g, t, 0, s, m.box, n, lo[0], lo[1], lo[2], sc[0], sc[1], sc[2], codes, idx);
+  if (radix_sort_pairs_u32(s, codes, codes2, idx, m.leaf, n, 0, 30, B + o_sort, sort_bytes) != 0)
+    return set_err(c, HCS_ERR_LIMIT, "LBVH build: too many tets to sort");
+  hipLaunchKernelGGL(k_check_order, g, t, 0, s, (const unsigned*)codes2, (const int*)m.leaf, n, (unsigned*)(B + o_seen),
+                     out);
+  hipLaunchKernelGGL(k_leaf_boxes, dim3(chunks), dim3(64), 0, s, (const double*)m.box, (const int*)m.leaf, n,
+                     (const BuildOut*)out, m.boxL, m.cbox);
+  if (n > 1) {
+    hipLaunchKernelGGL(k_box_chunks, dim3(schunks), dim3(64), 0, s, (const double*)m.cbox, chunks, sbox);
+    hipLaunchKernelGGL(k_karras, gi, t, 0, s, (const unsigned*)codes2, (const int*)m.leaf, n, (const BuildOut*)out,
+                       m.nodes, np, lp, range);
+    hipLaunchKernelGGL(k_node_boxes, dim3((n - 1 + 63) / 64), dim3(64), 0, s, (const double*)m.boxL,
+                       (const double*)m.cbox, (const double*)sbox, (const int2*)range, n - 1, (const BuildOut*)out, ubox);
+    hipLaunchKernelGGL(k_fill_nodes, gi, t, 0, s, (const double*)ubox, (const double*)m.box, n - 1,
+                       (const BuildOut*)out, m.nodes, m.wnodes);
+    hipLaunchKernelGGL(k_tree_height, g, t, 0, s, (const int*)lp, (const int*)np, n, out);
+  }
+  hipLaunchKernelGGL(k_frontiers, dim3(1), dim3(HCS_ROOTS / 2), 0, s, (const Node*)m.nodes, n - 1, out, m.roots);
+  rc = hip_check(c, hipGetLastError(), "LBVH build");
+  BuildOut* got = (BuildOut*)c->pin_down; /* (at least 64 KB) */
+  static_assert(sizeof(BuildOut) <= (64 << 10), "build result fits the pinned block");
+  if (!rc) rc = hip_check(c, hipMemcpyAsync(got, out, sizeof *got, hipMemcpyDeviceToHost, s), "memcpy");
+  if (!rc) rc = hip_check(c, hipStreamSynchronize(s), "sync");
+  if (c->d_build.bytes > HCS_SPARE_BYTES) {
+    (void)hipStreamSynchronize(s);
+    (void)hipFree(c->d_build.ptr);
+    c->d_build = DBuf();
+  }
+  if (rc) return rc;
+  if (got->bad) return set_err(c, HCS_ERR_HIP, "LBVH build: the Morton sort returned an invalid order");
+  m.height = got->height;
+  std::memcpy(m.roots_h, got->roots, sizeof m.roots_h);
+  if (3 * ((m.height + 1) / 2) + 1 > HCS_STACK)
+    return set_err(c, HCS_ERR_LIMIT, "LBVH height " + std::to_string(m.height) + " exceeds the traversal stack");
+  return HCS_OK;
 }
 
 /* Frontier depth of each triangle / soft pair's items, chosen from sizes
@@ -1427,10 +1496,11 @@ int hcs_destroy(hcs_ctx* h) {
   (void)hipStreamSynchronize(c->stream);
   while (!c->batches.empty()) hcs_batch_destroy(*c->batches.begin());
   for (auto& m : c->meshes) free_mesh(m);
+  if (c->spare) (void)hipFree(c->spare);
   pipe_free(c->pipe);
   for (DBuf* b : {&c->d_envs, &c->d_state, &c->d_items, &c->d_face_rec, &c->d_face_key, &c->d_face_cnt, &c->d_poly_rec, &c->d_poly_key, &c->d_poly_cnt,
                   &c->d_cand, &c->d_cand_cnt, &c->d_tx_cnt, &c->d_tx_off, &c->d_tx_list, &c->d_tx_out,
-                  &c->d_tx_grid})
+                  &c->d_tx_grid, &c->d_build})
     if (b->ptr) (void)hipFree(b->ptr);
   TaxelSensorBufs& T = c->ts;
   for (DBuf* b : {&T.mask, &T.k64, &T.kp, &T.idx, &T.cnt, &T.nfan, &T.fan_off, &T.tmp, &T.tris, &T.surf, &T.scnt, &T.soff,
@@ -1472,19 +1542,30 @@ static int make_soft(Ctx* c, const double* V, int32_t nv, const int32_t* T, int3
   m.props = *props;
   m.nv = nv;
   m.nelem = nt;
-  int rc = upload(c, (void**)&m.V, V, 3 * sizeof(double) * nv);
-  if (rc == HCS_OK) rc = upload(c, (void**)&m.E, T, 4 * sizeof(int32_t) * nt);
-  if (rc == HCS_OK) rc = upload(c, (void**)&m.p, pr, sizeof(double) * nv);
-  if (rc == HCS_OK) rc = hip_check(c, hipMalloc((void**)&m.rec, (size_t)HCS_TREC * sizeof(double) * nt), "hipMalloc");
-  if (rc == HCS_OK) rc = hip_check(c, hipMalloc((void**)&m.box, 6 * sizeof(double) * (size_t)nt), "hipMalloc");
-  if (rc == HCS_OK) rc = hip_check(c, hipMalloc((void**)&m.fpl, 16 * sizeof(float) * (size_t)nt), "hipMalloc");
-  if (rc == HCS_OK) {
+  const size_t n = nt, ni = n > 1 ? n - 1 : 1;
+  Slices S;
+  const size_t oV = S.take<double>(3 * (size_t)nv), oE = S.take<int32_t>(4 * n), op = S.take<double>(nv),
+               orec = S.take<double>(HCS_TREC * n), obox = S.take<double>(6 * n), ofpl = S.take<float>(16 * n),
+               onodes = S.take<Node>(ni), ow = S.take<WNode>(ni), oleaf = S.take<int32_t>(n), oL = S.take<double>(6 * n),
+               oc = S.take<double>(6 * ((n + 63) / 64)), oroots = S.take<int32_t>(HCS_ROOTS);
+  int rc = mesh_alloc(c, m, S.bytes);
+  if (rc != HCS_OK) {
+    m = Mesh();
+    return rc;
+  }
+  char* P = (char*)m.mem;
+  m.V = (double*)(P + oV), m.E = (int32_t*)(P + oE), m.p = (double*)(P + op), m.rec = (double*)(P + orec);
+  m.box = (double*)(P + obox), m.fpl = (float*)(P + ofpl), m.nodes = (Node*)(P + onodes), m.wnodes = (WNode*)(P + ow);
+  m.leaf = (int32_t*)(P + oleaf), m.boxL = (double*)(P + oL), m.cbox = (double*)(P + oc), m.roots = (int32_t*)(P + oroots);
+  rc = hip_check(c, hipMemcpyAsync(m.V, V, 3 * sizeof(double) * nv, hipMemcpyHostToDevice, c->stream), "upload");
+  if (!rc) rc = hip_check(c, hipMemcpyAsync(m.E, T, 4 * sizeof(int32_t) * nt, hipMemcpyHostToDevice, c->stream), "upload");
+  if (!rc) rc = hip_check(c, hipMemcpyAsync(m.p, pr, sizeof(double) * nv, hipMemcpyHostToDevice, c->stream), "upload");
+  if (!rc) {
     hipLaunchKernelGGL(k_tet_precompute, dim3((nt + 127) / 128), dim3(128), 0, c->stream, m.V, m.E, m.p, nt, m.rec,
                        m.box, (float4*)m.fpl);
     rc = hip_check(c, hipGetLastError(), "k_tet_precompute");
   }
-  if (rc == HCS_OK) rc = build_bvh(c, m);
-  if (rc == HCS_OK) rc = build_item_tables(c, m);
+  if (!rc) rc = build_bvh(c, m, V);
   if (rc != HCS_OK) {
     (void)hipStreamSynchronize(c->stream);
     free_mesh(m);
@@ -1507,56 +1588,68 @@ static int make_rigid(Ctx* c, const double* V, int32_t nv, const int32_t* F, int
   m.props = *props;
   m.nv = nv;
   m.nelem = ntri;
-  int rc = upload(c, (void**)&m.V, V, 3 * sizeof(double) * nv);
-  if (rc == HCS_OK) rc = upload(c, (void**)&m.E, F, 3 * sizeof(int32_t) * ntri);
-  if (rc == HCS_OK) {
-    /* query order: triangles sorted by the Morton code of their centroids,
-     * so a work item's 64 triangles are spatially compact */
-    std::vector<double> cen(3 * (size_t)ntri);
-    double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-    for (int32_t t = 0; t < ntri; ++t)
-      for (int k = 0; k < 3; ++k) {
-        const double x = (V[3 * F[3 * t] + k] + V[3 * F[3 * t + 1] + k] + V[3 * F[3 * t + 2] + k]) / 3.0;
-        cen[3 * (size_t)t + k] = x;
-        lo[k] = std::min(lo[k], x), hi[k] = std::max(hi[k], x);
-      }
-    auto spread = [](uint32_t v) {
-      v = (v * 0x00010001u) & 0xFF0000FFu;
-      v = (v * 0x00000101u) & 0x0F00F00Fu;
-      v = (v * 0x00000011u) & 0xC30C30C3u;
-      v = (v * 0x00000005u) & 0x49249249u;
-      return v;
-    };
-    std::vector<uint32_t> code(ntri);
-    for (int32_t t = 0; t < ntri; ++t) {
-      uint32_t q[3];
-      for (int k = 0; k < 3; ++k) {
-        const double u = hi[k] > lo[k] ? (cen[3 * (size_t)t + k] - lo[k]) / (hi[k] - lo[k]) * 1023.0 : 0.0;
-        q[k] = (uint32_t)std::min(1023.0, std::max(0.0, u));
-      }
-      code[t] = (spread(q[0]) << 2) | (spread(q[1]) << 1) | spread(q[2]);
+  const size_t n = ntri, chunks = (n + 63) / 64;
+  Slices S;
+  const size_t oV = S.take<double>(3 * (size_t)nv), oE = S.take<int32_t>(3 * n), oq = S.take<int32_t>(n),
+               on = S.take<double>(3 * n), oc = S.take<double>(6 * (chunks + 1));
+  int rc = mesh_alloc(c, m, S.bytes);
+  if (rc != HCS_OK) {
+    m = Mesh();
+    return rc;
+  }
+  char* P = (char*)m.mem;
+  m.V = (double*)(P + oV), m.E = (int32_t*)(P + oE), m.qorder = (int32_t*)(P + oq), m.nrm = (double*)(P + on);
+  m.cbox = (double*)(P + oc);
+  rc = hip_check(c, hipMemcpyAsync(m.V, V, 3 * sizeof(double) * nv, hipMemcpyHostToDevice, c->stream), "upload");
+  if (!rc) rc = hip_check(c, hipMemcpyAsync(m.E, F, 3 * sizeof(int32_t) * ntri, hipMemcpyHostToDevice, c->stream), "upload");
+  /* query order: triangles sorted by the Morton code of their centroids,
+   * so a work item's 64 triangles are spatially compact */
+  std::vector<double> cen(3 * (size_t)ntri);
+  double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+  for (int32_t t = 0; t < ntri; ++t)
+    for (int k = 0; k < 3; ++k) {
+      const double x = (V[3 * F[3 * t] + k] + V[3 * F[3 * t + 1] + k] + V[3 * F[3 * t + 2] + k]) / 3.0;
+      cen[3 * (size_t)t + k] = x;
+      lo[k] = std::min(lo[k], x), hi[k] = std::max(hi[k], x);
     }
-    std::vector<int32_t> order(ntri);
-    for (int32_t t = 0; t < ntri; ++t) order[t] = t;
-    std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return code[a] < code[b]; });
-    rc = upload(c, (void**)&m.qorder, order.data(), sizeof(int32_t) * (size_t)ntri);
+  auto spread = [](uint32_t v) {
+    v = (v * 0x00010001u) & 0xFF0000FFu;
+    v = (v * 0x00000101u) & 0x0F00F00Fu;
+    v = (v * 0x00000011u) & 0xC30C30C3u;
+    v = (v * 0x00000005u) & 0x49249249u;
+    return v;
+  };
+  std::vector<uint32_t> code(ntri);
+  for (int32_t t = 0; t < ntri; ++t) {
+    uint32_t q[3];
+    for (int k = 0; k < 3; ++k) {
+      const double u = hi[k] > lo[k] ? (cen[3 * (size_t)t + k] - lo[k]) / (hi[k] - lo[k]) * 1023.0 : 0.0;
+      q[k] = (uint32_t)std::min(1023.0, std::max(0.0, u));
+    }
+    code[t] = (spread(q[0]) << 2) | (spread(q[1]) << 1) | spread(q[2]);
   }
-  if (rc == HCS_OK) rc = hip_check(c, hipMalloc((void**)&m.nrm, 3 * sizeof(double) * (size_t)ntri), "hipMalloc");
-  if (rc == HCS_OK) {
-    hipLaunchKernelGGL(k_tri_normals, dim3((ntri + 127) / 128), dim3(128), 0, c->stream, m.V, m.E, ntri, m.nrm);
-    rc = hip_check(c, hipGetLastError(), "k_tri_normals");
-  }
+  std::vector<int32_t> order(ntri);
+  for (int32_t t = 0; t < ntri; ++t) order[t] = t;
+  std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return code[a] < code[b]; });
+  if (!rc)
+    rc = hip_check(c, hipMemcpyAsync(m.qorder, order.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice, c->stream), "upload");
   double vbox[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
-  if (rc == HCS_OK) rc = build_chunk_boxes(c, m, 3, m.qorder);
-  if (rc == HCS_OK) {
-    for (int32_t v = 0; v < nv; ++v)
-      for (int k = 0; k < 3; ++k)
-        vbox[k] = std::fmin(vbox[k], V[3 * (size_t)v + k]), vbox[3 + k] = std::fmax(vbox[3 + k], V[3 * (size_t)v + k]);
-    rc = hip_check(c, hipMemcpyAsync(m.cbox + 6 * (size_t)((ntri + 63) / 64), vbox, sizeof vbox, hipMemcpyHostToDevice,
-                                     c->stream), "upload");
+  for (int32_t v = 0; v < nv; ++v)
+    for (int k = 0; k < 3; ++k)
+      vbox[k] = std::fmin(vbox[k], V[3 * (size_t)v + k]), vbox[3 + k] = std::fmax(vbox[3 + k], V[3 * (size_t)v + k]);
+  if (!rc)
+    rc = hip_check(c, hipMemcpyAsync(m.cbox + 6 * chunks, vbox, sizeof vbox, hipMemcpyHostToDevice, c->stream), "upload");
+  if (!rc) {
+    hipLaunchKernelGGL(k_tri_normals, dim3((ntri + 127) / 128), dim3(128), 0, c->stream, m.V, m.E, ntri, m.nrm);
+    hipLaunchKernelGGL(k_chunk_boxes, dim3((unsigned)chunks), dim3(64), 0, c->stream, m.V, m.E, 3,
+                       (const int32_t*)m.qorder, ntri, m.cbox);
+    rc = hip_check(c, hipGetLastError(), "rigid mesh kernels");
   }
-  if (rc == HCS_OK) rc = hip_check(c, hipStreamSynchronize(c->stream), "sync");
-  if (rc != HCS_OK) free_mesh(m);
+  if (!rc) rc = hip_check(c, hipStreamSynchronize(c->stream), "sync");
+  if (rc != HCS_OK) {
+    (void)hipStreamSynchronize(c->stream);
+    free_mesh(m);
+  }
   return rc;
 }
 
@@ -1569,7 +1662,7 @@ static int install_mesh(Ctx* c, int32_t handle, Mesh& m) {
     free_mesh(m);
     return rc;
   }
-  free_mesh(c->meshes[handle]);
+  retire_mesh(c, c->meshes[handle]);
   c->meshes[handle] = m;
   c->last_valid = 0;
   return batches_refresh(c, handle);

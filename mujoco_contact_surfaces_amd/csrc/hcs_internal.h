@@ -18,6 +18,9 @@ struct Mesh {
   int32_t geom_id = 0;
   hcs_props props{};
   int32_t nv = 0, nelem = 0, height = 0;
+  /* the arrays below are slices of one allocation */
+  void* mem = nullptr;
+  size_t mem_bytes = 0;
   double* V = nullptr;
   int32_t* E = nullptr; /* T (soft) or F (rigid) */
   double* p = nullptr;
@@ -105,6 +108,10 @@ struct Ctx {
   DBuf d_cand, d_cand_cnt;
   DBuf d_tx_cnt, d_tx_off, d_tx_list, d_tx_out, d_tx_grid;
   TaxelSensorBufs ts;
+  DBuf d_build; /* scratch of the LBVH build */
+  /* memory of the last replaced mesh, for the next one */
+  void* spare = nullptr;
+  size_t spare_bytes = 0;
   /* last contact step's polygons (for taxels) */
   int64_t last_npoly = 0;
   int last_valid = 0;

@@ -5,7 +5,8 @@
  * 32- or 64-bit keys with int32 values (Morton codes of the LBVH build,
  * polygon keys of the sensors).
  *
- * Scan (reduce-then-scan, three launches, no atomics, no waits): tiles of
+ * Scan (reduce-then-scan, three launches, no atomics, no waits; one block and
+ * one launch up to 32768 counts): tiles of
  * 2048 counts (256 threads x 8), a per-tile sum, one block scanning the
  * tile sums, then every tile scanned again with its offset.  Within a block
  * each thread sums its 8 contiguous counts, a wave scans the thread sums
@@ -115,6 +116,34 @@ __global__ __launch_bounds__(kThreads) void k_scan_apply(const unsigned* in, lon
   }
 }
 
+/* A short scan (at most kOneTiles tiles) in one launch of one block: three
+ * launches and their gaps cost more than a block's passes over it (6400
+ * digit counts of a 51k-key sort pass: 10 us and two gaps -> 7.6 us). */
+constexpr int kOneTile = kSumThreads * kPer;
+constexpr int kOneTiles = 4;
+__global__ __launch_bounds__(kSumThreads) void k_scan_one(const unsigned* in, int n, unsigned* out) {
+  __shared__ unsigned lds[kSumThreads / 64];
+  unsigned carry = 0;
+  for (int t0 = 0; t0 < n; t0 += kOneTile) {
+    const int base = t0 + threadIdx.x * kPer;
+    unsigned v[kPer];
+    unsigned s = 0;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      v[j] = base + j < n ? in[base + j] : 0u;
+      s += v[j];
+    }
+    unsigned total;
+    unsigned run = carry + block_excl_scan(s, lds, &total);
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      if (base + j < n) out[base + j] = run;
+      run += v[j];
+    }
+    carry += total;
+  }
+}
+
 template <class K>
 __global__ __launch_bounds__(kThreads) void k_radix_hist(const K* __restrict__ keys, long long n, int shift,
                                                         unsigned dmask, int ntiles, unsigned* __restrict__ hist) {
@@ -187,6 +216,10 @@ int exclusive_scan_u32(hipStream_t s, const unsigned* in, unsigned* out, long lo
   if (n <= 0) return 0;
   const long long tiles = (n + kTile - 1) / kTile;
   if (tiles > (long long)kSumThreads * kMaxSumPer || tmp_bytes < scan_temp_bytes(n)) return -1;
+  if (n <= (long long)kOneTiles * kOneTile) {
+    hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(kSumThreads), 0, s, in, (int)n, out);
+    return 0;
+  }
   const int per = (int)((tiles + kSumThreads - 1) / kSumThreads);
   unsigned* sums = (unsigned*)tmp;
   hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)tiles), dim3(kThreads), 0, s, in, n, sums);

@@ -82,3 +82,32 @@ def test_many_pairs_with_and_without_contact(engine, n):
     assert rc == 0, engine.lib.hcs_last_error(engine.h)
     Wn = np.frombuffer(got, np.float64).reshape(n, 16)[:, :12]
     np.testing.assert_array_equal(Wn, W)
+
+
+@pytest.mark.parametrize("sizes", [[(3, 2), (3, 3), (3, 2), (3, 1)], [(4, 4), (1, 1), (4, 4), (4, 3), (0, 1)]],
+                         ids=["alike", "very different"])
+def test_replaced_meshes(sizes):
+    """A soft geom re-meshed again and again (its memory is reused where it
+    fits) steps like a new one of that mesh, tree height included."""
+    from mujoco_contact_surfaces_amd import Engine
+
+    sc = S.tactile_pad(5, L=2, K=2, m=16)
+    s, r = sc["soft"], sc["rigid"]
+    e = Engine(0)
+    ha = e.add_soft_mesh(s["V"], s["T"], s["p"], s["props"], 0)
+    hb = e.add_rigid_mesh(r["V"], r["F"], r["props"], 1)
+    for L, K in sizes:
+        V, T, p = S.soft_mesh(L, K, 1, 0.04, 0.03, 0.02, 5e4)
+        e.replace_soft_mesh(ha, V, T, p)
+        W, cnt = e.contact_step([(ha, hb, sc["X_WA"], sc["X_WB"], sc["V_WA"], sc["V_WB"])])
+        hn = e.add_soft_mesh(V, T, p, s["props"], 0)
+        Wn, cn = e.contact_step([(hn, hb, sc["X_WA"], sc["X_WB"], sc["V_WA"], sc["V_WB"])])
+        np.testing.assert_array_equal(cnt, cn)
+        np.testing.assert_array_equal(W, Wn)
+        np.testing.assert_array_equal(e.tet_records(ha), e.tet_records(hn))
+        assert e.mesh_info(ha) == e.mesh_info(hn) and (T.shape[0] == 1 or e.mesh_info(ha)["bvh_height"] > 0)
+        ref = O.soft_rigid(V, T, p, r["V"], r["F"], sc["X_WA"], sc["X_WB"], sc["V_WA"], sc["V_WB"], 5e4,
+                           s["props"]["dissipation"], s["props"]["dynamic_friction"], r["props"]["dynamic_friction"])
+        np.testing.assert_array_equal(cnt[0], ref["counts"])
+        assert_wrench_close(W[0], ref["wrench"])
+    e.close()
