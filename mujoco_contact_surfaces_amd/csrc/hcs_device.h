@@ -399,6 +399,11 @@ __device__ inline T polygon_centroid(const Poly<T>& p, const T* nrm, T* C) {
   return W;
 }
 
+/* Lanes of mask m below this lane. */
+__device__ inline unsigned lane_prefix(unsigned long long m) {
+  return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+}
+
 /* ------------------------------------------------------------ force law */
 
 /* Everything of one pair a face evaluation needs (W frame). */

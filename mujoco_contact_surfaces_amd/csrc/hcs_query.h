@@ -94,11 +94,6 @@ __device__ inline void make_item_ctx<Dual>(const EnvDesc& E, const double* st, i
   c.repr = E.repr;
 }
 
-/* Lanes of mask m below this lane. */
-__device__ inline unsigned lane_prefix(unsigned long long m) {
-  return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-}
-
 struct OutPtrs {
   double* face_rec;
   int64_t* face_key;

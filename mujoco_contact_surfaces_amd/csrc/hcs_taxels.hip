@@ -70,14 +70,15 @@ __global__ __launch_bounds__(64) void k_tx_sample(const double* __restrict__ pol
   if (threadIdx.x == 0) out[x + g.cx * y] = v;
 }
 
-/* The same, fan-major (double, S^2 <= HCS_TX_RAYS). */
-__global__ __launch_bounds__(64) void k_tx_sample_fan(const double* __restrict__ poly, const int64_t* __restrict__ key,
+/* The same, fan-major (double, S^2 <= HCS_TX_RAYS), W waves per taxel. */
+template <int W>
+__global__ __launch_bounds__(64 * W) void k_tx_sample_fan(const double* __restrict__ poly, const int64_t* __restrict__ key,
                                                       TaxelGridDev g, const unsigned* __restrict__ off,
                                                       const unsigned* __restrict__ cnt, const int* __restrict__ list,
                                                       double* __restrict__ out) {
   const int cell = blockIdx.x;
   const int x = cell % g.cx, y = cell / g.cx;
-  const double v = sample_cell_scatter(poly, key, g, off[cell], cnt[cell], list, x, y);
+  const double v = sample_cell_scatter<W>(poly, key, g, off[cell], cnt[cell], list, x, y);
   if (threadIdx.x == 0) out[x + g.cx * y] = v;
 }
 
@@ -116,9 +117,16 @@ int run_taxels(Ctx* c, const TaxelGridDev& g, const unsigned char* d_mask, const
   if (ptan)
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_tx_sample<Dual>), dim3(ncell), dim3(64), 0, c->stream, poly, ptan, key, g,
                        Xd, (const unsigned*)off, (const unsigned*)cnt, (const int*)c->d_tx_list.ptr, d_out);
-  else if (g.S * g.S <= HCS_TX_RAYS && c->last_pairs.size() < (1u << 19))
-    hipLaunchKernelGGL(k_tx_sample_fan, dim3(ncell), dim3(64), 0, c->stream, poly, key, g, (const unsigned*)off,
-                       (const unsigned*)cnt, (const int*)c->d_tx_list.ptr, d_out);
+  else if (g.S * g.S <= HCS_TX_RAYS && c->last_pairs.size() < (1u << 19)) {
+    /* up to eight taxels a CU, four waves share a taxel: 256 taxels 52 -> 22
+     * us, 1600 taxels 21 -> 14 us; with 3600 taxels 14 -> 16 us */
+    auto run = [&](auto kernel, int waves) {
+      hipLaunchKernelGGL(kernel, dim3(ncell), dim3(64 * waves), 0, c->stream, poly, key, g, (const unsigned*)off,
+                         (const unsigned*)cnt, (const int*)c->d_tx_list.ptr, d_out);
+    };
+    if (ncell <= 8 * c->num_cu) run(k_tx_sample_fan<4>, 4);
+    else run(k_tx_sample_fan<1>, 1);
+  }
   else
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_tx_sample<double>), dim3(ncell), dim3(64), 0, c->stream, poly,
                        (const double*)nullptr, key, g, (const double*)nullptr, (const unsigned*)off,
