@@ -167,19 +167,16 @@ int hcs_taxel_jacobian(hcs_ctx* h, const hcs_pair_in* pair, const hcs_step_opts*
   int rc = hcs_contact_step(h, 1, pair, &oc, &po, nullptr);
   if (rc) return rc;
   const int64_t cap = std::max<int64_t>(1, po.n_polygons);
-  DBuf prec, ptan, pkey, dXd, dmask, dout;
+  DBuf prec, ptan, pkey, dXd;
   auto cleanup = [&]() {
-    for (DBuf* b : {&prec, &ptan, &pkey, &dXd, &dmask, &dout})
+    for (DBuf* b : {&prec, &ptan, &pkey, &dXd})
       if (b->ptr) (void)hipFree(b->ptr);
   };
   if ((rc = ensure(c, prec, sizeof(double) * HCS_PREC * cap)) || (rc = ensure(c, ptan, sizeof(double) * HCS_PREC * cap)) ||
-      (rc = ensure(c, pkey, sizeof(int64_t) * 3 * cap)) || (rc = ensure(c, dXd, sizeof(double) * 12)) ||
-      (rc = ensure(c, dmask, 8)) || (rc = ensure(c, dout, sizeof(double) * ncell))) {
+      (rc = ensure(c, pkey, sizeof(int64_t) * 3 * cap)) || (rc = ensure(c, dXd, sizeof(double) * 12))) {
     cleanup();
     return rc;
   }
-  const unsigned char one = 1;
-  rc = hip_check(c, hipMemcpyAsync(dmask.ptr, &one, 1, hipMemcpyHostToDevice, c->stream), "upload");
   const double* R = pair->X_WB;
   for (int d = 0; d < kDirs && !rc; ++d) {
     /* tangent of the sensor pose (the sensor rides on geometry B) */
@@ -203,13 +200,9 @@ int hcs_taxel_jacobian(hcs_ctx* h, const hcs_pair_in* pair, const hcs_step_opts*
     rc = tangent_pass(c, 1, pair, &o, d, 1, (double*)prec.ptr, (double*)ptan.ptr, (int64_t*)pkey.ptr, cap, plan, &np);
     if (rc) break;
     const int64_t n = std::min<int64_t>((int64_t)np, cap);
-    rc = run_taxels(c, g, (const unsigned char*)dmask.ptr, (const double*)prec.ptr, (const double*)ptan.ptr,
-                    (const int64_t*)pkey.ptr, n, (const double*)dXd.ptr, (double*)dout.ptr);
     std::vector<double> col(ncell);
-    if (!rc)
-      rc = hip_check(c, hipMemcpyAsync(col.data(), dout.ptr, sizeof(double) * ncell, hipMemcpyDeviceToHost, c->stream),
-                     "dl");
-    if (!rc) rc = hip_check(c, hipStreamSynchronize(c->stream), "sync");
+    rc = run_taxels(c, g, {1}, (const double*)prec.ptr, (const double*)ptan.ptr, (const int64_t*)pkey.ptr, n,
+                    (const double*)dXd.ptr, col.data());
     for (int k = 0; k < ncell && !rc; ++k) Jt[(size_t)k * kDirs + d] = col[k];
   }
   cleanup();

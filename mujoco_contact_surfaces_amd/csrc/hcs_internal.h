@@ -106,7 +106,7 @@ struct Ctx {
   DBuf d_face_rec, d_face_key, d_face_cnt;
   DBuf d_poly_rec, d_poly_key, d_poly_cnt;
   DBuf d_cand, d_cand_cnt;
-  DBuf d_tx_cnt, d_tx_off, d_tx_list, d_tx_out, d_tx_grid;
+  DBuf d_tx_cnt, d_tx_off, d_tx_foot, d_tx_list, d_tx_out, d_tx_grid;
   TaxelSensorBufs ts;
   DBuf d_build; /* scratch of the LBVH build */
   /* memory of the last replaced mesh, for the next one */
@@ -218,8 +218,8 @@ void launch_prep(hipStream_t s, const EnvDesc* envs, const double* state, double
 void launch_fill_u32(hipStream_t s, unsigned int* p, unsigned int v, int n);
 
 int taxel_grid_dev(const hcs_taxel_grid& G, TaxelGridDev& g);
-int run_taxels(Ctx* c, const TaxelGridDev& g, const unsigned char* d_mask, const double* poly, const double* ptan,
-               const int64_t* key, int64_t np, const double* Xd, double* d_out);
+int run_taxels(Ctx* c, const TaxelGridDev& g, const std::vector<unsigned char>& seen, const double* poly,
+               const double* ptan, const int64_t* key, int64_t np, const double* Xd, double* out);
 
 /* Flat tactile sensors of a batch (hcs_batch_set_sensors): sensor s samples
  * the polygons of its pair only, at the pose of one of the pair's two
@@ -231,7 +231,8 @@ struct BatchTaxels {
   int ncell = 0; /* taxels of all sensors */
   DBuf grid /* TaxelGridDev per sensor, pose written per step */, src /* int per sensor: 36 pair + 12 side */,
       cell_base /* int[n + 1] */, cell_sensor /* int per taxel */, psoff /* int[npairs + 1] */, psens /* int[n] */,
-      mask /* uchar per pair: has a sensor */, poly_rec, poly_key, poly_cnt /* ull */, cnt /* unsigned[ncell + 1] */,
+      mask /* uchar per pair: has a sensor */, poly_rec, poly_key, foot /* int4 per polygon */,
+      poly_cnt /* ull */, cnt /* unsigned[ncell + 1] */,
       cursor /* unsigned[ncell] */, off /* unsigned[ncell + 1] */, scan_tmp, list /* int[list_cap] */,
       out /* double per taxel */, live /* int[ncell]: taxels with candidate polygons */;
   int64_t poly_cap = 0, list_cap = 0;

@@ -16,16 +16,22 @@
 
 namespace hcs {
 
+/* The taxels that polygon P's vertices span.  All eight vertex slots are read
+ * at once (a record holds them all): a loop to n waited for memory at every
+ * vertex. */
 __device__ inline void footprint(const double* P, const TaxelGridDev& g, int& x0, int& x1, int& y0, int& y1) {
   const int n = (int)P[0];
+  double v[24];
+#pragma unroll
+  for (int i = 0; i < 24; ++i) v[i] = P[1 + i];
   double lo[2] = {1e300, 1e300}, hi[2] = {-1e300, -1e300};
-  for (int i = 0; i < n; ++i) {
-    const double* v = P + 1 + 3 * i;
-    double d[3] = {v[0] - g.X[9], v[1] - g.X[10], v[2] - g.X[11]};
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const double d[3] = {v[3 * i] - g.X[9], v[3 * i + 1] - g.X[10], v[3 * i + 2] - g.X[11]};
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
-      double l = (g.X[c] * d[0] + g.X[3 + c] * d[1]) + g.X[6 + c] * d[2];
-      lo[c] = fmin(lo[c], l), hi[c] = fmax(hi[c], l);
+      const double l = (g.X[c] * d[0] + g.X[3 + c] * d[1]) + g.X[6 + c] * d[2];
+      lo[c] = i < n ? fmin(lo[c], l) : lo[c], hi[c] = i < n ? fmax(hi[c], l) : hi[c];
     }
   }
   const double m = 1e-9;

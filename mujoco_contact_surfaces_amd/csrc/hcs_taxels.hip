@@ -37,36 +37,98 @@ using namespace hcs;
 
 namespace hcs {
 
-__global__ void k_tx_bin(const double* __restrict__ poly, const int64_t* __restrict__ key, int64_t np,
-                         const unsigned char* __restrict__ env_mask, TaxelGridDev g, unsigned* __restrict__ cnt,
-                         const unsigned* __restrict__ off, unsigned* __restrict__ cursor, int* __restrict__ list) {
+/* Pairs whose polygons a sensor sees: bits for up to 256 pairs (they travel
+ * with the launch), a byte per pair in device memory beyond. */
+struct TxPairs {
+  unsigned long long bits[4];
+  const unsigned char* mask;
+  __device__ bool has(int64_t e) const { return mask ? mask[e] != 0 : (bits[e >> 6] >> (e & 63) & 1) != 0; }
+};
+
+/* Adds one to counter[cell] for every lane with on set and returns the lane's
+ * place; lanes of one cell share an atomic, for the first HCS_TX_SHARE cells
+ * (the rest go by themselves).  Neighbouring small polygons lie in few taxels,
+ * whose counters share cache lines, and atomics on one line complete one after
+ * another; large polygons have their taxels to themselves, and looking for
+ * company costs (none / 6 / 10 / 16 / all cells: a pad of 6.8k polygons 46, 17,
+ * 13, 13 and 12 us; one of 3 mm polygons under 100 x 100 taxels 12, 21, 25, 30
+ * and 38 us).  Called by whole
+ * waves. */
+#define HCS_TX_SHARE 10
+__device__ inline unsigned count_cell(unsigned* __restrict__ counter, int cell, bool on) {
+  const int lane = threadIdx.x & 63;
+  int lead = lane;
+  unsigned rank = 0, n = 1;
+  unsigned long long todo = __ballot(on);
+  for (int r = 0; r < HCS_TX_SHARE && todo != 0; ++r) {
+    const int l = __builtin_ctzll(todo);
+    const bool same = on && cell == __shfl(cell, l, 64);
+    const unsigned long long m = __ballot(same);
+    if (same) lead = l, rank = lane_prefix(m), n = (unsigned)__popcll(m);
+    todo &= ~m;
+  }
+  unsigned base = 0;
+  if (on && lane == lead) base = atomicAdd(counter + cell, n);
+  return __shfl(base, lead, 64) + rank;
+}
+
+/* The taxels of footprint f, numbered base + x + cx y, counted (FILL = 0) or
+ * given polygon q (FILL = 1).  Called by whole waves (an empty footprint: no
+ * polygon). */
+template <int FILL>
+__device__ inline void bin_polygon(int q, const int4& f, int cx, int base, unsigned* __restrict__ counter,
+                                   const unsigned* __restrict__ off, int* __restrict__ list, int64_t list_cap) {
+  int x = f.x, y = f.z;
+  bool on = f.x <= f.y && f.z <= f.w;
+  while (__any(on)) {
+    const int cell = on ? base + x + cx * y : -1;
+    const unsigned k = count_cell(counter, cell, on);
+    if (FILL && on && (int64_t)off[cell] + k < list_cap) list[off[cell] + k] = q;
+    if (++x > f.y) x = f.x, ++y;
+    on = on && y <= f.w;
+  }
+}
+
+/* Binning, one polygon per thread.  FILL = 0 notes the taxels its footprint
+ * covers and counts it there; FILL = 1 writes it into their lists.  Bound by
+ * the latency of one polygon (a few thousand): 64 threads a block, the record
+ * read at once and only in the first pass and shared atomics (count_cell) took
+ * the pair of launches from 50 to 13 us (6.8k polygons). */
+template <int FILL>
+__global__ __launch_bounds__(64) void k_tx_bin(const double* __restrict__ poly, const int64_t* __restrict__ key,
+                                               int64_t np, TxPairs pairs, TaxelGridDev g, int4* __restrict__ foot,
+                                               unsigned* __restrict__ cnt, const unsigned* __restrict__ off,
+                                               int* __restrict__ list, int64_t list_cap) {
   const int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (q >= np) return;
-  if (!env_mask[key[3 * q]]) return;
-  const double* P = poly + q * HCS_PREC;
-  int x0, x1, y0, y1;
-  footprint(P, g, x0, x1, y0, y1);
-  for (int y = y0; y <= y1; ++y)
-    for (int x = x0; x <= x1; ++x) {
-      const int cell = x + g.cx * y;
-      if (!off) {
-        atomicAdd(cnt + cell, 1u);
-      } else {
-        const unsigned slot = atomicAdd(cursor + cell, 1u);
-        list[off[cell] + slot] = (int)q;
-      }
+  int4 f = make_int4(0, -1, 0, -1);
+  if (q < np) {
+    if (FILL) {
+      f = foot[q];
+    } else {
+      if (pairs.has(key[3 * q])) footprint(poly + q * HCS_PREC, g, f.x, f.y, f.z, f.w);
+      foot[q] = f;
     }
+  }
+  bin_polygon<FILL>((int)q, f, g.cx, 0, cnt, off, list, list_cap);
+}
+
+/* A taxel's list: off[cell] .. off[cell + 1], or none of it when it does not
+ * fit the list buffer (the caller sees the total and runs again). */
+__device__ inline unsigned tx_count(const unsigned* __restrict__ off, int cell, int64_t list_cap) {
+  const unsigned a = off[cell], b = off[cell + 1];
+  return a <= b && (int64_t)b <= list_cap ? b - a : 0u;
 }
 
 template <class T>
 __global__ __launch_bounds__(64) void k_tx_sample(const double* __restrict__ poly, const double* __restrict__ ptan,
                                                    const int64_t* __restrict__ key, TaxelGridDev g,
                                                    const double* __restrict__ Xd, const unsigned* __restrict__ off,
-                                                   const unsigned* __restrict__ cnt, const int* __restrict__ list,
+                                                   const int* __restrict__ list, int64_t list_cap,
                                                    double* __restrict__ out) {
   const int cell = blockIdx.x;
   const int x = cell % g.cx, y = cell / g.cx;
-  const double v = sample_cell<T>(poly, ptan, key, g, Xd, off[cell], cnt[cell], list, x, y);
+  if (cell == 0 && threadIdx.x == 0) out[gridDim.x] = (double)off[gridDim.x];
+  const double v = sample_cell<T>(poly, ptan, key, g, Xd, off[cell], tx_count(off, cell, list_cap), list, x, y);
   if (threadIdx.x == 0) out[x + g.cx * y] = v;
 }
 
@@ -74,64 +136,95 @@ __global__ __launch_bounds__(64) void k_tx_sample(const double* __restrict__ pol
 template <int W>
 __global__ __launch_bounds__(64 * W) void k_tx_sample_fan(const double* __restrict__ poly, const int64_t* __restrict__ key,
                                                       TaxelGridDev g, const unsigned* __restrict__ off,
-                                                      const unsigned* __restrict__ cnt, const int* __restrict__ list,
+                                                      const int* __restrict__ list, int64_t list_cap,
                                                       double* __restrict__ out) {
   const int cell = blockIdx.x;
   const int x = cell % g.cx, y = cell / g.cx;
-  const double v = sample_cell_scatter<W>(poly, key, g, off[cell], cnt[cell], list, x, y);
+  if (cell == 0 && threadIdx.x == 0) out[gridDim.x] = (double)off[gridDim.x];
+  const double v = sample_cell_scatter<W>(poly, key, g, off[cell], tx_count(off, cell, list_cap), list, x, y);
   if (threadIdx.x == 0) out[x + g.cx * y] = v;
 }
 
-/* Bins polygons of the masked pairs into the taxel grid and samples it.
- * ptan/Xd select the tangent pass (nullptr: values). */
-int run_taxels(Ctx* c, const TaxelGridDev& g, const unsigned char* d_mask, const double* poly, const double* ptan,
-               const int64_t* key, int64_t np, const double* Xd, double* d_out) {
+/* Bins the polygons of the pairs with seen[e] != 0 into the taxel grid,
+ * samples it and returns the taxels in out (host).  ptan/Xd select the tangent
+ * pass (nullptr: values).  The counts are scanned on the device and the last
+ * kernel writes to pinned memory, so a call waits once; a list buffer that was
+ * too small shows in the total that comes with the taxels, and the lists are
+ * made again. */
+int run_taxels(Ctx* c, const TaxelGridDev& g, const std::vector<unsigned char>& seen, const double* poly,
+               const double* ptan, const int64_t* key, int64_t np, const double* Xd, double* out) {
   const int ncell = g.cx * g.cy;
+  const size_t scan_bytes = scan_temp_bytes((long long)ncell + 1);
   int rc;
-  if ((rc = ensure(c, c->d_tx_cnt, sizeof(unsigned) * 2 * ncell)) ||
-      (rc = ensure(c, c->d_tx_off, sizeof(unsigned) * (ncell + 1))))
+  if ((rc = ensure(c, c->d_tx_cnt, sizeof(unsigned) * ((size_t)ncell + 1))) ||
+      (rc = ensure(c, c->d_tx_off, sizeof(unsigned) * ((size_t)ncell + 1) + scan_bytes + 8)) ||
+      (rc = ensure(c, c->d_tx_foot, sizeof(int4) * (size_t)std::max<int64_t>(1, np))) ||
+      (rc = ensure(c, c->d_tx_list, sizeof(int) * (size_t)std::max<int64_t>(4096, 4 * np))) ||
+      (rc = pinned(c, c->pin_down, c->pin_down_bytes, sizeof(double) * ((size_t)ncell + 1))))
     return rc;
-  unsigned* cnt = (unsigned*)c->d_tx_cnt.ptr;
-  unsigned* cursor = cnt + ncell;
-  unsigned* off = (unsigned*)c->d_tx_off.ptr;
-  rc = hip_check(c, hipMemsetAsync(cnt, 0, sizeof(unsigned) * 2 * ncell, c->stream), "memset");
-  if (rc) return rc;
-  const int64_t nb = (np + 255) / 256;
-  if (np > 0)
-    hipLaunchKernelGGL(k_tx_bin, dim3((unsigned)nb), dim3(256), 0, c->stream, poly, key, np, d_mask, g, cnt,
-                       (const unsigned*)nullptr, (unsigned*)nullptr, (int*)nullptr);
-  std::vector<unsigned> hc(ncell), ho(ncell + 1);
-  rc = hip_check(c, hipMemcpyAsync(hc.data(), cnt, sizeof(unsigned) * ncell, hipMemcpyDeviceToHost, c->stream),
-                 "download counts");
-  if (!rc) rc = hip_check(c, hipStreamSynchronize(c->stream), "sync");
-  if (rc) return rc;
-  ho[0] = 0;
-  for (int i = 0; i < ncell; ++i) ho[i + 1] = ho[i] + hc[i];
-  if ((rc = ensure(c, c->d_tx_list, sizeof(int) * std::max<unsigned>(1, ho[ncell])))) return rc;
-  rc = hip_check(c, hipMemcpyAsync(off, ho.data(), sizeof(unsigned) * (ncell + 1), hipMemcpyHostToDevice, c->stream),
-                 "upload offsets");
-  if (rc) return rc;
-  if (np > 0)
-    hipLaunchKernelGGL(k_tx_bin, dim3((unsigned)nb), dim3(256), 0, c->stream, poly, key, np, d_mask, g, cnt,
-                       (const unsigned*)off, cursor, (int*)c->d_tx_list.ptr);
-  if (ptan)
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_tx_sample<Dual>), dim3(ncell), dim3(64), 0, c->stream, poly, ptan, key, g,
-                       Xd, (const unsigned*)off, (const unsigned*)cnt, (const int*)c->d_tx_list.ptr, d_out);
-  else if (g.S * g.S <= HCS_TX_RAYS && c->last_pairs.size() < (1u << 19)) {
-    /* up to eight taxels a CU, four waves share a taxel: 256 taxels 52 -> 22
-     * us, 1600 taxels 21 -> 14 us; with 3600 taxels 14 -> 16 us */
-    auto run = [&](auto kernel, int waves) {
-      hipLaunchKernelGGL(kernel, dim3(ncell), dim3(64 * waves), 0, c->stream, poly, key, g, (const unsigned*)off,
-                         (const unsigned*)cnt, (const int*)c->d_tx_list.ptr, d_out);
-    };
-    if (ncell <= 8 * c->num_cu) run(k_tx_sample_fan<4>, 4);
-    else run(k_tx_sample_fan<1>, 1);
+  TxPairs pairs{};
+  if (seen.size() > 256) {
+    if ((rc = ensure(c, c->d_tx_grid, seen.size())) ||
+        (rc = hip_check(c, hipMemcpyAsync(c->d_tx_grid.ptr, seen.data(), seen.size(), hipMemcpyHostToDevice, c->stream),
+                        "upload mask")))
+      return rc;
+    pairs.mask = (const unsigned char*)c->d_tx_grid.ptr;
+  } else {
+    for (size_t e = 0; e < seen.size(); ++e)
+      if (seen[e]) pairs.bits[e >> 6] |= 1ull << (e & 63);
   }
-  else
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_tx_sample<double>), dim3(ncell), dim3(64), 0, c->stream, poly,
-                       (const double*)nullptr, key, g, (const double*)nullptr, (const unsigned*)off,
-                       (const unsigned*)cnt, (const int*)c->d_tx_list.ptr, d_out);
-  return hip_check(c, hipGetLastError(), "taxel kernels");
+  /* small grids: the kernel writes the pinned memory itself */
+  double* got = (double*)c->pin_down;
+  double* d_out = got;
+  if (ncell > 8192) {
+    if ((rc = ensure(c, c->d_tx_out, sizeof(double) * ((size_t)ncell + 1)))) return rc;
+    d_out = (double*)c->d_tx_out.ptr;
+  }
+  unsigned* cnt = (unsigned*)c->d_tx_cnt.ptr;
+  unsigned* off = (unsigned*)c->d_tx_off.ptr;
+  void* scan_tmp = (char*)off + (sizeof(unsigned) * ((size_t)ncell + 1) + 7) / 8 * 8;
+  const dim3 nb((unsigned)((np + 63) / 64));
+  launch_fill_u32(c->stream, cnt, 0u, ncell + 1);
+  if (np > 0)
+    hipLaunchKernelGGL(k_tx_bin<0>, nb, dim3(64), 0, c->stream, poly, key, np, pairs, g, (int4*)c->d_tx_foot.ptr, cnt,
+                       (const unsigned*)nullptr, (int*)nullptr, (int64_t)0);
+  if (exclusive_scan_u32(c->stream, cnt, off, (long long)ncell + 1, scan_tmp, scan_bytes) != 0)
+    return set_err(c, HCS_ERR_LIMIT, "taxel grid too large");
+  for (;;) {
+    const int64_t list_cap = (int64_t)(c->d_tx_list.bytes / sizeof(int));
+    int* list = (int*)c->d_tx_list.ptr;
+    launch_fill_u32(c->stream, cnt, 0u, ncell + 1);
+    if (np > 0)
+      hipLaunchKernelGGL(k_tx_bin<1>, nb, dim3(64), 0, c->stream, poly, key, np, pairs, g, (int4*)c->d_tx_foot.ptr, cnt,
+                         (const unsigned*)off, list, list_cap);
+    if (ptan) {
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_tx_sample<Dual>), dim3(ncell), dim3(64), 0, c->stream, poly, ptan, key, g,
+                         Xd, (const unsigned*)off, (const int*)list, list_cap, d_out);
+    } else if (g.S * g.S <= HCS_TX_RAYS && c->last_pairs.size() < (1u << 19)) {
+      /* up to eight taxels a CU, four waves share a taxel: 256 taxels 52 -> 22
+       * us, 1600 taxels 21 -> 14 us; with 3600 taxels 14 -> 16 us */
+      auto run = [&](auto kernel, int waves) {
+        hipLaunchKernelGGL(kernel, dim3(ncell), dim3(64 * waves), 0, c->stream, poly, key, g, (const unsigned*)off,
+                           (const int*)list, list_cap, d_out);
+      };
+      if (ncell <= 8 * c->num_cu) run(k_tx_sample_fan<4>, 4);
+      else run(k_tx_sample_fan<1>, 1);
+    } else {
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_tx_sample<double>), dim3(ncell), dim3(64), 0, c->stream, poly,
+                         (const double*)nullptr, key, g, (const double*)nullptr, (const unsigned*)off,
+                         (const int*)list, list_cap, d_out);
+    }
+    rc = hip_check(c, hipGetLastError(), "taxel kernels");
+    if (!rc && d_out != got)
+      rc = hip_check(c, hipMemcpyAsync(got, d_out, sizeof(double) * ((size_t)ncell + 1), hipMemcpyDeviceToHost, c->stream),
+                     "download taxels");
+    if (!rc) rc = hip_check(c, hipStreamSynchronize(c->stream), "sync");
+    if (rc) return rc;
+    if ((int64_t)got[ncell] <= list_cap) break;
+    if ((rc = ensure(c, c->d_tx_list, sizeof(int) * (size_t)got[ncell]))) return rc;
+  }
+  std::memcpy(out, got, sizeof(double) * (size_t)ncell);
+  return HCS_OK;
 }
 
 int taxel_grid_dev(const hcs_taxel_grid& G, TaxelGridDev& g) {
@@ -150,45 +243,56 @@ int taxel_grid_dev(const hcs_taxel_grid& G, TaxelGridDev& g) {
  * step, which is re-run when a buffer overflowed).
  * =================================================================== */
 
-/* Sensor poses: the 12 doubles (rotation, position) at src[s] in the state. */
-__global__ void k_txb_pose(TaxelGridDev* __restrict__ g, const int* __restrict__ src, const double* __restrict__ state,
-                           int n) {
+/* Sensor poses, the 12 doubles (rotation, position) at src[s] in the state,
+ * and the step's counters cleared. */
+__global__ __launch_bounds__(256) void k_txb_begin(TaxelGridDev* __restrict__ g, const int* __restrict__ src,
+                                                   const double* __restrict__ state, int n, unsigned* __restrict__ cnt,
+                                                   unsigned* __restrict__ cursor, int ncell,
+                                                   unsigned* __restrict__ nlive) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= 12 * n) return;
-  const int s = t / 12, k = t % 12;
-  g[s].X[k] = state[src[s] + k];
+  if (t < 12 * n) g[t / 12].X[t % 12] = state[src[t / 12] + t % 12];
+  if (t <= ncell) cnt[t] = 0;
+  if (t < ncell) cursor[t] = 0;
+  if (t == 0) *nlive = 0;
 }
 
 /* Polygons strided over the grid; each polygon goes to every sensor of its
- * pair, into the taxels its footprint covers.  FILL = 0 counts per taxel;
- * FILL = 1 writes the polygon into the taxel's list slice. */
+ * pair, into the taxels its footprint covers.  FILL = 0 counts per taxel and
+ * keeps the footprint on the pair's first sensor; FILL = 1 writes the polygon
+ * into the taxel's list slice.  Bound by reading the records (320 B a polygon,
+ * 64-byte pieces of it), which the second pass now mostly leaves out: 1024
+ * pads 131 + 185 us -> 153 + 67 us, with shared atomics. */
 template <int FILL>
 __global__ __launch_bounds__(256) void k_txb_bin(const double* __restrict__ poly, const int64_t* __restrict__ key,
                                                  const unsigned long long* __restrict__ poly_cnt, int64_t poly_cap,
                                                  const int* __restrict__ psoff, const int* __restrict__ psens,
                                                  const TaxelGridDev* __restrict__ grids,
-                                                 const int* __restrict__ cell_base, unsigned* __restrict__ cnt,
-                                                 const unsigned* __restrict__ off, unsigned* __restrict__ cursor,
-                                                 int* __restrict__ list, int64_t list_cap) {
+                                                 const int* __restrict__ cell_base, int4* __restrict__ foot,
+                                                 unsigned* __restrict__ cnt, const unsigned* __restrict__ off,
+                                                 unsigned* __restrict__ cursor, int* __restrict__ list,
+                                                 int64_t list_cap) {
   const int64_t np = min((int64_t)*poly_cnt, poly_cap);
-  for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < np; q += (int64_t)gridDim.x * blockDim.x) {
-    const int e = (int)key[3 * q];
-    const double* P = poly + q * HCS_PREC;
-    for (int k = psoff[e]; k < psoff[e + 1]; ++k) {
-      const int s = psens[k];
-      const TaxelGridDev& g = grids[s];
-      int x0, x1, y0, y1;
-      footprint(P, g, x0, x1, y0, y1);
-      for (int y = y0; y <= y1; ++y)
-        for (int x = x0; x <= x1; ++x) {
-          const int cell = cell_base[s] + x + g.cx * y;
-          if (!FILL) {
-            atomicAdd(cnt + cell, 1u);
-          } else {
-            const int64_t slot = (int64_t)off[cell] + atomicAdd(cursor + cell, 1u);
-            if (slot < list_cap) list[slot] = (int)q;
-          }
-        }
+  const int64_t step = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t q0 = blockIdx.x * (int64_t)blockDim.x; q0 < np; q0 += step) {
+    const int64_t q = q0 + threadIdx.x;
+    int k = 0, k1 = 0;
+    bool first = true;
+    if (q < np) {
+      const int e = (int)key[3 * q];
+      k = psoff[e], k1 = psoff[e + 1];
+    }
+    while (__any(k < k1)) {
+      int4 f = make_int4(0, -1, 0, -1);
+      int cx = 1, base = 0;
+      if (k < k1) {
+        const int s = psens[k];
+        cx = grids[s].cx, base = cell_base[s];
+        if (FILL && first) f = foot[q];
+        else footprint(poly + q * HCS_PREC, grids[s], f.x, f.y, f.z, f.w);
+        if (!FILL && first) foot[q] = f;
+      }
+      bin_polygon<FILL>((int)q, f, cx, base, FILL ? cursor : cnt, off, list, list_cap);
+      first = false, ++k;
     }
   }
 }
@@ -197,15 +301,16 @@ __global__ __launch_bounds__(256) void k_txb_bin(const double* __restrict__ poly
  * buffer; an overflowed list is re-run after the step with a larger one),
  * appended to live[] with one atomic per block of HCS_TXB_LIVE threads
  * (atomics on the one counter complete one after another, so one per wave
- * would queue thousands); every other taxel is 0 (the output is cleared
- * before). */
+ * would queue thousands); every other taxel is 0. */
 #define HCS_TXB_LIVE 1024
 __global__ __launch_bounds__(HCS_TXB_LIVE) void k_txb_live(const unsigned* __restrict__ cnt,
                                                            const unsigned* __restrict__ off, int ncell,
                                                            int64_t list_cap, int* __restrict__ live,
-                                                           unsigned* __restrict__ nlive) {
+                                                           unsigned* __restrict__ nlive,
+                                                           double* __restrict__ out) {
   __shared__ unsigned s_off[HCS_TXB_LIVE / 64 + 1];
   const int cell = blockIdx.x * blockDim.x + threadIdx.x;
+  if (cell < ncell) out[cell] = 0.0;
   const bool on = cell < ncell && cnt[cell] > 0 && (int64_t)off[cell] + cnt[cell] <= list_cap;
   const unsigned long long m = __ballot(on);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -321,7 +426,8 @@ int batch_taxels_reserve(Ctx* c, BatchTaxels& t, int64_t poly_cap, int64_t list_
   if (list_cap > 0xffffffffLL) return set_err(c, HCS_ERR_CAPACITY, "taxel polygon lists exceed 2^32 entries");
   int rc;
   if ((rc = ensure(c, t.poly_rec, sizeof(double) * HCS_PREC * poly_cap)) ||
-      (rc = ensure(c, t.poly_key, sizeof(int64_t) * 3 * poly_cap)) || (rc = ensure(c, t.list, sizeof(int) * list_cap)))
+      (rc = ensure(c, t.poly_key, sizeof(int64_t) * 3 * poly_cap)) ||
+      (rc = ensure(c, t.foot, sizeof(int4) * poly_cap)) || (rc = ensure(c, t.list, sizeof(int) * list_cap)))
     return rc;
   t.poly_cap = poly_cap, t.list_cap = list_cap;
   return HCS_OK;
@@ -331,26 +437,23 @@ void batch_taxels_enqueue(Ctx* c, BatchTaxels& t, const double* state) {
   if (t.n == 0) return;
   hipStream_t s = c->stream;
   TaxelGridDev* g = (TaxelGridDev*)t.grid.ptr;
-  hipLaunchKernelGGL(k_txb_pose, dim3((12 * t.n + 255) / 256), dim3(256), 0, s, g, (const int*)t.src.ptr, state, t.n);
-  launch_fill_u32(s, (unsigned*)t.cnt.ptr, 0u, t.ncell + 1);
-  launch_fill_u32(s, (unsigned*)t.cursor.ptr, 0u, t.ncell);
+  unsigned* nlive = (unsigned*)t.poly_cnt.ptr + 2;
+  hipLaunchKernelGGL(k_txb_begin, dim3((std::max(12 * t.n, t.ncell + 1) + 255) / 256), dim3(256), 0, s, g,
+                     (const int*)t.src.ptr, state, t.n, (unsigned*)t.cnt.ptr, (unsigned*)t.cursor.ptr, t.ncell, nlive);
   const unsigned long long* pc = (const unsigned long long*)t.poly_cnt.ptr;
   hipLaunchKernelGGL(HIP_KERNEL_NAME(k_txb_bin<0>), dim3(t.bin_grid), dim3(256), 0, s, (const double*)t.poly_rec.ptr,
                      (const int64_t*)t.poly_key.ptr, pc, t.poly_cap, (const int*)t.psoff.ptr, (const int*)t.psens.ptr,
-                     (const TaxelGridDev*)g, (const int*)t.cell_base.ptr, (unsigned*)t.cnt.ptr,
+                     (const TaxelGridDev*)g, (const int*)t.cell_base.ptr, (int4*)t.foot.ptr, (unsigned*)t.cnt.ptr,
                      (const unsigned*)nullptr, (unsigned*)nullptr, (int*)nullptr, (int64_t)0);
   (void)exclusive_scan_u32(s, (const unsigned*)t.cnt.ptr, (unsigned*)t.off.ptr, (long long)t.ncell + 1,
                            t.scan_tmp.ptr, t.scan_bytes);
   hipLaunchKernelGGL(HIP_KERNEL_NAME(k_txb_bin<1>), dim3(t.bin_grid), dim3(256), 0, s, (const double*)t.poly_rec.ptr,
                      (const int64_t*)t.poly_key.ptr, pc, t.poly_cap, (const int*)t.psoff.ptr, (const int*)t.psens.ptr,
-                     (const TaxelGridDev*)g, (const int*)t.cell_base.ptr, (unsigned*)t.cnt.ptr,
+                     (const TaxelGridDev*)g, (const int*)t.cell_base.ptr, (int4*)t.foot.ptr, (unsigned*)t.cnt.ptr,
                      (const unsigned*)t.off.ptr, (unsigned*)t.cursor.ptr, (int*)t.list.ptr, t.list_cap);
-  unsigned* nlive = (unsigned*)t.poly_cnt.ptr + 2;
-  launch_fill_u32(s, nlive, 0u, 1);
-  launch_fill_u32(s, (unsigned*)t.out.ptr, 0u, 2 * t.ncell);
   hipLaunchKernelGGL(k_txb_live, dim3((t.ncell + HCS_TXB_LIVE - 1) / HCS_TXB_LIVE), dim3(HCS_TXB_LIVE), 0, s,
                      (const unsigned*)t.cnt.ptr,
-                     (const unsigned*)t.off.ptr, t.ncell, t.list_cap, (int*)t.live.ptr, nlive);
+                     (const unsigned*)t.off.ptr, t.ncell, t.list_cap, (int*)t.live.ptr, nlive, (double*)t.out.ptr);
   const dim3 grid(std::max(1, std::min(t.ncell, c->num_cu * 16)));
   if (t.max_rays <= HCS_TX_RAYS)
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_txb_sample<true>), grid, dim3(64), 0, s, (const double*)t.poly_rec.ptr,
@@ -379,7 +482,7 @@ int batch_taxels_demand(Ctx* c, BatchTaxels& t, int64_t& npoly, int64_t& nlist) 
 }
 
 void batch_taxels_free(BatchTaxels& t) {
-  for (DBuf* b : {&t.grid, &t.src, &t.cell_base, &t.cell_sensor, &t.psoff, &t.psens, &t.mask, &t.poly_rec, &t.poly_key,
+  for (DBuf* b : {&t.grid, &t.src, &t.cell_base, &t.cell_sensor, &t.psoff, &t.psens, &t.mask, &t.poly_rec, &t.poly_key, &t.foot,
                   &t.poly_cnt, &t.cnt, &t.cursor, &t.off, &t.scan_tmp, &t.list, &t.out, &t.live})
     if (b->ptr) (void)hipFree(b->ptr), b->ptr = nullptr, b->bytes = 0;
   t = BatchTaxels();
@@ -411,21 +514,11 @@ int hcs_taxels(hcs_ctx* h, int32_t nsensors, const hcs_taxel_grid* grids, double
     TaxelGridDev g;
     if (taxel_grid_dev(G, g) != HCS_OK) return set_err(c, HCS_ERR_ARG, "invalid taxel grid");
     const int ncell = g.cx * g.cy;
-    std::vector<unsigned char> mask(std::max(1, npairs), 0);
+    std::vector<unsigned char> seen(npairs, 0);
     for (int e = 0; e < npairs; ++e)
-      mask[e] = (c->last_geoms[2 * e] == G.geom || c->last_geoms[2 * e + 1] == G.geom) ? 1 : 0;
-    if ((rc = ensure(c, c->d_tx_grid, mask.size())) || (rc = ensure(c, c->d_tx_out, sizeof(double) * ncell)))
-      return rc;
-    rc = hip_check(c, hipMemcpyAsync(c->d_tx_grid.ptr, mask.data(), mask.size(), hipMemcpyHostToDevice, c->stream),
-                   "upload mask");
-    if (!rc)
-      rc = run_taxels(c, g, (const unsigned char*)c->d_tx_grid.ptr, (const double*)c->d_poly_rec.ptr, nullptr,
-                      (const int64_t*)c->d_poly_key.ptr, c->last_npoly, nullptr, (double*)c->d_tx_out.ptr);
-    if (!rc)
-      rc = hip_check(c, hipMemcpyAsync(out + off_out, c->d_tx_out.ptr, sizeof(double) * ncell, hipMemcpyDeviceToHost,
-                                       c->stream),
-                     "download taxels");
-    if (!rc) rc = hip_check(c, hipStreamSynchronize(c->stream), "sync");
+      seen[e] = (c->last_geoms[2 * e] == G.geom || c->last_geoms[2 * e + 1] == G.geom) ? 1 : 0;
+    rc = run_taxels(c, g, seen, (const double*)c->d_poly_rec.ptr, nullptr, (const int64_t*)c->d_poly_key.ptr,
+                    c->last_npoly, nullptr, out + off_out);
     if (rc) return rc;
     off_out += ncell;
   }

@@ -28,12 +28,30 @@ FINE, COARSE, TINY = dict(L=4, K=4, m=48), dict(L=2, K=2, m=4), dict(L=1, K=1, m
     (COARSE, 16, 8, 0, 0.0),  # a range of 8 x 8 rays: the largest small fan
     (COARSE, 16, 9, 0, 0.0),
     (TINY, 5, 24, 1, 0.3),
+    (TINY, 60, 3, 0, 0.0),  # few polygons over many taxels: the lists outgrow their first buffer
+    (COARSE, 91, 2, 0, 0.0),  # 8281 taxels: more than the kernel writes to host memory itself
 ])
 def test_flat_sensor_work_split(engine, shape, taxels, rays, window, sigma):
     print("[case] flat", shape, taxels, rays, window, flush=True)
     sc = S.tactile_pad(5, **shape)
     ha, hb = add_scene(engine, sc)
     engine.contact_step([pair_of(sc, ha, hb)], keep_polygons=True)
+    _check(engine, sc, hb, taxels, rays, window, sigma)
+
+
+@pytest.mark.parametrize("pairs", [256, 257])
+def test_flat_sensor_sees_its_pairs_only(engine, pairs):
+    """The pairs a sensor sees travel with the launch up to 256 of them: the
+    last pair's pad under its sensor, the others in contact with another."""
+    print("[case] pairs", pairs, flush=True)
+    sc, other = S.tactile_pad(5, **FINE), S.tactile_pad(6, **COARSE)
+    ha, hb = add_scene(engine, sc)
+    hc, hd = add_scene(engine, other)
+    engine.contact_step([pair_of(other, hc, hd)] * (pairs - 1) + [pair_of(sc, ha, hb)], keep_polygons=True)
+    _check(engine, sc, hb, 9, 12, 0, 0.0)
+
+
+def _check(engine, sc, hb, taxels, rays, window, sigma):
     ref = oracle_soft_rigid(sc)
     zs = sc["grid"]["half_size"][2]
     half = (0.0303, 0.0303, zs)  # rays off the polygons' edges
