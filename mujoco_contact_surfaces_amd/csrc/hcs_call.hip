@@ -32,6 +32,14 @@
 
 namespace hcs {
 
+/* The candidates a spread plan's items are cut to: 1 / (32 num_cu) of the
+ * expected total, within these.  (256 .. 1024 cut more items that turn out
+ * nearly empty: 2048 objects 1.06 ms for 0.90; 1024 .. 4096: 400 objects 397
+ * us for 370.) */
+#define HCS_CUT_MIN 512
+#define HCS_CUT_MAX 2048
+#define HCS_CUT_SHARES 32
+
 namespace {
 
 constexpr int kMaxCounters = 8;
@@ -63,11 +71,8 @@ __global__ __launch_bounds__(256) void k_call_front(FrontArgs f) {
     for (int64_t i = t; i < f.n16; i += n) f.dst[i] = f.src[i];
 }
 
-/* Whether a chunk's box Q can meet the subtree `root` of A under pose X (the
- * test of the batched cull). */
-__device__ inline bool may_meet_subtree(const EnvDesc& E, const double* X, const double* Q, int root) {
-  if (root == HCS_WNONE) return false;
-  double T[6];
+/* The box of the subtree `root` of A. */
+__device__ inline void subtree_box(const EnvDesc& E, int root, double* T) {
   if (E.ntA == 1 || root < 0) {
     const HCS_GPTR double* b = E.boxA + 6 * (size_t)(E.ntA == 1 ? 0 : ~root);
 #pragma unroll
@@ -77,7 +82,45 @@ __device__ inline bool may_meet_subtree(const EnvDesc& E, const double* X, const
 #pragma unroll
     for (int c = 0; c < 3; ++c) T[c] = fmin(N.b[c], N.b[6 + c]), T[3 + c] = fmax(N.b[3 + c], N.b[9 + c]);
   }
+}
+
+/* Whether a chunk's box Q can meet the subtree `root` of A under pose X (the
+ * test of the batched cull). */
+__device__ inline bool may_meet_subtree(const EnvDesc& E, const double* X, const double* Q, int root) {
+  if (root == HCS_WNONE) return false;
+  double T[6];
+  subtree_box(E, root, T);
   return boxes_may_overlap(X, Q, T);
+}
+
+/* About how many of a chunk's queries x a subtree's tets are candidates: the
+ * queries spread evenly over the chunk's box (in A's frame) with their mean
+ * extents, the tets over the subtree's with those of a filled box, each axis
+ * by itself.  Only the cut of the items depends on it. */
+__device__ inline unsigned expected_candidates(const EnvDesc& E, const double* X, int chunk, int root, int leaves) {
+  double Q[6], T[6];
+#pragma unroll
+  for (int c = 0; c < 6; ++c) Q[c] = E.cboxQ[6 * (size_t)chunk + c];
+  subtree_box(E, root, T);
+  const float nt = (float)leaves, nq = (float)min(64, E.nB - 64 * chunk);
+  float lt[3], vol = 1.f;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) lt[c] = fmaxf((float)(T[3 + c] - T[c]), 1e-30f), vol *= lt[c];
+  const float s = 1.8f * cbrtf(vol / nt);
+  float p = nt * nq;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    float c1 = (float)X[9 + i], h1 = 1e-30f, hq = 0.f;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const float r = (float)X[3 * i + k];
+      c1 += r * (float)(0.5 * (Q[k] + Q[3 + k])), h1 += fabsf(r) * (float)(0.5 * (Q[3 + k] - Q[k]));
+      hq += fabsf(r) * (float)E.csizeQ[3 * (size_t)chunk + k];
+    }
+    const float in = fminf(c1 + h1, (float)T[3 + i]) - fmaxf(c1 - h1, (float)T[i]);
+    p *= fminf(1.f, (fmaxf(in, 0.f) + s) / lt[i]) * fminf(1.f, (2.f * hq + s) / (2.f * h1));
+  }
+  return (unsigned)fminf(fmaxf(p, 0.f), 1e9f);
 }
 
 __device__ inline void chunk_box(const EnvDesc& E, int chunk, double* Q) {
@@ -113,6 +156,33 @@ __device__ inline int expand_levels(unsigned n1, unsigned budget) {
   int e = 0;
   while (e < HCS_ROOT_DEPTH && ((unsigned long long)n1 << (e + 1)) <= budget) ++e;
   return e;
+}
+
+/* An item's expected candidates, and the levels it can be cut (to about 16
+ * tets), in one word.  A soft query's candidate costs about four of a
+ * triangle's. */
+constexpr unsigned kEstMask = (1u << 28) - 1;
+__device__ inline unsigned cut_word(const EnvDesc& E, const double* X, int chunk, int root) {
+  if (!is_tree(E)) return 0u;
+  const int leaves = root < 0 || E.ntA == 1 ? 1 : E.nodesA[root].leaves;
+  unsigned n = 0;
+  while (n < 15 && (leaves >> n) > 16) ++n;
+  const unsigned est = min(expected_candidates(E, X, chunk, root, leaves), 1u << 25);
+  return (E.kind == KIND_SOFT ? 4 * est : est) | n << 28;
+}
+/* The pieces an item is cut into: halved until at most the target is left. */
+__device__ inline unsigned cut_slots(unsigned word, unsigned target) {
+  const unsigned q = (word & kEstMask) / target;
+  return 1u << min(q > 0 ? 32u - (unsigned)__builtin_clz(q) : 0u, word >> 28);
+}
+/* Subtree number sub of the 2^n below root; a leaf reached earlier is its
+ * first subtree only. */
+__device__ inline int cut_root(const EnvDesc& E, int root, int n, int sub) {
+  for (int b = n - 1; b >= 0; --b) {
+    if (root < 0) return (sub & ((2 << b) - 1)) == 0 ? root : HCS_WNONE;
+    root = E.nodesA[root].c[sub >> b & 1];
+  }
+  return root;
 }
 
 constexpr int kGenWaves = HCS_GEN_THREADS / 64;
@@ -166,6 +236,21 @@ __device__ inline unsigned kept_before(const unsigned* __restrict__ cnt, bool sc
   return pos + lane_prefix(m);
 }
 
+/* Adds the block's expected candidates to *sum (whole numbers, so the sum and
+ * with it the cut do not depend on the order). */
+__device__ inline void add_expected(unsigned word, unsigned long long* __restrict__ sum) {
+  __shared__ unsigned long long part[kGenWaves];
+  const unsigned long long v = (unsigned long long)wave_sum_i((int64_t)(word & kEstMask));
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned long long all = 0;
+#pragma unroll
+    for (int k = 0; k < kGenWaves; ++k) all += part[k];
+    if (all) atomicAdd(sum, all);
+  }
+}
+
 /* First cull: one block per HCS_GEN_THREADS items of one pair. */
 __global__ __launch_bounds__(HCS_GEN_THREADS) void k_call_cull1(const EnvDesc* __restrict__ envs,
                                                                 const int2* __restrict__ blocks,
@@ -188,6 +273,8 @@ __global__ __launch_bounds__(HCS_GEN_THREADS) void k_call_place1(const EnvDesc* 
                                                                  const int* __restrict__ xenv,
                                                                  const double* __restrict__ xf,
                                                                  double* __restrict__ xtri, int4* __restrict__ item,
+                                                                 unsigned* __restrict__ cut,
+                                                                 unsigned long long* __restrict__ cut_sum,
                                                                  unsigned* __restrict__ n1) {
   if ((int)blockIdx.x >= nblk) {
     const int e = xenv[blockIdx.x - nblk];
@@ -198,11 +285,22 @@ __global__ __launch_bounds__(HCS_GEN_THREADS) void k_call_place1(const EnvDesc* 
   unsigned through;
   const unsigned pos = kept_before(cnt, scanned, mask, keep, through);
   if (threadIdx.x == 0 && (int)blockIdx.x == nblk - 1) *n1 = through;
-  if (!keep) return;
   const int2 b = blocks[blockIdx.x];
   const EnvDesc& E = envs[b.x];
   const int depth = is_tree(E) ? E.depth : 0, i = b.y + threadIdx.x;
-  item[pos] = make_int4(b.x, i >> depth, (1 << depth) + (i & ((1 << depth) - 1)), 0);
+  const int chunk = i >> depth, node = (1 << depth) + (i & ((1 << depth) - 1));
+  if (!cut) {
+    if (keep) item[pos] = make_int4(b.x, chunk, node, 0);
+    return;
+  }
+  unsigned word = 0;
+  if (keep) {
+    const int root = is_tree(E) ? E.rootsA[node] : 0;
+    word = cut_word(E, xf + 12 * (size_t)b.x, chunk, root);
+    item[pos] = make_int4(b.x, chunk, root, 0);
+    cut[pos] = word;
+  }
+  add_expected(word, cut_sum);
 }
 
 /* Second cull: the kept items cut e levels deeper, e the same for the launch
@@ -240,6 +338,20 @@ __global__ __launch_bounds__(HCS_GEN_THREADS) void k_call_cull2(const EnvDesc* _
   block_counts(keep, cnt, mask);
 }
 
+/* The pairs' first live items: a pair's from its first item (sub 0, placed
+ * at pos), also for the pairs without items before it. */
+__device__ inline void first_of_pair(const int4* __restrict__ item, int i, int pos, int* __restrict__ pair_lo) {
+  for (int q = i > 0 ? item[i - 1].x + 1 : 0; q <= item[i].x; ++q) pair_lo[q] = pos;
+}
+__device__ inline void after_last_pair(const int4* __restrict__ item, unsigned n1, int npairs, int total,
+                                       int* __restrict__ pair_lo) {
+  for (int e = n1 ? item[n1 - 1].x + 1 : 0; e <= npairs; ++e) pair_lo[e] = total;
+}
+__device__ inline int4 live_record(const EnvDesc& E, const int4& it, int root) {
+  const int nq = is_tree(E) ? E.nB : E.ntA;
+  return make_int4(it.x, 64 * it.y, min(64, nq - 64 * it.y), is_tree(E) ? root : 0);
+}
+
 /* The live items in order, and each pair's first. */
 __global__ __launch_bounds__(HCS_GEN_THREADS) void k_call_place2(const EnvDesc* __restrict__ envs,
                                                                  const int4* __restrict__ item,
@@ -254,23 +366,135 @@ __global__ __launch_bounds__(HCS_GEN_THREADS) void k_call_place2(const EnvDesc* 
   const unsigned pos = kept_before(cnt, scanned, mask, keep, through);
   const unsigned n1 = *n1p, t = blockIdx.x * HCS_GEN_THREADS + threadIdx.x;
   if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
-    /* the pairs after the last one with an item */
     *live_cnt = through;
-    for (int e = n1 ? item[n1 - 1].x + 1 : 0; e <= npairs; ++e) pair_lo[e] = (int)through;
+    after_last_pair(item, n1, npairs, (int)through, pair_lo);
   }
   int i, sub, node;
   const bool on = second_item(envs, item, n1, budget, t, i, sub, node);
-  if (on && sub == 0) {
-    /* the first item of a pair: its place, also for the pairs without items
-     * before it */
-    const int e = item[i].x;
-    for (int q = i > 0 ? item[i - 1].x + 1 : 0; q <= e; ++q) pair_lo[q] = (int)pos;
-  }
+  if (on && sub == 0) first_of_pair(item, i, (int)pos, pair_lo);
   if (!keep) return;
   const int4 it = item[i];
   const EnvDesc& E = envs[it.x];
-  const int nq = is_tree(E) ? E.nB : E.ntA;
-  live_item[pos] = make_int4(it.x, 64 * it.y, min(64, nq - 64 * it.y), is_tree(E) && node > 1 ? E.rootsA[node] : 0);
+  live_item[pos] = live_record(E, it, is_tree(E) ? E.rootsA[node] : 0);
+}
+
+/* ---- spread plans: batches of many pairs, whose items differ too much for
+ * one number of levels (some chunks are a few large triangles that meet a
+ * whole mesh: 147k candidates in one item of 2048 objects, where a wave's
+ * share was 4k).  The items that the first cull keeps are cut by their
+ * expected candidates and culled again.  2048 objects, k_cand:
+ * 3.28 -> 0.90 ms; 400 objects 746 -> 370 us, 64 objects 325 -> 145 us, 200
+ * soft pairs 1.83 -> 1.36 ms.  (A second round of cuts with expectations for
+ * the smaller boxes found little more to cut and cost its launches.) */
+
+/* The candidates an item is cut to: a share of the total that gives every
+ * wave several items, and few enough pieces for the room (an item of est
+ * candidates has fewer than 1 + 2 est / target pieces). */
+struct CutArgs {
+  const unsigned* n;             /* items */
+  const unsigned long long* sum; /* of their expected candidates */
+  unsigned shares, room;
+};
+__device__ inline unsigned cut_target(const CutArgs& c) {
+  const unsigned long long sum = *c.sum, room = c.room - min(c.room, *c.n);
+  unsigned long long t = min(max(sum / c.shares, (unsigned long long)HCS_CUT_MIN), (unsigned long long)HCS_CUT_MAX);
+  t = max(t, 2 * sum / max(1ull, room) + 1);
+  return (unsigned)min(t, (unsigned long long)kEstMask);
+}
+__device__ inline unsigned block_exclusive(unsigned v, unsigned& total) {
+  __shared__ unsigned part[kGenWaves];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  unsigned inc = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const unsigned u = __shfl_up(inc, o, 64);
+    if (lane >= o) inc += u;
+  }
+  if (lane == 63) part[w] = inc;
+  __syncthreads();
+  unsigned before = inc - v;
+  total = 0;
+#pragma unroll
+  for (int k = 0; k < kGenWaves; ++k) before += k < w ? part[k] : 0u, total += part[k];
+  return before;
+}
+/* Pieces per block of items. */
+__global__ __launch_bounds__(HCS_GEN_THREADS) void k_cut_count(CutArgs c, const unsigned* __restrict__ word,
+                                                               unsigned* __restrict__ cnt) {
+  const unsigned n = *c.n, i = blockIdx.x * HCS_GEN_THREADS + threadIdx.x;
+  unsigned total;
+  (void)block_exclusive(i < n ? cut_slots(word[i], cut_target(c)) : 0u, total);
+  if (threadIdx.x == 0) cnt[blockIdx.x] = total;
+}
+/* First piece of every item, off[n] their number; in place of the words. */
+__global__ __launch_bounds__(HCS_GEN_THREADS) void k_cut_place(CutArgs c, const unsigned* __restrict__ cnt,
+                                                               unsigned* __restrict__ off) {
+  const unsigned n = *c.n, i = blockIdx.x * HCS_GEN_THREADS + threadIdx.x;
+  if (blockIdx.x * HCS_GEN_THREADS > n) return;
+  unsigned v = 0, before, all;
+  for (unsigned k = threadIdx.x; k < blockIdx.x; k += HCS_GEN_THREADS) v += cnt[k];
+  (void)block_exclusive(v, before);
+  __syncthreads();
+  v = i < n ? cut_slots(off[i], cut_target(c)) : 0u;
+  before += block_exclusive(v, all);
+  if (i <= n) off[i] = before;
+}
+/* The item that piece t belongs to. */
+__device__ inline bool piece(const unsigned* __restrict__ off, unsigned n, unsigned t, int& i, int& sub, int& levels) {
+  if (n == 0 || t >= off[n]) return false;
+  unsigned lo = 0, hi = n;
+  while (hi - lo > 1) {
+    const unsigned mid = (lo + hi) / 2;
+    if (off[mid] <= t) lo = mid;
+    else hi = mid;
+  }
+  const unsigned first = off[lo];
+  i = (int)lo, sub = (int)(t - first), levels = __builtin_ctz(off[lo + 1] - first);
+  return true;
+}
+__global__ __launch_bounds__(HCS_GEN_THREADS) void k_cut_cull(const EnvDesc* __restrict__ envs,
+                                                              const double* __restrict__ xf,
+                                                              const int4* __restrict__ item,
+                                                              const unsigned* __restrict__ n,
+                                                              const unsigned* __restrict__ off,
+                                                              unsigned* __restrict__ cnt,
+                                                              unsigned long long* __restrict__ mask) {
+  int i, sub, levels;
+  bool keep = piece(off, *n, blockIdx.x * HCS_GEN_THREADS + threadIdx.x, i, sub, levels);
+  if (keep && levels > 0) {
+    const int4 it = item[i];
+    const EnvDesc& E = envs[it.x];
+    double Q[6];
+    chunk_box(E, it.y, Q);
+    keep = may_meet_subtree(E, xf + 12 * (size_t)it.x, Q, cut_root(E, it.z, levels, sub));
+  }
+  block_counts(keep, cnt, mask);
+}
+/* The kept pieces are the live items; and each pair's first. */
+__global__ __launch_bounds__(HCS_GEN_THREADS) void k_cut_keep(const EnvDesc* __restrict__ envs,
+                                                              const int4* __restrict__ item,
+                                                              const unsigned* __restrict__ np,
+                                                              const unsigned* __restrict__ off,
+                                                              const unsigned* __restrict__ cnt,
+                                                              const unsigned long long* __restrict__ mask, int npairs,
+                                                              int4* __restrict__ live_item,
+                                                              unsigned* __restrict__ live_cnt,
+                                                              int* __restrict__ pair_lo) {
+  bool keep;
+  unsigned through;
+  const unsigned pos = kept_before(cnt, false, mask, keep, through);
+  const unsigned n = *np;
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+    *live_cnt = through;
+    after_last_pair(item, n, npairs, (int)through, pair_lo);
+  }
+  int i, sub, levels;
+  const bool on = piece(off, n, blockIdx.x * HCS_GEN_THREADS + threadIdx.x, i, sub, levels);
+  if (on && sub == 0) first_of_pair(item, i, (int)pos, pair_lo);
+  if (!keep) return;
+  const int4 it = item[i];
+  const EnvDesc& E = envs[it.x];
+  live_item[pos] = live_record(E, it, cut_root(E, it.z, levels, sub));
 }
 
 /* Exclusive scan of the live items' survivor counts (off[n] = total), one
@@ -373,8 +597,8 @@ CallSizes call_sizes(const Plan& plan) {
   CallSizes z;
   z.blocks1 = plan.blocks.size();
   z.items = (size_t)std::max(1, plan.nitems);
-  z.expand = HCS_EXPAND_BUDGET;
-  z.live = std::max<size_t>(z.items, z.expand);
+  z.expand = plan.spread ? HCS_SPREAD_BUDGET : HCS_EXPAND_BUDGET;
+  z.live = plan.spread ? z.items + z.expand : std::max<size_t>(z.items, z.expand);
   z.blocks2 = (z.live + HCS_GEN_THREADS - 1) / HCS_GEN_THREADS;
   /* slices of a pair's contributions: about 1024 waves in all, at most 64 per
    * pair */
@@ -413,7 +637,8 @@ int call_reserve(Ctx* c, Pipe& p, const Plan& plan, const CallBlob& b, int64_t c
       (rc = ensure(c, p.xtri, sizeof(double) * HCS_XTRI * std::max<int64_t>(1, plan.ntx))) ||
       (rc = ensure(c, p.gen_cnt, sizeof(unsigned) * (nb + 1))) ||
       (rc = ensure(c, p.gen_mask, sizeof(unsigned long long) * nb * kGenWaves)) ||
-      (rc = ensure(c, p.gen_item, sizeof(int4) * z.items)) || (rc = ensure(c, p.pair_lo, sizeof(int) * (np + 1))) ||
+      (rc = ensure(c, p.gen_item, sizeof(int4) * z.items)) ||
+      (plan.spread && (rc = ensure(c, p.gen_off, sizeof(unsigned) * (z.items + 1)))) || (rc = ensure(c, p.pair_lo, sizeof(int) * (np + 1))) ||
       (rc = ensure(c, p.live_item, sizeof(int4) * z.live)) || (rc = ensure(c, p.ncand, sizeof(int) * z.live)) ||
       (rc = ensure(c, p.nsurv, sizeof(unsigned) * (z.live + 1))) ||
       (rc = ensure(c, p.off, sizeof(unsigned) * (z.live + 1))) ||
@@ -479,14 +704,30 @@ int call_front(Ctx* c, Pipe& p, const QueryArgs& a, const Plan& plan, const Call
   unsigned *n1 = (unsigned*)p.err.ptr + 4, *live_cnt = (unsigned*)p.counter.ptr + HCS_QUEUES;
   /* beyond a few thousand blocks the sums of the counts before each block
    * would cost more than a scan */
+  /* (the error block's words past the error and the zero counter) */
+  unsigned* off = plan.spread ? (unsigned*)p.gen_off.ptr : nullptr;
+  unsigned long long* sum = (unsigned long long*)((char*)p.err.ptr + 24);
   const bool scan1 = z.blocks1 > 4096, scan2 = z.blocks2 > 4096;
   int rc = 0;
   hipLaunchKernelGGL(k_call_cull1, dim3(nblk), dim3(HCS_GEN_THREADS), 0, s, a.envs, blocks, a.xf, cnt1, mask1);
   if (scan1) rc = exclusive_scan_u32(s, cnt1, cnt1, nblk, p.scan_tmp.ptr, p.scan_bytes);
   hipLaunchKernelGGL(k_call_place1, dim3(nblk + (unsigned)plan.xenv.size()), dim3(HCS_GEN_THREADS), 0, s, a.envs,
                      blocks, nblk, (const unsigned*)cnt1, scan1, (const unsigned long long*)mask1,
-                     (const int*)(blob + b.xenv), a.xf, (double*)p.xtri.ptr, item, n1);
+                     (const int*)(blob + b.xenv), a.xf, (double*)p.xtri.ptr, item, off, sum, n1);
   const dim3 g2((unsigned)z.blocks2);
+  if (rc) return set_err(c, HCS_ERR_LIMIT, "too many work items to scan");
+  if (off) {
+    const CutArgs cut{n1, sum, (unsigned)c->num_cu * HCS_CUT_SHARES, (unsigned)z.live};
+    const dim3 t(HCS_GEN_THREADS), g1((unsigned)(z.items / HCS_GEN_THREADS + 1));
+    hipLaunchKernelGGL(k_cut_count, g1, t, 0, s, cut, (const unsigned*)off, cnt2);
+    hipLaunchKernelGGL(k_cut_place, g1, t, 0, s, cut, (const unsigned*)cnt2, off);
+    hipLaunchKernelGGL(k_cut_cull, g2, t, 0, s, a.envs, a.xf, (const int4*)item, (const unsigned*)n1,
+                       (const unsigned*)off, cnt2, mask2);
+    hipLaunchKernelGGL(k_cut_keep, g2, t, 0, s, a.envs, (const int4*)item, (const unsigned*)n1, (const unsigned*)off,
+                       (const unsigned*)cnt2, (const unsigned long long*)mask2, np, (int4*)p.live_item.ptr, live_cnt,
+                       (int*)p.pair_lo.ptr);
+    return HCS_OK;
+  }
   const unsigned budget = (unsigned)z.expand;
   hipLaunchKernelGGL(k_call_cull2, g2, dim3(HCS_GEN_THREADS), 0, s, a.envs, a.xf, (const int4*)item,
                      (const unsigned*)n1, budget, cnt2, mask2);

@@ -268,11 +268,22 @@ __device__ inline void box_union(double* u, const double* b) {
   for (int c = 0; c < 3; ++c) u[c] = fmin(u[c], b[c]), u[3 + c] = fmax(u[3 + c], b[3 + c]);
 }
 
-/* Boxes of the leaves in Morton order and of their chunks of 64, one wave per
- * chunk. */
+/* The mean half-extents of a wave's boxes (lanes with on), for chunk
+ * blockIdx.x. */
+__device__ inline void mean_half_extents(bool on, const double* lo, const double* hi, double* __restrict__ csize) {
+  const double n = (double)__popcll(__ballot(on));
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const double h = wave_sum<double>(on ? 0.5 * (hi[c] - lo[c]) : 0.0);
+    if (threadIdx.x == c) csize[3 * (size_t)blockIdx.x + c] = n > 0 ? h / n : 0.0;
+  }
+}
+
+/* Boxes of the leaves in Morton order and of their chunks of 64, and the mean
+ * size of a chunk's, one wave per chunk. */
 __global__ __launch_bounds__(64) void k_leaf_boxes(const double* __restrict__ box, const int* __restrict__ idx, int n,
                                                    const BuildOut* __restrict__ out, double* __restrict__ boxL,
-                                                   double* __restrict__ cbox) {
+                                                   double* __restrict__ cbox, double* __restrict__ csize) {
   const int i = blockIdx.x * 64 + threadIdx.x;
   const double inf = __builtin_inf();
   double u[6] = {inf, inf, inf, -inf, -inf, -inf};
@@ -282,6 +293,7 @@ __global__ __launch_bounds__(64) void k_leaf_boxes(const double* __restrict__ bo
 #pragma unroll
     for (int c = 0; c < 6; ++c) u[c] = b[c], boxL[6 * (size_t)i + c] = u[c];
   }
+  mean_half_extents(i < n, u, u + 3, csize);
 #pragma unroll
   for (int c = 0; c < 3; ++c) u[c] = wave_min(u[c]), u[3 + c] = wave_max(u[3 + c]);
   if (threadIdx.x < 6) {
@@ -343,10 +355,12 @@ __global__ __launch_bounds__(64) void k_node_boxes(const double* __restrict__ bo
 /* The children's boxes of every internal node, and its 4-wide node (the
  * layout of make_wide_node: grandchildren, a leaf child standing for itself). */
 __global__ __launch_bounds__(256) void k_fill_nodes(const double* __restrict__ ubox, const double* __restrict__ box,
-                                                    int n_int, const BuildOut* __restrict__ out, Node* nodes,
+                                                    const int2* __restrict__ range, int n_int,
+                                                    const BuildOut* __restrict__ out, Node* nodes,
                                                     WNode* __restrict__ wide) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n_int || out->bad) return;
+  nodes[i].leaves = range[i].y - range[i].x + 1;
   WNode& w = wide[i];
   int m = 0;
   auto put = [&](int ch) {
@@ -424,7 +438,7 @@ __global__ __launch_bounds__(64) void k_xtri(const EnvDesc* __restrict__ envs, c
  * `order`, in the mesh's own frame, one wave per chunk. */
 __global__ __launch_bounds__(64) void k_chunk_boxes(const double* __restrict__ V, const int32_t* __restrict__ el, int nv,
                                                     const int32_t* __restrict__ order, int n,
-                                                    double* __restrict__ cbox) {
+                                                    double* __restrict__ cbox, double* __restrict__ csize) {
   const int i = blockIdx.x * 64 + threadIdx.x;
   const double inf = __builtin_inf();
   double lo[3] = {inf, inf, inf}, hi[3] = {-inf, -inf, -inf};
@@ -436,6 +450,7 @@ __global__ __launch_bounds__(64) void k_chunk_boxes(const double* __restrict__ V
       for (int c = 0; c < 3; ++c) lo[c] = fmin(lo[c], v[c]), hi[c] = fmax(hi[c], v[c]);
     }
   }
+  mean_half_extents(i < n, lo, hi, csize);
 #pragma unroll
   for (int c = 0; c < 3; ++c) lo[c] = wave_min(lo[c]), hi[c] = wave_max(hi[c]);
   if (threadIdx.x < 6) {
@@ -1147,7 +1162,7 @@ int pipe_plan(Ctx* c, Pipe& p, const EnvDesc* envs, const Item* items, const Pla
 void pipe_free(Pipe& p) {
   for (DBuf* b : {&p.counter, &p.surv, &p.surv_cnt, &p.ncand, &p.nsurv, &p.off, &p.scan_tmp, &p.contrib, &p.out, &p.err,
                   &p.xf, &p.ibox, &p.live, &p.live_item, &p.qseg, &p.xtri, &p.xenv, &p.order, &p.item_o, &p.part, &p.rtab,
-                  &p.ptab, &p.blob, &p.gen_cnt, &p.gen_mask, &p.gen_item, &p.pair_lo})
+                  &p.ptab, &p.blob, &p.gen_cnt, &p.gen_mask, &p.gen_item, &p.gen_off, &p.pair_lo})
     if (b->ptr) (void)hipFree(b->ptr), b->ptr = nullptr, b->bytes = 0;
 }
 
@@ -1268,15 +1283,15 @@ static int build_bvh(Ctx* c, Mesh& m, const double* V) {
   hipLaunchKernelGGL(k_check_order, g, t, 0, s, (const unsigned*)codes2, (const int*)m.leaf, n, (unsigned*)(B + o_seen),
                      out);
   hipLaunchKernelGGL(k_leaf_boxes, dim3(chunks), dim3(64), 0, s, (const double*)m.box, (const int*)m.leaf, n,
-                     (const BuildOut*)out, m.boxL, m.cbox);
+                     (const BuildOut*)out, m.boxL, m.cbox, m.csize);
   if (n > 1) {
     hipLaunchKernelGGL(k_box_chunks, dim3(schunks), dim3(64), 0, s, (const double*)m.cbox, chunks, sbox);
     hipLaunchKernelGGL(k_karras, gi, t, 0, s, (const unsigned*)codes2, (const int*)m.leaf, n, (const BuildOut*)out,
                        m.nodes, np, lp, range);
     hipLaunchKernelGGL(k_node_boxes, dim3((n - 1 + 63) / 64), dim3(64), 0, s, (const double*)m.boxL,
                        (const double*)m.cbox, (const double*)sbox, (const int2*)range, n - 1, (const BuildOut*)out, ubox);
-    hipLaunchKernelGGL(k_fill_nodes, gi, t, 0, s, (const double*)ubox, (const double*)m.box, n - 1,
-                       (const BuildOut*)out, m.nodes, m.wnodes);
+    hipLaunchKernelGGL(k_fill_nodes, gi, t, 0, s, (const double*)ubox, (const double*)m.box,
+                       (const int2*)range, n - 1, (const BuildOut*)out, m.nodes, m.wnodes);
     hipLaunchKernelGGL(k_tree_height, g, t, 0, s, (const int*)lp, (const int*)np, n, out);
   }
   hipLaunchKernelGGL(k_frontiers, dim3(1), dim3(HCS_ROOTS / 2), 0, s, (const Node*)m.nodes, n - 1, out, m.roots);
@@ -1410,6 +1425,7 @@ int build_plan(Ctx* c, int npairs, const int32_t* geoms, const hcs_step_opts* o,
     plan.pair_kind[e] = E.kind;
     const bool tree = E.kind == KIND_TRI || E.kind == KIND_SOFT;
     E.cboxQ = hcs_gptr((const double*)(tree ? B.cbox : A.cbox));
+    E.csizeQ = hcs_gptr((const double*)(tree ? B.csize : A.csize));
     E.boxB = hcs_gptr((const double*)(E.kind == KIND_TET ? B.cbox + 6 * (size_t)((B.nelem + 63) / 64) : nullptr));
     E.item_count = (nq + chunk - 1) / chunk;
   }
@@ -1547,7 +1563,8 @@ static int make_soft(Ctx* c, const double* V, int32_t nv, const int32_t* T, int3
   const size_t oV = S.take<double>(3 * (size_t)nv), oE = S.take<int32_t>(4 * n), op = S.take<double>(nv),
                orec = S.take<double>(HCS_TREC * n), obox = S.take<double>(6 * n), ofpl = S.take<float>(16 * n),
                onodes = S.take<Node>(ni), ow = S.take<WNode>(ni), oleaf = S.take<int32_t>(n), oL = S.take<double>(6 * n),
-               oc = S.take<double>(6 * ((n + 63) / 64)), oroots = S.take<int32_t>(HCS_ROOTS);
+               oc = S.take<double>(6 * ((n + 63) / 64)), os = S.take<double>(3 * ((n + 63) / 64)),
+               oroots = S.take<int32_t>(HCS_ROOTS);
   int rc = mesh_alloc(c, m, S.bytes);
   if (rc != HCS_OK) {
     m = Mesh();
@@ -1556,7 +1573,8 @@ static int make_soft(Ctx* c, const double* V, int32_t nv, const int32_t* T, int3
   char* P = (char*)m.mem;
   m.V = (double*)(P + oV), m.E = (int32_t*)(P + oE), m.p = (double*)(P + op), m.rec = (double*)(P + orec);
   m.box = (double*)(P + obox), m.fpl = (float*)(P + ofpl), m.nodes = (Node*)(P + onodes), m.wnodes = (WNode*)(P + ow);
-  m.leaf = (int32_t*)(P + oleaf), m.boxL = (double*)(P + oL), m.cbox = (double*)(P + oc), m.roots = (int32_t*)(P + oroots);
+  m.leaf = (int32_t*)(P + oleaf), m.boxL = (double*)(P + oL), m.cbox = (double*)(P + oc);
+  m.csize = (double*)(P + os), m.roots = (int32_t*)(P + oroots);
   rc = hip_check(c, hipMemcpyAsync(m.V, V, 3 * sizeof(double) * nv, hipMemcpyHostToDevice, c->stream), "upload");
   if (!rc) rc = hip_check(c, hipMemcpyAsync(m.E, T, 4 * sizeof(int32_t) * nt, hipMemcpyHostToDevice, c->stream), "upload");
   if (!rc) rc = hip_check(c, hipMemcpyAsync(m.p, pr, sizeof(double) * nv, hipMemcpyHostToDevice, c->stream), "upload");
@@ -1591,7 +1609,7 @@ static int make_rigid(Ctx* c, const double* V, int32_t nv, const int32_t* F, int
   const size_t n = ntri, chunks = (n + 63) / 64;
   Slices S;
   const size_t oV = S.take<double>(3 * (size_t)nv), oE = S.take<int32_t>(3 * n), oq = S.take<int32_t>(n),
-               on = S.take<double>(3 * n), oc = S.take<double>(6 * (chunks + 1));
+               on = S.take<double>(3 * n), oc = S.take<double>(6 * (chunks + 1)), os = S.take<double>(3 * chunks);
   int rc = mesh_alloc(c, m, S.bytes);
   if (rc != HCS_OK) {
     m = Mesh();
@@ -1599,7 +1617,7 @@ static int make_rigid(Ctx* c, const double* V, int32_t nv, const int32_t* F, int
   }
   char* P = (char*)m.mem;
   m.V = (double*)(P + oV), m.E = (int32_t*)(P + oE), m.qorder = (int32_t*)(P + oq), m.nrm = (double*)(P + on);
-  m.cbox = (double*)(P + oc);
+  m.cbox = (double*)(P + oc), m.csize = (double*)(P + os);
   rc = hip_check(c, hipMemcpyAsync(m.V, V, 3 * sizeof(double) * nv, hipMemcpyHostToDevice, c->stream), "upload");
   if (!rc) rc = hip_check(c, hipMemcpyAsync(m.E, F, 3 * sizeof(int32_t) * ntri, hipMemcpyHostToDevice, c->stream), "upload");
   /* query order: triangles sorted by the Morton code of their centroids,
@@ -1642,7 +1660,7 @@ static int make_rigid(Ctx* c, const double* V, int32_t nv, const int32_t* F, int
   if (!rc) {
     hipLaunchKernelGGL(k_tri_normals, dim3((ntri + 127) / 128), dim3(128), 0, c->stream, m.V, m.E, ntri, m.nrm);
     hipLaunchKernelGGL(k_chunk_boxes, dim3((unsigned)chunks), dim3(64), 0, c->stream, m.V, m.E, 3,
-                       (const int32_t*)m.qorder, ntri, m.cbox);
+                       (const int32_t*)m.qorder, ntri, m.cbox, m.csize);
     rc = hip_check(c, hipGetLastError(), "rigid mesh kernels");
   }
   if (!rc) rc = hip_check(c, hipStreamSynchronize(c->stream), "sync");

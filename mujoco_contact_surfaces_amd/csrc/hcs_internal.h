@@ -34,6 +34,7 @@ struct Mesh {
   double* boxL = nullptr;   /* their AABBs in that order */
   double* nrm = nullptr;
   double* cbox = nullptr;    /* boxes of the chunks of 64 elements in leaf / query order, then (rigid) of the vertices */
+  double* csize = nullptr;   /* mean half-extents of the chunks' elements */
   int32_t* roots = nullptr;  /* soft: LBVH frontiers (HCS_ROOTS) */
   int32_t roots_h[HCS_ROOTS] = {}; /* their host copy */
 };
@@ -58,7 +59,8 @@ struct Pipe {
       /* per-call steps: the uploaded descriptors, state and tables; kept
        * items per block and their lane masks, and the items of the first
        * cull; first live item per pair */
-      blob, gen_cnt, gen_mask, gen_item, pair_lo;
+      blob, gen_cnt, gen_mask, gen_item, pair_lo,
+      gen_off /* spread plans: first pieces of the first cull's items */;
   int64_t cap = 0;
   size_t scan_bytes = 0;
   std::vector<int> qseg_host; /* host copy of the queue segments (the upload source) */
@@ -86,6 +88,7 @@ struct Plan {
   std::vector<int> pair_kind;
   std::vector<int> xenv; /* pairs in tet-query mode */
   int64_t ntx = 0;       /* their triangles in total */
+  bool spread = false; /* implicit plan: items cut by their expected candidates, each its own number of levels */
   std::vector<int> order; /* items by decreasing measured work (empty: item order) */
 };
 
@@ -145,6 +148,7 @@ int build_plan(Ctx* c, int npairs, const int32_t* geoms, const hcs_step_opts* o,
 #define HCS_GEN_THREADS 256
 #define HCS_ITEM_BUDGET 65536
 #define HCS_EXPAND_BUDGET 16384
+#define HCS_SPREAD_BUDGET 262144
 struct CallSizes {
   size_t blocks1, blocks2, items, live, expand;
   int slices;

@@ -47,7 +47,8 @@ struct Node {
   double b[12];   /* child 0 lo[3] hi[3], child 1 lo[3] hi[3] */
   int32_t c[2];   /* >= 0 internal node, < 0 leaf: ~element */
   int32_t h[2];   /* subtree heights (leaf 0) */
-  int32_t pad[4];
+  int32_t leaves; /* under this node (device build) */
+  int32_t pad[3];
 };
 static_assert(sizeof(Node) == 128, "one LBVH node per cache line");
 
@@ -143,6 +144,7 @@ struct EnvDesc {
   int32_t item_first, item_count;
   const HCS_GPTR double* cboxQ; /* boxes of the chunks of 64 queries, in their own frame (6 doubles each) */
   const HCS_GPTR double* boxB;  /* tet queries: B's vertex box */
+  const HCS_GPTR double* csizeQ;  /* mean half-extents of their elements (3 doubles each) */
   const HCS_GPTR int32_t* rootsA; /* A's LBVH frontiers (HCS_ROOTS) */
   int32_t depth;    /* triangle / soft queries: items over the frontier of depth `depth` */
   int32_t pad;

@@ -36,7 +36,7 @@ constexpr int kThreads = 256;
 constexpr int kPer = 8;
 constexpr int kTile = kThreads * kPer;
 constexpr int kSumThreads = 1024;
-constexpr int kMaxSumPer = 64; /* at most this many tile sums per thread of the middle pass */
+constexpr int kMaxSumPer = 1024; /* at most this many tile sums per thread of the middle pass */
 
 __device__ inline unsigned wave_incl_scan(unsigned v) {
   const int lane = threadIdx.x & 63;

@@ -111,3 +111,34 @@ def test_replaced_meshes(sizes):
         np.testing.assert_array_equal(cnt[0], ref["counts"])
         assert_wrench_close(W[0], ref["wrench"])
     e.close()
+
+
+@pytest.mark.parametrize("n", [60, 250])
+def test_batch_items_cut_by_expected_candidates(engine, n):
+    """Batches of enough items that each is cut by itself: fine pads, soft
+    pairs, a ball on a box and a fine body on one huge triangle's neighbours
+    (chunks of a dozen triangles that meet a whole mesh), every third pair
+    lifted away.  Results are those of calls of one pair."""
+    print("[case] spread", n, flush=True)
+    base = _scenes(engine)
+    big = S.tactile_pad(4, L=4, K=4, m=2)
+    ha, hb = add_scene(engine, big)
+    base.append(pair_of(big, ha, hb))
+    away = [(a, b, XA + np.r_[np.zeros(11), 5.0], XB, VA, VB) for a, b, XA, XB, VA, VB in base]
+    W1, c1 = zip(*[engine.contact_step([p]) for p in base])
+    pairs = [(away if k % 3 == 1 else base)[k // 3 % 4] for k in range(n)]
+    b = engine.batch([p[:2] for p in pairs])
+    b.set_state(np.array([np.concatenate(p[2:]) for p in pairs]))
+    for _ in range(2):
+        b.step()
+        W, cnt = b.get()
+        for k in range(n):
+            if k % 3 == 1:
+                assert cnt[k, 1] == 0 and not W[k].any()
+                continue
+            np.testing.assert_array_equal(cnt[k], c1[k // 3 % 4][0])
+            assert_wrench_close(W[k], W1[k // 3 % 4][0], rtol=1e-12)
+    first, _ = b.get()
+    b.step()
+    np.testing.assert_array_equal(b.get()[0], first)  # the cut does not depend on the order of the sums
+    b.close()
