@@ -206,7 +206,6 @@ __device__ inline int delta(const unsigned* codes, int n, int i, int j) {
 struct BuildOut {
   int bad;    /* the sort did not return a permutation in code order: nothing is built on it */
   int height; /* of the tree: the depth of its deepest leaf */
-  int32_t roots[HCS_ROOTS];
 };
 
 /* The leaf order must be a permutation in code order before a tree is built
@@ -463,7 +462,8 @@ __global__ __launch_bounds__(64) void k_chunk_boxes(const double* __restrict__ V
 
 /* The LBVH's frontiers (HCS_ROOTS), one block, level by level. */
 __global__ __launch_bounds__(HCS_ROOTS / 2) void k_frontiers(const Node* __restrict__ nodes, int n_int,
-                                                             BuildOut* __restrict__ out, int32_t* __restrict__ heap) {
+                                                             const BuildOut* __restrict__ out,
+                                                             int32_t* __restrict__ heap) {
   __shared__ int32_t h[HCS_ROOTS];
   const int t = threadIdx.x;
   if (out->bad) return;
@@ -479,7 +479,7 @@ __global__ __launch_bounds__(HCS_ROOTS / 2) void k_frontiers(const Node* __restr
     __syncthreads();
   }
 #pragma unroll
-  for (int k = 0; k < 2; ++k) heap[k * (HCS_ROOTS / 2) + t] = out->roots[k * (HCS_ROOTS / 2) + t] = h[k * (HCS_ROOTS / 2) + t];
+  for (int k = 0; k < 2; ++k) heap[k * (HCS_ROOTS / 2) + t] = h[k * (HCS_ROOTS / 2) + t];
 }
 
 /* Static boxes of one item per wave: [0..5] its query elements in their own
@@ -1294,7 +1294,8 @@ static int build_bvh(Ctx* c, Mesh& m, const double* V) {
                        (const int2*)range, n - 1, (const BuildOut*)out, m.nodes, m.wnodes);
     hipLaunchKernelGGL(k_tree_height, g, t, 0, s, (const int*)lp, (const int*)np, n, out);
   }
-  hipLaunchKernelGGL(k_frontiers, dim3(1), dim3(HCS_ROOTS / 2), 0, s, (const Node*)m.nodes, n - 1, out, m.roots);
+  hipLaunchKernelGGL(k_frontiers, dim3(1), dim3(HCS_ROOTS / 2), 0, s, (const Node*)m.nodes, n - 1,
+                     (const BuildOut*)out, m.roots);
   rc = hip_check(c, hipGetLastError(), "LBVH build");
   BuildOut* got = (BuildOut*)c->pin_down; /* (at least 64 KB) */
   static_assert(sizeof(BuildOut) <= (64 << 10), "build result fits the pinned block");
@@ -1308,7 +1309,6 @@ static int build_bvh(Ctx* c, Mesh& m, const double* V) {
   if (rc) return rc;
   if (got->bad) return set_err(c, HCS_ERR_HIP, "LBVH build: the Morton sort returned an invalid order");
   m.height = got->height;
-  std::memcpy(m.roots_h, got->roots, sizeof m.roots_h);
   if (3 * ((m.height + 1) / 2) + 1 > HCS_STACK)
     return set_err(c, HCS_ERR_LIMIT, "LBVH height " + std::to_string(m.height) + " exceeds the traversal stack");
   return HCS_OK;
@@ -1429,7 +1429,7 @@ int build_plan(Ctx* c, int npairs, const int32_t* geoms, const hcs_step_opts* o,
     E.boxB = hcs_gptr((const double*)(E.kind == KIND_TET ? B.cbox + 6 * (size_t)((B.nelem + 63) / 64) : nullptr));
     E.item_count = (nq + chunk - 1) / chunk;
   }
-  if (mode != ITEMS_WHOLE) static_depths(plan);
+  if (mode == ITEMS_IMPLICIT) static_depths(plan);
   int64_t total = 0;
   for (int e = 0; e < npairs; ++e) {
     EnvDesc& E = plan.envs[e];
@@ -1441,12 +1441,7 @@ int build_plan(Ctx* c, int npairs, const int32_t* geoms, const hcs_step_opts* o,
       for (int i = 0; i < E.item_count; i += HCS_GEN_THREADS) plan.blocks.push_back(make_int2(e, i));
     } else {
       /* (root 0: the whole LBVH of A) */
-      const int32_t* roots = c->meshes[geoms[2 * e]].roots_h + (1 << E.depth);
-      for (int k = 0; k < chunks; ++k)
-        for (int s = 0; s < (1 << E.depth); ++s) {
-          const int32_t root = E.depth ? roots[s] : 0;
-          if (root != HCS_WNONE) plan.items.push_back(Item{e, 64 * k, std::min(64, nq - 64 * k), root});
-        }
+      for (int k = 0; k < chunks; ++k) plan.items.push_back(Item{e, 64 * k, std::min(64, nq - 64 * k), 0});
       E.item_count = (int)plan.items.size() - E.item_first;
     }
     total += E.item_count;

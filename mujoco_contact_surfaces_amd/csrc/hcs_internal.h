@@ -36,7 +36,6 @@ struct Mesh {
   double* cbox = nullptr;    /* boxes of the chunks of 64 elements in leaf / query order, then (rigid) of the vertices */
   double* csize = nullptr;   /* mean half-extents of the chunks' elements */
   int32_t* roots = nullptr;  /* soft: LBVH frontiers (HCS_ROOTS) */
-  int32_t roots_h[HCS_ROOTS] = {}; /* their host copy */
 };
 
 /* Grow-only device buffer.  A fixed buffer is a view of memory the library
@@ -136,8 +135,7 @@ struct Ctx {
  * lane of the candidate kernel's wave).  Returns HCS_OK or an error. */
 enum PlanItems {
   ITEMS_WHOLE,    /* one item per chunk over A's whole tree (measured splitting follows) */
-  ITEMS_SPLIT,    /* over the static frontiers of static_depths() */
-  ITEMS_IMPLICIT, /* the same items, enumerated on the device */
+  ITEMS_IMPLICIT, /* over the static frontiers of static_depths(), enumerated on the device */
 };
 int build_plan(Ctx* c, int npairs, const int32_t* geoms, const hcs_step_opts* o, int tet_mode_max_tris,
                Plan& plan, PlanItems mode = ITEMS_WHOLE);
