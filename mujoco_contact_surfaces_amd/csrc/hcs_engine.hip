@@ -867,8 +867,8 @@ __global__ __launch_bounds__(256, 2) void k_clip(QueryArgs A, ClipArgs C, int di
  * from the plan's table sums slice j of the pair's contributions (a fixed
  * split of its slot range) lane-strided in order, then a fixed butterfly,
  * and the slice's items' candidate counts likewise; grid.y = direction.
- * k_env_combine adds a pair's slices in order, so results do not depend on
- * timing, and a heavy pair (K_e grows with its item count) no longer sets
+ * k_env_combine adds a pair's slices by a fixed butterfly, so results do not
+ * depend on timing, and a heavy pair (K_e grows with its item count) no longer sets
  * the time of the whole reduction. */
 __global__ __launch_bounds__(64) void k_env_reduce(const EnvDesc* __restrict__ envs, const int4* __restrict__ rtab,
                                                    int nred, const unsigned* __restrict__ off,
@@ -890,36 +890,29 @@ __global__ __launch_bounds__(64) void k_env_reduce(const EnvDesc* __restrict__ e
   if (threadIdx.x == 0) part[(int64_t)d * nred + w.w + j] = r;
 }
 
-/* One thread per (pair, direction): the pair's slices in order. */
-__global__ void k_env_combine(const int2* __restrict__ ptab, int nred, const RedPart* __restrict__ part,
-                              const unsigned long long* __restrict__ surv_cnt, int64_t surv_cap,
-                              const int* __restrict__ err, PairOut* __restrict__ out, int n, int ndir) {
-  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (t >= (int64_t)n * ndir) return;
-  const int e = (int)(t % n), d = (int)(t / n);
+/* One wave per (pair, direction): the pair's K <= 64 slices, one per lane, by
+ * a fixed butterfly (a thread that added them in order: 20 us for 4096 pairs,
+ * 31 us for 256 pairs of 64 slices; this: 9 and 4). */
+__global__ __launch_bounds__(64) void k_env_combine(const int2* __restrict__ ptab, int nred,
+                                                    const RedPart* __restrict__ part,
+                                                    const unsigned long long* __restrict__ surv_cnt, int64_t surv_cap,
+                                                    const int* __restrict__ err, PairOut* __restrict__ out, int n) {
+  const int e = (int)(blockIdx.x % (unsigned)n), d = (int)(blockIdx.x / (unsigned)n), lane = threadIdx.x;
   const int2 pe = ptab[e];
-  const RedPart* p = part + (int64_t)d * nred + pe.x;
-  double F[3] = {0, 0, 0}, tA[3] = {0, 0, 0}, tB[3] = {0, 0, 0};
-  int64_t np = 0, nf = 0, nc = 0;
-  auto add = [&](const RedPart& q) {
+  RedPart q{};
+  if (lane < pe.y) q = part[(int64_t)d * nred + pe.x + lane];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) F[c] = F[c] + q.F[c], tA[c] = tA[c] + q.tA[c], tB[c] = tB[c] + q.tB[c];
-    np += q.np, nf += q.nf, nc += q.nc;
-  };
-  /* in slice order; four slices loaded before they are added */
-  int j = 0;
-  for (; j + 3 < pe.y; j += 4) {
-    const RedPart q0 = p[j], q1 = p[j + 1], q2 = p[j + 2], q3 = p[j + 3];
-    add(q0), add(q1), add(q2), add(q3);
-  }
-  for (; j < pe.y; ++j) add(p[j]);
+  for (int c = 0; c < 3; ++c)
+    q.F[c] = wave_sum<double>(q.F[c]), q.tA[c] = wave_sum<double>(q.tA[c]), q.tB[c] = wave_sum<double>(q.tB[c]);
+  q.np = wave_sum_i(q.np), q.nf = wave_sum_i(q.nf), q.nc = wave_sum_i(q.nc);
+  if (lane != 0) return;
   const bool over = (int64_t)*surv_cnt > surv_cap;
   PairOut r;
 #pragma unroll
-  for (int c = 0; c < 3; ++c) r.F_A[c] = F[c], r.tau_A[c] = tA[c], r.F_B[c] = -F[c], r.tau_B[c] = tB[c];
-  r.n_candidates = nc, r.n_polygons = np, r.n_faces = nf;
+  for (int c = 0; c < 3; ++c) r.F_A[c] = q.F[c], r.tau_A[c] = q.tA[c], r.F_B[c] = -q.F[c], r.tau_B[c] = q.tB[c];
+  r.n_candidates = q.nc, r.n_polygons = q.np, r.n_faces = q.nf;
   r.status = (err && *err) ? HCS_ERR_LIMIT : (over ? HCS_ERR_CAPACITY : 0);
-  out[t] = r;
+  out[blockIdx.x] = r;
 }
 
 void launch_prep(hipStream_t s, const EnvDesc* envs, const double* state, double* xf, int n) {
@@ -1062,9 +1055,9 @@ static void pipe_back(Ctx* c, Pipe& p, const QueryArgs& a, int npairs, int clip_
     hipLaunchKernelGGL(k_env_reduce, dim3(p.nred, nd), dim3(64), 0, s, a.envs, (const int4*)p.rtab.ptr, p.nred,
                        (const unsigned*)p.off.ptr, (const int*)p.ncand.ptr, (const unsigned long long*)p.surv_cnt.ptr,
                        p.cap, (const Contrib*)p.contrib.ptr, (int64_t)p.cap, (RedPart*)p.part.ptr);
-    hipLaunchKernelGGL(k_env_combine, dim3((npairs * nd + 127) / 128), dim3(128), 0, s, (const int2*)p.ptab.ptr,
-                       p.nred, (const RedPart*)p.part.ptr, (const unsigned long long*)p.surv_cnt.ptr, p.cap,
-                       (const int*)p.err.ptr, (PairOut*)p.out.ptr, npairs, nd);
+    hipLaunchKernelGGL(k_env_combine, dim3(npairs * nd), dim3(64), 0, s, (const int2*)p.ptab.ptr, p.nred,
+                       (const RedPart*)p.part.ptr, (const unsigned long long*)p.surv_cnt.ptr, p.cap,
+                       (const int*)p.err.ptr, (PairOut*)p.out.ptr, npairs);
   }
 }
 
@@ -1081,14 +1074,19 @@ void launch_clip_reduce(Ctx* c, Pipe& p, const QueryArgs& a, int npairs, int cli
   pipe_back(c, p, a, npairs, clip_grid, 0, nullptr, nullptr, 0, e_clip, e_reduce);
 }
 
-/* Reduction slices: a pair of n items gets ceil(n / 8) waves (at most 64;
- * a split heavy pair has many items).  rt: per wave (pair, slice, slices,
- * first partial of the pair); pt: per pair (first partial, slices). */
+/* Reduction slices: a pair of n items gets ceil(n / 8) waves (a split heavy
+ * pair has many items), at most 32, or 64 where the pairs are few: a wave's
+ * sums end in a butterfly of 72 dependent shuffles, and 256 soft pairs of 64
+ * slices each were mostly those (30 us, 20 with 32).  Many uneven pairs are
+ * bound by reading the contributions (4096 objects: 88 us, 210 MB).  rt: per
+ * wave (pair, slice, slices, first partial of the pair); pt: per pair (first
+ * partial, slices). */
 void reduction_slices(const Plan& plan, std::vector<int4>& rt, std::vector<int2>& pt) {
   rt.clear();
   pt.assign(std::max<size_t>(1, plan.envs.size()), make_int2(0, 0));
+  const int most = std::max(32, std::min(64, 4096 / (int)std::max<size_t>(1, plan.envs.size())));
   for (size_t e = 0; e < plan.envs.size(); ++e) {
-    const int K = std::max(1, std::min(64, (plan.envs[e].item_count + 7) / 8));
+    const int K = std::max(1, std::min(most, (plan.envs[e].item_count + 7) / 8));
     pt[e] = make_int2((int)rt.size(), K);
     for (int j = 0; j < K; ++j) rt.push_back(make_int4((int)e, j, K, (int)rt.size() - j));
   }

@@ -142,3 +142,25 @@ def test_batch_items_cut_by_expected_candidates(engine, n):
     b.step()
     np.testing.assert_array_equal(b.get()[0], first)  # the cut does not depend on the order of the sums
     b.close()
+
+
+@pytest.mark.parametrize("n", [1, 64, 65, 129])
+def test_batch_reduction_slices(engine, n):
+    """Pairs of several hundred items in a measured batch: 64 reduction slices
+    a pair up to 64 pairs, fewer beyond, 32 from 128 on."""
+    print("[case] slices", n, flush=True)
+    sc = S.tactile_pad(7, L=4, K=3, m=40, depth=0.006)
+    ha, hb = add_scene(engine, sc)
+    pair = pair_of(sc, ha, hb)
+    W1, c1 = engine.contact_step([pair])
+    b = engine.batch([pair[:2]] * n)
+    b.set_state(np.tile(np.concatenate(pair[2:]), (n, 1)))
+    b.set_config(12, 1, 0, 64, 1, 1)
+    b.step()
+    W, cnt = b.get()
+    assert len(b.item_stats()) > 8 * 64 * n  # more than 64 slices of 8 items a pair without a limit
+    for k in range(n):
+        np.testing.assert_array_equal(cnt[k], c1[0])
+        assert_wrench_close(W[k], W1[0], rtol=1e-12)
+    np.testing.assert_array_equal(W, np.tile(W[:1], (n, 1)))
+    b.close()
