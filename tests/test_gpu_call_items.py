@@ -164,3 +164,23 @@ def test_batch_reduction_slices(engine, n):
         assert_wrench_close(W[k], W1[0], rtol=1e-12)
     np.testing.assert_array_equal(W, np.tile(W[:1], (n, 1)))
     b.close()
+
+
+# tets: below one tile of 2048 keys, a few tiles, and on both sides of the 64
+# tiles up to which a sort pass adds up its counts itself
+@pytest.mark.parametrize("L,K", [(2, 3), (4, 2), (5, 3), (5, 4)])
+def test_sorted_leaves(engine, L, K):
+    """The LBVH over Morton-sorted tets finds every candidate (its build
+    refuses an order that is not sorted)."""
+    V, T, p = S.soft_mesh(L, K, 1, 0.04, 0.03, 0.02, 5e4)
+    print("[case] sort", len(T), flush=True)
+    VR, FR = S.rigid_mesh(1, 6, 0.4)
+    sp = dict(S.SOFT_PROPS, hydroelastic_modulus=5e4)
+    ha, hb = engine.add_soft_mesh(V, T, p, sp, 0), engine.add_rigid_mesh(VR, FR, S.RIGID_PROPS, 1)
+    XA, XB, z = S.pose(np.eye(3), [0.013, 0.007, 0.017]), S.pose(np.eye(3), [0, 0, 0]), np.zeros(6)
+    W, cnt = engine.contact_step([(ha, hb, XA, XB, z, z)])
+    ref = O.soft_rigid(V, T, p, VR, FR, XA, XB, z, z, 5e4, sp["dissipation"], sp["dynamic_friction"],
+                       S.RIGID_PROPS["dynamic_friction"])
+    np.testing.assert_array_equal(cnt[0], ref["counts"])
+    assert cnt[0, 1] > 0
+    assert_wrench_close(W[0], ref["wrench"])
