@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "hcs_internal.h"
+#include "hcs_clip.h"
 #include "hcs_prim.h"
 #include "hcs_query.h"
 #include "hcs_reduce.h"
@@ -863,6 +864,16 @@ __global__ __launch_bounds__(256, 2) void k_clip(QueryArgs A, ClipArgs C, int di
     clip_survivor<T, KS, kCol>(A, C, i, dir, dst, op, col + threadIdx.x, 256);
 }
 
+/* Launches that mix kinds: 64 survivors per wave (grid-stride). */
+__global__ __launch_bounds__(64, 2) void k_clip_mixed(QueryArgs A, ClipArgs C, Contrib* out) {
+  __shared__ ClipLds L;
+  const OutPtrs o{A.face_rec, A.face_key, A.face_cnt, A.face_cap, A.poly_rec,
+                  A.poly_key, A.poly_cnt, A.poly_cap, A.poly_tan, A.poly_env};
+  const unsigned long long cnt = *A.surv_cnt;
+  const int64_t n = (int64_t)cnt < A.surv_cap ? (int64_t)cnt : A.surv_cap;
+  clip_wave(L, A, C, blockIdx.x * (int64_t)64, (int64_t)gridDim.x * 64, n, o, out);
+}
+
 /* Per pair, in K_e waves: wave w = (pair e, slice j, K_e, first partial)
  * from the plan's table sums slice j of the pair's contributions (a fixed
  * split of its slot range) lane-strided in order, then a fixed butterfly,
@@ -1029,7 +1040,7 @@ void launch_clip(Ctx* c, const Pipe& p, const QueryArgs& a, int clip_grid) {
     case KIND_SOFT: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_clip<double, KIND_SOFT>), g, dim3(256), 0, s, a, C, -1, out, zero); break;
     case KIND_TET: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_clip<double, KIND_TET>), g, dim3(256), 0, s, a, C, -1, out, zero); break;
     case KIND_PLANE: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_clip<double, KIND_PLANE>), g, dim3(256), 0, s, a, C, -1, out, zero); break;
-    default: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_clip<double, -1>), g, dim3(256), 0, s, a, C, -1, out, zero); break;
+    default: hipLaunchKernelGGL(k_clip_mixed, dim3(4 * g.x), dim3(64), 0, s, a, C, out); break;
   }
 }
 

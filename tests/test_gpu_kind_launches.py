@@ -50,3 +50,38 @@ def test_half_space_launch(engine, sizes, queues):
         assert_wrench_close(W[i], r["wrench"])
         assert_wrench_close(Wb[i], r["wrench"])
         assert st[st[:, 0] == i, 5].sum() == r["counts"][0]
+
+
+# few survivors (less than a wave), some hundred, some thousand a pair
+@pytest.mark.parametrize("size", [(0, 1), (1, 1), (3, 2)], ids=["20", "80", "5120"])
+@pytest.mark.parametrize("representation", [0, 1])
+@pytest.mark.parametrize("friction", [True, False])
+def test_mixed_launch_clips_like_the_launches_of_one_kind(engine, size, representation, friction):
+    """A half-space, a triangle and a soft pair in one call against calls of
+    one pair: the same faces, record for record; the wrenches' sums differ in
+    order only."""
+    print("[case] mixed clip", size, representation, friction, flush=True)
+    plane, _ = _plane_scene(engine, 1, *size)
+    pad = S.tactile_pad(3, L=size[0], K=size[1], m=20, depth=0.006)
+    soft = S.soft_soft_env(3, 0, nt_range=(3e3, 6e3))
+    pairs = [plane]
+    for sc in (pad, soft):
+        pairs.append(pair_of(sc, *add_scene(engine, sc)))
+    opts = dict(representation=representation, apply_forces=friction, face_capacity=1 << 18)
+
+    def ordered(rec, key):
+        o = np.lexsort(key.T[::-1])
+        return rec[o], key[o]
+
+    W, cnt, (rec, key) = engine.contact_step(pairs, **opts)
+    rec, key = ordered(rec, key)
+    assert (cnt[:, 2] > 0).all() and len(rec) == cnt[:, 2].sum()
+    for k, p in enumerate(pairs):
+        W1, c1, (r1, k1) = engine.contact_step([p], **opts)
+        np.testing.assert_array_equal(cnt[k], c1[0])
+        if friction:
+            assert_wrench_close(W[k], W1[0], rtol=1e-12)
+        r1, k1 = ordered(r1, k1)
+        mine = key[:, 0] == k
+        np.testing.assert_array_equal(key[mine][:, 1:], k1[:, 1:])
+        np.testing.assert_array_equal(rec[mine], r1)
