@@ -153,6 +153,9 @@ __global__ __launch_bounds__(64 * W) void k_tx_sample_fan(const double* __restri
  * made again. */
 int run_taxels(Ctx* c, const TaxelGridDev& g, const std::vector<unsigned char>& seen, const double* poly,
                const double* ptan, const int64_t* key, int64_t np, const double* Xd, double* out) {
+  /* taxels that the kernel writes to pinned memory itself, and that go there
+   * by a copy; beyond, straight to the caller */
+  constexpr int kDirect = 8192, kPinned = 1 << 20;
   const int ncell = g.cx * g.cy;
   const size_t scan_bytes = scan_temp_bytes((long long)ncell + 1);
   int rc;
@@ -160,7 +163,7 @@ int run_taxels(Ctx* c, const TaxelGridDev& g, const std::vector<unsigned char>& 
       (rc = ensure(c, c->d_tx_off, sizeof(unsigned) * ((size_t)ncell + 1) + scan_bytes + 8)) ||
       (rc = ensure(c, c->d_tx_foot, sizeof(int4) * (size_t)std::max<int64_t>(1, np))) ||
       (rc = ensure(c, c->d_tx_list, sizeof(int) * (size_t)std::max<int64_t>(4096, 4 * np))) ||
-      (rc = pinned(c, c->pin_down, c->pin_down_bytes, sizeof(double) * ((size_t)ncell + 1))))
+      (rc = pinned(c, c->pin_down, c->pin_down_bytes, sizeof(double) * (std::min<size_t>(ncell, kPinned) + 1))))
     return rc;
   TxPairs pairs{};
   if (seen.size() > 256) {
@@ -173,10 +176,10 @@ int run_taxels(Ctx* c, const TaxelGridDev& g, const std::vector<unsigned char>& 
     for (size_t e = 0; e < seen.size(); ++e)
       if (seen[e]) pairs.bits[e >> 6] |= 1ull << (e & 63);
   }
-  /* small grids: the kernel writes the pinned memory itself */
   double* got = (double*)c->pin_down;
   double* d_out = got;
-  if (ncell > 8192) {
+  const double* total = got + (ncell > kPinned ? 0 : ncell);
+  if (ncell > kDirect) {
     if ((rc = ensure(c, c->d_tx_out, sizeof(double) * ((size_t)ncell + 1)))) return rc;
     d_out = (double*)c->d_tx_out.ptr;
   }
@@ -215,15 +218,21 @@ int run_taxels(Ctx* c, const TaxelGridDev& g, const std::vector<unsigned char>& 
                          (const int*)list, list_cap, d_out);
     }
     rc = hip_check(c, hipGetLastError(), "taxel kernels");
-    if (!rc && d_out != got)
+    if (!rc && ncell > kPinned) {
+      rc = hip_check(c, hipMemcpyAsync(out, d_out, sizeof(double) * (size_t)ncell, hipMemcpyDeviceToHost, c->stream),
+                     "download taxels");
+      if (!rc)
+        rc = hip_check(c, hipMemcpyAsync(got, d_out + ncell, sizeof(double), hipMemcpyDeviceToHost, c->stream), "download");
+    } else if (!rc && d_out != got) {
       rc = hip_check(c, hipMemcpyAsync(got, d_out, sizeof(double) * ((size_t)ncell + 1), hipMemcpyDeviceToHost, c->stream),
                      "download taxels");
+    }
     if (!rc) rc = hip_check(c, hipStreamSynchronize(c->stream), "sync");
     if (rc) return rc;
-    if ((int64_t)got[ncell] <= list_cap) break;
-    if ((rc = ensure(c, c->d_tx_list, sizeof(int) * (size_t)got[ncell]))) return rc;
+    if ((int64_t)*total <= list_cap) break;
+    if ((rc = ensure(c, c->d_tx_list, sizeof(int) * (size_t)*total))) return rc;
   }
-  std::memcpy(out, got, sizeof(double) * (size_t)ncell);
+  if (ncell <= kPinned) std::memcpy(out, got, sizeof(double) * (size_t)ncell);
   return HCS_OK;
 }
 

@@ -30,6 +30,7 @@ FINE, COARSE, TINY = dict(L=4, K=4, m=48), dict(L=2, K=2, m=4), dict(L=1, K=1, m
     (TINY, 5, 24, 1, 0.3),
     (TINY, 60, 3, 0, 0.0),  # few polygons over many taxels: the lists outgrow their first buffer
     (COARSE, 91, 2, 0, 0.0),  # 8281 taxels: more than the kernel writes to host memory itself
+    (TINY, 1025, 1, 0, 0.0),  # more than a million: copied straight to the caller
 ])
 def test_flat_sensor_work_split(engine, shape, taxels, rays, window, sigma):
     print("[case] flat", shape, taxels, rays, window, flush=True)
