@@ -229,7 +229,9 @@ int hcs_taxels(hcs_ctx* ctx, int32_t nsensors, const hcs_taxel_grid* g, double* 
 /* TaxelSensor::internal_update (S/src/taxel_sensor.cpp:158-478) on the
  * polygons of the last hcs_contact_step run with keep_polygons = 1.
  * values (ntaxels, in/out): taxels no sample reaches keep their value, as
- * the reference's message does; *nsamples (optional) = surface samples. */
+ * the reference's message does; *nsamples (optional) = surface samples.  A
+ * sample_resolution that asks for more than 2^32 - 1 of them is refused
+ * (HCS_ERR_LIMIT). */
 int hcs_taxel_sensor_update(hcs_ctx* ctx, const hcs_taxel_sensor* sensor, double* values, int64_t* nsamples);
 /* CurvedSensor::internal_update (S/src/curved_sensor.cpp:388-481) on the
  * polygons of the last hcs_contact_step run with keep_polygons = 1: one ray

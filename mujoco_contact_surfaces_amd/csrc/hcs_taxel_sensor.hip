@@ -36,6 +36,7 @@
 #include "hcs_internal.h"
 #include "hcs_prim.h"
 #include "hcs_query.h"
+#include "hcs_samples.h"
 
 #pragma clang fp contract(off)
 
@@ -49,12 +50,14 @@ namespace hcs {
  * into the bits the pairs and meshes need when those fit 64 (ba, bb >= 0:
  * bits of the elements), else (element of A, element of B) with the pair in
  * kp.  Unselected polygons sort last.  For the rank sort, its counters are
- * cleared here and every place is empty (-1) until a polygon takes it. */
+ * cleared here and every place is empty (-1) until a polygon takes it.  The
+ * sampler's total is cleared too. */
 __global__ void k_ts_keys(const int64_t* __restrict__ key, int64_t np, const unsigned char* __restrict__ mask, int ba,
                           int bb, unsigned long long* __restrict__ k64, unsigned* __restrict__ kp,
-                          int* __restrict__ idx, unsigned* __restrict__ rank) {
+                          int* __restrict__ idx, unsigned* __restrict__ rank, TsTotal* __restrict__ total) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= np) return;
+  if (i == 0) *total = TsTotal{};
   const unsigned long long pair = key[3 * i], a = key[3 * i + 1], b = key[3 * i + 2];
   const bool on = mask[pair] != 0;
   if (ba >= 0) {
@@ -232,10 +235,11 @@ __global__ void k_ts_areas(const double* __restrict__ tris, const int* __restric
 
 #define HCS_TS_CHAIN 1024
 __global__ __launch_bounds__(64) void k_ts_chain(const int* __restrict__ surf, int64_t nt,
-                                                 const int* __restrict__ surf0, unsigned* __restrict__ nsurf,
+                                                 const int* __restrict__ surf0, const unsigned* __restrict__ nsurf,
                                                  double res, bool write, double* __restrict__ at,
-                                                 unsigned* __restrict__ count, const unsigned* __restrict__ off,
-                                                 double* __restrict__ acc_out, int2* __restrict__ tri_out) {
+                                                 unsigned* __restrict__ count, TsTotal* __restrict__ total,
+                                                 const unsigned* __restrict__ off, double* __restrict__ acc_out,
+                                                 int2* __restrict__ tri_out) {
   __shared__ double L[HCS_TS_CHAIN];
   const int lane = threadIdx.x;
   if (blockIdx.x >= *nsurf) return;
@@ -282,18 +286,14 @@ __global__ __launch_bounds__(64) void k_ts_chain(const int* __restrict__ surf, i
   top = wave_max(top);
   const double step = res * at[t1 - 1];
   const unsigned base = write ? off[id] : 0u;
-  unsigned n = 0;
-  for (double acc = 0.0; acc < top; ++n) {
-    if (write && lane == 0) acc_out[base + n] = acc, tri_out[base + n] = make_int2((int)t0, (int)t1 - 1);
-    const double next = acc + step;
-    if (next == acc) {
-      /* a step below the rounding of acc would never reach the end */
-      if (lane == 0) nsurf[1] = 1u;
-      break;
-    }
-    acc = next;
-  }
-  if (!write && lane == 0) count[id] = n;
+  bool too_many;
+  const unsigned n = area_chain(top, step, too_many, [&](unsigned k, double acc) {
+    if (write && lane == 0) acc_out[base + k] = acc, tri_out[base + k] = make_int2((int)t0, (int)t1 - 1);
+  });
+  if (write || lane != 0) return;
+  count[id] = n;
+  atomicAdd(&total->n, (unsigned long long)n);
+  if (too_many) total->too_many = 1;
 }
 
 /* x * 16807^e modulo 2^31 - 1 */
@@ -642,7 +642,7 @@ static int sensor_fans(Ctx* c, int32_t geom, unsigned& ntri) {
     const bool rank = packed && np <= HCS_TS_RANK;
     const unsigned nb = (unsigned)((np + 255) / 256);
     hipLaunchKernelGGL(k_ts_keys, dim3(nb), dim3(256), 0, s, (const int64_t*)c->d_poly_key.ptr, np, dmask,
-                       packed ? ba : -1, bb, k64, kp, rank ? order : idx, rank ? kp : nullptr);
+                       packed ? ba : -1, bb, k64, kp, rank ? order : idx, rank ? kp : nullptr, (TsTotal*)B.cnt.ptr);
     if (rank) {
       const int slices = (int)std::max<int64_t>(1, std::min<int64_t>(nb, 512 / nb));
       const int per = (int)((np + slices - 1) / slices);
@@ -689,6 +689,18 @@ static int sensor_fans(Ctx* c, int32_t geom, unsigned& ntri) {
   return hip_check(c, hipGetLastError(), "sensor triangles");
 }
 
+/* The sampler's count, when it is not refused. */
+static int sample_total(Ctx* c, unsigned long long& m) {
+  TsTotal t{};
+  int rc = hip_check(c, hipMemcpyAsync(&t, c->ts.cnt.ptr, sizeof t, hipMemcpyDeviceToHost, c->stream), "dl");
+  if (!rc) rc = hip_check(c, hipStreamSynchronize(c->stream), "sync");
+  if (rc) return rc;
+  if (t.too_many || t.n > HCS_TS_MAX)
+    return set_err(c, HCS_ERR_LIMIT, "sensor: sample_resolution asks for more than 2^32 - 1 samples");
+  m = t.n;
+  return HCS_OK;
+}
+
 int hcs_taxel_sensor_update(hcs_ctx* h, const hcs_taxel_sensor* S, double* values, int64_t* nsamples) {
   if (!h || !S || !values || S->ntaxels < 0 || (S->ntaxels > 0 && !S->taxels) || S->method < 0 || S->method > 3 ||
       S->sample_method < 0 || S->sample_method > 1 || !(S->sample_resolution > 0) || !(S->include_margin >= 0))
@@ -721,28 +733,22 @@ int hcs_taxel_sensor_update(hcs_ctx* h, const hcs_taxel_sensor* S, double* value
     m = m32;
   } else if (ntri > 0) {
     /* areas and prefix sums; per pair the first triangle (in no order), the
-     * sample count and its scan; [surfaces, stalled] */
+     * sample count and its scan; the surfaces */
     const size_t np1 = c->last_pairs.size() + 1;
-    if ((rc = ensure(c, B.area, sizeof(double) * ntri)) || (rc = ensure(c, B.pair_u, sizeof(unsigned) * (3 * np1 + 2))) ||
+    if ((rc = ensure(c, B.area, sizeof(double) * ntri)) || (rc = ensure(c, B.pair_u, sizeof(unsigned) * (3 * np1 + 1))) ||
         (rc = ensure(c, B.tmp, std::max<size_t>(scan_temp_bytes((long long)np1), 8))))
       return rc;
     unsigned* cnt = (unsigned*)B.pair_u.ptr;
-    nsurf = cnt + np1, soff = nsurf + 2, surf0 = (int*)(soff + np1);
-    launch_fill_u32(s, cnt, 0u, (int)np1 + 2);
+    nsurf = cnt + np1, soff = nsurf + 1, surf0 = (int*)(soff + np1);
+    launch_fill_u32(s, cnt, 0u, (int)np1 + 1);
     hipLaunchKernelGGL(k_ts_areas, dim3((ntri + 255) / 256), dim3(256), 0, s, (const double*)B.tris.ptr,
                        (const int*)B.surf.ptr, (int64_t)ntri, (double*)B.area.ptr, surf0, nsurf);
     hipLaunchKernelGGL(k_ts_chain, dim3((unsigned)c->last_pairs.size()), dim3(64), 0, s, (const int*)B.surf.ptr,
                        (int64_t)ntri, surf0, nsurf, S->sample_resolution, false, (double*)B.area.ptr, cnt,
-                       (const unsigned*)soff, (double*)nullptr, (int2*)nullptr);
+                       (TsTotal*)B.cnt.ptr, (const unsigned*)soff, (double*)nullptr, (int2*)nullptr);
     if (exclusive_scan_u32(s, cnt, soff, (long long)np1, B.tmp.ptr, B.tmp.bytes) != 0)
       return set_err(c, HCS_ERR_LIMIT, "sensor: too many pairs to scan");
-    unsigned got[2] = {0, 0}; /* stalled, samples */
-    rc = hip_check(c, hipMemcpyAsync(got, nsurf + 1, sizeof(unsigned), hipMemcpyDeviceToHost, s), "dl");
-    if (!rc) rc = hip_check(c, hipMemcpyAsync(got + 1, soff + np1 - 1, sizeof(unsigned), hipMemcpyDeviceToHost, s), "dl");
-    if (!rc) rc = hip_check(c, hipStreamSynchronize(s), "sync");
-    if (rc) return rc;
-    if (got[0]) return set_err(c, HCS_ERR_LIMIT, "sensor: sample_resolution is below the rounding of the surface's area");
-    m = got[1];
+    if ((rc = sample_total(c, m))) return rc;
   }
   if (nsamples) *nsamples = (int64_t)m;
   if (m == 0) {
@@ -762,7 +768,7 @@ int hcs_taxel_sensor_update(hcs_ctx* h, const hcs_taxel_sensor* S, double* value
     int2* range = (int2*)(acc + m);
     hipLaunchKernelGGL(k_ts_chain, dim3((unsigned)c->last_pairs.size()), dim3(64), 0, s, (const int*)B.surf.ptr,
                        (int64_t)ntri, surf0, nsurf, S->sample_resolution, true, (double*)B.area.ptr,
-                       (unsigned*)nullptr, (const unsigned*)soff, acc, range);
+                       (unsigned*)nullptr, (TsTotal*)nullptr, (const unsigned*)soff, acc, range);
     hipLaunchKernelGGL(k_ts_draw, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, (const double*)B.tris.ptr,
                        (const double*)B.area.ptr, (const double*)acc, (const int2*)range, (int64_t)m,
                        (double*)B.P.ptr, (double*)B.E.ptr);

@@ -1,0 +1,35 @@
+"""Taxel sensors that ask for more samples than 32-bit offsets number are
+refused before a buffer is sized by the count; the next call is served."""
+import numpy as np
+import pytest
+
+from mujoco_contact_surfaces_amd import scenes as S
+from mujoco_contact_surfaces_amd.engine import HcsError
+from test_gpu_parity import add_scene, pair_of
+
+pytestmark = pytest.mark.gpu
+
+HCS_ERR_LIMIT = -6
+TAXELS = np.array([[x, 0.0, 0.002] for x in np.linspace(-0.02, 0.02, 5)])
+
+
+def _step(engine, npairs):
+    sc = S.tactile_pad(3, L=1, K=1, m=2)
+    ha, hb = add_scene(engine, sc)
+    _, cnt = engine.contact_step([pair_of(sc, ha, hb)] * npairs, keep_polygons=True)
+    assert (cnt[:, 1] > 0).all()
+    return hb, sc["X_WB"]
+
+
+# one surface of 1 / resolution samples, and 1100 surfaces of 4e6 each: no
+# surface's count passes 32 bits there, the sum 4.4e9 does (and would wrap to
+# 1e8)
+@pytest.mark.parametrize("npairs,resolution", [(1, 1e-10), (1, 1e-17), (1100, 2.5e-7)])
+def test_area_importance_samples_beyond_32_bits(engine, npairs, resolution):
+    print("[case] area importance", npairs, resolution, flush=True)
+    geom, X = _step(engine, npairs)
+    with pytest.raises(HcsError) as e:
+        engine.taxel_sensor(geom, X, TAXELS, 0.004, resolution, "squared", "area_importance")
+    assert e.value.code == HCS_ERR_LIMIT
+    _, m = engine.taxel_sensor(geom, X, TAXELS, 0.004, 0.002, "squared", "area_importance")
+    assert 499 * npairs <= m <= 502 * npairs
