@@ -136,38 +136,20 @@ __global__ void k_ts_fans(const double* __restrict__ poly, const int64_t* __rest
   }
 }
 
-__device__ inline double ts_len(const double* a, const double* b) {
-  const double d[3] = {a[0] - b[0], a[1] - b[1], a[2] - b[2]};
-  return sqrt(dot3(d, d));
-}
-
-/* the reference's loop counts of one triangle */
-__device__ inline void ts_steps(const double* T, double res, int& st, int& st2) {
-  const int st0 = (int)(ts_len(T + 3, T) / res) + 1;
-  const int st1 = (int)(ts_len(T + 6, T) / res) + 1;
-  st2 = (int)(ts_len(T + 6, T) / res) + 1;
-  st = st0 > st1 ? st0 : st1;
-}
-
 __device__ inline void ts_sample(const double* T, double b0, double b1, double b2, double* p, double* e) {
 #pragma unroll
   for (int c = 0; c < 3; ++c) p[c] = (b0 * T[c] + b1 * T[3 + c]) + b2 * T[6 + c];
   *e = (b0 * T[9] + b1 * T[10]) + b2 * T[11];
 }
 
-__global__ void k_ts_count(const double* __restrict__ tris, int64_t nt, double res, unsigned* __restrict__ cnt) {
+__global__ __launch_bounds__(256) void k_ts_count(const double* __restrict__ tris, int64_t nt, double res,
+                                                  unsigned* __restrict__ cnt, TsTotal* __restrict__ total) {
   const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (t > nt) return;
-  if (t == nt) {
-    cnt[t] = 0;
-    return;
-  }
-  int st, st2;
-  ts_steps(tris + HCS_TS_TRI * t, res, st, st2);
-  unsigned na = 0, nb = 0;
-  for (double a = 0; a <= 1; a += 1. / st) ++na;
-  for (double b = 0; b <= 1; b += 1. / st2) ++nb;
-  cnt[t] = na * nb;
+  const unsigned long long n = t < nt ? grid_samples(tris + HCS_TS_TRI * t, res) : 0ull;
+  if (t <= nt) cnt[t] = (unsigned)n;
+  if (n > HCS_TS_MAX) total->too_many = 1;
+  const int64_t sum = wave_sum_i((int64_t)n);
+  if ((threadIdx.x & 63) == 0) atomicAdd(&total->n, (unsigned long long)sum);
 }
 
 __global__ void k_ts_gen(const double* __restrict__ tris, int64_t nt, double res, const unsigned* __restrict__ off,
@@ -176,7 +158,7 @@ __global__ void k_ts_gen(const double* __restrict__ tris, int64_t nt, double res
   if (t >= nt) return;
   const double* T = tris + HCS_TS_TRI * t;
   int st, st2;
-  ts_steps(T, res, st, st2);
+  if (!grid_steps(T, res, st, st2)) return;
   size_t j = off[t];
   for (double a = 0; a <= 1; a += 1. / st)
     for (double b = 0; b <= 1; b += 1. / st2) {
@@ -720,17 +702,12 @@ int hcs_taxel_sensor_update(hcs_ctx* h, const hcs_taxel_sensor* S, double* value
   int* surf0 = nullptr;
   if (ntri > 0 && S->sample_method == 0) {
     hipLaunchKernelGGL(k_ts_count, dim3((ntri + 1 + 255) / 256), dim3(256), 0, s, (const double*)B.tris.ptr,
-                       (int64_t)ntri, S->sample_resolution, (unsigned*)B.scnt.ptr);
+                       (int64_t)ntri, S->sample_resolution, (unsigned*)B.scnt.ptr, (TsTotal*)B.cnt.ptr);
     if ((rc = ensure(c, B.tmp, std::max<size_t>(scan_temp_bytes((long long)ntri + 1), 8)))) return rc;
     if (exclusive_scan_u32(s, (const unsigned*)B.scnt.ptr, (unsigned*)B.soff.ptr, (long long)ntri + 1, B.tmp.ptr,
                            B.tmp.bytes) != 0)
       return set_err(c, HCS_ERR_LIMIT, "sensor: too many triangles to scan");
-    unsigned m32 = 0;
-    rc = hip_check(c, hipMemcpyAsync(&m32, (unsigned*)B.soff.ptr + ntri, sizeof(unsigned), hipMemcpyDeviceToHost, s),
-                   "dl");
-    if (!rc) rc = hip_check(c, hipStreamSynchronize(s), "sync");
-    if (rc) return rc;
-    m = m32;
+    if ((rc = sample_total(c, m))) return rc;
   } else if (ntri > 0) {
     /* areas and prefix sums; per pair the first triangle (in no order), the
      * sample count and its scan; the surfaces */

@@ -22,4 +22,10 @@ int64_t emu_area_chain(double top, double step, double* acc, int64_t cap) {
   return too_many ? -1 : (int64_t)n;
 }
 
+/* The samples of one triangle (9 coordinates, DEFAULT), or -1. */
+int64_t emu_grid_samples(const double* tri, double res) {
+  const unsigned long long n = grid_samples(tri, res);
+  return n > HCS_TS_MAX ? -1 : (int64_t)n;
+}
+
 }  // extern "C"

@@ -23,6 +23,8 @@ def emu(tmp_path_factory):
     lib = C.CDLL(out)
     lib.emu_area_chain.restype = C.c_int64
     lib.emu_area_chain.argtypes = [C.c_double, C.c_double, _D, C.c_int64]
+    lib.emu_grid_samples.restype = C.c_int64
+    lib.emu_grid_samples.argtypes = [_D, C.c_double]
     return lib
 
 
@@ -44,3 +46,32 @@ def test_area_chain_counts_the_sums_below_the_top(emu, top, step):
 @pytest.mark.parametrize("top", [1e-4, 1.0, 3e5])
 def test_area_chain_refuses_more_than_32_bits_count(emu, top, res):
     assert emu.emu_area_chain(top, res * top, None, 0) == -1
+
+
+def _triangle(l01, l02):
+    return np.array([0.1, 0.2, 0.3, 0.1 + l01, 0.2, 0.3, 0.1, 0.2 + l02, 0.3])
+
+
+def _passes(st):
+    n, a = 0, 0.0
+    while a <= 1:
+        n, a = n + 1, a + 1.0 / st
+    return n
+
+
+@pytest.mark.parametrize("l01,l02,res", [(1e-3, 2e-3, 5e-3), (3e-3, 1e-3, 1e-3), (0.02, 0.013, 3.7e-4), (0.3, 1e-4, 1e-3),
+                                         (0.0, 0.0, 1e-3), (0.1, 1e-6, 1e-6)])
+def test_grid_samples_are_the_passes_of_the_loops(emu, l01, l02, res):
+    t = _triangle(l01, l02)
+    n0, n1 = np.linalg.norm(t[3:6] - t[:3]) / res, np.linalg.norm(t[6:9] - t[:3]) / res
+    st2 = int(n1) + 1
+    st = max(int(n0) + 1, st2)
+    assert emu.emu_grid_samples(t.ctypes.data_as(_D), res) == _passes(st) * _passes(st2)
+
+
+# 1e5 x 1e5 passes (a product that wraps 32 bits), steps beyond an int, and
+# edges without an end
+@pytest.mark.parametrize("l01,l02,res", [(0.05, 0.05, 5e-7), (0.05, 0.05, 2e-11), (0.05, 1e-9, 1e-18),
+                                         (1e-9, 0.05, 1e-300), (np.inf, 0.05, 1e-3)])
+def test_grid_samples_refuse_more_than_32_bits_count(emu, l01, l02, res):
+    assert emu.emu_grid_samples(_triangle(l01, l02).ctypes.data_as(_D), res) == -1

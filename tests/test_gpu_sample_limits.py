@@ -33,3 +33,17 @@ def test_area_importance_samples_beyond_32_bits(engine, npairs, resolution):
     assert e.value.code == HCS_ERR_LIMIT
     _, m = engine.taxel_sensor(geom, X, TAXELS, 0.004, 0.002, "squared", "area_importance")
     assert 499 * npairs <= m <= 502 * npairs
+
+
+# one triangle's samples pass 32 bits; its steps pass an int; and 1100 pairs
+# of 1.8e7 samples each, whose sum does (2e10)
+@pytest.mark.parametrize("npairs,resolution", [(1, 2e-7), (1, 1e-12), (1100, 1.5e-5)])
+def test_default_samples_beyond_32_bits(engine, npairs, resolution):
+    print("[case] default", npairs, resolution, flush=True)
+    geom, X = _step(engine, npairs)
+    _, one = engine.taxel_sensor(geom, X, TAXELS, 0.004, 0.002)
+    with pytest.raises(HcsError) as e:
+        engine.taxel_sensor(geom, X, TAXELS, 0.004, resolution)
+    assert e.value.code == HCS_ERR_LIMIT
+    _, m = engine.taxel_sensor(geom, X, TAXELS, 0.004, 0.002)
+    assert m == one > 0
