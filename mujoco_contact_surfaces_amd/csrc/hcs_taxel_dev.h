@@ -284,8 +284,7 @@ __device__ inline double sample_cell(const double* __restrict__ poly, const doub
  * triangle and runs the hit test on the rays of its sample range only; the
  * nearest hit per ray is found with LDS atomics: the least t (its IEEE bits
  * order like t, t > 0), then among hits at that t the least (polygon key,
- * fan index), the tie rule of the ray-major loop above.  The packed key
- * kq * 8 + k needs kq < 2^61, i.e. pair indices below 2^19.
+ * fan index), the tie rule of the ray-major loop above.
  *
  * The first pass also records, per ray, the fan whose atomic lowered t
  * (the owner) and flags a ray when a hit matched the t already there (a
@@ -313,13 +312,25 @@ __device__ inline double sample_cell(const double* __restrict__ poly, const doub
  * 128.) */
 #define HCS_TX_SMALL 64
 static_assert(HCS_TX_RAYS == 24 * 24 && 64 * HCS_TX_SMALL < 65536, "codes of the fan-major sampler");
-/* A taxel's rays (7.5 KB) and each wave's fans (6 KB).  A fan's id: list
- * position * 64 + its vertices k * 8 + k1. */
+/* A fan's id: its polygon's position in the taxel's list * 16 + its vertex k * 2
+ * + whether the next vertex is the first.  In a list of up to HCS_TX_POLYS no id
+ * is HCS_TX_NONE; the callers take the ray-major sampler where a list could be
+ * longer (as many kept polygons are 86 GB). */
+#define HCS_TX_POLYS ((1ll << 28) - 1)
+#define HCS_TX_NONE 0xffffffffu
+__device__ inline unsigned fan_id(unsigned pos, int k, int k1) {
+  return pos << 4 | (unsigned)k << 1 | (k1 == 0 ? 1u : 0u);
+}
+__device__ inline unsigned fan_pos(unsigned id) { return id >> 4; }
+__device__ inline int fan_k(unsigned id) { return (int)(id >> 1 & 7); }
+__device__ inline int fan_k1(unsigned id) { return id & 1 ? 0 : fan_k(id) + 1; }
+
+/* A taxel's rays (7.5 KB) and each wave's fans (6 KB). */
 struct TxHits {
   unsigned long long tmin[HCS_TX_RAYS];
   /* first pass: the fan of the hit that lowered t last; second pass: of the
-   * least (key, fan) among the hits at tmin, -1 before the first */
-  int own[HCS_TX_RAYS];
+   * least (key, fan) among the hits at tmin, HCS_TX_NONE before the first */
+  unsigned own[HCS_TX_RAYS];
   unsigned char flag[HCS_TX_RAYS]; /* the ray needs the second pass */
   int again;
 };
@@ -534,24 +545,25 @@ __device__ inline int round_lane(const TxScatter& L, int t, int shift) {
 }
 
 /* Whether fan a comes before fan b (the least key, then the least fan). */
-__device__ inline bool fan_before(const int64_t* __restrict__ key, const int* __restrict__ list, int a, int b) {
-  const int64_t ka = pkey(key, list[a >> 6]), kb = pkey(key, list[b >> 6]);
-  return ka < kb || (ka == kb && (a >> 3 & 7) < (b >> 3 & 7));
+__device__ inline bool fan_before(const int64_t* __restrict__ key, const int* __restrict__ list, unsigned a,
+                                  unsigned b) {
+  const int64_t ka = pkey(key, list[fan_pos(a)]), kb = pkey(key, list[fan_pos(b)]);
+  return ka < kb || (ka == kb && fan_k(a) < fan_k(b));
 }
 
 /* A hit of ray s at t by fan id: PASS 0 keeps the least t per ray, PASS 1 the
  * least (key, fan) among hits at that t. */
 template <int PASS>
 __device__ inline void keep_hit(TxHits& H, const int64_t* __restrict__ key, const int* __restrict__ list, int s,
-                                double t, int id) {
+                                double t, unsigned id) {
   const unsigned long long tb = (unsigned long long)__double_as_longlong(t);
   if (PASS == 0) {
     const unsigned long long old = atomicMin(&H.tmin[s], tb);
     if (tb < old) H.own[s] = id;
     else if (tb == old) H.flag[s] = 1;
   } else if (tb == H.tmin[s]) {
-    int cur = __atomic_load_n(&H.own[s], __ATOMIC_RELAXED);
-    while ((cur < 0 || fan_before(key, list, id, cur)) &&
+    unsigned cur = __atomic_load_n(&H.own[s], __ATOMIC_RELAXED);
+    while ((cur == HCS_TX_NONE || fan_before(key, list, id, cur)) &&
            !__atomic_compare_exchange_n(&H.own[s], &cur, id, false, __ATOMIC_RELAXED, __ATOMIC_RELAXED)) {
     }
   }
@@ -579,7 +591,7 @@ __device__ inline void scatter_chunk(TxHits& H, TxScatter& L, const double* __re
       TxFan c;
       if (fan_setup(P, k, k1, g, R, c)) {
         const int w = c.j1 - c.j0 + 1, h = c.i1 - c.i0 + 1;
-        L.id[lane] = (unsigned short)(l << 6 | k << 3 | k1);
+        L.id[lane] = (unsigned short)fan_id((unsigned)l, k, k1);
         L.box[lane] = (unsigned short)(c.i0 | c.j0 << 5 | w << 10);
         work = w * h <= HCS_TX_SMALL ? (unsigned)(w * h) : (unsigned)h << 16;
 #pragma unroll
@@ -605,13 +617,14 @@ __device__ inline void scatter_chunk(TxHits& H, TxScatter& L, const double* __re
       const double e1[3] = {L.fan[3][w], L.fan[4][w], L.fan[5][w]};
       const double e2[3] = {L.fan[6][w], L.fan[7][w], L.fan[8][w]};
       const double th = fan_hit(v0, e1, e2, L.fan[9][w], g, R, i, j);
-      if (th > 0.0) keep_hit<PASS>(H, key, list, s, th, (int)(c0 << 6) + L.id[w]);
+      if (th > 0.0) keep_hit<PASS>(H, key, list, s, th, (c0 << 4) + L.id[w]);
     }
     for (int t = lane; t < (int)(tot >> 16); t += 64) {
-      const int w = round_lane(L, t, 16), id = L.id[w];
-      const double* P = poly + (size_t)L.q[id >> 6] * HCS_PREC;
+      const int w = round_lane(L, t, 16);
+      const unsigned id = L.id[w];
+      const double* P = poly + (size_t)L.q[fan_pos(id)] * HCS_PREC;
       TxFan c;
-      if (!fan_setup(P, id >> 3 & 7, id & 7, g, R, c)) continue;
+      if (!fan_setup(P, fan_k(id), fan_k1(id), g, R, c)) continue;
       const int i = c.i0 + t - (int)(L.pre[w] >> 16);
       int ja, jb;
       fan_row(c, g, R, i, ja, jb);
@@ -619,7 +632,7 @@ __device__ inline void scatter_chunk(TxHits& H, TxScatter& L, const double* __re
         const int s = i * g.S + j;
         if (PASS == 1 && !H.flag[s]) continue;
         const double th = fan_hit(c.v0, c.e1, c.e2, c.f, g, R, i, j);
-        if (th > 0.0) keep_hit<PASS>(H, key, list, s, th, (int)(c0 << 6) + id);
+        if (th > 0.0) keep_hit<PASS>(H, key, list, s, th, (c0 << 4) + id);
       }
     }
     wave_sync();
@@ -680,9 +693,9 @@ __device__ inline double sample_cell_scatter(const double* __restrict__ poly, co
   if (g.window == 1) rsigma_squared = 0.5 / (g.sigma * g.sigma);
   if (g.window == 2) rtukey = 1. / g.sigma * S * S;
   const double PI = 3.14159265358979323846;
-  auto value = [&](int s, int id, double& t) {
-    const int i = s / S, j = s % S, q = one_chunk ? L.q[id >> 6] : list[id >> 6];
-    const double raw = fan_pressure(poly + (size_t)q * HCS_PREC, id >> 3 & 7, id & 7, g, R, i, j, t) * rmean;
+  auto value = [&](int s, unsigned id, double& t) {
+    const int i = s / S, j = s % S, q = one_chunk ? L.q[fan_pos(id)] : list[fan_pos(id)];
+    const double raw = fan_pressure(poly + (size_t)q * HCS_PREC, fan_k(id), fan_k1(id), g, R, i, j, t) * rmean;
     double weight = 1.0;
     if (g.window == 1) {
       const double dist = hypot(di_factor * i + sub_halfwidth, di_factor * j + sub_halfwidth) / max_dist;
@@ -708,7 +721,7 @@ __device__ inline double sample_cell_scatter(const double* __restrict__ poly, co
       if (!(t < 1.5 * g.zs)) w = 0.0;
     }
     if (settled) H.tmin[s] = (unsigned long long)__double_as_longlong(w);
-    else H.flag[s] = 1, H.own[s] = -1, H.again = 1;
+    else H.flag[s] = 1, H.own[s] = HCS_TX_NONE, H.again = 1;
   }
   __syncthreads();
   if (H.again) {
@@ -721,7 +734,7 @@ __device__ inline double sample_cell_scatter(const double* __restrict__ poly, co
     for (int s = tid; s < nr; s += 64 * W)
       if (H.flag[s]) {
         double t, w = 0.0;
-        if (__longlong_as_double((long long)H.tmin[s]) < 1.5 * g.zs && H.own[s] >= 0) w = value(s, H.own[s], t);
+        if (__longlong_as_double((long long)H.tmin[s]) < 1.5 * g.zs && H.own[s] != HCS_TX_NONE) w = value(s, H.own[s], t);
         H.tmin[s] = (unsigned long long)__double_as_longlong(w);
       }
     __syncthreads();

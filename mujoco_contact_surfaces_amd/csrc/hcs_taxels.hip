@@ -21,7 +21,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <climits>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -132,7 +131,8 @@ __global__ __launch_bounds__(64) void k_tx_sample(const double* __restrict__ pol
   if (threadIdx.x == 0) out[x + g.cx * y] = v;
 }
 
-/* The same, fan-major (double, S^2 <= HCS_TX_RAYS), W waves per taxel. */
+/* The same, fan-major (double, S^2 <= HCS_TX_RAYS, np <= HCS_TX_POLYS), W
+ * waves per taxel. */
 template <int W>
 __global__ __launch_bounds__(64 * W) void k_tx_sample_fan(const double* __restrict__ poly, const int64_t* __restrict__ key,
                                                       TaxelGridDev g, const unsigned* __restrict__ off,
@@ -203,7 +203,7 @@ int run_taxels(Ctx* c, const TaxelGridDev& g, const std::vector<unsigned char>& 
     if (ptan) {
       hipLaunchKernelGGL(HIP_KERNEL_NAME(k_tx_sample<Dual>), dim3(ncell), dim3(64), 0, c->stream, poly, ptan, key, g,
                          Xd, (const unsigned*)off, (const int*)list, list_cap, d_out);
-    } else if (g.S * g.S <= HCS_TX_RAYS && c->last_pairs.size() < (1u << 19)) {
+    } else if (g.S * g.S <= HCS_TX_RAYS && np <= HCS_TX_POLYS) {
       /* up to eight taxels a CU, four waves share a taxel: 256 taxels 52 -> 22
        * us, 1600 taxels 21 -> 14 us; with 3600 taxels 14 -> 16 us */
       auto run = [&](auto kernel, int waves) {
@@ -341,7 +341,8 @@ __global__ __launch_bounds__(HCS_TXB_LIVE) void k_txb_live(const unsigned* __res
 }
 
 /* One wave per live taxel of any sensor, strided over the grid; FAN: the
- * fan-major sampler (every sensor has S^2 <= HCS_TX_RAYS). */
+ * fan-major sampler (every sensor has S^2 <= HCS_TX_RAYS, and there is room for
+ * at most HCS_TX_POLYS polygons). */
 template <bool FAN>
 __global__ __launch_bounds__(64) void k_txb_sample(const double* __restrict__ poly, const int64_t* __restrict__ key,
                                                    const TaxelGridDev* __restrict__ grids,
@@ -422,8 +423,6 @@ int batch_taxels_setup(Ctx* c, BatchTaxels& t, int npairs, const int32_t* geoms,
   t.n = n, t.ncell = ncell;
   t.max_rays = 0;
   for (int k = 0; k < n; ++k) t.max_rays = std::max(t.max_rays, g[k].S * g[k].S);
-  /* the fan-major sampler packs pair indices into 19 bits */
-  if (npairs >= (1 << 19)) t.max_rays = INT_MAX;
   t.bin_grid = std::max(1, c->num_cu * 4);
   return hip_check(c, hipStreamSynchronize(c->stream), "sync");
 }
@@ -464,7 +463,7 @@ void batch_taxels_enqueue(Ctx* c, BatchTaxels& t, const double* state) {
                      (const unsigned*)t.cnt.ptr,
                      (const unsigned*)t.off.ptr, t.ncell, t.list_cap, (int*)t.live.ptr, nlive, (double*)t.out.ptr);
   const dim3 grid(std::max(1, std::min(t.ncell, c->num_cu * 16)));
-  if (t.max_rays <= HCS_TX_RAYS)
+  if (t.max_rays <= HCS_TX_RAYS && t.poly_cap <= HCS_TX_POLYS)
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_txb_sample<true>), grid, dim3(64), 0, s, (const double*)t.poly_rec.ptr,
                        (const int64_t*)t.poly_key.ptr, (const TaxelGridDev*)g, (const int*)t.cell_base.ptr,
                        (const int*)t.cell_sensor.ptr, (const unsigned*)t.off.ptr, (const unsigned*)t.cnt.ptr,

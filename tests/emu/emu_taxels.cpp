@@ -62,4 +62,11 @@ int emu_taxels(const double* polys, int64_t np, const int64_t* keys, const doubl
   return 0;
 }
 
+/* The id of fan (k, k1) of list entry pos, and what is read back from it. */
+unsigned emu_fan_id(unsigned pos, int k, int k1, unsigned* back) {
+  const unsigned id = fan_id(pos, k, k1);
+  back[0] = fan_pos(id), back[1] = (unsigned)fan_k(id), back[2] = (unsigned)fan_k1(id);
+  return id;
+}
+
 }  // extern "C"

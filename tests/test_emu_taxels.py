@@ -91,3 +91,19 @@ def test_fan_major_sampler_equals_ray_major_and_oracle(emu, case, window, sigma)
     assert np.abs(ref).max() > 0
     np.testing.assert_array_equal(b, a)
     np.testing.assert_allclose(b, ref, rtol=1e-10, atol=1e-10 * np.abs(ref).max())
+
+
+# list positions up to the longest list the fan-major sampler is given: the
+# first, the last, and where an id passes 31 bits
+@pytest.mark.parametrize("pos", [0, 1, 2 ** 25 - 1, 2 ** 25, 2 ** 27, 2 ** 28 - 2])
+def test_fan_ids_hold_every_list_position(emu, pos):
+    emu.emu_fan_id.restype = C.c_uint32
+    emu.emu_fan_id.argtypes = [C.c_uint32, C.c_int, C.c_int, C.POINTER(C.c_uint32)]
+    ids = set()
+    for nv in range(3, 9):
+        for k in range(nv):
+            k1 = (k + 1) % nv
+            back = (C.c_uint32 * 3)()
+            ids.add((emu.emu_fan_id(pos, k, k1, back), k, k1))
+            assert tuple(back) == (pos, k, k1)
+    assert len({i for i, _, _ in ids}) == len(ids) and 0xffffffff not in {i for i, _, _ in ids}
