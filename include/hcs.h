@@ -252,7 +252,11 @@ int hcs_batch_get(hcs_batch* batch, hcs_pair_out* out);
 /* Autotuner: times the launch shapes on the current state, keeps the best.
  * Re-planning (here and in hcs_batch_set_config) measures one step on the
  * current state and splits heavy work items over subtrees; results never
- * depend on the plan beyond the order of floating-point sums. */
+ * depend on the plan beyond the order of floating-point sums.  Without a state
+ * there is nothing to measure: a configuration set before the first
+ * hcs_batch_set_state is planned in that call.  A batch that was never tuned
+ * or configured is not measured at all: each step culls and splits its items
+ * on the device. */
 int hcs_batch_tune(hcs_batch* batch, int32_t reps, double* best_ms);
 /* Launch configuration: cfg = [persistent blocks per CU, queries per lane
  * (must be 1: larger values are rejected), largest rigid mesh handled in

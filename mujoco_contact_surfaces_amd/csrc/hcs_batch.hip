@@ -43,7 +43,7 @@ struct hcs_batch {
   bool shape_set = false; /* hcs_batch_set_config or hcs_batch_tune chose the shape */
   bool whole = false;     /* plan whole items without a measurement (item statistics) */
   DBuf envs, state, items;
-  /* Until a step can be measured (a shape set or tuned with a state), the
+  /* Until a shape was set or tuned and a state is there to measure it with, the
    * items are enumerated, culled and split on the device in every step, as in
    * a per-call step: an unmeasured plan has no way to tell the heavy items. */
   bool implicit = false;
@@ -282,11 +282,11 @@ static int batch_split(hcs_batch* b) {
   return HCS_OK;
 }
 
-/* (Re)builds the plan for the current shape and uploads it; with a state
- * set, heavy items are split and all items ordered by measured steps. */
+/* (Re)builds the plan for the current shape and uploads it; with a shape and a
+ * state set, heavy items are split and all items ordered by measured steps. */
 static int batch_plan(hcs_batch* b) {
   batch_free_graph(b);
-  b->implicit = !b->has_state && !b->whole;
+  b->implicit = !(b->shape_set && b->has_state) && !b->whole;
   int rc = build_plan(b->c, b->npairs, b->geoms.data(), &b->opts, b->tet_max, b->plan,
                       b->implicit ? ITEMS_IMPLICIT : ITEMS_WHOLE);
   b->plan.order.clear();
@@ -297,8 +297,8 @@ static int batch_plan(hcs_batch* b) {
                                [](const EnvDesc& E) { return E.kind == KIND_TRI || E.kind == KIND_SOFT; });
   if (b->implicit) return rc ? rc : batch_upload_implicit(b);
   if (!rc) rc = batch_upload(b);
-  if (!rc && b->has_state) rc = batch_split(b);
-  if (!rc && b->has_state) rc = batch_order(b);
+  if (!rc && !b->whole) rc = batch_split(b);
+  if (!rc && !b->whole) rc = batch_order(b);
   return rc;
 }
 
@@ -415,7 +415,11 @@ int hcs_batch_set_state(hcs_batch* b, const double* state) {
                      "upload state");
   if (rc) return rc;
   b->has_state = true;
-  return hip_check(c, hipStreamSynchronize(c->stream), "sync");
+  if ((rc = hip_check(c, hipStreamSynchronize(c->stream), "sync"))) return rc;
+  if (!b->shape_set || !b->implicit) return HCS_OK;
+  /* a shape set before there was a state: measured now */
+  rc = batch_plan(b);
+  return rc ? rc : batch_capture(b);
 }
 
 int hcs_batch_step(hcs_batch* b) {
