@@ -280,7 +280,10 @@ int hcs_batch_kernel_times(hcs_batch* batch, int32_t reps, double* ms);
  * production steps, candidates, cheap-test survivors, n elements of B,
  * wall-clock start, wall-clock end (constant-rate device counter; 0 for
  * items culled in that step)]; *nitems = number of items (capacity 0
- * queries it). */
+ * queries it).  A batch that is not planned yet (never configured, or without
+ * a state) has no items of its own between steps: the profile is then of a step
+ * over whole items (64 queries against the whole of A), beside the batch's own
+ * step. */
 int hcs_batch_item_stats(hcs_batch* batch, int64_t* out, int64_t capacity, int64_t* nitems);
 /* Work-unit counts of the last step: [candidates, polygons, faces]. */
 int hcs_batch_counts(hcs_batch* batch, int64_t* counts);

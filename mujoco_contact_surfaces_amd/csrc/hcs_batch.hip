@@ -597,20 +597,25 @@ int hcs_batch_item_stats(hcs_batch* b, int64_t* out, int64_t capacity, int64_t* 
   if (!b || !nitems || capacity < 0 || (capacity > 0 && !out)) return HCS_ERR_ARG;
   Ctx* c = b->c;
   if (b->implicit) {
-    /* per item of a plan of whole items: a batch of its own for the call */
+    if (capacity == 0) {
+      Plan whole;
+      const int rc = build_plan(c, b->npairs, b->geoms.data(), &b->opts, b->tet_max, whole);
+      if (!rc) *nitems = (int64_t)whole.items.size();
+      return rc;
+    }
+    /* per item of a plan of whole items: a batch of its own for the call; and
+     * the step that the profile of a planned batch runs */
     hcs_batch* w = nullptr;
     int rc = batch_create(c, b->npairs, b->geoms.data(), &b->opts, b->tet_max, true, &w);
     if (!rc)
       rc = hip_check(c, hipMemcpyAsync(w->state.ptr, b->state.ptr, sizeof(double) * HCS_STATE * b->npairs,
                                        hipMemcpyDeviceToDevice, c->stream), "copy state");
-    if (!rc && capacity > 0) {
-      rc = hcs_batch_step(w);
-      std::vector<hcs_pair_out> o(b->npairs);
-      if (!rc) rc = hcs_batch_get(w, o.data());
-    }
+    if (!rc) rc = hcs_batch_step(w);
+    std::vector<hcs_pair_out> o(b->npairs);
+    if (!rc) rc = hcs_batch_get(w, o.data());
     if (!rc) rc = hcs_batch_item_stats(w, out, capacity, nitems);
     if (w) hcs_batch_destroy(w);
-    return rc;
+    return rc ? rc : hcs_batch_step(b);
   }
   const int n = (int)b->plan.items.size();
   *nitems = n;

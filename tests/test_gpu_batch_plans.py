@@ -64,3 +64,26 @@ def test_unconfigured_batch_after_a_mesh_is_replaced(engine):
     np.testing.assert_array_equal(got[0][1], got[1][1])
     assert len(got[0][2]) == len(got[1][2]) and got[0][1][0, 1] > 0
     b.close(), fresh.close()
+
+
+def test_item_profile_runs_the_step(engine):
+    """The profile of a batch that is not planned steps the batch, as that of a
+    planned one does."""
+    pairs = _pairs(engine)
+    moved = _state(pairs)
+    moved[:, 23] -= 0.0005
+    b, ref = engine.batch([p[:2] for p in pairs]), engine.batch([p[:2] for p in pairs])
+    b.set_state(_state(pairs))
+    b.step()
+    b.get()
+    ref.set_state(moved)
+    ref.step()
+    b.set_state(moved)
+    st = b.item_stats()
+    W, cnt = b.get()
+    Wr, cr = ref.get()
+    np.testing.assert_array_equal(cnt, cr)
+    np.testing.assert_array_equal(W, Wr)
+    for k in range(len(pairs)):
+        assert st[st[:, 0] == k, 5].sum() == cnt[k, 0]
+    b.close(), ref.close()
