@@ -1,5 +1,6 @@
 /*
- * hcs_samples.h -- sample counts of the taxel sensor's samplers.
+ * hcs_samples.h -- sample counts of the taxel sensor's samplers, and the ray
+ * cull of the curved sensor.
  */
 #pragma once
 #include "hcs_device.h"
@@ -66,6 +67,40 @@ __device__ inline unsigned area_chain(double top, double step, bool& too_many, F
     each(n, acc);
   }
   return n;
+}
+
+/* Whether a ray's line can be accepted by the hit test of a triangle: not when
+ * it misses the triangle's bounding sphere (centre C, radius r), widened.  The
+ * computed barycentrics err by at most 16 eps |D| (|s| + L) L^2 / |det| in
+ * position, s the vector from the triangle to the ray's origin, D its
+ * direction, L <= 2r the longest edge, and the hit test rejects |det| < 1e-10,
+ * so an accepted hit lies within 3.6e-5 |D| (|s| + L) L^2 of the triangle; the
+ * sphere is widened by more than four times that (|s| bounded through the
+ * largest coordinates, |D| by dmax >= 1), by 1e-9 of the ray's largest
+ * coordinate, and the comparison by 1e-14 |s|^2 for the cancellation in
+ * |s|^2 - (s.D)^2 / |D|^2.  A NaN or infinity fails the comparison, so nothing
+ * is skipped on it. */
+#define HCS_SPHERE 5 /* C, r with its part of the widening, factor of the ray's part */
+__device__ inline void fan_sphere(const double* T, double dmax, double* b) {
+  double C[3], tm = 0.0, r2 = 0.0;
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+    C[c] = ((T[c] + T[3 + c]) + T[6 + c]) * (1.0 / 3.0),
+    tm = fmax(tm, fmax(fabs(T[c]), fmax(fabs(T[3 + c]), fabs(T[6 + c]))));
+#pragma unroll
+  for (int v = 0; v < 3; ++v) {
+    const double d[3] = {T[3 * v] - C[0], T[3 * v + 1] - C[1], T[3 * v + 2] - C[2]};
+    r2 = fmax(r2, dot3(d, d));
+  }
+  const double r = sqrt(r2), k = 1.2e-3 * r2 * dmax;
+  b[0] = C[0], b[1] = C[1], b[2] = C[2], b[3] = r + k * (tm + r), b[4] = k;
+}
+/* sc: the ray's largest coordinate, sl = 1e-9 sc + 1e-300, iD2 = 1 / |D|^2 */
+__device__ inline bool line_misses(const double* b, const double* O, const double* D, double iD2, double sc,
+                                   double sl) {
+  const double s[3] = {b[0] - O[0], b[1] - O[1], b[2] - O[2]};
+  const double ss = dot3(s, s), sd = dot3(s, D), re = (b[3] + b[4] * sc) + sl;
+  return ss - (sd * sd) * iD2 > re * re + 1e-14 * ss;
 }
 
 }  // namespace hcs

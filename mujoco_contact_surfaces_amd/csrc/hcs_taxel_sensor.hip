@@ -424,15 +424,9 @@ struct CsHit {
  * (S/src/bvh.cpp:49-74) in FP64 over the fan triangles, nearest t (first
  * triangle in order on ties).
  *
- * Triangles whose bounding sphere (centre C, radius r) the ray's line misses
- * are skipped.  The computed barycentrics err by at most
- * 16 eps (|s| + L) L^2 / |det| in position, s the vector from the triangle to
- * the ray's origin, L <= 2r the longest edge, and the hit test rejects
- * |det| < 1e-10, so an accepted hit lies within 3.6e-5 (|s| + L) L^2 of the
- * triangle; the sphere is widened by more than four times that (|s| bounded
- * through the largest coordinates), by 1e-9 of the ray's largest coordinate,
- * and the comparison by 1e-14 |s|^2 for the cancellation in |s|^2 - (s.D)^2.
- * A NaN or infinity fails the comparison, so nothing is skipped on it.
+ * Triangles that the ray's line misses by more than the rounding of the hit
+ * test are skipped (line_misses); the spheres are widened for the longest of
+ * the wave's directions.
  *
  * One lane per ray, one wave per (64 rays, slice of the triangles): with a
  * thread walking every triangle, 2601 rays were 41 waves on 256 CUs, each a
@@ -447,46 +441,27 @@ struct CsHit {
 __global__ __launch_bounds__(64) void k_cs_rays(const double* __restrict__ tris, int64_t nt, CsArgs a,
                                                 const double* __restrict__ pts, const double* __restrict__ nrms, int m,
                                                 CsHit* __restrict__ part) {
-  __shared__ double sph[64][6];
+  __shared__ double sph[64][6]; /* (HCS_SPHERE, padded) */
   const int lane = threadIdx.x, j = blockIdx.x * 64 + lane, jr = j < m ? j : m - 1;
   double pw[3], nw[3], O[3], D[3], sc = 0.0;
   xform(a.X, pts + 3 * (size_t)jr, pw);
   rot(a.X, nrms + 3 * (size_t)jr, nw);
 #pragma unroll
   for (int c = 0; c < 3; ++c) O[c] = pw[c] + nw[c] * 1e-8, D[c] = -nw[c], sc = fmax(sc, fabs(O[c]));
-  const double iD2 = 1.0 / dot3(D, D), sl = 1e-9 * sc + 1e-300;
+  const double D2 = dot3(D, D), iD2 = 1.0 / D2, sl = 1e-9 * sc + 1e-300;
+  const double dmax = wave_max(fmax(1.0, sqrt(D2)));
   double best = 1e30, bu = 0.0, bv = 0.0;
   int64_t bt = -1;
   const int64_t t0 = nt * blockIdx.y / gridDim.y, t1 = nt * (blockIdx.y + 1) / gridDim.y;
   for (int64_t c0 = t0; c0 < t1; c0 += 64) {
     const int cn = (int)(t1 - c0 < 64 ? t1 - c0 : 64);
     __syncthreads();
-    if (lane < cn) {
-      const double* T = tris + HCS_TS_TRI * (c0 + lane);
-      double C[3], tm = 0.0, r2 = 0.0;
-#pragma unroll
-      for (int c = 0; c < 3; ++c)
-        C[c] = ((T[c] + T[3 + c]) + T[6 + c]) * (1.0 / 3.0),
-        tm = fmax(tm, fmax(fabs(T[c]), fmax(fabs(T[3 + c]), fabs(T[6 + c]))));
-#pragma unroll
-      for (int v = 0; v < 3; ++v) {
-        const double d[3] = {T[3 * v] - C[0], T[3 * v + 1] - C[1], T[3 * v + 2] - C[2]};
-        r2 = fmax(r2, dot3(d, d));
-      }
-      const double r = sqrt(r2), k = 1.2e-3 * r2;
-      sph[lane][0] = C[0], sph[lane][1] = C[1], sph[lane][2] = C[2];
-      sph[lane][3] = r + k * (tm + r), sph[lane][4] = k;
-    }
+    if (lane < cn) fan_sphere(tris + HCS_TS_TRI * (c0 + lane), dmax, sph[lane]);
     __syncthreads();
     /* the lane's triangles of the tile, then their hit tests in order */
     unsigned long long todo = 0;
 #pragma unroll 8
-    for (int k = 0; k < 64; ++k) {
-      const double* b = sph[k];
-      const double s[3] = {b[0] - O[0], b[1] - O[1], b[2] - O[2]};
-      const double ss = dot3(s, s), sd = dot3(s, D), re = (b[3] + b[4] * sc) + sl;
-      todo |= ss - (sd * sd) * iD2 > re * re + 1e-14 * ss ? 0ull : 1ull << k;
-    }
+    for (int k = 0; k < 64; ++k) todo |= line_misses(sph[k], O, D, iD2, sc, sl) ? 0ull : 1ull << k;
     todo &= ~0ull >> (64 - cn);
     while (todo) {
       const int64_t t = c0 + __builtin_ctzll(todo);

@@ -1,5 +1,5 @@
-// CPU build of the taxel sensor's sample counts (hcs_samples.h), test
-// infrastructure only.
+// CPU build of the taxel sensor's sample counts and the curved sensor's ray
+// cull (hcs_samples.h), test infrastructure only.
 #include <hip/hip_runtime.h>
 
 #include "hcs_samples.h"
@@ -26,6 +26,19 @@ int64_t emu_area_chain(double top, double step, double* acc, int64_t cap) {
 int64_t emu_grid_samples(const double* tri, double res) {
   const unsigned long long n = grid_samples(tri, res);
   return n > HCS_TS_MAX ? -1 : (int64_t)n;
+}
+
+/* skip[i]: the line of ray i (origin O, direction D) is skipped for triangle
+ * i. */
+void emu_lines_miss(const double* T, const double* O, const double* D, int64_t n, unsigned char* skip) {
+  for (int64_t i = 0; i < n; ++i) {
+    const double *o = O + 3 * i, *d = D + 3 * i;
+    double b[HCS_SPHERE], sc = 0.0;
+    for (int c = 0; c < 3; ++c) sc = fmax(sc, fabs(o[c]));
+    const double D2 = dot3(d, d);
+    fan_sphere(T + 9 * i, fmax(1.0, sqrt(D2)), b);
+    skip[i] = line_misses(b, o, d, 1.0 / D2, sc, 1e-9 * sc + 1e-300);
+  }
 }
 
 }  // extern "C"
