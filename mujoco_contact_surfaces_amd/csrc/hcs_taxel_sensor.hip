@@ -121,8 +121,9 @@ __global__ void k_ts_nfan(const double* __restrict__ poly, const int64_t* __rest
 
 __global__ void k_ts_fans(const double* __restrict__ poly, const int64_t* __restrict__ key,
                           const int* __restrict__ order, int n, const unsigned* __restrict__ off,
-                          double* __restrict__ tris, int* __restrict__ surf) {
+                          double* __restrict__ tris, int* __restrict__ surf, unsigned* __restrict__ cnt_end) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0) *cnt_end = 0; /* (of k_ts_count) */
   if (i >= n || off[i] == off[i + 1]) return;
   const double* P = poly + HCS_PREC * (size_t)order[i];
   const int nv = (int)P[0];
@@ -142,11 +143,23 @@ __device__ inline void ts_sample(const double* T, double b0, double b1, double b
   *e = (b0 * T[9] + b1 * T[10]) + b2 * T[11];
 }
 
-__global__ __launch_bounds__(256) void k_ts_count(const double* __restrict__ tris, int64_t nt, double res,
-                                                  unsigned* __restrict__ cnt, TsTotal* __restrict__ total) {
+/* Samples per triangle.  Their sum is at most HCS_TS_MAX when each is at most
+ * an nt-th of it; one that is more raises cnt[nt] (cleared before), and the sum
+ * is then made in 64 bits (k_ts_sum).  (Summing in 64 bits every time, one
+ * atomic per wave, took 7.1 us for 3.5.) */
+__global__ void k_ts_count(const double* __restrict__ tris, int64_t nt, double res, unsigned long long each,
+                           unsigned* __restrict__ cnt) {
+  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (t >= nt) return;
+  const unsigned long long n = grid_samples(tris + HCS_TS_TRI * t, res);
+  cnt[t] = (unsigned)n;
+  if (n > each) cnt[nt] = 1;
+}
+
+__global__ __launch_bounds__(256) void k_ts_sum(const double* __restrict__ tris, int64_t nt, double res,
+                                                TsTotal* __restrict__ total) {
   const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   const unsigned long long n = t < nt ? grid_samples(tris + HCS_TS_TRI * t, res) : 0ull;
-  if (t <= nt) cnt[t] = (unsigned)n;
   if (n > HCS_TS_MAX) total->too_many = 1;
   const int64_t sum = wave_sum_i((int64_t)n);
   if ((threadIdx.x & 63) == 0) atomicAdd(&total->n, (unsigned long long)sum);
@@ -637,12 +650,13 @@ static int sensor_fans(Ctx* c, int32_t geom, unsigned& ntri) {
   }
   const size_t nt1 = std::max<size_t>(1, ntri);
   if ((rc = ensure(c, B.tris, sizeof(double) * HCS_TS_TRI * nt1)) || (rc = ensure(c, B.surf, sizeof(int) * nt1)) ||
-      (rc = ensure(c, B.scnt, sizeof(unsigned) * (nt1 + 1))) || (rc = ensure(c, B.soff, sizeof(unsigned) * (nt1 + 1))))
+      (rc = ensure(c, B.scnt, sizeof(unsigned) * (nt1 + 2))) || (rc = ensure(c, B.soff, sizeof(unsigned) * (nt1 + 2))))
     return rc;
   if (ntri > 0)
     hipLaunchKernelGGL(k_ts_fans, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, s,
                        (const double*)c->d_poly_rec.ptr, (const int64_t*)c->d_poly_key.ptr, order, (int)np,
-                       (const unsigned*)B.fan_off.ptr, (double*)B.tris.ptr, (int*)B.surf.ptr);
+                       (const unsigned*)B.fan_off.ptr, (double*)B.tris.ptr, (int*)B.surf.ptr,
+                       (unsigned*)B.scnt.ptr + ntri);
   return hip_check(c, hipGetLastError(), "sensor triangles");
 }
 
@@ -676,13 +690,25 @@ int hcs_taxel_sensor_update(hcs_ctx* h, const hcs_taxel_sensor* S, double* value
   unsigned *nsurf = nullptr, *soff = nullptr;
   int* surf0 = nullptr;
   if (ntri > 0 && S->sample_method == 0) {
-    hipLaunchKernelGGL(k_ts_count, dim3((ntri + 1 + 255) / 256), dim3(256), 0, s, (const double*)B.tris.ptr,
-                       (int64_t)ntri, S->sample_resolution, (unsigned*)B.scnt.ptr, (TsTotal*)B.cnt.ptr);
-    if ((rc = ensure(c, B.tmp, std::max<size_t>(scan_temp_bytes((long long)ntri + 1), 8)))) return rc;
-    if (exclusive_scan_u32(s, (const unsigned*)B.scnt.ptr, (unsigned*)B.soff.ptr, (long long)ntri + 1, B.tmp.ptr,
+    const dim3 g((ntri + 255) / 256);
+    const unsigned* soff32 = (const unsigned*)B.soff.ptr;
+    hipLaunchKernelGGL(k_ts_count, g, dim3(256), 0, s, (const double*)B.tris.ptr, (int64_t)ntri, S->sample_resolution,
+                       HCS_TS_MAX / ntri, (unsigned*)B.scnt.ptr);
+    if ((rc = ensure(c, B.tmp, std::max<size_t>(scan_temp_bytes((long long)ntri + 2), 8)))) return rc;
+    /* offsets, their end, and the end plus cnt[ntri] */
+    if (exclusive_scan_u32(s, (const unsigned*)B.scnt.ptr, (unsigned*)B.soff.ptr, (long long)ntri + 2, B.tmp.ptr,
                            B.tmp.bytes) != 0)
       return set_err(c, HCS_ERR_LIMIT, "sensor: too many triangles to scan");
-    if ((rc = sample_total(c, m))) return rc;
+    unsigned end[2] = {0, 0};
+    rc = hip_check(c, hipMemcpyAsync(end, soff32 + ntri, sizeof end, hipMemcpyDeviceToHost, s), "dl");
+    if (!rc) rc = hip_check(c, hipStreamSynchronize(s), "sync");
+    if (rc) return rc;
+    m = end[0];
+    if (end[1] != end[0]) {
+      hipLaunchKernelGGL(k_ts_sum, g, dim3(256), 0, s, (const double*)B.tris.ptr, (int64_t)ntri, S->sample_resolution,
+                         (TsTotal*)B.cnt.ptr);
+      if ((rc = sample_total(c, m))) return rc;
+    }
   } else if (ntri > 0) {
     /* areas and prefix sums; per pair the first triangle (in no order), the
      * sample count and its scan; the surfaces */
