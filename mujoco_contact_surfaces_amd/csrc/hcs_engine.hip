@@ -1520,7 +1520,7 @@ int hcs_destroy(hcs_ctx* h) {
   pipe_free(c->pipe);
   for (DBuf* b : {&c->d_envs, &c->d_state, &c->d_items, &c->d_face_rec, &c->d_face_key, &c->d_face_cnt, &c->d_poly_rec, &c->d_poly_key, &c->d_poly_cnt,
                   &c->d_cand, &c->d_cand_cnt, &c->d_tx_cnt, &c->d_tx_off, &c->d_tx_foot, &c->d_tx_list, &c->d_tx_out,
-                  &c->d_tx_grid, &c->d_build})
+                  &c->d_tx_grid, &c->d_tx_total, &c->d_build})
     if (b->ptr) (void)hipFree(b->ptr);
   TaxelSensorBufs& T = c->ts;
   for (DBuf* b : {&T.mask, &T.k64, &T.kp, &T.idx, &T.cnt, &T.nfan, &T.fan_off, &T.tmp, &T.tris, &T.surf, &T.scnt, &T.soff,

@@ -108,7 +108,7 @@ struct Ctx {
   DBuf d_face_rec, d_face_key, d_face_cnt;
   DBuf d_poly_rec, d_poly_key, d_poly_cnt;
   DBuf d_cand, d_cand_cnt;
-  DBuf d_tx_cnt, d_tx_off, d_tx_foot, d_tx_list, d_tx_out, d_tx_grid;
+  DBuf d_tx_cnt, d_tx_off, d_tx_foot, d_tx_list, d_tx_out, d_tx_grid, d_tx_total;
   TaxelSensorBufs ts;
   DBuf d_build; /* scratch of the LBVH build */
   /* memory of the last replaced mesh, for the next one */
@@ -241,6 +241,7 @@ struct BatchTaxels {
   size_t scan_bytes = 0;
   int bin_grid = 1;
   int max_rays = 0; /* the largest S^2 of the sensors */
+  int64_t pair_cells = 1; /* the most taxels of one pair's sensors */
 };
 int batch_taxels_setup(Ctx* c, BatchTaxels& t, int npairs, const int32_t* geoms, int n, const int32_t* pair,
                        const hcs_taxel_grid* grids);

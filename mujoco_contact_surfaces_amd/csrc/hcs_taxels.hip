@@ -28,6 +28,7 @@
 #include "hcs_device.h"
 #include "hcs_internal.h"
 #include "hcs_prim.h"
+#include "hcs_query.h"
 #include "hcs_taxel_dev.h"
 
 #pragma clang fp contract(off)
@@ -111,6 +112,36 @@ __global__ __launch_bounds__(64) void k_tx_bin(const double* __restrict__ poly, 
   bin_polygon<FILL>((int)q, f, g.cx, 0, cnt, off, list, list_cap);
 }
 
+/* Entries of all lists, in 64 bits: their offsets are 32-bit, and a sum beyond
+ * that is refused.  Only made where the number of polygons and taxels does not
+ * exclude it. */
+__device__ inline void add_entries(const int4& f, bool on, unsigned long long* __restrict__ total) {
+  const int64_t n = on && f.x <= f.y && f.z <= f.w ? (int64_t)(f.y - f.x + 1) * (f.w - f.z + 1) : 0;
+  const int64_t sum = wave_sum_i(n);
+  if ((threadIdx.x & 63) == 0 && sum > 0) atomicAdd(total, (unsigned long long)sum);
+}
+__global__ __launch_bounds__(64) void k_tx_total(const int4* __restrict__ foot, int64_t np,
+                                                 unsigned long long* __restrict__ total) {
+  const int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  add_entries(q < np ? foot[q] : make_int4(0, -1, 0, -1), q < np, total);
+}
+constexpr unsigned long long kMaxEntries = 0xffffffffull;
+/* The sum of a k_tx_total / k_txb_total launch made by enqueue(total). */
+template <class F>
+static int check_entries(Ctx* c, F enqueue) {
+  int rc = ensure(c, c->d_tx_total, 8);
+  if (rc) return rc;
+  unsigned long long* total = (unsigned long long*)c->d_tx_total.ptr;
+  launch_fill_u32(c->stream, (unsigned*)total, 0u, 2);
+  enqueue(total);
+  unsigned long long n = 0;
+  rc = hip_check(c, hipMemcpyAsync(&n, total, 8, hipMemcpyDeviceToHost, c->stream), "dl");
+  if (!rc) rc = hip_check(c, hipStreamSynchronize(c->stream), "sync");
+  if (rc) return rc;
+  if (n > kMaxEntries) return set_err(c, HCS_ERR_CAPACITY, "taxel polygon lists exceed 2^32 entries");
+  return HCS_OK;
+}
+
 /* A taxel's list: off[cell] .. off[cell + 1], or none of it when it does not
  * fit the list buffer (the caller sees the total and runs again). */
 __device__ inline unsigned tx_count(const unsigned* __restrict__ off, int cell, int64_t list_cap) {
@@ -191,6 +222,12 @@ int run_taxels(Ctx* c, const TaxelGridDev& g, const std::vector<unsigned char>& 
   if (np > 0)
     hipLaunchKernelGGL(k_tx_bin<0>, nb, dim3(64), 0, c->stream, poly, key, np, pairs, g, (int4*)c->d_tx_foot.ptr, cnt,
                        (const unsigned*)nullptr, (int*)nullptr, (int64_t)0);
+  if ((unsigned long long)np > kMaxEntries / (unsigned)ncell) {
+    rc = check_entries(c, [&](unsigned long long* t) {
+      hipLaunchKernelGGL(k_tx_total, nb, dim3(64), 0, c->stream, (const int4*)c->d_tx_foot.ptr, np, t);
+    });
+    if (rc) return rc;
+  }
   if (exclusive_scan_u32(c->stream, cnt, off, (long long)ncell + 1, scan_tmp, scan_bytes) != 0)
     return set_err(c, HCS_ERR_LIMIT, "taxel grid too large");
   for (;;) {
@@ -302,6 +339,27 @@ __global__ __launch_bounds__(256) void k_txb_bin(const double* __restrict__ poly
       }
       bin_polygon<FILL>((int)q, f, cx, base, FILL ? cursor : cnt, off, list, list_cap);
       first = false, ++k;
+    }
+  }
+}
+
+/* The entries that k_txb_bin counts, in 64 bits. */
+__global__ __launch_bounds__(256) void k_txb_total(const double* __restrict__ poly, const int64_t* __restrict__ key,
+                                                   int64_t np, const int* __restrict__ psoff,
+                                                   const int* __restrict__ psens, const TaxelGridDev* __restrict__ grids,
+                                                   unsigned long long* __restrict__ total) {
+  const int64_t step = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t q0 = blockIdx.x * (int64_t)blockDim.x; q0 < np; q0 += step) {
+    const int64_t q = q0 + threadIdx.x;
+    int k = 0, k1 = 0;
+    if (q < np) {
+      const int e = (int)key[3 * q];
+      k = psoff[e], k1 = psoff[e + 1];
+    }
+    for (; __any(k < k1); ++k) {
+      int4 f = make_int4(0, -1, 0, -1);
+      if (k < k1) footprint(poly + q * HCS_PREC, grids[psens[k]], f.x, f.y, f.z, f.w);
+      add_entries(f, k < k1, total);
     }
   }
 }
@@ -423,6 +481,9 @@ int batch_taxels_setup(Ctx* c, BatchTaxels& t, int npairs, const int32_t* geoms,
   t.n = n, t.ncell = ncell;
   t.max_rays = 0;
   for (int k = 0; k < n; ++k) t.max_rays = std::max(t.max_rays, g[k].S * g[k].S);
+  std::vector<int64_t> cells(npairs, 0);
+  for (int k = 0; k < n; ++k) cells[pair[k]] += (int64_t)g[k].cx * g[k].cy;
+  t.pair_cells = *std::max_element(cells.begin(), cells.end());
   t.bin_grid = std::max(1, c->num_cu * 4);
   return hip_check(c, hipStreamSynchronize(c->stream), "sync");
 }
@@ -486,7 +547,13 @@ int batch_taxels_demand(Ctx* c, BatchTaxels& t, int64_t& npoly, int64_t& nlist) 
                    "dl");
   if (!rc) rc = hip_check(c, hipStreamSynchronize(c->stream), "sync");
   npoly = (int64_t)np, nlist = (int64_t)nl;
-  return rc;
+  /* (polygons beyond the record buffer are counted when it has grown) */
+  if (rc || npoly > t.poly_cap || np <= kMaxEntries / (unsigned long long)t.pair_cells) return rc;
+  return check_entries(c, [&](unsigned long long* total) {
+    hipLaunchKernelGGL(k_txb_total, dim3(t.bin_grid), dim3(256), 0, c->stream, (const double*)t.poly_rec.ptr,
+                       (const int64_t*)t.poly_key.ptr, npoly, (const int*)t.psoff.ptr, (const int*)t.psens.ptr,
+                       (const TaxelGridDev*)t.grid.ptr, total);
+  });
 }
 
 void batch_taxels_free(BatchTaxels& t) {
