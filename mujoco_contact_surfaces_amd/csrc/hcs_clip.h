@@ -4,18 +4,20 @@
  * per survivor.  The arithmetic is process_candidate's (hcs_query.h), value
  * for value; what differs is how the work lies on the lanes.
  *
- * Such a launch is a few thousand survivors of a step of a few pairs, bound by
- * the time of one wave: the register build for all kinds needs private memory
- * and issues each kind's polygon and up to eight faces for all lanes.  Here
+ * The register build for all kinds needs private memory and issues each kind's
+ * polygon and up to eight faces for all lanes.  Here
  *   - polygons live in LDS, one column per lane, and a clipping plane computes
  *     its two crossings (read back by index) instead of one per possible edge;
  *   - the faces of all 64 polygons are dealt out to the lanes, 64 at a time,
  *     and each polygon's lane adds its faces' results in order;
  *   - divisions by 3 and by a face's slip speed are done with fused
  *     multiply-adds from one reciprocal and rounded as a division would be.
- * A scene of 12 pairs: 42 -> 25 us.  Launches of one kind keep the register
- * builds: with millions of survivors the LDS round trips of every plane and
- * face cost more than the instructions saved (2.6M: 0.70 against 0.72 ms).
+ * Against the register build for all kinds: 12 pairs of a scene 42 -> 25 us, a
+ * batch of tet-query and triangle pairs 26 -> 20 us (16 pairs, 3.6k polygons),
+ * 150 -> 115 (512, 169k) and 685 -> 512 (4096, 1.35M).  Launches of one kind
+ * keep their own register builds: with millions of survivors the LDS round
+ * trips of every plane and face cost more there than the instructions saved
+ * (2.6M: 0.70 against 0.72 ms).
  */
 #pragma once
 #include "hcs_query.h"
@@ -171,8 +173,6 @@ __device__ inline double column_centroid(const double* col, int n, const double*
   return W;
 }
 
-/* One survivor's polygon in the lane's column: n vertices (0: none), the
- * normal nS, the field (gA, cA) of A's tet, and the constants of its faces. */
 /* Has the values loaded here, where nothing else waits, and not where each is
  * first used. */
 template <int N>
@@ -181,6 +181,8 @@ __device__ inline void loaded(double* v) {
   for (int i = 0; i < N; ++i) asm volatile("" : "+v"(v[i]));
 }
 
+/* One survivor's polygon in the lane's column: n vertices (0: none), the
+ * normal nS, the field (gA, cA) of A's tet, and the constants of its faces. */
 struct LanePoly {
   int n;
   double nS[3], gA[3], cA, C[3], W2;

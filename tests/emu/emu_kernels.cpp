@@ -14,6 +14,7 @@
 #include <thread>
 #include <vector>
 
+#include "hcs_clip.h"
 #include "hcs_oracle.h"
 #include "hcs_query.h"
 
@@ -23,6 +24,10 @@ WaveEmu* g_wave;
 /* emu_set_options: run the general candidate kernel (the one mixed-kind
  * launches use) instead of the kind's own */
 int g_generic = 0;
+/* contributions of the last pair that the clip of mixed-kind launches
+ * (clip_wave) makes different from clip_survivor's in any bit but a zero's
+ * sign */
+int64_t g_clip_differences = -1;
 
 using namespace hcs;
 
@@ -288,6 +293,28 @@ int emu_pair(const double* VA, int nva, const int32_t* TA, int nta, const double
       else if (dir < 0) clip_survivor<double>(Q, C, (int64_t)i, dir, con.data(), nullptr);
       else clip_survivor<Dual>(Q, C, (int64_t)i, dir, con.data(), nullptr);
     }
+    if (dir < 0) {
+      /* the same survivors, 64 at a time by one wave */
+      std::vector<Contrib> mixed(con.size());
+      ClipLds* L = new ClipLds();
+      const OutPtrs none{};
+      std::vector<std::thread> th;
+      for (int lane = 0; lane < 64; ++lane)
+        th.emplace_back([&, lane] {
+          g_lane = lane;
+          threadIdx.x = lane;
+          clip_wave(*L, Q, C, 0, 64, (int64_t)scnt, none, mixed.data());
+        });
+      for (auto& t : th) t.join();
+      delete L;
+      g_clip_differences = 0;
+      for (unsigned k = 0; k < off[nitems]; ++k) {
+        const Contrib &a = con[k], &b = mixed[k];
+        bool same = a.np == b.np && a.nf == b.nf;
+        for (int c = 0; c < 3; ++c) same = same && a.F[c] == b.F[c] && a.tA[c] == b.tA[c] && a.tB[c] == b.tB[c];
+        g_clip_differences += !same;
+      }
+    }
     double F[3] = {0, 0, 0}, tA[3] = {0, 0, 0}, tB[3] = {0, 0, 0};
     int64_t np = 0, nf = 0;
     for (unsigned k = 0; k < off[nitems]; ++k) {
@@ -307,6 +334,39 @@ int emu_pair(const double* VA, int nva, const int32_t* TA, int nta, const double
 extern "C" {
 
 void emu_set_options(int generic) { g_generic = generic; }
+int64_t emu_clip_differences() { return g_clip_differences; }
+
+/* x / 3 and x / b as the clip of mixed-kind launches divides. */
+void emu_div3(const double* x, int64_t n, double* q) {
+  for (int64_t i = 0; i < n; ++i) q[i] = div3(x[i]);
+}
+void emu_div_by(const double* x, const double* b, int64_t n, double* q) {
+  for (int64_t i = 0; i < n; ++i) q[i] = div_by(x[i], b[i], 1.0 / b[i]);
+}
+
+/* Polygons of n[i] <= 7 vertices (v: 8 x 3 each) cut by plane i (normal,
+ * offset) in place, with the clip of mixed-kind launches (wave) or with the
+ * one-kind launches' column clip. */
+void emu_clip_planes(double* v, int32_t* n, const double* planes, int64_t count, int wave) {
+  std::vector<double> lds(3 * HCS_MAXV * HCS_CLIP_ST);
+  for (int64_t i = 0; i < count; ++i) {
+    double *p = v + 24 * i, *col = lds.data();
+    const double* h = planes + 4 * i;
+    const int st = wave ? HCS_CLIP_ST : 1;
+    for (int k = 0; k < 24; ++k) col[k * st] = p[k];
+    int m = n[i];
+    ColPoly P{col, st, m};
+    switch (m) {
+      case 3: wave ? clip_plane<3>(col, m, h, h[3]) : clip_halfspace_col<3>(P, h, h[3]); break;
+      case 4: wave ? clip_plane<4>(col, m, h, h[3]) : clip_halfspace_col<4>(P, h, h[3]); break;
+      case 5: wave ? clip_plane<5>(col, m, h, h[3]) : clip_halfspace_col<5>(P, h, h[3]); break;
+      case 6: wave ? clip_plane<6>(col, m, h, h[3]) : clip_halfspace_col<6>(P, h, h[3]); break;
+      default: wave ? clip_plane<7>(col, m, h, h[3]) : clip_halfspace_col<7>(P, h, h[3]); break;
+    }
+    n[i] = wave ? m : P.n;
+    for (int k = 0; k < 24; ++k) p[k] = k < 3 * n[i] ? col[k * st] : 0.0;
+  }
+}
 
 /* A wave whose even and odd lanes reach two different ballots: the
  * emulation must abort on it (a collective under divergent control flow). */
