@@ -694,8 +694,6 @@ __global__ __launch_bounds__(64, KS == KIND_TRI ? 3 : 2) void k_cand(QueryArgs A
     const unsigned n = A.live_cnt[0], G = gridDim.x;
     const int base = A.live ? A.qseg[0] : 0;
     const unsigned v = blockIdx.x;
-    /* tet and half-space items are alike and short: dealt out by index */
-    constexpr bool fixed = KS == KIND_PLANE || KS == KIND_TET;
     if (v < n) {
       int idx = A.live ? A.live[base + v] : (int)v;
       int4 rec = A.live_item[base + v];
@@ -707,13 +705,13 @@ __global__ __launch_bounds__(64, KS == KIND_TRI ? 3 : 2) void k_cand(QueryArgs A
         if (vn < n) {
           nidx = A.live ? A.live[base + vn] : (int)vn;
           nrec = A.live_item[base + vn];
-          if (!fixed && k > 0 && lane == 0) raw = atomicAdd(A.counter, 1u);
+          if (k > 0 && lane == 0) raw = atomicAdd(A.counter, 1u);
         }
         run_cand<MODE, KS>(L, A, idx, Item{rec.x, rec.y, rec.z, rec.w}, s_next, s_end);
         if (vn >= n) break;
         idx = nidx;
         rec = nrec;
-        vn = fixed ? vn + G : k == 0 ? v + 2 * G : __shfl(raw, 0, 64) + 3 * G;
+        vn = k == 0 ? v + 2 * G : __shfl(raw, 0, 64) + 3 * G;
       }
     }
   } else if (A.live) {
