@@ -290,9 +290,9 @@ static int batch_plan(hcs_batch* b) {
   int rc = build_plan(b->c, b->npairs, b->geoms.data(), &b->opts, b->tet_max, b->plan,
                       b->implicit ? ITEMS_IMPLICIT : ITEMS_WHOLE);
   b->plan.order.clear();
-  /* few items are cut evenly (20 pairs: 185 against 187 us a step), and a
-   * million go as they are */
-  b->plan.spread = b->implicit && b->plan.nitems > 4096 && b->plan.nitems <= HCS_SPREAD_BUDGET &&
+  /* few items are cut evenly (20 pairs: 185 against 187 us a step), and
+   * millions go as they are */
+  b->plan.spread = b->implicit && b->plan.nitems > 4096 && b->plan.nitems <= HCS_SPREAD_ITEMS &&
                    std::any_of(b->plan.envs.begin(), b->plan.envs.end(),
                                [](const EnvDesc& E) { return E.kind == KIND_TRI || E.kind == KIND_SOFT; });
   if (b->implicit) return rc ? rc : batch_upload_implicit(b);

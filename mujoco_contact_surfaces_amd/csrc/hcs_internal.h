@@ -141,12 +141,19 @@ int build_plan(Ctx* c, int npairs, const int32_t* geoms, const hcs_step_opts* o,
                Plan& plan, PlanItems mode = ITEMS_WHOLE);
 
 /* Per-call steps: threads (items) per block of the item enumeration; items
- * that a split may lead to in all; sizes of the tables that follow from a
- * plan (blocks of both culls, places of live items, reduction slices). */
+ * that a split may lead to in all (HCS_SPREAD_BUDGET beyond the first cull's in
+ * a spread plan); sizes of the tables that follow from a plan (blocks of both
+ * culls, places of live items, reduction slices). */
 #define HCS_GEN_THREADS 256
 #define HCS_ITEM_BUDGET 65536
 #define HCS_EXPAND_BUDGET 16384
 #define HCS_SPREAD_BUDGET 262144
+/* Items up to which an unmeasured batch has them cut by their expected
+ * candidates (28 bytes an item).  With objects of up to 20k triangles, cut
+ * against whole: 8192 pairs (327k items) 3.28 against 6.05 ms a step, 32768
+ * pairs (1.3M) 11.8 against 13.2; with 65536 pairs (2.6M) 23.0 both ways, the
+ * chip has whole items enough. */
+#define HCS_SPREAD_ITEMS (1 << 21)
 struct CallSizes {
   size_t blocks1, blocks2, items, live, expand;
   int slices;
