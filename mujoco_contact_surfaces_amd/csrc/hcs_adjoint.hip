@@ -84,7 +84,7 @@ static int tangent_pass(Ctx* c, int npairs, const hcs_pair_in* in, const hcs_ste
       a.poly_cnt = (unsigned long long*)c->d_poly_cnt.ptr;
     }
     pipe_enqueue(c, P, a, npairs, nitems, clip_grid_for(c, P.cap), ndir, (const double*)dseed.ptr,
-                 (const double*)dseed.ptr + npairs, false, dir0);
+                 (const double*)dseed.ptr + npairs, dir0);
     rc = hip_check(c, hipGetLastError(), "tangent pass");
     unsigned long long ns = 0;
     if (!rc) rc = hip_check(c, hipMemcpyAsync(&ns, P.surv_cnt.ptr, 8, hipMemcpyDeviceToHost, c->stream), "dl");

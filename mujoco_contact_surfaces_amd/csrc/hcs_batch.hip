@@ -106,7 +106,7 @@ static void batch_enqueue(hcs_batch* b, const QueryArgs& a) {
   }
   if (b->tx.n > 0) launch_fill_u32(b->c->stream, (unsigned*)b->tx.poly_cnt.ptr, 0u, 2);
   pipe_enqueue(b->c, b->pipe, a, b->npairs, grid_of(b), clip_grid_for(b->c, b->pipe.cap), 0, nullptr, nullptr,
-               false, 0);
+               0);
   batch_taxels_enqueue(b->c, b->tx, (const double*)b->state.ptr);
 }
 
@@ -171,7 +171,7 @@ static int batch_measure(hcs_batch* b, std::vector<int>& nc) {
   /* counts only: no survivors, no clipping */
   const QueryArgs a = batch_args(b);
   pipe_front(c, b->pipe, a, b->npairs);
-  launch_cand(c->stream, a, grid_of(b), CAND_COUNT);
+  launch_cand(c, a, grid_of(b), CAND_COUNT);
   int rc = hip_check(c, hipGetLastError(), "measure step");
   if (!rc)
     rc = hip_check(c, hipMemcpyAsync(nc.data(), b->pipe.ncand.ptr, sizeof(int) * n, hipMemcpyDeviceToHost, c->stream),
@@ -195,7 +195,7 @@ static int batch_measure_cycles(hcs_batch* b, std::vector<unsigned long long>& c
   QueryArgs a = batch_args(b);
   a.item_stats = (unsigned long long*)d.ptr;
   pipe_front(c, b->pipe, a, b->npairs);
-  launch_cand(c->stream, a, grid_of(b), CAND_STEP);
+  launch_cand(c, a, grid_of(b), CAND_STEP);
   std::vector<unsigned long long> h(6 * (size_t)n);
   rc = hip_check(c, hipGetLastError(), "cycles step");
   if (!rc) rc = hip_check(c, hipMemcpyAsync(h.data(), d.ptr, bytes, hipMemcpyDeviceToHost, c->stream), "dl");
@@ -690,7 +690,7 @@ int hcs_batch_kernel_times(hcs_batch* b, int32_t reps, double* ms) {
     if (b->implicit) (void)call_front(c, P, a, b->plan, b->blob, nullptr, 0);
     else pipe_front(c, P, a, b->npairs);
     (void)hipEventRecord(ev[0], s);
-    launch_cand(s, a, cand_grid(b), CAND_STEP);
+    launch_cand(c, a, cand_grid(b), CAND_STEP);
     (void)hipEventRecord(ev[1], s);
     if (b->implicit)
       (void)call_back(c, P, a, b->plan, (PairOut*)P.out.ptr, (CallTail*)((PairOut*)P.out.ptr + b->npairs), ev[2], ev[4]);

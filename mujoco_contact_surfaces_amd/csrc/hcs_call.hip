@@ -551,7 +551,7 @@ __global__ __launch_bounds__(64) void k_call_reduce(const int* __restrict__ pair
 
 struct CombineArgs {
   const RedPart* part;
-  int K, npairs;
+  int K;
   const unsigned long long *surv_cnt, *poly_cnt, *face_cnt, *cand_cnt;
   int64_t surv_cap;
   const int* err;
@@ -763,7 +763,7 @@ int call_back(Ctx* c, Pipe& p, const QueryArgs& a, const Plan& plan, PairOut* ou
                      (const int*)a.item_ncand, (const unsigned long long*)a.surv_cnt, p.cap,
                      (const Contrib*)p.contrib.ptr, (RedPart*)p.part.ptr);
   CombineArgs q{};
-  q.part = (const RedPart*)p.part.ptr, q.K = K, q.npairs = np;
+  q.part = (const RedPart*)p.part.ptr, q.K = K;
   q.surv_cnt = a.surv_cnt, q.surv_cap = p.cap, q.err = a.error, q.out = out, q.tail = tail;
   /* a counter the step does not have reads as cleared words of the error
    * block */
@@ -778,7 +778,7 @@ int call_enqueue(Ctx* c, Pipe& p, const QueryArgs& a, const Plan& plan, const Ca
                  int ncounters, bool keys, int cand_grid, PairOut* out, CallTail* tail) {
   int rc = call_front(c, p, a, plan, b, counters, ncounters);
   if (rc) return rc;
-  launch_cand(c->stream, a, std::min(a.nitems, cand_grid), keys ? CAND_KEYS : CAND_STEP);
+  launch_cand(c, a, std::min(a.nitems, cand_grid), keys ? CAND_KEYS : CAND_STEP);
   return keys ? HCS_OK : call_back(c, p, a, plan, out, tail, nullptr, nullptr);
 }
 

@@ -246,7 +246,6 @@ __global__ void k_karras(const unsigned* __restrict__ codes, const int* __restri
   const int lo = i < j ? i : j, hi = i < j ? j : i;
   range[i] = make_int2(lo, hi);
   Node* N = nodes + i;
-  N->h[0] = N->h[1] = 0;
   if (lo == gamma) {
     N->c[0] = ~idx[gamma];
     leaf_parent[gamma] = i;
@@ -352,8 +351,7 @@ __global__ __launch_bounds__(64) void k_node_boxes(const double* __restrict__ bo
   for (int c = 0; c < 6; ++c) ubox[6 * (size_t)i + c] = u[c];
 }
 
-/* The children's boxes of every internal node, and its 4-wide node (the
- * layout of make_wide_node: grandchildren, a leaf child standing for itself). */
+/* The children's boxes of every internal node, and its 4-wide node. */
 __global__ __launch_bounds__(256) void k_fill_nodes(const double* __restrict__ ubox, const double* __restrict__ box,
                                                     const int2* __restrict__ range, int n_int,
                                                     const BuildOut* __restrict__ out, Node* nodes,
@@ -361,35 +359,14 @@ __global__ __launch_bounds__(256) void k_fill_nodes(const double* __restrict__ u
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n_int || out->bad) return;
   nodes[i].leaves = range[i].y - range[i].x + 1;
-  WNode& w = wide[i];
-  int m = 0;
-  auto put = [&](int ch) {
-    const double* b = ch < 0 ? box + 6 * (size_t)~ch : ubox + 6 * (size_t)ch;
-#pragma unroll
-    for (int c = 0; c < 6; ++c) w.b[6 * m + c] = b[c];
-    w.ch[m++] = ch;
-  };
+  auto child = [&](int ch) { return ch < 0 ? box + 6 * (size_t)~ch : ubox + 6 * (size_t)ch; };
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
-    const int ch = nodes[i].c[s];
-    const double* b = ch < 0 ? box + 6 * (size_t)~ch : ubox + 6 * (size_t)ch;
+    const double* b = child(nodes[i].c[s]);
 #pragma unroll
     for (int c = 0; c < 6; ++c) nodes[i].b[6 * s + c] = b[c];
-    if (ch < 0) {
-      put(ch);
-    } else {
-      const int g0 = nodes[ch].c[0], g1 = nodes[ch].c[1];
-      put(g0);
-      put(g1);
-    }
   }
-  for (; m < 4; ++m) {
-#pragma unroll
-    for (int c = 0; c < 3; ++c) w.b[6 * m + c] = __builtin_inf(), w.b[6 * m + 3 + c] = -__builtin_inf();
-    w.ch[m] = HCS_WNONE;
-  }
-#pragma unroll
-  for (int k = 0; k < 12; ++k) w.pad[k] = 0;
+  make_wide_node(nodes, i, wide[i], child);
 }
 
 /* Depth of the deepest leaf: every leaf counts its ancestors. */
@@ -1016,12 +993,13 @@ static void launch_cand_mode(hipStream_t s, const QueryArgs& a, int grid) {
   }
 }
 
-void launch_cand(hipStream_t s, const QueryArgs& a, int grid, int mode) {
+void launch_cand(Ctx* c, const QueryArgs& a, int grid, int mode) {
+  hipStream_t s = c->stream;
   if (a.nitems <= 0 || grid <= 0) return;
   if (mode == CAND_KEYS) launch_cand_mode<CAND_KEYS>(s, a, grid);
   else if (mode == CAND_COUNT) launch_cand_mode<CAND_COUNT>(s, a, grid);
   else if (launch_kind(a) == KIND_PLANE)
-    hipLaunchKernelGGL(k_cand_plane, dim3(std::min((a.nitems + HCS_PLANE_ITEMS - 1) / HCS_PLANE_ITEMS, 256 * 4)),
+    hipLaunchKernelGGL(k_cand_plane, dim3(std::min((a.nitems + HCS_PLANE_ITEMS - 1) / HCS_PLANE_ITEMS, c->num_cu * 4)),
                        dim3(64 * HCS_PLANE_WAVES), 0, s, a);
   else launch_cand_mode<CAND_STEP>(s, a, grid);
 }
@@ -1071,10 +1049,9 @@ static void pipe_back(Ctx* c, Pipe& p, const QueryArgs& a, int npairs, int clip_
 }
 
 void pipe_enqueue(Ctx* c, Pipe& p, const QueryArgs& a, int npairs, int cand_grid, int clip_grid, int ndir,
-                  const double* dstar_dE, const double* invE, bool cand_only, int dir0) {
+                  const double* dstar_dE, const double* invE, int dir0) {
   pipe_front(c, p, a, npairs);
-  launch_cand(c->stream, a, cand_grid, a.cand_key ? CAND_KEYS : CAND_STEP);
-  if (cand_only) return;
+  launch_cand(c, a, cand_grid, CAND_STEP);
   pipe_back(c, p, a, npairs, clip_grid, ndir, dstar_dE, invE, dir0, nullptr, nullptr);
 }
 

@@ -192,7 +192,7 @@ QueryArgs pipe_args(const Pipe& p, const EnvDesc* envs, const double* state, con
 /* ndir = 0: forward (double); ndir > 0: tangent directions dir0 ..
  * dir0+ndir-1 (contributions and outputs indexed by direction - dir0). */
 void pipe_enqueue(Ctx* c, Pipe& p, const QueryArgs& a, int npairs, int cand_grid, int clip_grid, int ndir,
-                  const double* dstar_dE, const double* invE, bool cand_only, int dir0);
+                  const double* dstar_dE, const double* invE, int dir0);
 /* Static boxes of the current items (once per plan, after the items and
  * env descriptors are on the device). */
 struct Plan;
@@ -206,7 +206,7 @@ int split_roots(Ctx* c, const EnvDesc* envs, const Item* items, const std::vecto
                 const std::vector<int>& depth, std::vector<int32_t>& out);
 void pipe_free(Pipe& p);
 /* mode: CandMode */
-void launch_cand(hipStream_t s, const QueryArgs& a, int grid, int mode);
+void launch_cand(Ctx* c, const QueryArgs& a, int grid, int mode);
 void launch_clip(Ctx* c, const Pipe& p, const QueryArgs& a, int clip_grid);
 int pinned(Ctx* c, void*& p, size_t& have, size_t bytes);
 void launch_clip_reduce(Ctx* c, Pipe& p, const QueryArgs& a, int npairs, int clip_grid, hipEvent_t e_clip,

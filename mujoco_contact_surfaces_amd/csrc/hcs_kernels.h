@@ -46,9 +46,8 @@ namespace hcs {
 struct Node {
   double b[12];   /* child 0 lo[3] hi[3], child 1 lo[3] hi[3] */
   int32_t c[2];   /* >= 0 internal node, < 0 leaf: ~element */
-  int32_t h[2];   /* subtree heights (leaf 0) */
-  int32_t leaves; /* under this node (device build) */
-  int32_t pad[3];
+  int32_t leaves; /* under this node */
+  int32_t pad[5];
 };
 static_assert(sizeof(Node) == 128, "one LBVH node per cache line");
 
@@ -66,27 +65,34 @@ struct WNode {
 static_assert(sizeof(WNode) == 256, "one wide node per two cache lines");
 #define HCS_WNONE INT32_MIN
 
-/* Builds the wide node of binary internal node i. */
-__host__ __device__ inline void make_wide_node(const Node* nodes, int i, WNode& w) {
-  const Node& n = nodes[i];
+/* Builds the wide node of binary internal node i from the nodes' children;
+ * box(ch): the 6 doubles of child code ch. */
+template <class Box>
+__host__ __device__ inline void make_wide_node(const Node* nodes, int i, WNode& w, Box box) {
   int m = 0;
-  auto put = [&](const double* b, int ch) {
+  auto put = [&](int ch) {
+    const double* b = box(ch);
+#pragma unroll
     for (int c = 0; c < 6; ++c) w.b[6 * m + c] = b[c];
     w.ch[m++] = ch;
   };
+#pragma unroll
   for (int s = 0; s < 2; ++s) {
-    const int c = n.c[s];
+    const int c = nodes[i].c[s];
     if (c < 0) {
-      put(n.b + 6 * s, c);
+      put(c);
     } else {
-      const Node& g = nodes[c];
-      for (int t = 0; t < 2; ++t) put(g.b + 6 * t, g.c[t]);
+      const int g0 = nodes[c].c[0], g1 = nodes[c].c[1];
+      put(g0);
+      put(g1);
     }
   }
   for (; m < 4; ++m) {
+#pragma unroll
     for (int c = 0; c < 3; ++c) w.b[6 * m + c] = INFINITY, w.b[6 * m + 3 + c] = -INFINITY;
     w.ch[m] = HCS_WNONE;
   }
+#pragma unroll
   for (int k = 0; k < 12; ++k) w.pad[k] = 0;
 }
 

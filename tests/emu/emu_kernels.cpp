@@ -120,21 +120,26 @@ void prepare(const double* V, int nv, const int32_t* T, int nt, const double* p,
     const double* b = &s.box[6 * (size_t)s.leaf[j]];
     int pc = lp[j], pp = pc >> 1, side = pc & 1;
     for (int c = 0; c < 6; ++c) s.nodes[pp].b[6 * side + c] = b[c];
-    s.nodes[pp].h[side] = 0;
     for (int guard = 0; guard < n; ++guard) {
       if (flags[pp]++ == 0) break;
       Node& N = s.nodes[pp];
       double u[6];
       for (int c = 0; c < 3; ++c) u[c] = std::fmin(N.b[c], N.b[6 + c]), u[3 + c] = std::fmax(N.b[3 + c], N.b[9 + c]);
-      const int h = 1 + std::max(N.h[0], N.h[1]);
       if (pp == 0) break;
       pc = np[pp], pp = pc >> 1, side = pc & 1;
       for (int c = 0; c < 6; ++c) s.nodes[pp].b[6 * side + c] = u[c];
-      s.nodes[pp].h[side] = h;
     }
   }
   s.wnodes.resize(std::max(1, n - 1));
-  for (int i = 0; i + 1 < n; ++i) make_wide_node(s.nodes.data(), i, s.wnodes[i]);
+  std::vector<double> ubox(6 * (size_t)n);
+  for (int i = 0; i + 1 < n; ++i) {
+    const Node& N = s.nodes[i];
+    double* u = &ubox[6 * (size_t)i];
+    for (int c = 0; c < 3; ++c) u[c] = std::fmin(N.b[c], N.b[6 + c]), u[3 + c] = std::fmax(N.b[3 + c], N.b[9 + c]);
+  }
+  for (int i = 0; i + 1 < n; ++i)
+    make_wide_node(s.nodes.data(), i, s.wnodes[i],
+                   [&](int ch) { return ch < 0 ? &s.box[6 * (size_t)~ch] : &ubox[6 * (size_t)ch]; });
 }
 
 }  // namespace
