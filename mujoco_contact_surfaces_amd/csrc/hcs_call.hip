@@ -498,8 +498,12 @@ __global__ __launch_bounds__(HCS_GEN_THREADS) void k_cut_keep(const EnvDesc* __r
 }
 
 /* Exclusive scan of the live items' survivor counts (off[n] = total), one
- * block: a few thousand items, one launch instead of three. */
-constexpr int kScanThreads = 1024, kScanPer = 8;
+ * block: 3 to 9 us for up to 8192 live items and as much again for every 8192
+ * more, where a scan of all places takes 9 us in three launches.  A small part
+ * of the places is live: with up to kScanPlaces of them this is 5 us less for
+ * 12 mixed pairs and 120 bodies on the ground, 3 for 250 and the same for 500
+ * bodies, whose places just fit. */
+constexpr int kScanThreads = 1024, kScanPer = 8, kScanPlaces = 65536;
 __global__ __launch_bounds__(kScanThreads) void k_call_scan(const unsigned* __restrict__ in,
                                                             const unsigned* __restrict__ live_cnt,
                                                             unsigned* __restrict__ off) {
@@ -748,7 +752,7 @@ int call_back(Ctx* c, Pipe& p, const QueryArgs& a, const Plan& plan, PairOut* ou
   const CallSizes z = call_sizes(plan);
   const int np = (int)plan.envs.size();
   unsigned* off = (unsigned*)p.off.ptr;
-  if (z.live <= (size_t)kScanThreads * kScanPer * 8) {
+  if (z.live <= (size_t)kScanPlaces) {
     hipLaunchKernelGGL(k_call_scan, dim3(1), dim3(kScanThreads), 0, s, (const unsigned*)a.item_nsurv,
                        (const unsigned*)a.live_cnt, off);
   } else if (exclusive_scan_u32(s, a.item_nsurv, off, (long long)z.live + 1, p.scan_tmp.ptr, p.scan_bytes) != 0) {

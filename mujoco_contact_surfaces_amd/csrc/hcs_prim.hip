@@ -6,7 +6,7 @@
  * polygon keys of the sensors).
  *
  * Scan (reduce-then-scan, three launches, no atomics, no waits; one block and
- * one launch up to 32768 counts): tiles of
+ * one launch up to 8192 counts): tiles of
  * 2048 counts (256 threads x 8), a per-tile sum, one block scanning the
  * tile sums, then every tile scanned again with its offset.  Within a block
  * each thread sums its 8 contiguous counts, a wave scans the thread sums
@@ -117,31 +117,27 @@ __global__ __launch_bounds__(kThreads) void k_scan_apply(const unsigned* in, lon
   }
 }
 
-/* A short scan (at most kOneTiles tiles) in one launch of one block: three
- * launches and their gaps cost more than a block's passes over it (6400
- * digit counts of a 51k-key sort pass: 10 us and two gaps -> 7.6 us). */
+/* A scan of up to one block's tile in one launch: three launches take 7.7 to
+ * 9.2 us whatever the size (300 to 65536 counts), this 2.6 us at 300 counts,
+ * 5.5 at 4096 and 8.9 at 8192; a second tile of the one block costs as much
+ * again (16 us at 16384, 30 at 32768). */
 constexpr int kOneTile = kSumThreads * kPer;
-constexpr int kOneTiles = 4;
 __global__ __launch_bounds__(kSumThreads) void k_scan_one(const unsigned* in, int n, unsigned* out) {
   __shared__ unsigned lds[kSumThreads / 64];
-  unsigned carry = 0;
-  for (int t0 = 0; t0 < n; t0 += kOneTile) {
-    const int base = t0 + threadIdx.x * kPer;
-    unsigned v[kPer];
-    unsigned s = 0;
+  const int base = threadIdx.x * kPer;
+  unsigned v[kPer];
+  unsigned s = 0;
 #pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-      v[j] = base + j < n ? in[base + j] : 0u;
-      s += v[j];
-    }
-    unsigned total;
-    unsigned run = carry + block_excl_scan(s, lds, &total);
+  for (int j = 0; j < kPer; ++j) {
+    v[j] = base + j < n ? in[base + j] : 0u;
+    s += v[j];
+  }
+  unsigned total;
+  unsigned run = block_excl_scan(s, lds, &total);
 #pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-      if (base + j < n) out[base + j] = run;
-      run += v[j];
-    }
-    carry += total;
+  for (int j = 0; j < kPer; ++j) {
+    if (base + j < n) out[base + j] = run;
+    run += v[j];
   }
 }
 
@@ -255,7 +251,7 @@ int exclusive_scan_u32(hipStream_t s, const unsigned* in, unsigned* out, long lo
   if (n <= 0) return 0;
   const long long tiles = (n + kTile - 1) / kTile;
   if (tiles > (long long)kSumThreads * kMaxSumPer || tmp_bytes < scan_temp_bytes(n)) return -1;
-  if (n <= (long long)kOneTiles * kOneTile) {
+  if (n <= kOneTile) {
     hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(kSumThreads), 0, s, in, (int)n, out);
     return 0;
   }
