@@ -208,8 +208,9 @@ int hcs_contact_step(hcs_ctx* ctx, int32_t npairs, const hcs_pair_in* in, const 
  * under HIP graph capture, tight serving loops, hosts that forbid
  * hipMalloc); no counterpart in the reference.  Wrenches and counts only
  * (no faces; keep_polygons must be 0).  Every device buffer of the step is
- * a slice of one static 64 MiB array per device, so the call allocates and
- * frees nothing; pairs, work items and survivors must fit it together (at
+ * a slice of one static array per device (64 MiB for what the call's sizes
+ * ask for, 4 MiB for the engine's own tables), so the call allocates and frees
+ * nothing; pairs, work items and survivors must fit the 64 MiB together (at
  * most about 690k survivors of the exact rejections) or the call returns
  * HCS_ERR_CAPACITY.  The array is shared by every call on one device:
  * calls that overlap on one device race. */

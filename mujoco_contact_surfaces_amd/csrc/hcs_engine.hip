@@ -744,8 +744,8 @@ __global__ __launch_bounds__(64, KS == KIND_TRI ? 3 : 2) void k_cand(QueryArgs A
  * waves 144 us; one wave per item with the general kernel's survivor chunks
  * 127 us, and the clip kernel read the chunks' padding; this form 55 us, and
  * the clip 98 -> 43 us with its own build and no padding).  Four items per
- * wave keep four chains item -> pair -> boxes -> records in flight, which is
- * what bounds it.  Survivors are numbered in lane order, as the general
+ * wave keep four chains item -> pair -> boxes -> records in flight; what bounds
+ * it now is the data path (busy 73% of the time) and HBM (0.29 GB).  Survivors are numbered in lane order, as the general
  * kernel does. */
 #define HCS_PLANE_WAVES 8
 #define HCS_PLANE_PER 4
@@ -983,25 +983,29 @@ static int launch_kind(const QueryArgs& a) {
 }
 
 template <int MODE>
-static void launch_cand_mode(hipStream_t s, const QueryArgs& a, int grid) {
+static void launch_cand_mode(Ctx* c, const QueryArgs& a, int grid) {
+  hipStream_t s = c->stream;
   switch (launch_kind(a)) {
     case KIND_TRI: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cand<MODE, KIND_TRI>), dim3(grid), dim3(64), 0, s, a); break;
     case KIND_SOFT: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cand<MODE, KIND_SOFT>), dim3(grid), dim3(64), 0, s, a); break;
     case KIND_TET: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cand<MODE, KIND_TET>), dim3(grid), dim3(64), 0, s, a); break;
-    case KIND_PLANE: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cand<MODE, KIND_PLANE>), dim3(grid), dim3(64), 0, s, a); break;
+    case KIND_PLANE:
+      if constexpr (MODE == CAND_STEP) {
+        const int blocks = std::min((a.nitems + HCS_PLANE_ITEMS - 1) / HCS_PLANE_ITEMS, c->num_cu * 4);
+        hipLaunchKernelGGL(k_cand_plane, dim3(blocks), dim3(64 * HCS_PLANE_WAVES), 0, s, a);
+      } else {
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cand<MODE, KIND_PLANE>), dim3(grid), dim3(64), 0, s, a);
+      }
+      break;
     default: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cand<MODE, -1>), dim3(grid), dim3(64), 0, s, a); break;
   }
 }
 
 void launch_cand(Ctx* c, const QueryArgs& a, int grid, int mode) {
-  hipStream_t s = c->stream;
   if (a.nitems <= 0 || grid <= 0) return;
-  if (mode == CAND_KEYS) launch_cand_mode<CAND_KEYS>(s, a, grid);
-  else if (mode == CAND_COUNT) launch_cand_mode<CAND_COUNT>(s, a, grid);
-  else if (launch_kind(a) == KIND_PLANE)
-    hipLaunchKernelGGL(k_cand_plane, dim3(std::min((a.nitems + HCS_PLANE_ITEMS - 1) / HCS_PLANE_ITEMS, c->num_cu * 4)),
-                       dim3(64 * HCS_PLANE_WAVES), 0, s, a);
-  else launch_cand_mode<CAND_STEP>(s, a, grid);
+  if (mode == CAND_KEYS) launch_cand_mode<CAND_KEYS>(c, a, grid);
+  else if (mode == CAND_COUNT) launch_cand_mode<CAND_COUNT>(c, a, grid);
+  else launch_cand_mode<CAND_STEP>(c, a, grid);
 }
 
 /* The forward clip kernel, built for the launch's kind. */

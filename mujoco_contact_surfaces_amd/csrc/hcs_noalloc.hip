@@ -7,10 +7,11 @@
  *
  * Every device buffer of the step (env descriptors, state, work items, the
  * pipeline's counters, survivors, contributions, scan storage, reduction
- * partials and per-pair outputs) is a slice of one file-scope array, `scratch`, of HCS_SCRATCH_BYTES on each device.  Its
- * device address comes from hipGetSymbolAddress, taken once per device
- * with that device current (hcs_create calls scratch_setup); host code only
- * ever uses that address.  The slices are laid out per call from the call's
+ * partials and per-pair outputs) is a slice of one file-scope array, `scratch`,
+ * of HCS_SCRATCH_BYTES + HCS_SCRATCH_EXTRA on each device.  Its device address
+ * comes from hipGetSymbolAddress, taken once per device with that device
+ * current (hcs_create calls scratch_setup); host code only ever uses that
+ * address.  The slices are laid out per call from the call's
  * sizes; a call that does not fit returns HCS_ERR_CAPACITY before anything
  * runs, or (survivors beyond the space left) after the step with every
  * pair's counts valid and its status HCS_ERR_CAPACITY.

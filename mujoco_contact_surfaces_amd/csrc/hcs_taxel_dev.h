@@ -296,8 +296,9 @@ __device__ inline double sample_cell(const double* __restrict__ poly, const doub
  * the same.
  *
  * Bound by FP64 instructions and the latency of their chains at 2 waves per
- * SIMD (about 205 VGPRs; held to 168 it spills and is no faster), so by the
- * hit tests and ranges a fan takes and by how evenly they fill the lanes.  A
+ * SIMD (207 VGPRs; held to 168 it spills and is no faster): 45% of the issue
+ * slots with 76% of the lanes active, the waves waiting half of the time; so by
+ * the hit tests and ranges a fan takes and by how evenly they fill the lanes.  A
  * fan covers 2 to 4 rays: sample ranges that end at the last ray inside (they
  * were rounded outward by up to a sample on each side), one evaluation per ray
  * (there were two) and row cuts without divisions by the spacing took 1024

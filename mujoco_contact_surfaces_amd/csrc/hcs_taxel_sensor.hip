@@ -343,7 +343,8 @@ struct TsPart {
  * once for the wave's taxels, and the slices fill the chip whatever the
  * number of taxels (one wave per taxel over all samples was 256 waves, each
  * a chain of 1600 loads of its own: 501 us for 256 taxels and 104k samples,
- * -> 24 us).  FP64 multiplies and adds bound it. */
+ * -> 27 us).  What bounds it is the latency of its loads and FP64 chains: 28%
+ * of the issue slots, the waves waiting 58% of the time. */
 #define HCS_TS_TX 8
 template <bool CLOSEST>
 __global__ __launch_bounds__(64) void k_ts_taxel(const double* __restrict__ P, const double* __restrict__ E,
