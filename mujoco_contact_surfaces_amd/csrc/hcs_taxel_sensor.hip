@@ -451,7 +451,7 @@ struct CsHit {
  * of its own mask, so a round serves one triangle of every lane.  (The box of the ray segment
  * against the triangle's box, the test before, let a fifth of the triangles
  * through for rays oblique to the axes, so most triangles were hit-tested
- * for some lane: 67 us.)  2601 rays on 11.5k triangles: 5522 -> 44 us. */
+ * for some lane: 67 us.)  2601 rays on 11.5k triangles: 5522 -> 45 us. */
 __global__ __launch_bounds__(64) void k_cs_rays(const double* __restrict__ tris, int64_t nt, CsArgs a,
                                                 const double* __restrict__ pts, const double* __restrict__ nrms, int m,
                                                 CsHit* __restrict__ part) {
