@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "hcs_clip.h"
+#include "hcs_items.h"
 #include "hcs_oracle.h"
 #include "hcs_query.h"
 
@@ -28,6 +29,14 @@ int g_generic = 0;
  * (clip_wave) makes different from clip_survivor's in any bit but a zero's
  * sign */
 int64_t g_clip_differences = -1;
+
+/* emu_set_items: items as a per-call step has them (1: cut evenly) or an
+ * unconfigured batch (2: by expected candidates), over the frontier of depth
+ * `depth` and with room for `room` pieces; 0: those of emu_pair's split */
+struct {
+  int mode = 0, depth = 0;
+  unsigned room = 0;
+} g_items;
 
 using namespace hcs;
 
@@ -142,6 +151,78 @@ void prepare(const double* V, int nv, const int32_t* T, int nt, const double* p,
                    [&](int ch) { return ch < 0 ? &s.box[6 * (size_t)~ch] : &ubox[6 * (size_t)ch]; });
 }
 
+/* the leaves under node code ch, in order */
+void leaves_under(const Soft& s, int ch, std::vector<int>& out) {
+  if (ch == HCS_WNONE) return;
+  if (ch < 0 || s.leaf.size() == 1) {
+    out.push_back(ch < 0 ? ~ch : s.leaf[0]);
+    return;
+  }
+  leaves_under(s, s.nodes[ch].c[0], out);
+  leaves_under(s, s.nodes[ch].c[1], out);
+}
+
+/* the LBVH's frontiers, as k_frontiers lays them out */
+std::vector<int32_t> frontiers(const Soft& s) {
+  std::vector<int32_t> h(HCS_ROOTS, HCS_WNONE);
+  h[1] = 0;
+  for (int i = 1; i < HCS_ROOTS / 2; ++i) {
+    const int c = h[i];
+    const bool node = c >= 0 && s.leaf.size() > 1;
+    h[2 * i] = node ? s.nodes[c].c[0] : c;
+    h[2 * i + 1] = node ? s.nodes[c].c[1] : HCS_WNONE;
+  }
+  return h;
+}
+
+/* the live items of one pair (E: with its chunk boxes and frontiers), as the
+ * kernels of hcs_call.hip enumerate, cull and cut them */
+std::vector<Item> live_items(const EnvDesc& E, const double* X, int chunks) {
+  std::vector<int4> item;
+  std::vector<unsigned> word;
+  unsigned long long sum = 0;
+  const int depth = is_tree(E) ? E.depth : 0;
+  for (int i = 0; i < chunks << depth; ++i) {
+    int chunk, node;
+    if (!first_item(E, X, i, chunk, node)) continue;
+    const int root = is_tree(E) ? E.rootsA[node] : 0;
+    item.push_back(make_int4(0, chunk, g_items.mode == 1 ? node : root, 0));
+    word.push_back(cut_word(E, X, chunk, root));
+    sum += word.back() & kEstMask;
+  }
+  const unsigned n = (unsigned)item.size();
+  std::vector<Item> out;
+  auto keep = [&](const int4& it, int root) {
+    const int4 r = live_record(E, it, root);
+    out.push_back(Item{r.x, r.y, r.z, r.w});
+  };
+  if (g_items.mode == 1) {
+    for (unsigned t = 0; t < std::max(n, g_items.room); ++t) {
+      int i, s, node;
+      if (!second_item(&E, item.data(), n, g_items.room, t, i, s, node)) continue;
+      double Q[6];
+      chunk_box(E, item[i].y, Q);
+      if (node != item[i].z && !may_meet_subtree(E, X, Q, E.rootsA[node])) continue;
+      keep(item[i], is_tree(E) ? E.rootsA[node] : 0);
+    }
+    return out;
+  }
+  const CutArgs c{&n, &sum, 8, n + g_items.room};
+  const unsigned target = std::max(1u, cut_target(c) / 64); /* (small pairs: the least target would cut nothing) */
+  std::vector<unsigned> off(n + 1, 0);
+  for (unsigned i = 0; i < n; ++i) off[i + 1] = off[i] + cut_slots(word[i], target);
+  for (unsigned t = 0; t < off[n] + 3; ++t) {
+    int i, s, levels;
+    if (!piece(off.data(), n, t, i, s, levels)) continue;
+    const int root = cut_root(E, item[i].z, levels, s);
+    double Q[6];
+    chunk_box(E, item[i].y, Q);
+    if (levels > 0 && !may_meet_subtree(E, X, Q, root)) continue;
+    keep(item[i], root);
+  }
+  return out;
+}
+
 }  // namespace
 
 extern "C" {
@@ -206,10 +287,51 @@ int emu_pair(const double* VA, int nva, const int32_t* TA, int nta, const double
   const int per = 64;
   for (int q = 0; q < nq; q += per)
     for (int r : roots) items.push_back(Item{0, q, std::min(per, nq - q), chunks_of_A ? 0 : r});
-  E.item_first = 0, E.item_count = (int)items.size();
-  const int nitems = (int)items.size();
   double X[12];
   orc_compose_SR(state, state + 12, X);
+  std::vector<double> cbox, csize, boxB(6);
+  std::vector<int32_t> heap;
+  if (g_items.mode) {
+    /* boxes of the chunks of queries and the mean half-extents of their
+     * elements (k_leaf_boxes, k_chunk_boxes), B's vertex box */
+    const int chunks = (nq + per - 1) / per;
+    const double inf = std::numeric_limits<double>::infinity();
+    for (int k = 0; k < chunks; ++k) {
+      double q[6] = {inf, inf, inf, -inf, -inf, -inf}, h[3] = {0, 0, 0};
+      const int cnt = std::min(per, nq - k * per);
+      for (int l = 0; l < cnt; ++l) {
+        double b[6] = {inf, inf, inf, -inf, -inf, -inf};
+        if (chunks_of_A) {
+          for (int c = 0; c < 6; ++c) b[c] = A.boxL[6 * (size_t)(k * per + l) + c];
+        } else {
+          const int nvq = kind == KIND_SOFT ? 4 : 3;
+          const int32_t* f = FB + nvq * (size_t)qorder[k * per + l];
+          for (int v = 0; v < nvq; ++v)
+            for (int c = 0; c < 3; ++c)
+              b[c] = std::fmin(b[c], VB[3 * f[v] + c]), b[3 + c] = std::fmax(b[3 + c], VB[3 * f[v] + c]);
+        }
+        for (int c = 0; c < 3; ++c)
+          q[c] = std::fmin(q[c], b[c]), q[3 + c] = std::fmax(q[3 + c], b[3 + c]), h[c] += 0.5 * (b[3 + c] - b[c]);
+      }
+      cbox.insert(cbox.end(), q, q + 6);
+      for (int c = 0; c < 3; ++c) csize.push_back(h[c] / cnt);
+    }
+    for (int c = 0; c < 3; ++c) boxB[c] = inf, boxB[3 + c] = -inf;
+    for (int v = 0; v < nvb; ++v)
+      for (int c = 0; c < 3; ++c)
+        boxB[c] = std::fmin(boxB[c], VB[3 * v + c]), boxB[3 + c] = std::fmax(boxB[3 + c], VB[3 * v + c]);
+    heap = frontiers(A);
+    for (int i = 0; i + 1 < nta; ++i) {
+      std::vector<int> l;
+      leaves_under(A, i, l);
+      A.nodes[i].leaves = (int)l.size();
+    }
+    E.cboxQ = cbox.data(), E.csizeQ = csize.data(), E.boxB = boxB.data(), E.rootsA = heap.data();
+    E.depth = g_items.depth;
+    items = live_items(E, X, chunks);
+  }
+  E.item_first = 0, E.item_count = (int)items.size();
+  const int nitems = (int)items.size();
   /* the cull decision of each item (k_item_boxes + k_cull) */
   std::vector<char> culled(nitems, 0);
   for (int i = 0; i < nitems; ++i) {
@@ -339,6 +461,60 @@ int emu_pair(const double* VA, int nva, const int32_t* TA, int nta, const double
 extern "C" {
 
 void emu_set_options(int generic) { g_generic = generic; }
+void emu_set_items(int mode, int depth, unsigned room) { g_items.mode = mode, g_items.depth = depth, g_items.room = room; }
+
+/* For a body's tree: frontiers, their subtrees and the cuts of every subtree
+ * that do not hold each of its leaves exactly once. */
+int emu_cover_errors(const double* V, int nv, const int32_t* T, int nt, const double* p) {
+  Soft A;
+  prepare(V, nv, T, nt, p, A);
+  const std::vector<int32_t> heap = frontiers(A);
+  EnvDesc E{};
+  E.nodesA = A.nodes.data(), E.ntA = nt, E.kind = KIND_TRI, E.rootsA = heap.data();
+  auto under = [&](int ch) {
+    std::vector<int> l;
+    leaves_under(A, ch, l);
+    return l;
+  };
+  int bad = 0;
+  const std::vector<int> all = under(0);
+  bad += (int)all.size() != nt;
+  for (int d = 0; d <= HCS_ROOT_DEPTH; ++d) {
+    std::vector<int> l;
+    for (int k = 0; k < 1 << d; ++k) leaves_under(A, heap[(1 << d) + k], l);
+    bad += l != all;
+    /* the second cull's subtrees of a place of the first */
+    E.depth = d;
+    const int n = levels_below(E, HCS_ROOT_DEPTH);
+    bad += d + n > HCS_ROOT_DEPTH;
+    for (int k = 0; k < 1 << d; ++k) {
+      std::vector<int> m;
+      for (int s = 0; s < 1 << n; ++s) leaves_under(A, heap[(((1 << d) + k) << n) + s], m);
+      bad += m != under(heap[(1 << d) + k]);
+    }
+  }
+  for (int z = 1; z < 16; ++z) {
+    if (heap[z] == HCS_WNONE) continue;
+    for (int n = 0; n < (nt == 1 ? 1 : 15); ++n) {
+      std::vector<int> m;
+      for (int s = 0; s < 1 << n; ++s) leaves_under(A, cut_root(E, heap[z], n, s), m);
+      bad += m != under(heap[z]);
+    }
+  }
+  return bad;
+}
+
+/* The pieces that items of these words are cut to, and their target: at most
+ * room in all. */
+int64_t emu_pieces(const unsigned* word, unsigned n, unsigned shares, unsigned room, unsigned* target) {
+  unsigned long long sum = 0;
+  for (unsigned i = 0; i < n; ++i) sum += word[i] & kEstMask;
+  const CutArgs c{&n, &sum, shares, room};
+  *target = cut_target(c);
+  int64_t all = 0;
+  for (unsigned i = 0; i < n; ++i) all += cut_slots(word[i], *target);
+  return all;
+}
 int64_t emu_clip_differences() { return g_clip_differences; }
 
 /* x / 3 and x / b as the clip of mixed-kind launches divides. */

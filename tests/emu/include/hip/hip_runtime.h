@@ -43,6 +43,9 @@ struct float4 {
 inline float4 make_float4(float a, float b, float c, float d) { return float4{a, b, c, d}; }
 inline int min(int a, int b) { return a < b ? a : b; }
 inline int max(int a, int b) { return a > b ? a : b; }
+inline unsigned min(unsigned a, unsigned b) { return a < b ? a : b; }
+inline unsigned long long min(unsigned long long a, unsigned long long b) { return a < b ? a : b; }
+inline unsigned long long max(unsigned long long a, unsigned long long b) { return a > b ? a : b; }
 
 struct Dim3 {
   unsigned x, y, z;
