@@ -224,7 +224,9 @@ int hcs_candidates(hcs_ctx* ctx, const hcs_pair_in* pair, int64_t* keys, int64_t
 /* ---- tactile sensors (FlatTactileSensor::bvh_update), on the polygons of
  * the last hcs_contact_step run with keep_polygons = 1.  out holds, per
  * sensor, cx * cy values at [x + cx * y] with cx = floor(2 xs / res + 0.1)
- * (S/src/flat_tactile_sensor.cpp:196-197). */
+ * (S/src/flat_tactile_sensor.cpp:196-197).  The polygons are listed per
+ * taxel they may cover; more than 2^32 - 1 entries of one sensor are refused
+ * (HCS_ERR_CAPACITY). */
 int hcs_taxel_dims(const hcs_taxel_grid* g, int32_t* cx, int32_t* cy);
 int hcs_taxels(hcs_ctx* ctx, int32_t nsensors, const hcs_taxel_grid* g, double* out);
 /* TaxelSensor::internal_update (S/src/taxel_sensor.cpp:158-478) on the
